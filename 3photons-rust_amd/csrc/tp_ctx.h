@@ -142,6 +142,7 @@ inline int grid_for(const Ctx *c, int source, int precision, uint64_t nb)
 // Device-side constants of a run, computed exactly as the reference does on
 // the host (coupling.rs, resacc.rs:59-100, evgen.rs:66-69, spinor.rs:37-44).
 tpd::Params make_params(const tp_params *p);
+tpd::Params make_event_params(const tp_params *p, int precision);
 tpd::FParams make_fparams(const tp_params *p);
 
 } // namespace tpe

@@ -61,7 +61,26 @@ tpd::Params make_params(const tp_params *p)
     P.kp_t = P.nt01re * P.g_bp;
     P.km_s = P.ns01re * P.g_bm;
     P.km_t = P.nt01re * P.g_bm;
+    P.unit = 1.;
     P.sort = p->sort_photons ? 1 : 0;
+    return P;
+}
+
+// The constants of the event loop: in f64 with energies in the unit that the
+// closed-form helicity sums ask for.  Scaling by a power of two keeps every
+// bit of the momenta and every cut decision.
+tpd::Params make_event_params(const tp_params *p, int precision)
+{
+    tpd::Params P = make_params(p);
+    if (precision != TP_PREC_F64)
+        return P;
+    const double up = tpd::energy_unit(p->e_total);
+    P.unit = 1. / up;
+    P.e_total *= up;
+    P.e_min *= up;
+    P.el_x *= up;
+    P.el_e *= up;
+    P.hk = tpd::helicity_constants(p->e_total, p->g_a, p->g_beta_p, p->g_beta_m, up);
     return P;
 }
 
@@ -1221,7 +1240,7 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     tpk::FusedArgs a;
     std::memset(&a, 0, sizeof a);
-    a.P = make_params(params);
+    a.P = make_event_params(params, params->precision);
     a.num_events = num_events;
     a.batch_size = batch_size;
     a.precision = params->precision;
@@ -1642,7 +1661,7 @@ extern "C" int tp_events(void *ctx, const tp_params *params, int rng_kind, const
         HIPCHK(c, hipSetDevice(c->device));
         tpk::FusedArgs a;
         std::memset(&a, 0, sizeof a);
-        a.P = make_params(params);
+        a.P = make_event_params(params, params->precision);
         a.precision = params->precision;
         rc = ensure_mt(c);
         if (rc)
@@ -1953,7 +1972,7 @@ extern "C" int tp_run_device_noalloc(void *ctx, const tp_params *params, int rng
             return fail(c, TP_ERR_INTERNAL, "tp_run_device_noalloc: grid differs from the set-up's");
         tpk::FusedArgs a;
         std::memset(&a, 0, sizeof a);
-        a.P = make_params(params);
+        a.P = make_event_params(params, params->precision);
         a.num_events = num_events;
         a.batch_size = TP_BATCH_SIZE;
         a.precision = params->precision;

@@ -579,7 +579,7 @@ extern "C" int tp_flow_run_device(void *flow, const tp_params *params, double al
             return rc;
         tpk::FusedArgs fa;
         std::memset(&fa, 0, sizeof fa);
-        fa.P = make_params(params);
+        fa.P = make_event_params(params, TP_PREC_F64);
         fa.num_events = num_events;
         fa.batch_size = bs;
         fa.precision = TP_PREC_F64;

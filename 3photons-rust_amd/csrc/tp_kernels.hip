@@ -400,7 +400,7 @@ __global__ __launch_bounds__(256) void events_kernel(FusedArgs a, uint32_t n, Ev
         for (int i = 0; i < 3; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                o.p[12ull * e + 4 * i + j] = p[i][j];
+                o.p[12ull * e + 4 * i + j] = p[i][j] * a.P.unit;
     if (o.keep)
         o.keep[e] = k ? 1 : 0;
     if (o.m)

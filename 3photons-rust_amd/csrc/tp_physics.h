@@ -6,9 +6,10 @@
 // L1-resident log and sin/cos tables of tp_math.h, whose routines return the
 // correctly rounded value but within ~0.002 ulp of a rounding boundary (the
 // reference calls the host libm; the two agree on > 99.8 % of arguments).  The
-// f64 path keeps the reference's operation order exactly (the translation
-// unit is compiled with -ffp-contract=off); it differs from the reference only
-// where the reference computes known zeros or exact negations:
+// f64 path keeps the reference's operation order through RAMBO, the sort and
+// the cuts (the translation unit is compiled with -ffp-contract=off) and takes
+// its helicity sums in closed form (tp_helicity.h); the all-f32 path keeps the
+// reference's order throughout, apart from known zeros and exact negations:
 //   * s(j,i) is taken as -s(i,j) (exactly equal but for the sign of a zero);
 //   * the helicity sums skip the zero amplitudes (adding +-0 to a non-zero sum
 //     is exact, so the sums are unchanged);
@@ -22,6 +23,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "tp_helicity.h"
 #include "tp_math.h"
 
 #include <type_traits>
@@ -39,9 +41,14 @@ struct Params {
     double xx1, f1re, f1im;       // positron spinor
     double ns01re, ns01im;        // -RAC8 * s(e-, e+)
     double nt01re, nt01im;        // -RAC8 * t(e-, e+)
-    // ns01re and nt01re times g_a, g_bp and g_bm (the f64 and mixed
-    // amplitudes' real scale factors; the imaginary parts are +-0)
+    // ns01re and nt01re times g_a, g_bp and g_bm (the mixed amplitudes' real
+    // scale factors; the imaginary parts are +-0)
     double ka_s, ka_t, kp_s, kp_t, km_s, km_t;
+    // f64 event path: energies above are in units of `unit` (a power of two
+    // that brings e_total into [64, 128)), hk gives the helicity sums in the
+    // caller's units
+    HelicityK hk;
+    double unit;
     int sort;
     int pad;
 };
@@ -260,15 +267,8 @@ template <class T> struct Spin {
     C<T> s[5][5]; // only off-diagonal entries are set
 };
 
-// a b - c d: with FAST one fma (the f64 event loop), otherwise the
-// reference's two products and a difference.
-template <bool FAST, class T> __device__ __forceinline__ T mul_sub(T a, T b, T c, T d)
-{
-    if constexpr (FAST)
-        return fma(a, b, -(c * d));
-    else
-        return a * b - c * d;
-}
+// a b + c d: with FAST one fma, otherwise the reference's two products and a
+// sum.
 template <bool FAST, class T> __device__ __forceinline__ T mul_add(T a, T b, T c, T d)
 {
     if constexpr (FAST)
@@ -277,7 +277,8 @@ template <bool FAST, class T> __device__ __forceinline__ T mul_add(T a, T b, T c
         return a * b + c * d;
 }
 
-template <class T, bool FAST = false>
+// The all-f32 parity path's spinor products: the reference's plain operations.
+template <class T>
 __device__ __forceinline__ void spinor_products(T xx0, T f0re, T f0im, T xx1, T f1re, T f1im, const T p[3][4],
                                                 Spin<T> &S)
 {
@@ -288,21 +289,15 @@ __device__ __forceinline__ void spinor_products(T xx0, T f0re, T f0im, T xx1, T 
         xx[k] = sq(p[k][3] + p[k][2]);
         // f32::MIN_POSITIVE / f64::MIN_POSITIVE
         const T minpos = sizeof(T) == 8 ? (T)2.2250738585072014e-308 : (T)1.17549435e-38f;
-        if (xx[k] > minpos) {
-            if constexpr (FAST) {
-                const T y = tpm::rcp_n(xx[k]);
-                fx[k] = mk<T>(p[k][0] * y, p[k][1] * y);
-            } else {
-                fx[k] = mk<T>(dv(p[k][0], xx[k]), dv(p[k][1], xx[k]));
-            }
-        }
+        if (xx[k] > minpos)
+            fx[k] = mk<T>(dv(p[k][0], xx[k]), dv(p[k][1], xx[k]));
         else
             fx[k] = mk<T>(sq((T)2. * p[k][3]), (T)0.);
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        C<T> s0k = mk<T>(mul_sub<FAST>(f0re, xx[k], fx[k].re, xx0), mul_sub<FAST>(f0im, xx[k], fx[k].im, xx0));
-        C<T> s1k = mk<T>(mul_sub<FAST>(f1re, xx[k], fx[k].re, xx1), mul_sub<FAST>(f1im, xx[k], fx[k].im, xx1));
+        C<T> s0k = mk<T>(f0re * xx[k] - fx[k].re * xx0, f0im * xx[k] - fx[k].im * xx0);
+        C<T> s1k = mk<T>(f1re * xx[k] - fx[k].re * xx1, f1im * xx[k] - fx[k].im * xx1);
         S.s[0][2 + k] = s0k;
         S.s[2 + k][0] = neg(s0k);
         S.s[1][2 + k] = s1k;
@@ -312,8 +307,7 @@ __device__ __forceinline__ void spinor_products(T xx0, T f0re, T f0im, T xx1, T 
     for (int k = 0; k < 3; ++k)
 #pragma unroll
         for (int l = k + 1; l < 3; ++l) {
-            C<T> skl = mk<T>(mul_sub<FAST>(fx[k].re, xx[l], fx[l].re, xx[k]),
-                             mul_sub<FAST>(fx[k].im, xx[l], fx[l].im, xx[k]));
+            C<T> skl = mk<T>(fx[k].re * xx[l] - fx[l].re * xx[k], fx[k].im * xx[l] - fx[l].im * xx[k]);
             S.s[2 + k][2 + l] = skl;
             S.s[2 + l][2 + k] = neg(skl);
         }
@@ -322,8 +316,7 @@ __device__ __forceinline__ void spinor_products(T xx0, T f0re, T f0im, T xx1, T 
 // Complex products of the amplitude algebra.  With FAST they contract
 // multiply-adds into fma and divide by multiplying with one reciprocal of
 // |b|^2 (in f64 the refined one, in f32 the hardware's), so the result moves
-// by an ulp or so (the f64 event loops, the mixed-precision path, the
-// adjoints).  Without FAST they are the reference's plain operations (the
+// by an ulp or so (the mixed-precision path, the adjoints).  Without FAST they are the reference's plain operations (the
 // all-f32 parity path).
 __device__ __forceinline__ C<double> cmul_fast(C<double> a, C<double> b)
 {
@@ -431,12 +424,10 @@ template <class T> struct ADen {
     C<T> d;
     T inv; // 1 / |d|^2
 };
-__device__ __forceinline__ double rcp_amp(double x) { return tpm::rcp_n(x); }
-__device__ __forceinline__ float rcp_amp(float x) { return __builtin_amdgcn_rcpf(x); }
-template <class T> __device__ __forceinline__ ADen<T> a_den(const Spin<T> &S, int a, int b)
+__device__ __forceinline__ ADen<float> a_den(const Spin<float> &S, int a, int b)
 {
-    const C<T> d = xmul<true>(xmul<true>(xmul<true>(S.s[0][a], S.s[0][b]), S.s[1][a]), S.s[1][b]);
-    return ADen<T>{d, rcp_amp(xnorm<true>(d))};
+    const C<float> d = xmul<true>(xmul<true>(xmul<true>(S.s[0][a], S.s[0][b]), S.s[1][a]), S.s[1][b]);
+    return ADen<float>{d, __builtin_amdgcn_rcpf(xnorm<true>(d))};
 }
 template <class T> __device__ __forceinline__ C<T> a_ppm_d(const Spin<T> &S, const AmpK<T> &K, const ADen<T> &D, int k3)
 {
@@ -447,7 +438,9 @@ template <class T> __device__ __forceinline__ C<T> a_pmm_d(const Spin<T> &S, con
     return rscale(xmul<true>(xsq<true>(tof(S.s[1][k1])), D.d), K.ka_t * D.inv);
 }
 
-// Helicity sums of the five matrix-element contributions (matelems.rs:53-86):
+// Helicity sums of the five matrix-element contributions (matelems.rs:53-86)
+// from the amplitudes (the f32 algebra of the mixed and all-f32 paths; the f64
+// paths use the closed form of tp_helicity.h):
 // m[0] = sum|A g_a|^2, m[1] = sum|B+ g_b+|^2, m[2] = sum|B- g_b-|^2,
 // m[3] + i m[4] = sum (2 A g_a) conj(B+ g_b+).  Helicities MMP..PPM carry A and
 // B+ (spinor.rs:72-98), MMM and PPP carry B- only (spinor.rs:100-113).  The
@@ -482,7 +475,7 @@ __device__ __forceinline__ void helicity_sums(const Spin<T> &S, const AmpK<T> &K
         }
     };
     if constexpr (FAST) {
-        const ADen<T> d23 = a_den(S, 2, 3), d24 = a_den(S, 2, 4), d34 = a_den(S, 3, 4);
+        const ADen<float> d23 = a_den(S, 2, 3), d24 = a_den(S, 2, 4), d34 = a_den(S, 3, 4);
         fold(0, a_pmm_d(S, K, d23, 4), bp_pmm<T, FAST>(S, K, 4, 2, 3));
         fold(1, a_pmm_d(S, K, d24, 3), bp_pmm<T, FAST>(S, K, 3, 2, 4));
         fold(2, a_ppm_d(S, K, d34, 2), bp_ppm<T, FAST>(S, K, 3, 4, 2));
@@ -767,11 +760,7 @@ template <class Walk> __device__ __forceinline__ bool generate_faster_f64(const 
 // Helicity sums m[5] of an event that passed the cuts.
 __device__ __forceinline__ void matrix_elements_f64(const Params &P, const double p[3][4], double m[5])
 {
-    Spin<double> S;
-    spinor_products<double, true>(P.xx0, P.f0re, P.f0im, P.xx1, P.f1re, P.f1im, p, S);
-    const AmpK<double> K{mk(P.ns01re, P.ns01im), mk(P.nt01re, P.nt01im), P.g_a, P.g_bp, P.g_bm,
-                         P.ka_s, P.ka_t, P.kp_s, P.kp_t, P.km_s, P.km_t};
-    helicity_sums<double, true>(S, K, m);
+    helicity_sums_closed(P.hk, p, m);
 }
 
 // Mixed precision keeps RAMBO (massless q, conformal map), the sort and the
