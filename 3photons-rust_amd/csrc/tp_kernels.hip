@@ -70,32 +70,42 @@ __device__ __forceinline__ void kahan(double &s, double &c, double x)
     s = t;
 }
 
+// In f64 the squares join their sums by fused multiply-adds, and the sum of
+// the weights, linear in m, is formed from the sums of m at the end
+// (acc_values); PREC 1 adds each of the twelve terms.
 template <int PREC> __device__ __forceinline__ void acc_add(Acc<PREC> &A, const Params &P, const double m[5])
 {
+    const double w = weight_f64<PREC == 0>(P, m);
+    A.n += 1;
+    if (PREC == 0) {
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            A.s[k] = A.s[k] + m[k];
+            A.s[5 + k] = fma(m[k], m[k], A.s[5 + k]);
+        }
+        A.s[11] = fma(w, w, A.s[11]);
+        return;
+    }
     double x[12];
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
         x[k] = m[k];
         x[5 + k] = m[k] * m[k];
     }
-    const double w = weight_f64(P, m);
     x[10] = w;
     x[11] = w * w;
-    A.n += 1;
 #pragma unroll
-    for (int j = 0; j < 12; ++j) {
-        if (PREC == 0)
-            A.s[j] = A.s[j] + x[j];
-        else
-            kahan(A.s[j], A.c[PREC ? j : 0], x[j]);
-    }
+    for (int j = 0; j < 12; ++j)
+        kahan(A.s[j], A.c[PREC ? j : 0], x[j]);
 }
 
-template <int PREC> __device__ __forceinline__ void acc_values(const Acc<PREC> &A, double v[12])
+template <int PREC> __device__ __forceinline__ void acc_values(const Acc<PREC> &A, const Params &P, double v[12])
 {
 #pragma unroll
     for (int j = 0; j < 12; ++j)
         v[j] = PREC ? A.s[j] - A.c[PREC ? j : 0] : A.s[j];
+    if (PREC == 0)
+        v[10] = weight_f64<true>(P, A.s);
 }
 
 // Fixed-shape wavefront butterfly then in-order wave combine; deterministic.
@@ -222,22 +232,21 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
         for (uint32_t k = 0; k < iters; ++k) {
             bool pass = false;
             double p[3][4];
-            int d[3]; // sort slots of the three photons
             const uint64_t qk = qnext;
             if (FE && k + 1 < len)
                 qnext = a.evq[wbase + (size_t)((k + 1) * 64 + lane)];
             if (k < len && SOURCE == 3) {
                 RanfWalk w{a.draws, a.qbase, qk, rb};
-                pass = generate_faster_f64(fresh_params(), w, p, d);
+                pass = generate_faster_f64(fresh_params(), w, p);
             } else if (k < len && SOURCE == 4) {
                 XoWalk w{a.xdraws, a.qbase, qk, rb};
-                pass = generate_faster_f64(fresh_params(), w, p, d);
+                pass = generate_faster_f64(fresh_params(), w, p);
             } else if (k < len) {
                 double u[12];
                 if (SOURCE == 0) {
 #pragma unroll
                     for (int j = 0; j < 12; ++j)
-                        u[j] = xo_uniform53(s);
+                        u[j] = xo_uniform64(s);
                 } else if (SOURCE == 1) {
                     const int32_t *e = src + 12 * (size_t)(k * 64 + lane);
 #pragma unroll
@@ -249,11 +258,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                     for (int j = 0; j < 12; ++j)
                         u[j] = a.u[j * a.u_stride + e];
                 }
-                pass = generate_f64<SOURCE == 0>(fresh_params(), u, p, d);
+                pass = generate_f64<SOURCE == 0>(fresh_params(), u, p);
             }
             const uint64_t mask = __ballot(pass);
             if (pass) {
                 const uint32_t slot = qn + (uint32_t)__popcll(mask & lanemask_lt);
+                int d[3] = {0, 1, 2}; // the f32 algebra of the mixed path takes the photons sorted
+                if (PREC == 1)
+                    sort_slots(p, fresh_params().sort, d);
 #pragma unroll
                 for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -304,7 +316,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
         }
         __syncthreads();
         double v[12];
-        acc_values(A, v);
+        acc_values(A, fresh_params(), v);
         block_reduce_store<1>(v, A.n, out + lb, red);
     }
 }
@@ -370,7 +382,7 @@ __global__ __launch_bounds__(256) void events_kernel(FusedArgs a, uint32_t n, Ev
                 gf2_apply(a.mt + 1024 * k, s);
 #pragma unroll
         for (int j = 0; j < 12; ++j)
-            u[j] = xo_uniform53(s); // u 2^53, as the fused kernel draws them
+            u[j] = xo_uniform64(s); // u 2^64, as the fused kernel draws them
     } else {
 #pragma unroll
         for (int j = 0; j < 12; ++j)
@@ -378,12 +390,13 @@ __global__ __launch_bounds__(256) void events_kernel(FusedArgs a, uint32_t n, Ev
     }
     double pu[3][4], p[3][4], m[5] = {0., 0., 0., 0., 0.};
     int d[3];
-    const bool k = generate_f64<SOURCE == 0>(a.P, u, pu, d);
+    const bool k = generate_f64<SOURCE == 0>(a.P, u, pu);
+    sort_slots(pu, a.P.sort, d);
     to_slots(pu, d, p);
     if (SOURCE == 0)
 #pragma unroll
         for (int j = 0; j < 12; ++j)
-            u[j] = u[j] * 0x1.0p-53;
+            u[j] = u[j] * 0x1.0p-64;
     if (k)
         matrix_elements<PREC>(a.P, p, m);
     if (!k) {

@@ -109,10 +109,26 @@ TPM_FN double sqrt_n(double x)
     g = __builtin_fma(d, h, g);
     return x == 0. ? x : g;
 }
+// sqrt_n for x that is 0 or positive: the seed of an exact 0 comes from
+// 2^-1000 instead, and every later product with x keeps it 0.
+TPM_FN double sqrt_nonneg(double x)
+{
+    const double y = __builtin_amdgcn_rsq(fmax(x, 0x1.0p-1000));
+    double g = x * y;
+    double h = y * 0.5;
+    const double r = __builtin_fma(-h, g, 0.5);
+    g = __builtin_fma(g, r, g);
+    h = __builtin_fma(h, r, h);
+    double d = __builtin_fma(-g, g, x);
+    g = __builtin_fma(d, h, g);
+    d = __builtin_fma(-g, g, x);
+    return __builtin_fma(d, h, g);
+}
 #else
 TPM_FN double div_n(double a, double b) { return a / b; }
 TPM_FN double rcp_n(double b) { return 1. / b; }
 TPM_FN double sqrt_n(double x) { return std::sqrt(x); }
+TPM_FN double sqrt_nonneg(double x) { return std::sqrt(x); }
 #endif
 
 // Natural logarithm of a positive normal double.

@@ -95,15 +95,14 @@ template <class T> __device__ __forceinline__ C<T> tof(C<T> s) { return C<T>{-s.
 // ---- RAMBO: evgen.rs:174-207 (generate_raw) and 89-118 (generate) ---------
 
 // Massless momentum of one photon from (cos theta, phi, e1, e2) uniforms.
-// SCALED: the uniforms come as u 2^53, the integers xoshiro256+'s x >> 11
-// holds (xo_uniform53), and the 2^-53 factors fold into the operations
-// exactly: 2u - 1 = fma(u', 2^-52, -1) (2u is exact, so the reference's two
-// roundings are one), 2 pi u = (2 pi 2^-53) u' and u1 u2 = (u1' u2') 2^-106,
-// each rounded once as before.
+// SCALED: the uniforms come as u 2^64 (xo_uniform64), and the 2^-64 factors
+// fold into the operations exactly: 2u - 1 = fma(u', 2^-63, -1) (2u is exact,
+// so the reference's two roundings are one), 2 pi u = (2 pi 2^-64) u' and
+// u1 u2 = (u1' u2') 2^-128, each rounded once as before.
 template <bool SCALED>
 __device__ __forceinline__ void raw_photon_f64(double uc, double uphi, double ue1, double ue2, double q[4])
 {
-    constexpr double S = SCALED ? 0x1.0p-53 : 1.;
+    constexpr double S = SCALED ? 0x1.0p-64 : 1.;
     const double two_pi = 2. * 3.14159265358979323846;
     double cos_t = __builtin_fma(uc, 2. * S, -1.);
     double phi = (two_pi * S) * uphi;
@@ -112,7 +111,7 @@ __device__ __forceinline__ void raw_photon_f64(double uc, double uphi, double ue
         em = em * (S * S);
     double sphi, cphi;
     tpm::sincos_f64(phi, sphi, cphi);
-    double st = sq(1. - cos_t * cos_t);
+    double st = tpm::sqrt_nonneg(1. - cos_t * cos_t); // |cos_t| <= 1
     double en = -tpm::log_pos(em + 2.2250738585072014e-308);
     q[0] = en * (st * sphi);
     q[1] = en * (st * cphi);
@@ -172,8 +171,9 @@ template <class T> __device__ __forceinline__ void sort3(T p[3][4])
 // comparisons of the unsorted energies.  It reproduces the swap sequence
 // exactly, ties and NaN included: step 2 compares photon 2 with the winner a
 // of step 1, step 3 compares the loser b with whatever step 2 left in slot 2.
-// The kernels keep the photons where RAMBO made them and apply the slots where
-// they store the event (no register shuffles).
+// The kernels keep the photons where RAMBO made them.  The closed-form sums of
+// the f64 path do not depend on the photons' order; the mixed path applies the
+// slots where it stores the event (no register shuffles).
 __host__ __device__ __forceinline__ void sort_slots(const double p[3][4], int sort, int d[3])
 {
     if (!sort) {
@@ -206,43 +206,34 @@ template <class T> __device__ __forceinline__ void to_slots(const T p[3][4], con
 }
 
 // ---- Cuts: evcut.rs:42-96 -------------------------------------------------
-// On the unsorted photons with their slots d: every test but the energy and
-// plane cuts treats the photons symmetrically (each dot product is the same
-// IEEE expression for (i,j) and (j,i)), the energy cut takes the slot-2
-// energy as the reference does after sorting, and the plane cut's normal
-// n = p_slot0 x p_slot1 only changes sign (exactly) when its two photons are
-// taken in the other order, which |num| and |n| do not see.  All tests are
-// evaluated (no early exit), which changes nothing: they have no side effects.
-__device__ __forceinline__ bool keep_f64(const Params &P, const double p[3][4], const int d[3])
+// On the unsorted photons.  Every test but the plane cut treats the photons
+// symmetrically: the energy cut takes the smallest energy, which is what the
+// reference's sort leaves in slot 2.  The beams run along x with
+// |el_x| = el_e, so |p_x el_x| > cut (E el_e) is tested as |p_x| > cut E, and
+// the dot products of the pair cut are fused: both move a boundary by an ulp
+// or so of the compared values, far below the spacing of the events (of 1e9
+// events about 1e-6 lie that close to a cut).  The plane cut's normal is the
+// cross product of the two photons outside slot 2 (its sign, which their
+// order changes, does not count).  All tests are evaluated (no early exit),
+// which changes nothing: they have no side effects.
+__device__ __forceinline__ bool keep_f64(const Params &P, const double p[3][4])
 {
-    // (selects between loaded values, never between array elements: the
-    // latter can turn into an address select that moves p to scratch)
-    const double E0 = p[0][3], E1 = p[1][3], E2 = p[2][3];
-    double emin;
-    if (P.sort) {
-        emin = d[0] == 2 ? E0 : (d[1] == 2 ? E1 : E2);
-    } else {
-        emin = E0;
-        emin = (emin < E1) ? emin : E1;
-        emin = (emin < E2) ? emin : E2;
-    }
-    bool ok = !(emin < P.e_min);
+    bool ok = !(fmin(fmin(p[0][3], p[1][3]), p[2][3]) < P.e_min);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        double num = p[i][0] * P.el_x;
-        double den = p[i][3] * P.el_e;
-        ok = ok & !(fabs(num) > P.cut_beam * den);
-    }
+    for (int i = 0; i < 3; ++i)
+        ok = ok & !(fabs(p[i][0]) > P.cut_beam * p[i][3]);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = i + 1; j < 3; ++j) {
-            double num = (p[i][0] * p[j][0] + p[i][1] * p[j][1]) + p[i][2] * p[j][2];
-            double den = p[i][3] * p[j][3];
-            ok = ok & !(num > P.cut_pp * den);
+            const double num = fma(p[i][2], p[j][2], fma(p[i][1], p[j][1], p[i][0] * p[j][0]));
+            ok = ok & !(num > P.cut_pp * (p[i][3] * p[j][3]));
         }
     if (P.cut_plane > 0.) {
-        // the two photons outside slot 2
+        // (selects between loaded values, never between array elements: the
+        // latter can turn into an address select that moves p to scratch)
+        int d[3];
+        sort_slots(p, P.sort, d);
         double a[3], b[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -551,10 +542,17 @@ __device__ __forceinline__ void spinor_products_f32(const Params &P, const float
         }
 }
 
-// Per-event weight: dot(m, sigma_contribs) as a left fold (resacc.rs:126).
-__device__ __forceinline__ double weight_f64(const Params &P, const double m[5])
+// Per-event weight: dot(m, sigma_contribs) as a left fold (resacc.rs:126),
+// with FUSED multiply-adds in the f64 path.
+template <bool FUSED> __device__ __forceinline__ double weight_f64(const Params &P, const double m[5])
 {
     double w = m[0] * P.sc[0];
+    if (FUSED) {
+#pragma unroll
+        for (int c = 1; c < 5; ++c)
+            w = fma(m[c], P.sc[c], w);
+        return w;
+    }
     w = w + m[1] * P.sc[1];
     w = w + m[2] * P.sc[2];
     w = w + m[3] * P.sc[3];
@@ -562,19 +560,17 @@ __device__ __forceinline__ double weight_f64(const Params &P, const double m[5])
     return w;
 }
 
-// RAMBO event from 12 uniforms (photons sorted) and its cut decision.
-// RAMBO event from 12 uniforms: photons as RAMBO makes them (unsorted), their
-// sort slots d, and the cut decision.
+// RAMBO event from 12 uniforms: photons as RAMBO makes them (unsorted) and
+// the cut decision.
 template <bool SCALED = false>
-__device__ __forceinline__ bool generate_f64(const Params &P, const double u[12], double p[3][4], int d[3])
+__device__ __forceinline__ bool generate_f64(const Params &P, const double u[12], double p[3][4])
 {
     double q[3][4];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
         raw_photon_f64<SCALED>(u[4 * i], u[4 * i + 1], u[4 * i + 2], u[4 * i + 3], q[i]);
     conformal_f64(P, q, p);
-    sort_slots(p, P.sort, d);
-    return keep_f64(P, p, d);
+    return keep_f64(P, p);
 }
 
 // ---- faster-evgen re-rolls from accept bits -------------------------------------
@@ -739,7 +735,7 @@ template <class Walk> __device__ __forceinline__ void raw_photons_faster_f64(Wal
         const double cx = x[i] * nrm, cy = y[i] * nrm;
         const double cos_t = 2. * r9[i] - 1.;
         const double em = r9[3 + i] * r9[6 + i];
-        const double st = sq(1. - cos_t * cos_t);
+        const double st = tpm::sqrt_nonneg(1. - cos_t * cos_t); // |cos_t| <= 1
         const double en = -tpm::log_pos(em + 2.2250738585072014e-308);
         q[i][0] = en * (st * cx);
         q[i][1] = en * (st * cy);
@@ -748,13 +744,12 @@ template <class Walk> __device__ __forceinline__ void raw_photons_faster_f64(Wal
     }
 }
 
-template <class Walk> __device__ __forceinline__ bool generate_faster_f64(const Params &P, Walk &w, double p[3][4], int d[3])
+template <class Walk> __device__ __forceinline__ bool generate_faster_f64(const Params &P, Walk &w, double p[3][4])
 {
     double q[3][4];
     raw_photons_faster_f64(w, q);
     conformal_f64(P, q, p);
-    sort_slots(p, P.sort, d);
-    return keep_f64(P, p, d);
+    return keep_f64(P, p);
 }
 
 // Helicity sums m[5] of an event that passed the cuts.

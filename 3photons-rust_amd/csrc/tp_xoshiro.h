@@ -47,10 +47,10 @@ __device__ __forceinline__ double xo_uniform(uint64_t s[4])
     return fma((double)hi, 0x1.0p-32, (double)(lo >> 11) * 0x1.0p-53);
 }
 
-// The same uniform times 2^53, i.e. the integer u64 >> 11 as an exact double
-// (hi * 2^21 + (lo >> 11) < 2^53), for code that folds the 2^-53 into its
-// own operations.
-__device__ __forceinline__ double xo_uniform53(uint64_t s[4])
+// The same uniform times 2^64, i.e. (u64 >> 11) 2^11 as an exact double, for
+// code that folds the 2^-64 into its own operations (masking the low bits is
+// a cheaper instruction than shifting them out).
+__device__ __forceinline__ double xo_uniform64(uint64_t s[4])
 {
     const uint64_t x = xo_next(s);
     uint32_t hi = (uint32_t)(x >> 32);
@@ -58,7 +58,7 @@ __device__ __forceinline__ double xo_uniform53(uint64_t s[4])
     // (an empty asm on hi: without it the compiler matches the two 32-bit
     // conversions as a 64-bit one and adds a +0.0 term)
     asm("" : "+v"(hi));
-    return fma((double)hi, 0x1.0p21, (double)(lo >> 11));
+    return fma((double)hi, 0x1.0p32, (double)(lo & 0xFFFFF800u));
 }
 
 // s <- M s.  Read through the constant address space so that the uniform
