@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "tp.h"
+#include "tp_kernels.h"
 #include "tp_physics.h"
 #include "tp_rng_host.h"
 
@@ -38,13 +39,24 @@ template <int N> struct ScopedBufs {
     }
 };
 
-struct Tables { // device copies of GF(2) jump tables for one (seeding, batch size, grid)
-    DevBuf bt, stride;
+struct Tables { // device copy of the powers 2^k of a GF(2) matrix
+    DevBuf bt;
     int kb = 0;
+};
+
+// xoshiro256+ skip tables of one device, filled once by the first tp_create on
+// it and only read afterwards (tp_kernels.h).
+struct XoTables {
+    int rc = TP_ERR_INTERNAL;
+    std::string err;
+    const uint64_t *m16 = nullptr;     // M^(v 16^j), M one draw
+    const uint64_t *b16[2] = {nullptr, nullptr}; // B^(v 16^j): M^(12 * 10 000), the 2^128 jump (by seeding)
+    const uint64_t *lanes = nullptr;   // lane tables of every run length
 };
 
 struct Ctx {
     int device = 0;
+    const XoTables *xo = nullptr;
     int cus = 1;                    // compute units of the device
     int blocks_per_cu[5][2] = {{1, 1}, {1, 1}, {1, 1}, {1, 1}, {1, 1}}; // resident fused workgroups per CU [source][precision]
     hipStream_t stream = nullptr;
@@ -55,6 +67,7 @@ struct Ctx {
     std::map<std::string, std::unique_ptr<Tables>> tables;
     std::map<std::string, std::vector<uint32_t>> ranf_polys; // host copies keyed by R
     DevBuf polys, draws, origin, p0, per_batch, merged, evq;
+    DevBuf parts; // sums of the parts of split batches (MAX_PARTS), allocated by tp_create
     DevBuf mt128, bt128, f32ev; // all-f32 mode: xoshiro128+ tables, per-event values
     std::string bt128_key;
     int bt128_kb = 0;
@@ -131,12 +144,63 @@ inline int ensure(Ctx *c, DevBuf &b, size_t bytes)
     return TP_OK;
 }
 
-// Persistent grid: as many batch workgroups as can be resident at once (CUs x
-// occupancy), each striding over batches; never more than there are batches.
-inline int grid_for(const Ctx *c, int source, int precision, uint64_t nb)
+// How a launch of nb batches of n events (each a wavefront's work, or split
+// over several) is laid out.
+struct Split {
+    uint32_t parts, run; // wavefronts per batch, events per lane of each
+    int grid;
+};
+constexpr uint64_t MAX_PARTS = 1u << 16;
+// The run length with the least estimated time.  A wavefront takes `run`
+// iterations and a start-up of about 2 (the xoshiro stream's skip; half an
+// iteration for streams read from memory).  `slots` wavefronts are resident at
+// once and share 4 SIMDs per CU: a SIMD with one wavefront spends 1.4 times
+// the issue time of an iteration (measured: 4900 cycles against 3400), one
+// with several their sum.  So 1000 batches take 2 parts each rather than leave
+// two wavefronts of three idle, 10 000 take 4 rather than fill a fourth round
+// of 3072 to a quarter, and one closure call takes a part per 64 events.
+inline Split split_for(const Ctx *c, int source, int precision, uint64_t nb, uint32_t n)
 {
-    const uint64_t g = static_cast<uint64_t>(c->cus) * static_cast<uint64_t>(c->blocks_per_cu[source][precision]);
-    return static_cast<int>(std::max<uint64_t>(1, std::min<uint64_t>(nb, g)));
+    const uint64_t simds = 4ull * c->cus, slots = (uint64_t)c->cus * c->blocks_per_cu[source][precision];
+    Split best{0, 0, 0};
+    double least = 0.;
+    for (uint32_t run : tpk::XO_RUNS) {
+        const uint64_t parts = (n + 64ull * run - 1) / (64ull * run), tasks = nb * parts;
+        if (parts > 1 && (parts > slots || tasks > MAX_PARTS))
+            continue;
+        const uint64_t iters = source == 0 ? std::min(run, n) : std::min<uint64_t>(run, (n + 63) / 64);
+        const uint64_t rest = tasks % slots;
+        const double turns = (double)(tasks / slots) * ((double)slots / (double)simds) +
+                             (rest ? std::max(1.4, (double)((rest + simds - 1) / simds)) : 0.);
+        const double cost = ((double)iters + (source == 0 ? 2. : 0.5)) * turns;
+        if (!best.parts || cost < least) {
+            least = cost;
+            // a wavefront that takes several parts keeps its place in the batch
+            best = Split{(uint32_t)parts, run, (int)std::min(tasks, slots / parts * parts)};
+        }
+    }
+    if (!best.parts) // batches of more than 64 * 157 events, in more parts than are resident
+        best = Split{1, (n + 63) / 64, (int)std::min(nb, slots)};
+    return best;
+}
+
+// The event loop on a.nb batches of n events, split as split_for says, with
+// the batches' sums in a.out.
+inline void launch_event_loop(const Ctx *c, tpk::FusedArgs &a, int source, uint32_t n)
+{
+    const Split s = split_for(c, source, a.precision, a.nb, n);
+    a.parts = s.parts;
+    a.run = s.run;
+    a.part_out = c->parts.p;
+    if (source == 0) {
+        a.lanes = nullptr;
+        for (int i = 0; i < tpk::XO_NRUNS; ++i)
+            if (tpk::XO_RUNS[i] == s.run)
+                a.lanes = c->xo->lanes + (size_t)i * tpk::XO_LANE_WORDS;
+    }
+    tpk::launch_fused(a, source, s.grid, c->stream);
+    if (s.parts > 1)
+        tpk::launch_batch_sums(a, c->stream);
 }
 
 // Device-side constants of a run, computed exactly as the reference does on

@@ -300,34 +300,21 @@ int bits_for(uint64_t n)
     return k;
 }
 
-// Batch-advance matrix B (skip-ahead: M^(12*batch_size); jump: the 2^128
-// jump) as pow2 table up to nb, plus B^grid.
-int ensure_tables(Ctx *c, int seeding, uint32_t batch_size, uint64_t nb, int grid, Tables **out)
+// The 2^128 jump as a table of its powers 2^k up to nb (faster-evgen with jump
+// seeding).
+int ensure_jump_table(Ctx *c, uint64_t nb, Tables **out)
 {
-    int kb = std::max(1, bits_for(nb));
-    std::string key = std::to_string(seeding) + ":" + std::to_string(batch_size) + ":" + std::to_string(grid);
+    const int kb = std::max(1, bits_for(nb));
+    const std::string key = "jump";
     auto it = c->tables.find(key);
     if (it != c->tables.end() && it->second->kb >= kb) {
         *out = it->second.get();
         return TP_OK;
     }
     tp::Gf2Mat B;
-    if (seeding == TP_SEED_JUMP)
-        tp::gf2_jump128(B);
-    else
-        tp::gf2_pow_from_table(tp::xoshiro_step_pow2(), 12ull * batch_size, B);
-    std::vector<tp::Gf2Mat> bt = tp::gf2_pow2_table(B, kb);
-    tp::Gf2Mat S;
-    tp::gf2_pow_from_table(bt, static_cast<uint64_t>(grid), S);
-    if (bits_for(static_cast<uint64_t>(grid)) > kb) {
-        std::vector<tp::Gf2Mat> bt2 = tp::gf2_pow2_table(B, bits_for(static_cast<uint64_t>(grid)));
-        tp::gf2_pow_from_table(bt2, static_cast<uint64_t>(grid), S);
-    }
+    tp::gf2_jump128(B);
     std::unique_ptr<Tables> t(new Tables);
-    int rc = upload_mats(c, t->bt, bt);
-    if (rc)
-        return rc;
-    rc = upload_mats(c, t->stride, std::vector<tp::Gf2Mat>(1, S));
+    int rc = upload_mats(c, t->bt, tp::gf2_pow2_table(B, kb));
     if (rc)
         return rc;
     t->kb = kb;
@@ -774,7 +761,7 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
             a.bstride = 0;
             a.evq = static_cast<const uint64_t *>(c->evq.p);
             a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-            tpk::launch_fused(a, source, grid_for(c, source, 0, a.nb), c->stream);
+            launch_event_loop(c, a, source, (uint32_t)std::min<uint64_t>(num_events, batch_size));
             HIPCHK(c, hipGetLastError());
         }
         if (!ok) // fe_starts is staged for the copy above
@@ -1025,7 +1012,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         a.bstride = PS;
         a.evq = static_cast<const uint64_t *>(c->evq.p);
         a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-        tpk::launch_fused(a, 3, grid_for(c, 3, 0, cnb), c->stream);
+        launch_event_loop(c, a, 3, (uint32_t)std::min<uint64_t>(num_events, batch_size));
         HIPCHK(c, hipGetLastError());
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
@@ -1053,7 +1040,7 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     Tables *t = nullptr;
-    int rc = ensure_tables(c, TP_SEED_JUMP, batch_size, nb, grid_for(c, 4, 0, chunk), &t);
+    int rc = ensure_jump_table(c, nb, &t);
     if (!rc)
         rc = ensure_lane_tables(c);
     if (!rc)
@@ -1122,7 +1109,7 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
             HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
             first = false;
         }
-        tpk::launch_fused(a, 4, grid_for(c, 4, 0, cnb), c->stream);
+        launch_event_loop(c, a, 4, (uint32_t)std::min<uint64_t>(num_events, batch_size));
         HIPCHK(c, hipGetLastError());
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
@@ -1233,6 +1220,21 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
     return TP_OK;
 }
 
+// The stream tables and batch range of a xoshiro256+ run of nb batches.  (The
+// powers of B are those of batches of 10 000 events; a closure call of another
+// size is one batch and uses none.)
+int xo_event_args(Ctx *c, tpk::FusedArgs &a, int seeding, uint64_t nb)
+{
+    if (!c->xo || c->xo->rc != TP_OK)
+        return fail(c, c->xo ? c->xo->rc : TP_ERR_UNSUPPORTED,
+                    "xoshiro256+ table set-up failed: " + (c->xo ? c->xo->err : std::string("device ordinal above 63")));
+    a.m16 = c->xo->m16;
+    a.b16 = c->xo->b16[seeding];
+    a.nb = nb;
+    a.b_first = 0;
+    return TP_OK;
+}
+
 // Enqueue a whole run (or one closure-sized batch when batch_size == n).
 int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, const void *state0,
                 uint64_t num_events, uint32_t batch_size, void *per_batch_dev)
@@ -1278,19 +1280,12 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     if (rng_kind == TP_RNG_XOSHIRO) {
         const tp_xoshiro_state *x = static_cast<const tp_xoshiro_state *>(state0);
         std::memcpy(a.s0, x->s, sizeof a.s0);
-        const int grid = grid_for(c, 0, a.precision, nb);
-        Tables *t = nullptr;
-        rc = ensure_tables(c, seeding, batch_size, nb, grid, &t);
+        rc = xo_event_args(c, a, seeding, nb);
         if (rc)
             return rc;
-        a.bt = static_cast<const uint64_t *>(t->bt.p);
-        a.stride = static_cast<const uint64_t *>(t->stride.p);
-        a.kb = t->kb;
-        a.nb = nb;
-        a.b_first = 0;
         a.out = per_batch_dev;
         HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-        tpk::launch_fused(a, 0, grid, c->stream);
+        launch_event_loop(c, a, 0, (uint32_t)std::min<uint64_t>(num_events, batch_size));
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         return TP_OK;
@@ -1395,7 +1390,7 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
             HIPCHK(c, hipGetLastError());
             tpk::launch_f32_accumulate(fa, f32_grid(c, cnb), c->stream);
         } else {
-            tpk::launch_fused(a, 1, grid_for(c, 1, a.precision, cnb), c->stream);
+            launch_event_loop(c, a, 1, (uint32_t)std::min<uint64_t>(num_events, batch_size));
         }
         HIPCHK(c, hipGetLastError());
     }
@@ -1413,69 +1408,79 @@ float elapsed(hipEvent_t a, hipEvent_t b)
 
 } // namespace
 
-// ---- tables of the no-allocation entry point ---------------------------------
-// tp_run_device_noalloc runs the xoshiro256+ event loop without allocating
-// device memory: the GF(2) tables its kernels read live in `scratch`, a
-// file-scope device array, filled once per device at set-up (tp_create) and
-// only read after that, so calls on one device that overlap do not race on
-// it.  Each device holds its own copy at its own address, which set-up takes
-// with hipGetSymbolAddress while that device is current; host code uses that
-// address, never the array's name.
-//   matrices [0, KM)                M^(2^k), the in-batch draw offsets
-//   [KM, KM + NS_KB)                B^(2^k), B = M^(12 * 10 000) (skip-ahead)
-//   [KM + NS_KB, KM + 2 NS_KB)      B^(2^k), B = the 2^128 jump (jump seeding)
-//   KM + 2 NS_KB + 2 seeding + p    B^grid of the full persistent grid, p = 0 f64, 1 mixed
-constexpr int NS_KB = 32;                            // runs of fewer than 2^32 batches
-constexpr int NS_BT = KM, NS_STRIDE = KM + 2 * NS_KB, NS_MATS = KM + 2 * NS_KB + 4;
-constexpr size_t NS_WORDS = (size_t)NS_MATS * 1024; // 100 matrices of 8 KiB: 800 KiB
-static_assert(sizeof(tp::Gf2Mat) == 1024 * sizeof(uint64_t), "matrix layout");
+// ---- xoshiro256+ skip tables ---------------------------------------------------
+// The GF(2) tables the xoshiro256+ event loop reads live in `scratch`, a
+// file-scope device array, so that tp_run_device_noalloc needs no allocation.
+// It is filled once per device at set-up (tp_create) and only read after that,
+// so calls on one device that overlap do not race on it.  Each device holds
+// its own copy at its own address, which set-up takes with hipGetSymbolAddress
+// while that device is current; host code uses that address, never the
+// array's name.
+constexpr size_t NS_M = 0;                                             // M^(v 16^j)
+constexpr size_t NS_B = NS_M + 15 * tpk::XO_M_DIGITS * tpk::XO_MAT_WORDS; // B^(v 16^j), skip-ahead then jump
+constexpr size_t NS_LANES = NS_B + 2 * 15 * tpk::XO_B_DIGITS * tpk::XO_MAT_WORDS;
+constexpr size_t NS_WORDS = NS_LANES + tpk::XO_NRUNS * tpk::XO_LANE_WORDS; // 24 MiB
+static_assert(sizeof(tp::Gf2Mat) == tpk::XO_MAT_WORDS * sizeof(uint64_t), "matrix layout");
 static __device__ __align__(256) uint64_t scratch[NS_WORDS];
 
 namespace {
 constexpr int NS_MAX_DEVICES = 64;
-struct NoallocSetup {
+struct XoSetup {
     std::once_flag once;
-    int rc = TP_ERR_INTERNAL;
-    std::string err;
-    uint64_t *ptr = nullptr; // this device's address of `scratch`
-    int full_grid[2] = {0, 0};
+    XoTables t;
 };
-NoallocSetup g_noalloc[NS_MAX_DEVICES];
+XoSetup g_xo[NS_MAX_DEVICES];
 
-// Once per device, with the device current: the array's address and its tables.
-void noalloc_setup(NoallocSetup &S, int cus, const int blocks[2])
+// Once per device, with the device current: the array's address and its
+// tables, from the powers of two of the three matrices.
+void xo_setup(XoTables &T, hipStream_t st)
 {
-    void *ptr = nullptr;
-    hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || !ptr) {
-        S.err = std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e);
-        S.rc = TP_ERR_HIP;
-        return;
-    }
-    std::vector<tp::Gf2Mat> mats(NS_MATS);
-    const std::vector<tp::Gf2Mat> &mt = tp::xoshiro_step_pow2();
-    for (int k = 0; k < KM; ++k)
-        mats[k] = mt[k];
-    tp::Gf2Mat B[2];
-    tp::gf2_pow_from_table(mt, 12ull * TP_BATCH_SIZE, B[0]);
-    tp::gf2_jump128(B[1]);
-    for (int sd = 0; sd < 2; ++sd) {
-        const std::vector<tp::Gf2Mat> bt = tp::gf2_pow2_table(B[sd], NS_KB);
-        for (int k = 0; k < NS_KB; ++k)
-            mats[NS_BT + sd * NS_KB + k] = bt[k];
-        for (int p = 0; p < 2; ++p) {
-            S.full_grid[p] = std::max(1, cus * blocks[p]);
-            tp::gf2_pow_from_table(bt, (uint64_t)S.full_grid[p], mats[NS_STRIDE + 2 * sd + p]);
+    void *ptr = nullptr, *pow2 = nullptr;
+    auto check = [&](hipError_t e, const char *what) {
+        if (e != hipSuccess && T.err.empty()) {
+            T.err = std::string(what) + ": " + hipGetErrorString(e);
+            T.rc = TP_ERR_HIP;
         }
-    }
-    e = hipMemcpy(ptr, mats.data(), NS_WORDS * sizeof(uint64_t), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-        S.err = std::string("scratch upload: ") + hipGetErrorString(e);
-        S.rc = TP_ERR_HIP;
+        return e == hipSuccess;
+    };
+    if (!check(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)"))
         return;
+    const std::vector<tp::Gf2Mat> &mt = tp::xoshiro_step_pow2();
+    const int digits[3] = {tpk::XO_M_DIGITS, tpk::XO_B_DIGITS, tpk::XO_B_DIGITS};
+    std::vector<tp::Gf2Mat> mats(mt.begin(), mt.begin() + 4 * digits[0]);
+    for (int sd = 0; sd < 2; ++sd) {
+        tp::Gf2Mat B;
+        if (sd == TP_SEED_JUMP)
+            tp::gf2_jump128(B);
+        else
+            tp::gf2_pow_from_table(mt, 12ull * TP_BATCH_SIZE, B);
+        const std::vector<tp::Gf2Mat> bt = tp::gf2_pow2_table(B, 4 * digits[1 + sd]);
+        mats.insert(mats.end(), bt.begin(), bt.end());
     }
-    S.ptr = static_cast<uint64_t *>(ptr);
-    S.rc = TP_OK;
+    uint64_t *t = static_cast<uint64_t *>(ptr);
+    const size_t bytes = mats.size() * sizeof(tp::Gf2Mat);
+    bool ok = check(hipMalloc(&pow2, bytes), "hipMalloc of the powers") &&
+              check(hipMemcpy(pow2, mats.data(), bytes, hipMemcpyHostToDevice), "upload of the powers");
+    if (ok) {
+        const uint64_t *p = static_cast<const uint64_t *>(pow2);
+        uint64_t *o = t + NS_M;
+        for (int d : digits) {
+            tpk::launch_xo_digit_table(p, d, o, st);
+            p += 4 * d * tpk::XO_MAT_WORDS;
+            o += 15 * d * tpk::XO_MAT_WORDS;
+        }
+        tpk::launch_xo_lane_tables(t + NS_M, t + NS_LANES, st);
+        ok = check(hipGetLastError(), "table kernels") && check(hipStreamSynchronize(st), "table kernels");
+    }
+    if (pow2)
+        (void)hipFree(pow2);
+    if (!ok)
+        return;
+    T.m16 = t + NS_M;
+    T.b16[TP_SEED_SKIPAHEAD] = t + NS_B;
+    T.b16[TP_SEED_JUMP] = t + NS_B + 15 * tpk::XO_B_DIGITS * tpk::XO_MAT_WORDS;
+    T.lanes = t + NS_LANES;
+    T.rc = TP_OK;
 }
 } // namespace
 
@@ -1509,9 +1514,14 @@ extern "C" int tp_create(int device, void **ctx_out)
         for (int src = 0; src < 5; ++src)
             for (int prec = 0; prec < 2; ++prec)
                 c->blocks_per_cu[src][prec] = tpk::fused_blocks_per_cu(src, prec);
-        if (device < NS_MAX_DEVICES) { // tables of tp_run_device_noalloc (device current)
-            NoallocSetup &S = g_noalloc[device];
-            std::call_once(S.once, [&] { noalloc_setup(S, c->cus, c->blocks_per_cu[0]); });
+        if (device < NS_MAX_DEVICES) { // xoshiro256+ tables (device current)
+            std::call_once(g_xo[device].once, [&] { xo_setup(g_xo[device].t, c->stream); });
+            c->xo = &g_xo[device].t;
+        }
+        const int rc = ensure(c, c->parts, MAX_PARTS * sizeof(tp_acc));
+        if (rc) {
+            tp_destroy(c);
+            return rc;
         }
         *ctx_out = c;
         return TP_OK;
@@ -1526,7 +1536,7 @@ extern "C" int tp_destroy(void *ctx)
             return TP_ERR_ARG;
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
-        for (DevBuf *b : {&c->mt, &c->polys, &c->draws, &c->origin, &c->p0, &c->per_batch, &c->merged, &c->evq,
+        for (DevBuf *b : {&c->parts, &c->mt, &c->polys, &c->draws, &c->origin, &c->p0, &c->per_batch, &c->merged, &c->evq,
                           &c->mt128, &c->bt128, &c->st128, &c->f32ev, &c->fe_lists, &c->fe_meta, &c->fe_piece,
                           &c->fe_flag, &c->fe_seq, &c->xo_states, &c->xo_draws, &c->xo128_states,
                           &c->xo128_draws, &c->xo128_pt, &c->xo_acc, &c->xo_lt, &c->xo128_lt, &c->fe_stat, &c->adj_u})
@@ -1535,8 +1545,6 @@ extern "C" int tp_destroy(void *ctx)
         for (auto &kv : c->tables) {
             if (kv.second->bt.p)
                 (void)hipFree(kv.second->bt.p);
-            if (kv.second->stride.p)
-                (void)hipFree(kv.second->stride.p);
         }
         for (auto &e : c->ev)
             if (e)
@@ -1958,18 +1966,9 @@ extern "C" int tp_run_device_noalloc(void *ctx, const tp_params *params, int rng
         if (!per_batch_dev)
             return fail(c, TP_ERR_ARG, "null per-batch output");
         const uint64_t nb = (num_events + TP_BATCH_SIZE - 1) / TP_BATCH_SIZE;
-        if (nb >= (1ull << NS_KB))
+        if (nb >= (1ull << 32))
             return fail(c, TP_ERR_ARG, "tp_run_device_noalloc: at most 2^32 - 1 batches of 10 000 events");
-        if (c->device >= NS_MAX_DEVICES)
-            return fail(c, TP_ERR_UNSUPPORTED, "tp_run_device_noalloc: device ordinal above 63");
-        const NoallocSetup &S = g_noalloc[c->device];
-        if (S.rc != TP_OK)
-            return fail(c, S.rc, "tp_run_device_noalloc set-up failed: " + S.err);
         HIPCHK(c, hipSetDevice(c->device));
-        const int p = params->precision == TP_PREC_MIXED ? 1 : 0;
-        const int grid = grid_for(c, 0, params->precision, nb);
-        if ((uint64_t)grid < nb && grid != S.full_grid[p])
-            return fail(c, TP_ERR_INTERNAL, "tp_run_device_noalloc: grid differs from the set-up's");
         tpk::FusedArgs a;
         std::memset(&a, 0, sizeof a);
         a.P = make_event_params(params, params->precision);
@@ -1977,17 +1976,13 @@ extern "C" int tp_run_device_noalloc(void *ctx, const tp_params *params, int rng
         a.batch_size = TP_BATCH_SIZE;
         a.precision = params->precision;
         std::memcpy(a.s0, static_cast<const tp_xoshiro_state *>(rng_state0)->s, sizeof a.s0);
-        a.mt = S.ptr;
-        a.km = KM;
-        a.bt = S.ptr + (size_t)(NS_BT + seeding * NS_KB) * 1024;
-        a.kb = std::max(1, bits_for(nb));
-        a.stride = S.ptr + (size_t)(NS_STRIDE + 2 * seeding + p) * 1024;
-        a.nb = nb;
-        a.b_first = 0;
+        rc = xo_event_args(c, a, seeding, nb);
+        if (rc)
+            return rc;
         a.out = per_batch_dev;
         HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
         HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-        tpk::launch_fused(a, 0, grid, c->stream);
+        launch_event_loop(c, a, 0, (uint32_t)std::min<uint64_t>(num_events, TP_BATCH_SIZE));
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         if (merged_dev) {

@@ -624,7 +624,7 @@ extern "C" int tp_flow_run_device(void *flow, const tp_params *params, double al
             fa.nb = b1 - b0;
             fa.b_first = b0;
             fa.out = per_batch_dev + b0;
-            tpk::launch_fused(fa, 2, grid_for(c, 2, 0, fa.nb), c->stream);
+            launch_event_loop(c, fa, 2, (uint32_t)std::min<uint64_t>(num_events, bs));
             FHIP(f, hipGetLastError());
         }
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));

@@ -19,13 +19,21 @@ struct FusedArgs {
     uint64_t num_events;   // events of the whole run (for the last, partial batch)
     uint32_t batch_size;   // events per full batch
     int32_t precision;     // tp_precision
-    // xoshiro source: state of batch b, thread chunk start e0 is
-    //   M^(12*e0) * B^b * s0  with B = M^(12*batch_size) or the 2^128 jump.
+    // A batch's events are split over `parts` wavefronts, each taking runs of
+    // `run` events per lane: part s holds events 64 run s .. of the batch.
+    // With more than one part each writes its sums to part_out[batch * parts + s]
+    // and launch_batch_sums adds them up.
+    uint32_t parts, run;
+    void *part_out;        // tp_acc*
+    // xoshiro source: part s of batch b starts at M^(12 * 64 run s) * B^b * s0
+    // with B = M^(12*batch_size) or the 2^128 jump, and its lane l
+    // 12 run l draws later.
     uint64_t s0[4];
-    const uint64_t *mt;    // M^(2^k), k < km, each 256x4 words
-    const uint64_t *bt;    // B^(2^k), k < kb
-    const uint64_t *stride;// B^(grid size)
-    int32_t km, kb;
+    const uint64_t *m16, *b16; // M^(v 16^j), B^(v 16^j), v = 1..15: digits of an exponent (tp_xoshiro.h)
+    const uint64_t *lanes;     // images of the state's nibbles under the lanes' skips for `run`
+    // tp_events: M^(2^k), k < km, each 256x4 words
+    const uint64_t *mt;
+    int32_t km;
     // buffer source: RANF values (int32 in [0, 1e9)) of this launch's batches,
     // batch (b - b_first) at offset 12*batch_size*(b - b_first).
     const int32_t *draws;
@@ -81,6 +89,22 @@ void launch_fused(const FusedArgs &a,
                   int source /*0 xoshiro, 1 buffer, 2 weighted, 3 faster-evgen RANF, 4 faster-evgen xoshiro (f64 only)*/,
                   int grid, hipStream_t st);
 int fused_blocks_per_cu(int source, int precision); // resident workgroups per CU (occupancy)
+// The sums of a.nb batches from their parts, in the order of the parts.
+void launch_batch_sums(const FusedArgs &a, hipStream_t st);
+
+// ---- xoshiro256+ skip tables (once per device) --------------------------------
+// Events per lane that a wavefront of the event loop may take, each with a
+// lane table of its own: a batch of 10 000 events in 1, 2, 3, 4, 8, 16, 32, 40,
+// 79 and 157 parts.
+constexpr uint32_t XO_RUNS[] = {157, 79, 53, 40, 20, 10, 5, 4, 2, 1};
+constexpr int XO_NRUNS = sizeof XO_RUNS / sizeof XO_RUNS[0];
+constexpr int XO_M_DIGITS = 12, XO_B_DIGITS = 8;         // exponents below 2^48 draws, 2^32 batches
+constexpr size_t XO_MAT_WORDS = 1024;                    // 256 columns of 4 words
+constexpr size_t XO_LANE_WORDS = 64 * 16 * 64 * 4;       // per run length: 2 MiB
+// tab16[(15 j + v - 1) * 1024 ..] = B^(v 16^j) from pow2[k * 1024 ..] = B^(2^k), k < 4 digits.
+void launch_xo_digit_table(const uint64_t *pow2, int digits, uint64_t *tab16, hipStream_t st);
+// The lane tables of every run length of XO_RUNS, in that order.
+void launch_xo_lane_tables(const uint64_t *m16, uint64_t *lanes, hipStream_t st);
 // Per-event diagnostics: one thread per event, same device code as the loop.
 // Event e draws from offset 12*e (xoshiro: a.s0 with a.mt; buffer: a.draws).
 struct EventOut {

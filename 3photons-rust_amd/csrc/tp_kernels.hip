@@ -1,12 +1,12 @@
 // tp_kernels.hip -- gfx950 kernels of the 3photons event loop.
 //
-//  fused_kernel      one wavefront per 10 000-event batch, grid-strided over
-//                    batches; uniforms from xoshiro256+ in registers or from
+//  fused_kernel      one wavefront per 10 000-event batch or part of one,
+//                    grid-strided over parts; uniforms from xoshiro256+ in registers or from
 //                    the expanded RANF stream, RAMBO -> cuts in registers,
 //                    passing events compacted through an LDS queue, spinors
 //                    -> amplitudes -> weight on full wavefronts, 12 running
 //                    sums per lane, butterfly reduction to one accumulator
-//                    per batch.
+//                    per part (batch_sums_kernel adds a batch's parts).
 //  ranf_expand       RANF stream into HBM, one wavefront per segment of R
 //                    rounds, 55 lanes = the 55 values of a round.
 //  ranf_seed         jump-mode origins, seeded_new(seed + 123456 b) per batch.
@@ -26,21 +26,6 @@ struct DevAcc { // layout of tp_acc
     uint64_t selected;
     double spm2[5], vars[5], sigma, variance;
 };
-
-// State of (batch b, draw offset off inside the batch): M^off B^b s0.
-__device__ __forceinline__ void xo_state_at(const FusedArgs &a, uint64_t b, uint64_t off, uint64_t s[4])
-{
-    s[0] = a.s0[0];
-    s[1] = a.s0[1];
-    s[2] = a.s0[2];
-    s[3] = a.s0[3];
-    for (int k = 0; k < a.kb; ++k)
-        if ((b >> k) & 1ull) // uniform across the workgroup
-            gf2_apply(a.bt + 1024 * k, s);
-    for (int k = 0; k < a.km; ++k)
-        if ((off >> k) & 1ull) // per lane
-            gf2_apply(a.mt + 1024 * k, s);
-}
 
 // ---- per-thread accumulation (resacc.rs:121-129) ---------------------------
 // Sums s = (spm2[5], vars[5], sigma, variance); the mixed-precision path
@@ -149,19 +134,28 @@ __device__ __forceinline__ void block_reduce_store(double v[12], uint32_t n, Dev
 
 // ---- the fused event loop ------------------------------------------------
 //
-// One wavefront per batch.  Each iteration every lane generates one event
-// (uniforms -> RAMBO -> sort slots -> cuts); the photon momenta of the events
-// that pass are appended to a queue in LDS (ballot + prefix count), each photon
-// into the row of its sort slot, and whenever 64
-// are queued the whole wavefront takes them and evaluates spinors, amplitudes
+// One wavefront per part of a batch, persistent: the grid holds as many
+// wavefronts as are resident and each strides over parts.  Each iteration every lane generates one event
+// (uniforms -> RAMBO -> cuts); the photon momenta of the events
+// that pass are appended to a queue in LDS (ballot + prefix count), and whenever 64
+// are queued the whole wavefront takes them and evaluates the helicity sums
 // and weights on full lanes.  Cut events therefore cost no amplitude work, and
 // the amplitude code never runs with masked-off lanes except for the final
-// partial flush of a batch.  The accumulation order is the queue order, a
+// partial flush of a part.  The accumulation order is the queue order, a
 // function of the data only, so results are reproducible run to run.
 //
-// Event assignment inside the batch: with the in-register xoshiro stream each
-// lane owns a contiguous chunk (one skip-ahead per chunk); with a stream read
+// Event assignment inside the part: with the in-register xoshiro stream each
+// lane owns a contiguous run (one skip-ahead per run); with a stream read
 // from HBM lane l takes events l, l+64, ... (coalesced loads).
+//
+// What bounds it: VALU issue, at the measured issue times (f64 fma 4.9 cycles,
+// add and mul 4.4, rcp and rsq 16.3, xor, mov and add_u32 2.7, shifts and
+// three-operand integer instructions 4.4) about 90 % busy at 1e9 events; one
+// wavefront per batch left a run of 1e7 events with one wavefront per SIMD of
+// the three that fit and a closure call with one on the whole chip, most of
+// whose time was the lanes' own skips of the stream (a call of 4321 events
+// 381 -> 42 us, 1.23e6 events with jump seeding 677 -> 93 us, 1e9 events
+// 26.8 -> 25.8 ms with parts and shared skips).
 constexpr int QCAP = 128;
 
 // Three wavefronts per SIMD (163 VGPRs at f64, no scratch): the LDS queue
@@ -190,38 +184,33 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
     __shared__ double red[1][13];
     const uint32_t lane = threadIdx.x;
     const uint64_t lanemask_lt = (1ull << lane) - 1ull;
-    uint64_t st[4] = {0, 0, 0, 0}; // xoshiro state at this lane's chunk start
+    uint64_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}; // xoshiro state at the part's first draw (uniform)
     bool have = false;
-    DevAcc *out = reinterpret_cast<DevAcc *>(a.out);
-    for (uint64_t lb = blockIdx.x; lb < a.nb; lb += gridDim.x) {
+    for (uint64_t t = blockIdx.x; t < a.nb * a.parts; t += gridDim.x) {
+        const uint64_t lb = a.parts == 1 ? t : t / a.parts;
+        const uint32_t first = (uint32_t)(t - lb * a.parts) * 64u * a.run; // the part's first event in the batch
         const uint64_t b = a.b_first + lb;
-        const uint64_t start = b * a.batch_size;
-        const uint64_t left = a.num_events - start;
-        const uint32_t n = left < a.batch_size ? (uint32_t)left : a.batch_size;
-        const uint32_t q = n / 64, r = n % 64;
-        const uint32_t iters = q + (r ? 1u : 0u);
-        uint32_t len, e0;
-        if (SOURCE == 0) {
-            len = q + (lane < r ? 1u : 0u);
-            e0 = lane * q + (lane < r ? lane : r);
-        } else {
-            len = q + (lane < r ? 1u : 0u); // events lane, lane+64, ...
-            e0 = lane;
-        }
+        const uint64_t left = a.num_events - b * a.batch_size;
+        const uint32_t nbatch = left < a.batch_size ? (uint32_t)left : a.batch_size;
+        const uint32_t n = first < nbatch ? min(nbatch - first, 64u * a.run) : 0u;
+        uint32_t len, iters;
         uint64_t s[4] = {0, 0, 0, 0};
         if (SOURCE == 0) {
-            if (!have || n != a.batch_size)
-                xo_state_at(a, b, 12ull * e0, st);
-            else
-                gf2_apply(a.stride, st);
+            len = lane * a.run < n ? min(n - lane * a.run, a.run) : 0u;
+            iters = min(n, a.run);
+            // every part of this wavefront has the same place in its batch
+            // (the grid is a multiple of `parts` wherever it strides)
+            xo_advance_uniform(a.b16, have ? gridDim.x / a.parts : b, sw);
+            if (!have)
+                xo_advance_uniform(a.m16, 12ull * first, sw);
             have = true;
-            s[0] = st[0];
-            s[1] = st[1];
-            s[2] = st[2];
-            s[3] = st[3];
+            xo_lane_states(a.lanes, sw, s);
+        } else {
+            len = n / 64 + (lane < n % 64 ? 1u : 0u); // events lane, lane+64, ...
+            iters = (n + 63) / 64;
         }
-        const int32_t *src = (SOURCE == 1) ? a.draws + (size_t)lb * 12 * a.batch_size : nullptr;
-        const size_t wbase = (size_t)lb * a.batch_size;
+        const int32_t *src = (SOURCE == 1) ? a.draws + 12 * ((size_t)lb * a.batch_size + first) : nullptr;
+        const size_t wbase = (size_t)lb * a.batch_size + first;
         const RerollBits rb{a.acc1, a.bbase, a.bstride ? (lb + 1) * a.bstride : a.blimit};
         Acc<PREC> A;
         acc_zero(A);
@@ -317,8 +306,99 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
         __syncthreads();
         double v[12];
         acc_values(A, fresh_params(), v);
-        block_reduce_store<1>(v, A.n, out + lb, red);
+        block_reduce_store<1>(v, A.n, reinterpret_cast<DevAcc *>(a.parts == 1 ? a.out : a.part_out) + t, red);
     }
+}
+
+// Parts' sums into their batch's: lane l adds parts l, l + 64, ..., then the
+// butterfly of block_reduce_store (the order depends on the number of parts
+// only).
+__global__ __launch_bounds__(64) void batch_sums_kernel(FusedArgs a)
+{
+    __shared__ double red[1][13];
+    const uint64_t lb = blockIdx.x;
+    const DevAcc *p = reinterpret_cast<const DevAcc *>(a.part_out) + lb * a.parts;
+    double v[12] = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
+    uint32_t n = 0;
+    for (uint32_t s = threadIdx.x; s < a.parts; s += 64) {
+        n += (uint32_t)p[s].selected;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+            v[j] = v[j] + p[s].spm2[j];
+            v[5 + j] = v[5 + j] + p[s].vars[j];
+        }
+        v[10] = v[10] + p[s].sigma;
+        v[11] = v[11] + p[s].variance;
+    }
+    block_reduce_store<1>(v, n, reinterpret_cast<DevAcc *>(a.out) + lb, red);
+}
+
+void launch_batch_sums(const FusedArgs &a, hipStream_t st)
+{
+    hipLaunchKernelGGL(batch_sums_kernel, dim3((unsigned)a.nb), dim3(64), 0, st, a);
+}
+
+// Column `col` of B^(v 16^j), one lane per column; the matrices are uniform.
+__global__ __launch_bounds__(64) void xo_digit_table_kernel(const uint64_t *pow2, uint64_t *tab16)
+{
+    const uint32_t j = blockIdx.x / 15, v = blockIdx.x % 15 + 1, col = 64 * blockIdx.y + threadIdx.x;
+    uint64_t s[4];
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w)
+        s[w] = w == blockIdx.y ? 1ull << threadIdx.x : 0;
+    for (uint32_t k = 0; k < 4; ++k)
+        if ((v >> k) & 1u)
+            gf2_apply(pow2 + XO_MAT_WORDS * (4 * j + k), s);
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+        tab16[XO_MAT_WORDS * blockIdx.x + 4 * col + w] = s[w];
+}
+
+void launch_xo_digit_table(const uint64_t *pow2, int digits, uint64_t *tab16, hipStream_t st)
+{
+    hipLaunchKernelGGL(xo_digit_table_kernel, dim3(15 * digits, 4), dim3(64), 0, st, pow2, tab16);
+}
+
+struct XoRuns {
+    uint32_t n[XO_NRUNS];
+};
+// Lane l's images of every value of nibble `threadIdx.x` of the state, for run
+// length runs.n[blockIdx.y] (l = blockIdx.x, so the skip matrices are uniform).
+__global__ __launch_bounds__(64) void xo_lane_table_kernel(const uint64_t *m16, uint64_t *lanes, XoRuns runs)
+{
+    const uint32_t l = blockIdx.x, ch = threadIdx.x;
+    uint64_t img[4][4]; // of the nibble's four bits
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w)
+            img[k][w] = w == ch / 16 ? 1ull << (4 * (ch % 16) + k) : 0;
+        const uint64_t *tab = m16;
+        for (uint32_t e = 12 * runs.n[blockIdx.y] * l; e; e >>= 4, tab += 15 * XO_MAT_WORDS)
+            if (e & 15u)
+                gf2_apply(tab + ((e & 15u) - 1) * XO_MAT_WORDS, img[k]);
+    }
+    uint64_t *out = lanes + XO_LANE_WORDS * blockIdx.y + 256 * (size_t)(16 * ch) + 2 * l;
+#pragma unroll
+    for (uint32_t v = 0; v < 16; ++v) {
+        uint64_t x[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k)
+#pragma unroll
+            for (uint32_t w = 0; w < 4; ++w)
+                x[w] ^= (v >> k) & 1u ? img[k][w] : 0;
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w)
+            out[256 * v + 128 * (w / 2) + w % 2] = x[w];
+    }
+}
+
+void launch_xo_lane_tables(const uint64_t *m16, uint64_t *lanes, hipStream_t st)
+{
+    XoRuns r;
+    for (int i = 0; i < XO_NRUNS; ++i)
+        r.n[i] = XO_RUNS[i];
+    hipLaunchKernelGGL(xo_lane_table_kernel, dim3(64, XO_NRUNS), dim3(64), 0, st, m16, lanes, r);
 }
 
 template <int SOURCE, int PREC> int blocks_per_cu()

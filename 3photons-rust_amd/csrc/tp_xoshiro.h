@@ -88,6 +88,86 @@ __device__ __forceinline__ void gf2_apply(const uint64_t *__restrict__ mg, uint6
     s[3] = r3;
 }
 
+// ---- states of a wavefront's lanes ------------------------------------------
+// A wavefront whose lanes each take a run of consecutive draws needs 64 states
+// a fixed number of draws apart.  A lane that skips to its own by itself
+// applies one 256x256 matrix per set bit of its offset, some 2500 instructions
+// each.  Instead the wavefront skips once to its first draw, all lanes on one
+// matrix together (gf2_uniform), and takes the lanes' offsets from a table of
+// their images of every nibble of the state (xo_lane_states): about 140
+// instructions per digit of the skip and 650 for all 64 lanes.
+
+// XOR over the wavefront's 64 lanes (all active); the result is uniform.
+template <int CTRL, int ROWS> __device__ __forceinline__ uint32_t xor_dpp(uint32_t x)
+{
+    return x ^ (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ uint32_t wave_xor(uint32_t x)
+{
+    x = xor_dpp<0x111, 0xf>(x); // row_shr:1, 2, 4, 8: lane 15 of each row of 16 holds the row's
+    x = xor_dpp<0x112, 0xf>(x);
+    x = xor_dpp<0x114, 0xf>(x);
+    x = xor_dpp<0x118, 0xf>(x);
+    x = xor_dpp<0x142, 0xa>(x); // row_bcast:15 into rows 1 and 3
+    x = xor_dpp<0x143, 0xc>(x); // row_bcast:31 into rows 2 and 3: lane 63 holds all
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
+// s <- M s for a state all lanes hold alike: lane l takes columns l, l + 64,
+// l + 128 and l + 192.
+__device__ __forceinline__ void gf2_uniform(const uint64_t *__restrict__ m, uint64_t s[4])
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint4 *c = reinterpret_cast<const uint4 *>(m) + 2 * lane;
+    uint32_t r[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const uint4 a = c[128 * w], b = c[128 * w + 1];
+        const uint32_t k = 0u - ((uint32_t)(s[w] >> lane) & 1u);
+        r[0] ^= a.x & k;
+        r[1] ^= a.y & k;
+        r[2] ^= a.z & k;
+        r[3] ^= a.w & k;
+        r[4] ^= b.x & k;
+        r[5] ^= b.y & k;
+        r[6] ^= b.z & k;
+        r[7] ^= b.w & k;
+    }
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+        s[w] = pack64(wave_xor(r[2 * w]), wave_xor(r[2 * w + 1]));
+}
+
+// s <- B^e s for a state and exponent all lanes hold alike, from the table
+// B^(v 16^j), v = 1..15, of e's hexadecimal digits j.
+__device__ __forceinline__ void xo_advance_uniform(const uint64_t *__restrict__ tab, uint64_t e, uint64_t s[4])
+{
+    for (; e; e >>= 4, tab += 15 * 1024)
+        if (e & 15u)
+            gf2_uniform(tab + ((e & 15u) - 1) * 1024, s);
+}
+
+// The lanes' states s_l = L^l s from the table of L^l (v << 4 ch), entry
+// [ch][v][2][lane][2 words] (ch the nibble of the state, v its value).
+__device__ __forceinline__ void xo_lane_states(const uint64_t *__restrict__ tab, const uint64_t s[4], uint64_t st[4])
+{
+    const ulonglong2 *t = reinterpret_cast<const ulonglong2 *>(tab) + (threadIdx.x & 63u);
+    st[0] = st[1] = st[2] = st[3] = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const uint64_t x = s[w];
+#pragma unroll 4
+        for (int k = 0; k < 16; ++k) {
+            const ulonglong2 *e = t + 128 * (16 * (16 * w + k) + (uint32_t)((x >> (4 * k)) & 15u));
+            const ulonglong2 a = e[0], b = e[64];
+            st[0] ^= a.x;
+            st[1] ^= a.y;
+            st[2] ^= b.x;
+            st[3] ^= b.y;
+        }
+    }
+}
+
 // ---- xoshiro128+ (the f32 generator of src/random/standard.rs) ---------------
 __device__ __forceinline__ uint32_t rotl32(uint32_t x, int k) { return (x << k) | (x >> (32 - k)); }
 

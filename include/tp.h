@@ -182,9 +182,11 @@ int tp_run_device(void *ctx, const tp_params *params, int rng_kind, int seeding,
  * runs the xoshiro256+ stream only (rng_kind TP_RNG_XOSHIRO, precision
  * TP_PREC_F64 or TP_PREC_MIXED, both seedings, no faster-evgen; anything else
  * returns TP_ERR_UNSUPPORTED) and at most 2^32 - 1 batches (TP_ERR_ARG
- * beyond).  Its skip-ahead tables sit in a static device array of 800 KiB
+ * beyond).  Its skip-ahead tables sit in a static device array of 24 MiB
  * per GPU, filled once by tp_create and only read afterwards, so calls that
- * overlap on one GPU share it without racing; per_batch_dev and merged_dev
+ * overlap on one GPU share it without racing; the sums of batches split over
+ * several wavefronts go through 6.5 MiB of the context's own, also allocated
+ * by tp_create; per_batch_dev and merged_dev
  * are the caller's, as for tp_run_device.  Returns when enqueued; tp_sync
  * waits. */
 int tp_run_device_noalloc(void *ctx, const tp_params *params, int rng_kind, int seeding,
