@@ -65,8 +65,9 @@ struct Ctx {
     DevBuf mt;       // M^(2^k)
     int km = 0;
     std::map<std::string, std::unique_ptr<Tables>> tables;
-    std::map<std::string, std::vector<uint32_t>> ranf_polys; // host copies keyed by R
-    DevBuf polys, draws, origin, p0, per_batch, merged, evq;
+    DevBuf r16;             // RANF: jump polynomials of the digits of a number of rounds
+    bool r16_ready = false;
+    DevBuf draws, origin, p0, per_batch, merged, evq;
     DevBuf parts; // sums of the parts of split batches (MAX_PARTS), allocated by tp_create
     DevBuf mt128, bt128, f32ev; // all-f32 mode: xoshiro128+ tables, per-event values
     std::string bt128_key;
@@ -197,6 +198,15 @@ inline void launch_event_loop(const Ctx *c, tpk::FusedArgs &a, int source, uint3
         for (int i = 0; i < tpk::XO_NRUNS; ++i)
             if (tpk::XO_RUNS[i] == s.run)
                 a.lanes = c->xo->lanes + (size_t)i * tpk::XO_LANE_WORDS;
+    }
+    a.rjump_rounds = 0;
+    const uint64_t stride = 12ull * a.batch_size * (s.grid / s.parts), part = 12ull * std::min<uint64_t>(64ull * s.run, n);
+    if (source == 1 && !a.rorigin && a.nb * s.parts > (uint64_t)s.grid) {
+        // the least number of rounds from the last one of a part to the first
+        // of the wavefront's next (a part of whole runs: that or one more)
+        a.rjump_rounds = (stride - part + 1) / 55;
+        const tp::RanfPoly q = tp::ranf_poly_rounds(a.rjump_rounds);
+        std::copy(q.begin(), q.end(), a.rjump);
     }
     tpk::launch_fused(a, source, s.grid, c->stream);
     if (s.parts > 1)

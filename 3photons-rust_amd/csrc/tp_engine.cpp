@@ -323,25 +323,18 @@ int ensure_jump_table(Ctx *c, uint64_t nb, Tables **out)
     return TP_OK;
 }
 
-// x^(55*R*2^k) mod (x^55 + x^31 - 1) for k < K, uploaded to c->polys.
-int ensure_polys(Ctx *c, int R, int K)
+// The jump polynomials of the digits of a number of RANF rounds, into c->r16
+// (once per context).
+int ensure_r16(Ctx *c)
 {
-    std::string key = std::to_string(R) + ":" + std::to_string(K);
-    auto it = c->ranf_polys.find(key);
-    if (it == c->ranf_polys.end()) {
-        std::vector<uint32_t> flat;
-        tp::RanfPoly q = tp::ranf_poly_xpow(55ull * static_cast<uint64_t>(R));
-        for (int k = 0; k < K; ++k) {
-            flat.insert(flat.end(), q.begin(), q.end());
-            q = tp::ranf_poly_mul(q, q);
-        }
-        it = c->ranf_polys.emplace(key, std::move(flat)).first;
-    }
-    int rc = ensure(c, c->polys, it->second.size() * sizeof(uint32_t));
+    if (c->r16_ready)
+        return TP_OK;
+    const std::vector<uint32_t> &t = tp::ranf_round_digits();
+    int rc = ensure(c, c->r16, t.size() * sizeof(uint32_t));
     if (rc)
         return rc;
-    HIPCHK(c, hipMemcpyAsync(c->polys.p, it->second.data(), it->second.size() * sizeof(uint32_t),
-                             hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipMemcpy(c->r16.p, t.data(), t.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    c->r16_ready = true;
     return TP_OK;
 }
 
@@ -421,7 +414,7 @@ int ensure_acc(Ctx *c, uint64_t np) { return ensure_acc_words(c, np * FE_XO_WORD
 // q_first at index 0), from the master origin uploaded by the caller, and
 // their accept bits (the unit-disc test of stream kind 0 or 1) into c->xo_acc
 // from *bbase, the first position of the first expansion segment, on.
-int fe_expand(Ctx *c, uint64_t p0_master, int K, uint64_t q_first, uint64_t q_last, int kind, uint64_t *bbase)
+int fe_expand(Ctx *c, uint64_t p0_master, uint64_t q_first, uint64_t q_last, int kind, uint64_t *bbase)
 {
     const uint64_t seg_first = q_first / 55 / RANF_R, nsegs = (q_last - 1) / 55 / RANF_R - seg_first + 1;
     int rc = ensure(c, c->draws, (q_last - q_first) * sizeof(int32_t));
@@ -433,8 +426,7 @@ int fe_expand(Ctx *c, uint64_t p0_master, int K, uint64_t q_first, uint64_t q_la
     std::memset(&r, 0, sizeof r);
     r.origin = static_cast<const int32_t *>(c->origin.p);
     r.p0 = static_cast<const int32_t *>(c->p0.p);
-    r.polys = static_cast<const uint32_t *>(c->polys.p);
-    r.K = K;
+    r.r16 = static_cast<const uint32_t *>(c->r16.p);
     r.R = RANF_R;
     r.out = static_cast<int32_t *>(c->draws.p);
     r.d_begin = q_first - p0_master;
@@ -455,7 +447,6 @@ int fe_expand(Ctx *c, uint64_t p0_master, int K, uint64_t q_first, uint64_t q_la
 struct FeStream {
     int kind = 0;                 // tpk::FeWalkArgs kind: 0 RANF f64, 1 RANF f32, 2 xoshiro256+
     uint64_t p0_master = 0;       // RANF: frame position of the master origin's next value
-    int K = 0;                    // RANF: segment-jump depth of c->polys
     const uint64_t *s0 = nullptr; // xoshiro256+: the run's state (position 0)
     const uint32_t *s0_128 = nullptr; // xoshiro128+ (kind 3): the run's state (position 0)
 };
@@ -549,7 +540,7 @@ int fe_stream_expand(Ctx *c, const FeStream &fs, uint64_t q_first, uint64_t q_la
 {
     if (fs.kind < 2) {
         *qbase = q_first;
-        return fe_expand(c, fs.p0_master, fs.K, q_first, q_last, fs.kind, bbase);
+        return fe_expand(c, fs.p0_master, q_first, q_last, fs.kind, bbase);
     }
     const uint64_t p_first = q_first / FE_XO_PIECE, p_end = (q_last + FE_XO_PIECE - 1) / FE_XO_PIECE;
     const uint64_t np = p_end - p_first;
@@ -784,9 +775,7 @@ int enqueue_ranf_faster_evgen(Ctx *c, tpk::FusedArgs &a, tpk::F32Args *fa, const
     FeStream fs;
     fs.kind = fa ? 1 : 0;
     fs.p0_master = 55u - rs->index; // position of the next value
-    // segment jumps cover positions up to 30 per event (the mean is 17.9)
-    fs.K = std::max(1, bits_for((fs.p0_master + 30 * (num_events + 1) + 4 * FE_OVERLAP) / 55 / RANF_R + 2));
-    int rc = ensure_polys(c, RANF_R, fs.K);
+    int rc = ensure_r16(c);
     if (!rc)
         rc = ensure(c, c->origin, 56 * sizeof(int32_t));
     if (!rc)
@@ -887,8 +876,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     const uint64_t PS = FE_JUMP_PIECE * ((batch_size + TP_BATCH_SIZE - 1) / TP_BATCH_SIZE);
     const uint64_t max_rounds = PS / 55 + 2;
-    const int K = std::max(1, bits_for(max_rounds / RANF_R + 1));
-    int rc = ensure_polys(c, RANF_R, K);
+    int rc = ensure_r16(c);
     if (!rc)
         rc = ensure(c, c->draws, chunk * PS * sizeof(int32_t));
     if (!rc)
@@ -924,8 +912,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         std::memset(&r, 0, sizeof r);
         r.origin = static_cast<const int32_t *>(c->origin.p) + 56 * first_piece;
         r.p0 = static_cast<const int32_t *>(c->p0.p) + first_piece;
-        r.polys = static_cast<const uint32_t *>(c->polys.p);
-        r.K = K;
+        r.r16 = static_cast<const uint32_t *>(c->r16.p);
         r.R = RANF_R;
         r.out = static_cast<int32_t *>(c->draws.p) + first_piece * PS;
         r.d_begin = d_begin;
@@ -1290,8 +1277,6 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         return TP_OK;
     }
-    // RANF: expand the stream of a chunk of batches into HBM, then run the
-    // fused kernel on it.
     const tp_ranf_state *rs = static_cast<const tp_ranf_state *>(state0);
     if (rs->index > 55)
         return fail(c, TP_ERR_ARG, "RANF state index out of range");
@@ -1302,6 +1287,36 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
             fa.source = 2;
         return enqueue_ranf_faster_evgen(c, a, f32 ? &fa : nullptr, rs, num_events, batch_size, per_batch_dev);
     }
+    rc = ensure_r16(c);
+    if (rc)
+        return rc;
+    if (!f32) { // the event loop makes its draws itself
+        std::memcpy(a.rround, rs->numbers, sizeof a.rround);
+        a.rp0 = 55u - rs->index;
+        a.r16 = static_cast<const uint32_t *>(c->r16.p);
+        a.nb = nb;
+        a.b_first = 0;
+        a.out = per_batch_dev;
+        HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+        if (seeding == TP_SEED_JUMP) {
+            rc = ensure(c, c->origin, nb * 56 * sizeof(int32_t));
+            if (!rc)
+                rc = ensure(c, c->p0, nb * sizeof(int32_t));
+            if (rc)
+                return rc;
+            tpk::launch_ranf_seed(rs->seed, 0, nb, static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p),
+                                  c->stream);
+            HIPCHK(c, hipGetLastError());
+            a.rorigin = static_cast<const int32_t *>(c->origin.p);
+        }
+        HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+        launch_event_loop(c, a, 1, (uint32_t)std::min<uint64_t>(num_events, batch_size));
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+        return TP_OK;
+    }
+    // All-f32 mode: the stream of a chunk of batches expanded into HBM, then
+    // its events.
     const uint64_t chunk = std::min<uint64_t>(nb, RANF_CHUNK_BATCHES);
     const size_t per_batch_draws = 12ull * batch_size;
     rc = ensure(c, c->draws, chunk * per_batch_draws * sizeof(int32_t));
@@ -1318,10 +1333,6 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     const uint64_t p0_master = 55u - rs->index;
     uint64_t max_rounds = (seeding == TP_SEED_JUMP) ? (per_batch_draws + 54) / 55 + 1
                                                     : (p0_master + total_draws + 54) / 55 + 1;
-    int K = std::max(1, bits_for(max_rounds / RANF_R + 1));
-    rc = ensure_polys(c, RANF_R, K);
-    if (rc)
-        return rc;
     HIPCHK(c, hipStreamSynchronize(c->stream)); // previous users of the staging copy are done
     int32_t *origin0 = c->origin0;
     std::memcpy(origin0, rs->numbers, sizeof c->origin0);
@@ -1335,8 +1346,7 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         std::memset(&r, 0, sizeof r);
         r.origin = static_cast<const int32_t *>(c->origin.p);
         r.p0 = static_cast<const int32_t *>(c->p0.p);
-        r.polys = static_cast<const uint32_t *>(c->polys.p);
-        r.K = K;
+        r.r16 = static_cast<const uint32_t *>(c->r16.p);
         r.R = RANF_R;
         r.out = static_cast<int32_t *>(c->draws.p);
         uint64_t npieces;
@@ -1373,25 +1383,17 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         }
         tpk::launch_ranf_expand(r, npieces, c->stream);
         HIPCHK(c, hipGetLastError());
-        a.nb = cnb;
-        a.b_first = b0;
-        a.draws = static_cast<const int32_t *>(c->draws.p);
-        a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
         if (first_kernel) {
             HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
             first_kernel = false;
         }
-        if (f32) {
-            fa.nb = cnb;
-            fa.b_first = b0;
-            fa.draws = a.draws;
-            fa.out = a.out;
-            tpk::launch_f32_events(fa, f32_grid(c, cnb), c->stream);
-            HIPCHK(c, hipGetLastError());
-            tpk::launch_f32_accumulate(fa, f32_grid(c, cnb), c->stream);
-        } else {
-            launch_event_loop(c, a, 1, (uint32_t)std::min<uint64_t>(num_events, batch_size));
-        }
+        fa.nb = cnb;
+        fa.b_first = b0;
+        fa.draws = static_cast<const int32_t *>(c->draws.p);
+        fa.out = static_cast<tp_acc *>(per_batch_dev) + b0;
+        tpk::launch_f32_events(fa, f32_grid(c, cnb), c->stream);
+        HIPCHK(c, hipGetLastError());
+        tpk::launch_f32_accumulate(fa, f32_grid(c, cnb), c->stream);
         HIPCHK(c, hipGetLastError());
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
@@ -1536,7 +1538,7 @@ extern "C" int tp_destroy(void *ctx)
             return TP_ERR_ARG;
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
-        for (DevBuf *b : {&c->parts, &c->mt, &c->polys, &c->draws, &c->origin, &c->p0, &c->per_batch, &c->merged, &c->evq,
+        for (DevBuf *b : {&c->parts, &c->mt, &c->r16, &c->draws, &c->origin, &c->p0, &c->per_batch, &c->merged, &c->evq,
                           &c->mt128, &c->bt128, &c->st128, &c->f32ev, &c->fe_lists, &c->fe_meta, &c->fe_piece,
                           &c->fe_flag, &c->fe_seq, &c->xo_states, &c->xo_draws, &c->xo128_states,
                           &c->xo128_draws, &c->xo128_pt, &c->xo_acc, &c->xo_lt, &c->xo128_lt, &c->fe_stat, &c->adj_u})
@@ -1695,9 +1697,7 @@ extern "C" int tp_events(void *ctx, const tp_params *params, int rng_kind, const
             HIPCHK(c, hipStreamSynchronize(c->stream));
             std::memcpy(c->origin0, rs->numbers, sizeof c->origin0);
             c->p00 = static_cast<int32_t>(55u - rs->index);
-            const uint64_t max_rounds = (c->p00 + D + 54) / 55 + 1;
-            const int K = std::max(1, bits_for(max_rounds / RANF_R + 1));
-            rc = ensure_polys(c, RANF_R, K);
+            rc = ensure_r16(c);
             if (rc)
                 return rc;
             HIPCHK(c, hipMemcpyAsync(c->origin.p, c->origin0, sizeof c->origin0, hipMemcpyHostToDevice, c->stream));
@@ -1706,8 +1706,7 @@ extern "C" int tp_events(void *ctx, const tp_params *params, int rng_kind, const
             std::memset(&r, 0, sizeof r);
             r.origin = static_cast<const int32_t *>(c->origin.p);
             r.p0 = static_cast<const int32_t *>(c->p0.p);
-            r.polys = static_cast<const uint32_t *>(c->polys.p);
-            r.K = K;
+            r.r16 = static_cast<const uint32_t *>(c->r16.p);
             r.R = RANF_R;
             r.out = static_cast<int32_t *>(c->draws.p);
             r.d_begin = 0;
@@ -1874,30 +1873,33 @@ extern "C" int tp_simulate_batch(void *ctx, const tp_params *params, int rng_kin
         if (rc)
             return rc;
         HIPCHK(c, hipMemcpyAsync(out, c->per_batch.p, sizeof(tp_acc), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
         // `&mut rng` side effect: 12 draws per event (evgen.rs:182-187), or the
-        // walk of the faster-evgen draws.
-        if (params->faster_evgen && rng_kind == TP_RNG_XOSHIRO) {
-            tp::xoshiro_advance(static_cast<tp_xoshiro_state *>(rng_state)->s, c->fe_xo_end);
-        } else if (params->faster_evgen && rng_kind == TP_RNG_XOSHIRO128) {
-            tp::xoshiro128_advance(static_cast<tp_xoshiro128_state *>(rng_state)->s, c->fe_xo_end);
-        } else if (params->faster_evgen) {
-            tp_ranf_state *s = static_cast<tp_ranf_state *>(rng_state);
-            std::memcpy(s->numbers, c->fe_end.numbers, sizeof s->numbers);
-            s->index = c->fe_end.index;
-        } else if (rng_kind == TP_RNG_XOSHIRO) {
-            tp::xoshiro_advance(static_cast<tp_xoshiro_state *>(rng_state)->s, 12ull * n);
-        } else if (rng_kind == TP_RNG_XOSHIRO128) {
-            tp::xoshiro128_advance(static_cast<tp_xoshiro128_state *>(rng_state)->s, 12ull * n);
-        } else {
+        // walk of the faster-evgen draws.  The new state is formed while the
+        // device works, and handed over once it is done.
+        if (rng_kind == TP_RNG_RANF) {
             tp_ranf_state *s = static_cast<tp_ranf_state *>(rng_state);
             tp::RanfState g;
-            std::memcpy(g.numbers, s->numbers, sizeof g.numbers);
-            g.index = s->index;
-            g.seed = s->seed;
-            tp::ranf_advance(g, 12ull * n);
+            if (params->faster_evgen) {
+                g = c->fe_end;
+            } else {
+                std::memcpy(g.numbers, s->numbers, sizeof g.numbers);
+                g.index = s->index;
+                g.seed = s->seed;
+                tp::ranf_advance(g, 12ull * n);
+            }
+            HIPCHK(c, hipStreamSynchronize(c->stream));
             std::memcpy(s->numbers, g.numbers, sizeof g.numbers);
             s->index = g.index;
+        } else if (rng_kind == TP_RNG_XOSHIRO) {
+            tp_xoshiro_state s = *static_cast<tp_xoshiro_state *>(rng_state);
+            tp::xoshiro_advance(s.s, params->faster_evgen ? c->fe_xo_end : 12ull * n);
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            *static_cast<tp_xoshiro_state *>(rng_state) = s;
+        } else {
+            tp_xoshiro128_state s = *static_cast<tp_xoshiro128_state *>(rng_state);
+            tp::xoshiro128_advance(s.s, params->faster_evgen ? c->fe_xo_end : 12ull * n);
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            *static_cast<tp_xoshiro128_state *>(rng_state) = s;
         }
         return TP_OK;
     });

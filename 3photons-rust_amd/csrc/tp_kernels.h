@@ -34,8 +34,19 @@ struct FusedArgs {
     // tp_events: M^(2^k), k < km, each 256x4 words
     const uint64_t *mt;
     int32_t km;
-    // buffer source: RANF values (int32 in [0, 1e9)) of this launch's batches,
-    // batch (b - b_first) at offset 12*batch_size*(b - b_first).
+    // RANF source: batch b's events draw from position rp0 + 12 batch_size b
+    // on of the stream whose round 0 is rround (X[1..55]); with jump seeding
+    // (rorigin non-null) batch b > 0 has a stream of its own, round 0 at
+    // rorigin[56 b] and positions from 0.  r16: x^(55 v 16^j) mod the
+    // recurrence's polynomial, 55 coefficients each, v = 1..15, for the digits
+    // of a number of rounds.
+    int32_t rround[56];
+    uint32_t rp0;
+    const int32_t *rorigin;
+    const uint32_t *r16;
+    uint32_t rjump[55];    // x^(55 rjump_rounds): from the end of a wavefront's part to near its next one
+    uint64_t rjump_rounds; // (0: none)
+    // expanded RANF values: faster-evgen (below), tp_events
     const int32_t *draws;
     // weighted source (importance sampling): uniforms (f64) and weight 1/q(u)
     // per event; event i = batch_size*(b - b_first) + e has its uniform j at
@@ -72,8 +83,7 @@ struct RanfArgs {
     uint64_t seg_first;    // first segment index of the window
     uint64_t nsegs;        // segments per piece in this launch
     uint64_t piece_stride; // output offset between pieces
-    const uint32_t *polys; // [K][55] x^(55*R*2^k) mod (x^55 + x^31 - 1)
-    int32_t K;
+    const uint32_t *r16;   // digits of a number of rounds, as FusedArgs
     int32_t R;             // rounds per segment
     int32_t *out;
     // faster-evgen: accept bits of every round the launch generates (bits 1:
@@ -86,7 +96,7 @@ struct RanfArgs {
 };
 
 void launch_fused(const FusedArgs &a,
-                  int source /*0 xoshiro, 1 buffer, 2 weighted, 3 faster-evgen RANF, 4 faster-evgen xoshiro (f64 only)*/,
+                  int source /*0 xoshiro, 1 RANF, 2 weighted, 3 faster-evgen RANF, 4 faster-evgen xoshiro (f64 only)*/,
                   int grid, hipStream_t st);
 int fused_blocks_per_cu(int source, int precision); // resident workgroups per CU (occupancy)
 // The sums of a.nb batches from their parts, in the order of the parts.

@@ -132,6 +132,109 @@ __device__ __forceinline__ void block_reduce_store(double v[12], uint32_t n, Dev
     __syncthreads();
 }
 
+// ---- RANF rounds -----------------------------------------------------------
+constexpr int32_t MODULO = 1000000000;
+
+// One RANF round in closed form (lane i - 1 holds X[i], i = 1..55):
+//   i <= 24:  X'[i] = X[i] - X[i+31]
+//   25..48:   X'[i] = X[i] - X'[i-24] = X[i] - X[i-24] + X[i+7]
+//   49..55:   X'[i] = X[i] - X[i-24] + X[i-48] - X[i-17]
+// (ranf.rs:106-119 applies the first two lines as in-place updates; the third
+// is the second with X'[i-24] expanded once more), all mod 1e9.  Every lane
+// evaluates (X[i] - b) + (c - d) with b, c, d read from other lanes of the
+// same wave by ds_bpermute (no LDS storage, no barrier).  Lanes 55..63 hold 0
+// and keep it, so a term a case does not have reads lane 63; each value is the
+// unique representative in [0, 1e9), so the sum order does not matter.  The
+// whole wave must be active: one wave holds one window.
+__device__ __forceinline__ uint32_t mod_sub(uint32_t a, uint32_t b) // (a - b) mod 1e9, a, b in [0, 1e9)
+{
+    const uint32_t t = a - b;
+    return min(t, t + (uint32_t)MODULO);
+}
+struct RanfLanes { // byte addresses for ds_bpermute of the lanes a lane reads
+    int b, c, d;
+};
+__device__ __forceinline__ RanfLanes ranf_lanes()
+{
+    const int lane = (int)(threadIdx.x & 63u), i = lane + 1;
+    const bool live = lane < 55;
+    RanfLanes l;
+    l.b = (live ? (i <= 24 ? i + 30 : i - 25) : 63) << 2;          // X[i+31] or X[i-24]
+    l.c = (live && i > 24 ? (i <= 48 ? i + 6 : i - 49) : 63) << 2; // X[i+7] or X[i-48]
+    l.d = (live && i > 48 ? i - 18 : 63) << 2;                     // X[i-17]
+    return l;
+}
+__device__ __forceinline__ int32_t ranf_next_round(int32_t x, const RanfLanes &l)
+{
+    const uint32_t wb = (uint32_t)__builtin_amdgcn_ds_bpermute(l.b, x);
+    const uint32_t wc = (uint32_t)__builtin_amdgcn_ds_bpermute(l.c, x);
+    const uint32_t wd = (uint32_t)__builtin_amdgcn_ds_bpermute(l.d, x);
+    const uint32_t v = mod_sub((uint32_t)x, wb) + mod_sub(wc, wd); // [0, 2e9)
+    return (int32_t)min(v, v - (uint32_t)MODULO);
+}
+
+// X_{r+m} from X_r with c = x^(55 m) mod P: X_{r+m}[i] = sum_k c_k Y[i-1+k]
+// over the window Y = (X_r, X_{r+1}).
+__device__ __forceinline__ int32_t ranf_jump(int32_t x, const uint32_t *__restrict__ c, int32_t *win)
+{
+    const int lane = threadIdx.x;
+    int32_t nx = ranf_next_round(x, ranf_lanes());
+    if (lane < 55) {
+        win[lane] = x;
+        win[55 + lane] = nx;
+    }
+    __syncthreads();
+    uint64_t acc = 0;
+    if (lane < 55) {
+#pragma unroll 5
+        for (int k = 0; k < 55; ++k) {
+            acc += (uint64_t)c[k] * (uint64_t)(uint32_t)win[lane + k];
+            if ((k & 15) == 15)
+                acc %= (uint64_t)MODULO;
+        }
+        acc %= (uint64_t)MODULO;
+    }
+    __syncthreads();
+    return lane < 55 ? (int32_t)acc : 0;
+}
+
+// X_{r+e} from X_r for a number of rounds e all lanes hold alike.  win: 110
+// ints of LDS, free before and after.
+__device__ __forceinline__ int32_t ranf_advance(int32_t x, const uint32_t *__restrict__ r16, uint64_t e, int32_t *win)
+{
+    for (; e; e >>= 4, r16 += 15 * 55)
+        if (e & 15u)
+            x = ranf_jump(x, r16 + 55 * ((uint32_t)(e & 15u) - 1), win);
+    return x;
+}
+
+// What bounds a round: a chain of one LDS permute and nine dependent integer
+// instructions, about 180 cycles, which three wavefronts per SIMD hide behind
+// the events (14 rounds of about 48 issue cycles for 64 events of 2500).
+// Against a stream expanded into HBM first, 48 bytes an event written and read
+// again: 1e9 events 43.4 -> 28.3 ms with the event loop's own gains, the
+// expansion having been 10.4 ms of them; 1e7 events 586 -> 414 us.
+//
+// The next `need` (at most 768) values of the stream into ring[0 ..] in
+// stream order: lane l holds X[l + 1] of the current round in x, whose next
+// unread value is its o-th (X[55 - o], o up to 55).  Rounds are written whole,
+// values past `need` (below ring[need + 54]) and lanes with nothing to write
+// (to ring[dump]) included.
+__device__ __forceinline__ void ranf_fill(int32_t &x, uint32_t &o, uint32_t need, int32_t *ring, uint32_t dump,
+                                          const RanfLanes &l)
+{
+    const int lane = (int)(threadIdx.x & 63u), at = 54 - lane - (int)o;
+    ring[lane < 55 && at >= 0 ? (uint32_t)at : dump] = x;
+    uint32_t p = lane < 55 ? (uint32_t)(at + 55) : dump;
+    const uint32_t step = lane < 55 ? 55u : 0u, rounds = (o + need + 54) / 55 - 1;
+    for (uint32_t r = 0; r < rounds; ++r) {
+        x = ranf_next_round(x, l);
+        ring[p] = x;
+        p += step;
+    }
+    o = o + need - 55 * rounds;
+}
+
 // ---- the fused event loop ------------------------------------------------
 //
 // One wavefront per part of a batch, persistent: the grid holds as many
@@ -145,8 +248,10 @@ __device__ __forceinline__ void block_reduce_store(double v[12], uint32_t n, Dev
 // function of the data only, so results are reproducible run to run.
 //
 // Event assignment inside the part: with the in-register xoshiro stream each
-// lane owns a contiguous run (one skip-ahead per run); with a stream read
-// from HBM lane l takes events l, l+64, ... (coalesced loads).
+// lane owns a contiguous run (one skip-ahead per run); the others take events
+// l, l+64, ... in lane l.  The RANF stream is made by the wavefront as a whole,
+// 55 values a round, into LDS (ranf_fill), where each lane picks its event's 12
+// values; values read from HBM then lie side by side across the lanes.
 //
 // What bounds it: VALU issue, at the measured issue times (f64 fma 4.9 cycles,
 // add and mul 4.4, rcp and rsq 16.3, xor, mov and add_u32 2.7, shifts and
@@ -179,12 +284,21 @@ __device__ __forceinline__ const Params &fresh_params()
 template <int SOURCE, int PREC>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void fused_kernel(FusedArgs a)
 {
-    __shared__ double queue[12][QCAP];      // momenta, structure of arrays
+    // momenta, structure of arrays, slots 0..63 and 64..127; between
+    // iterations fewer than 64 events wait, so with the RANF source the upper
+    // half holds an iteration's draws until its events are pushed
+    __shared__ __align__(16) double queue[2][12][64];
+    auto slot_of = [&](uint32_t s) -> double * { return &queue[0][0][0] + (s >> 6) * (12 * 64) + (s & 63u); };
+    int32_t *ring = reinterpret_cast<int32_t *>(&queue[1][0][0]);
+    constexpr uint32_t RING_DUMP = 1400; // past the 768 + 54 values written, below the half's 1536
     __shared__ uint32_t qev[SOURCE == 2 ? QCAP : 1]; // weighted source: the event's index in the chunk
     __shared__ double red[1][13];
     const uint32_t lane = threadIdx.x;
     const uint64_t lanemask_lt = (1ull << lane) - 1ull;
     uint64_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}; // xoshiro state at the part's first draw (uniform)
+    int32_t rx = 0;      // RANF: X[lane + 1] of the current round,
+    uint32_t ro = 0;     // the place of the next unread value in it,
+    uint64_t rround = 0; // and the round's number at the end of the part
     bool have = false;
     for (uint64_t t = blockIdx.x; t < a.nb * a.parts; t += gridDim.x) {
         const uint64_t lb = a.parts == 1 ? t : t / a.parts;
@@ -209,7 +323,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
             len = n / 64 + (lane < n % 64 ? 1u : 0u); // events lane, lane+64, ...
             iters = (n + 63) / 64;
         }
-        const int32_t *src = (SOURCE == 1) ? a.draws + 12 * ((size_t)lb * a.batch_size + first) : nullptr;
+        const RanfLanes rl = ranf_lanes();
+        if (SOURCE == 1 && n) {
+            const bool own = a.rorigin && b > 0;
+            const uint64_t q = (own ? 0 : a.rp0) + 12ull * (first + (a.rorigin ? 0 : b * a.batch_size));
+            uint64_t skip = q / 55;
+            if (have && a.rjump_rounds && rround + a.rjump_rounds <= skip) { // on from the previous part
+                rx = ranf_jump(rx, a.rjump, ring);
+                skip -= rround + a.rjump_rounds;
+            } else {
+                rx = lane < 55 ? (own ? a.rorigin[56 * b + lane + 1] : a.rround[lane + 1]) : 0;
+            }
+            if (skip < 4) // (a round costs a twentieth of a jump)
+                for (; skip; --skip)
+                    rx = ranf_next_round(rx, rl);
+            rx = ranf_advance(rx, a.r16, skip, ring);
+            ro = (uint32_t)(q % 55);
+            // the round the part leaves in rx (ranf_fill stops at the last one it reads)
+            rround = (q + 12ull * n - 1) / 55;
+            have = true;
+        }
         const size_t wbase = (size_t)lb * a.batch_size + first;
         const RerollBits rb{a.acc1, a.bbase, a.bstride ? (lb + 1) * a.bstride : a.blimit};
         Acc<PREC> A;
@@ -224,6 +357,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
             const uint64_t qk = qnext;
             if (FE && k + 1 < len)
                 qnext = a.evq[wbase + (size_t)((k + 1) * 64 + lane)];
+            int4 rd[3]; // RANF: the lane's 12 draws
+            if (SOURCE == 1) {
+                ranf_fill(rx, ro, 12 * min(64u, n - 64 * k), ring, RING_DUMP, rl);
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    rd[j] = reinterpret_cast<const int4 *>(ring)[3 * lane + j];
+                __syncthreads(); // read before the events are pushed
+            }
             if (k < len && SOURCE == 3) {
                 RanfWalk w{a.draws, a.qbase, qk, rb};
                 pass = generate_faster_f64(fresh_params(), w, p);
@@ -237,10 +379,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                     for (int j = 0; j < 12; ++j)
                         u[j] = xo_uniform64(s);
                 } else if (SOURCE == 1) {
-                    const int32_t *e = src + 12 * (size_t)(k * 64 + lane);
 #pragma unroll
-                    for (int j = 0; j < 12; ++j)
-                        u[j] = (double)e[j] * 1e-9;
+                    for (int j = 0; j < 3; ++j) {
+                        u[4 * j] = (double)rd[j].x * 1e-9;
+                        u[4 * j + 1] = (double)rd[j].y * 1e-9;
+                        u[4 * j + 2] = (double)rd[j].z * 1e-9;
+                        u[4 * j + 3] = (double)rd[j].w * 1e-9;
+                    }
                 } else {
                     const size_t e = wbase + (size_t)(k * 64 + lane);
 #pragma unroll
@@ -259,7 +404,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                 for (int i = 0; i < 3; ++i)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        queue[4 * d[i] + j][slot] = p[i][j];
+                        slot_of(slot)[64 * (4 * d[i] + j)] = p[i][j];
                 if (SOURCE == 2)
                     qev[slot] = (uint32_t)(wbase + (size_t)(k * 64 + lane));
             }
@@ -272,7 +417,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                 for (int i = 0; i < 3; ++i)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        pq[i][j] = queue[4 * i + j][slot];
+                        pq[i][j] = slot_of(slot)[64 * (4 * i + j)];
                 const double wq = SOURCE == 2 ? a.invq[qev[slot]] : 1.;
                 __syncthreads();
                 qn -= 64;
@@ -292,7 +437,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                 for (int i = 0; i < 3; ++i)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        pq[i][j] = queue[4 * i + j][lane];
+                        pq[i][j] = slot_of(lane)[64 * (4 * i + j)];
                 matrix_elements<PREC>(fresh_params(), pq, m);
                 if (SOURCE == 2) {
                     const double wq = a.invq[qev[lane]];
@@ -519,80 +664,6 @@ void launch_events(const FusedArgs &a, int source, uint32_t n, const EventOut &o
 }
 
 // ---- RANF expansion ------------------------------------------------------
-constexpr int32_t MODULO = 1000000000;
-
-__device__ __forceinline__ int32_t norm_mod(int32_t v)
-{
-    v += (v < 0) ? MODULO : 0;
-    v += (v < 0) ? MODULO : 0;
-    v -= (v >= MODULO) ? MODULO : 0;
-    v -= (v >= MODULO) ? MODULO : 0;
-    return v;
-}
-
-// One RANF round in closed form (lane i - 1 holds X[i], i = 1..55):
-//   i <= 24:  X'[i] = X[i] - X[i+31]
-//   25..48:   X'[i] = X[i] - X'[i-24] = X[i] - X[i-24] + X[i+7]
-//   49..55:   X'[i] = X[i] - X[i-24] + X[i-48] - X[i-17]
-// (ranf.rs:106-119 applies the first two lines as in-place updates; the third
-// is the second with X'[i-24] expanded once more), all mod 1e9.  Every lane
-// evaluates (X[i] - b) + (c - d) with b, c, d read from other lanes of the
-// same wave by ds_bpermute (no LDS storage, no barrier).  Lanes 55..63 hold 0
-// and keep it, so a term a case does not have reads lane 63; each value is the
-// unique representative in [0, 1e9), so the sum order does not matter.  The
-// whole wave must be active: one wave holds one window.
-__device__ __forceinline__ uint32_t mod_sub(uint32_t a, uint32_t b) // (a - b) mod 1e9, a, b in [0, 1e9)
-{
-    const uint32_t t = a - b;
-    return min(t, t + (uint32_t)MODULO);
-}
-struct RanfLanes { // byte addresses for ds_bpermute of the lanes a lane reads
-    int b, c, d;
-};
-__device__ __forceinline__ RanfLanes ranf_lanes()
-{
-    const int lane = (int)(threadIdx.x & 63u), i = lane + 1;
-    const bool live = lane < 55;
-    RanfLanes l;
-    l.b = (live ? (i <= 24 ? i + 30 : i - 25) : 63) << 2;          // X[i+31] or X[i-24]
-    l.c = (live && i > 24 ? (i <= 48 ? i + 6 : i - 49) : 63) << 2; // X[i+7] or X[i-48]
-    l.d = (live && i > 48 ? i - 18 : 63) << 2;                     // X[i-17]
-    return l;
-}
-__device__ __forceinline__ int32_t ranf_next_round(int32_t x, const RanfLanes &l)
-{
-    const uint32_t wb = (uint32_t)__builtin_amdgcn_ds_bpermute(l.b, x);
-    const uint32_t wc = (uint32_t)__builtin_amdgcn_ds_bpermute(l.c, x);
-    const uint32_t wd = (uint32_t)__builtin_amdgcn_ds_bpermute(l.d, x);
-    const uint32_t v = mod_sub((uint32_t)x, wb) + mod_sub(wc, wd); // [0, 2e9)
-    return (int32_t)min(v, v - (uint32_t)MODULO);
-}
-
-// X_{r+m} from X_r with c = x^(55 m) mod P: X_{r+m}[i] = sum_k c_k Y[i-1+k]
-// over the window Y = (X_r, X_{r+1}).
-__device__ __forceinline__ int32_t ranf_jump(int32_t x, const uint32_t *__restrict__ c, int32_t *win)
-{
-    const int lane = threadIdx.x;
-    int32_t nx = ranf_next_round(x, ranf_lanes());
-    if (lane < 55) {
-        win[lane] = x;
-        win[55 + lane] = nx;
-    }
-    __syncthreads();
-    uint64_t acc = 0;
-    if (lane < 55) {
-#pragma unroll 5
-        for (int k = 0; k < 55; ++k) {
-            acc += (uint64_t)c[k] * (uint64_t)(uint32_t)win[lane + k];
-            if ((k & 15) == 15)
-                acc %= (uint64_t)MODULO;
-        }
-        acc %= (uint64_t)MODULO;
-    }
-    __syncthreads();
-    return lane < 55 ? (int32_t)acc : 0;
-}
-
 // Outcome of the unit-disc test on the point (x, y) = 2u - 1 of two
 // uniforms: r2 above 1 re-rolls, and in f64 so does r2 below MIN_POSITIVE^2
 // (f32's MIN_POSITIVE^2 is 0).  The walk sums (0 + x*x) + y*y for the six
@@ -714,9 +785,7 @@ template <int BITS> __global__ __launch_bounds__(64) void ranf_expand_kernel(Ran
     if (r_begin * 55 >= q_end)
         return; // whole workgroup
     int32_t x = lane < 55 ? a.origin[56 * piece + lane + 1] : 0;
-    for (int k = 0; k < a.K; ++k)
-        if ((seg >> k) & 1ull)
-            x = ranf_jump(x, a.polys + 55 * k, win);
+    x = ranf_advance(x, a.r16, seg * (uint64_t)a.R, win);
     int32_t *out = a.out + piece * a.piece_stride;
     const RanfLanes l = ranf_lanes();
     __shared__ uint64_t bm[2][BITS ? 32 : 1];

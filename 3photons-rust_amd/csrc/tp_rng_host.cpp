@@ -54,29 +54,57 @@ void ranf_seeded(RanfState &g, int32_t seed)
         ranf_round(g.numbers);
 }
 
-static inline uint64_t mulmod(uint64_t a, uint64_t b) { return (a * b) % RANF_MODULO; }
-
 RanfPoly ranf_poly_mul(const RanfPoly &a, const RanfPoly &b)
 {
-    // Product of degree <= 108, then reduce with x^55 = 1 - x^31.
+    // Product of degree <= 108 (sums of 16 products below 1e18 fit 64 bits),
+    // then reduced with x^55 = 1 - x^31.
     uint64_t prod[109] = {0};
     for (int i = 0; i < 55; ++i) {
-        if (!a[i])
-            continue;
         for (int j = 0; j < 55; ++j)
-            prod[i + j] = (prod[i + j] + mulmod(a[i], b[j])) % RANF_MODULO;
+            prod[i + j] += static_cast<uint64_t>(a[i]) * b[j];
+        if (i % 16 == 15 || i == 54)
+            for (uint64_t &v : prod)
+                v %= RANF_MODULO;
     }
     for (int d = 108; d >= 55; --d) {
-        uint64_t c = prod[d];
-        if (!c)
-            continue;
-        prod[d] = 0;
+        const uint64_t c = prod[d];
         prod[d - 55] = (prod[d - 55] + c) % RANF_MODULO;
         prod[d - 24] = (prod[d - 24] + RANF_MODULO - c) % RANF_MODULO;
     }
     RanfPoly r(55);
     for (int i = 0; i < 55; ++i)
         r[i] = static_cast<uint32_t>(prod[i]);
+    return r;
+}
+
+const std::vector<uint32_t> &ranf_round_digits()
+{
+    static std::vector<uint32_t> tab;
+    static std::once_flag once;
+    std::call_once(once, [] {
+        RanfPoly base = ranf_poly_xpow(55); // x^(55 16^j)
+        for (int j = 0; j < RANF_DIGITS; ++j) {
+            RanfPoly q = base;
+            for (int v = 1; v < 16; ++v) {
+                tab.insert(tab.end(), q.begin(), q.end());
+                q = ranf_poly_mul(q, base);
+            }
+            base = q;
+        }
+    });
+    return tab;
+}
+
+RanfPoly ranf_poly_rounds(uint64_t rounds)
+{
+    const std::vector<uint32_t> &t = ranf_round_digits();
+    RanfPoly r(55, 0);
+    r[0] = 1;
+    for (size_t at = 0; rounds; rounds >>= 4, at += 15 * 55)
+        if (rounds & 15u) {
+            const auto q = t.begin() + at + 55 * ((rounds & 15u) - 1);
+            r = ranf_poly_mul(r, RanfPoly(q, q + 55));
+        }
     return r;
 }
 
@@ -96,7 +124,7 @@ RanfPoly ranf_poly_xpow(uint64_t n)
     return result;
 }
 
-void ranf_apply_round_jump(const RanfPoly &c, const int32_t *x_in, int32_t *x_out)
+void ranf_apply_round_jump(const uint32_t *c, const int32_t *x_in, int32_t *x_out)
 {
     // Window Y[0..109] = X_r[1..55], X_{r+1}[1..55]; X_{r+m}[i] = sum_k c_k Y[i-1+k].
     int32_t next[56];
@@ -107,13 +135,17 @@ void ranf_apply_round_jump(const RanfPoly &c, const int32_t *x_in, int32_t *x_ou
         y[i] = static_cast<uint64_t>(x_in[i + 1]);
         y[55 + i] = static_cast<uint64_t>(next[i + 1]);
     }
-    x_out[0] = 0;
-    for (int i = 0; i < 55; ++i) {
-        uint64_t acc = 0;
-        for (int k = 0; k < 55; ++k)
-            acc = (acc + mulmod(c[k], y[i + k])) % RANF_MODULO;
-        x_out[i + 1] = static_cast<int32_t>(acc);
+    uint64_t acc[55] = {0};
+    for (int k = 0; k < 55; ++k) {
+        for (int i = 0; i < 55; ++i)
+            acc[i] += c[k] * y[i + k];
+        if (k % 8 == 7 || k == 54)
+            for (uint64_t &v : acc)
+                v %= RANF_MODULO;
     }
+    x_out[0] = 0;
+    for (int i = 0; i < 55; ++i)
+        x_out[i + 1] = static_cast<int32_t>(acc[i]);
 }
 
 void ranf_advance(RanfState &g, uint64_t n)
@@ -124,10 +156,13 @@ void ranf_advance(RanfState &g, uint64_t n)
     }
     uint64_t rest = n - g.index;
     uint64_t rounds = (rest + 54) / 55;
-    RanfPoly c = ranf_poly_xpow(55 * rounds);
+    const uint32_t *tab = ranf_round_digits().data(); // of the hexadecimal digits of `rounds`
     int32_t out[56];
-    ranf_apply_round_jump(c, g.numbers, out);
-    std::memcpy(g.numbers, out, sizeof out);
+    for (uint64_t e = rounds; e; e >>= 4, tab += 15 * 55)
+        if (e & 15u) {
+            ranf_apply_round_jump(tab + ((e & 15u) - 1) * 55, g.numbers, out);
+            std::memcpy(g.numbers, out, sizeof out);
+        }
     g.index = static_cast<uint32_t>(55 * rounds - rest);
 }
 

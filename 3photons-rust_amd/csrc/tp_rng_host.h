@@ -35,8 +35,13 @@ void ranf_round(int32_t *numbers /*[56]*/);       // IRN55 (ranf.rs:106-119)
 using RanfPoly = std::vector<uint32_t>; // 55 coefficients, c[k] of x^k
 RanfPoly ranf_poly_xpow(uint64_t n);       // x^n mod P
 RanfPoly ranf_poly_mul(const RanfPoly &a, const RanfPoly &b);
-// Apply a jump polynomial (x^(55 m)) to the round X[1..55]: returns X_{r+m}.
-void ranf_apply_round_jump(const RanfPoly &c, const int32_t *x_in /*[56]*/, int32_t *x_out /*[56]*/);
+// Apply a jump polynomial (x^(55 m), 55 coefficients) to the round X[1..55]: returns X_{r+m}.
+void ranf_apply_round_jump(const uint32_t *c, const int32_t *x_in /*[56]*/, int32_t *x_out /*[56]*/);
+// x^(55 v 16^j) mod P at [55 (15 j + v - 1) ..], v = 1..15, for the hexadecimal
+// digits j < RANF_DIGITS of a number of rounds (built once, cached).
+constexpr int RANF_DIGITS = 15;
+const std::vector<uint32_t> &ranf_round_digits();
+RanfPoly ranf_poly_rounds(uint64_t rounds); // x^(55 rounds) mod P, from those
 // Advance a generator state by n single draws (same effect as n random()).
 void ranf_advance(RanfState &g, uint64_t n);
 
