@@ -44,7 +44,7 @@ struct Tables { // device copy of the powers 2^k of a GF(2) matrix
     int kb = 0;
 };
 
-// xoshiro256+ skip tables of one device, filled once by the first tp_create on
+// xoshiro skip tables of one device, filled once by the first tp_create on
 // it and only read afterwards (tp_kernels.h).
 struct XoTables {
     int rc = TP_ERR_INTERNAL;
@@ -52,6 +52,7 @@ struct XoTables {
     const uint64_t *m16 = nullptr;     // M^(v 16^j), M one draw
     const uint64_t *b16[2] = {nullptr, nullptr}; // B^(v 16^j): M^(12 * 10 000), the 2^128 jump (by seeding)
     const uint64_t *lanes = nullptr;   // lane tables of every run length
+    const uint32_t *m16_128 = nullptr, *b16_128[2] = {nullptr, nullptr}, *lanes128 = nullptr; // the same of xoshiro128+
 };
 
 struct Ctx {
@@ -59,6 +60,7 @@ struct Ctx {
     const XoTables *xo = nullptr;
     int cus = 1;                    // compute units of the device
     int blocks_per_cu[5][2] = {{1, 1}, {1, 1}, {1, 1}, {1, 1}, {1, 1}}; // resident fused workgroups per CU [source][precision]
+    int f32_blocks[4] = {1, 1, 1, 1}; // resident all-f32 wavefronts per CU [source]
     hipStream_t stream = nullptr;
     hipEvent_t ev[5] = {nullptr, nullptr, nullptr, nullptr, nullptr}; // [4]: the device walk's status copy
     std::string err;
@@ -69,11 +71,7 @@ struct Ctx {
     bool r16_ready = false;
     DevBuf draws, origin, p0, per_batch, merged, evq;
     DevBuf parts; // sums of the parts of split batches (MAX_PARTS), allocated by tp_create
-    DevBuf mt128, bt128, f32ev; // all-f32 mode: xoshiro128+ tables, per-event values
-    std::string bt128_key;
-    int bt128_kb = 0;
-    DevBuf st128;               // all-f32 mode: B^grid, the grid-stride advance
-    std::string st128_key;
+    DevBuf f32ev, f32cnt;       // all-f32 mode: per-event values, accepted events of the parts
     tp_stats last{};
     bool timed = false;
     // Host staging of the RANF origin: must outlive the asynchronous copies.
@@ -106,11 +104,6 @@ struct Ctx {
 
 constexpr int KM = 32;              // intra-call offsets < 2^32 draws
 constexpr int RANF_R = 2048;        // RANF rounds per expansion segment (one jump per segment)
-// Batches per RANF expansion + event-loop launch: two full strides of the
-// 3072-wavefront persistent grid (one wavefront per batch), so no launch ends
-// on a partly idle stride; 6144 * 120000 int32 = 2.95 GB of stream.
-constexpr uint64_t RANF_CHUNK_BATCHES = 6144;
-
 // Where tp_guard stores an exception's message for tp_last_error.
 inline std::string *ctx_err(void *ctx) { return ctx ? &static_cast<Ctx *>(ctx)->err : nullptr; }
 
@@ -152,65 +145,160 @@ struct Split {
     int grid;
 };
 constexpr uint64_t MAX_PARTS = 1u << 16;
-// The run length with the least estimated time.  A wavefront takes `run`
-// iterations and a start-up of about 2 (the xoshiro stream's skip; half an
-// iteration for streams read from memory).  `slots` wavefronts are resident at
-// once and share 4 SIMDs per CU: a SIMD with one wavefront spends 1.4 times
-// the issue time of an iteration (measured: 4900 cycles against 3400), one
-// with several their sum.  So 1000 batches take 2 parts each rather than leave
-// two wavefronts of three idle, 10 000 take 4 rather than fill a fourth round
-// of 3072 to a quarter, and one closure call takes a part per 64 events.
-inline Split split_for(const Ctx *c, int source, int precision, uint64_t nb, uint32_t n)
+// What a kernel's part costs, in issue times of one of its iterations (64
+// events): `startup` iterations a part, and `wait` for latencies that other
+// wavefronts do not cover, once where the SIMDs' issue is the bound (wavefronts
+// that finish early leave their SIMD's time to the others), or `per_round` of
+// resident wavefronts where loads are.  `join` is the kernel that joins the
+// parts' sums, per `join_batches` batches, `most` the parts it takes; a split
+// has to take less than `gain` of the unsplit time.
+struct PartCost {
+    double startup, wait;
+    bool per_round;
+    double gain = 1.;
+    uint64_t most = MAX_PARTS;
+    double join = 0.;
+    uint64_t join_batches = 1;
+};
+// Measured at 100 to 10 000 batches with every run length.  A wavefront with a
+// SIMD to itself takes 1.45 of an iteration's issue time (RANF, 1000 batches:
+// 481 us in one part each, 405 in two, 381 in three, 368 in four, 378 in eight),
+// a part some 3.5 iterations beside its events (10 000 batches: 2.53 ms whole,
+// 2.72 in two parts); event loops that read their draws from HBM wait 2.6
+// iterations a round (faster-evgen, 1000 batches: 780 us whole, 540 in two
+// parts, 414 in three, which fill the chip once, 478 in four); the weighted
+// loop's rows of uniforms come in best in long runs (2000 batches: 4.12 ms whole
+// with the flow, 4.21 in two parts; 1000: 2.20 and 2.11); the all-f32 loop waits
+// 0.8, its separate sums take 42 us per 1536 batches (1000 batches: 560 us in
+// two parts, 494 in four, 475 in eight; 10 000: 3.13 ms whole, 3.72 in three).
+inline PartCost event_part_cost(int source)
 {
-    const uint64_t simds = 4ull * c->cus, slots = (uint64_t)c->cus * c->blocks_per_cu[source][precision];
+    return source < 2 ? PartCost{3.5, 0.45, false} : source == 2 ? PartCost{3.5, 0.45, false, 0.85} : PartCost{1.5, 2.6, true};
+}
+inline PartCost f32_part_cost(int source)
+{
+    return source == 0   ? PartCost{4., 0.8, false}
+           : source == 1 ? PartCost{1., 0.8, false, 1., tpk::F32_MAX_PARTS, 21., 1536}
+                         : PartCost{1., 2.6, true, 1., tpk::F32_MAX_PARTS, 21., 1536};
+}
+// The run length with the least estimated time for nb batches of n events on
+// `blocks` resident wavefronts per CU.  lane_runs: a lane takes consecutive
+// events, so a short batch leaves lanes idle.
+inline Split split_for(uint64_t cus, uint64_t blocks, uint64_t nb, uint32_t n, bool lane_runs, const PartCost &k)
+{
+    const uint64_t simds = 4 * cus, slots = cus * blocks;
+    auto up = [&](uint64_t tasks) { return (double)((tasks + simds - 1) / simds); };
     Split best{0, 0, 0};
     double least = 0.;
     for (uint32_t run : tpk::XO_RUNS) {
         const uint64_t parts = (n + 64ull * run - 1) / (64ull * run), tasks = nb * parts;
-        if (parts > 1 && (parts > slots || tasks > MAX_PARTS))
+        if (parts > 1 && (parts > std::min(slots, k.most) || tasks > MAX_PARTS))
             continue;
-        const uint64_t iters = source == 0 ? std::min(run, n) : std::min<uint64_t>(run, (n + 63) / 64);
+        const uint64_t iters = lane_runs ? std::min(run, n) : std::min<uint64_t>(run, (n + 63) / 64);
         const uint64_t rest = tasks % slots;
-        const double turns = (double)(tasks / slots) * ((double)slots / (double)simds) +
-                             (rest ? std::max(1.4, (double)((rest + simds - 1) / simds)) : 0.);
-        const double cost = ((double)iters + (source == 0 ? 2. : 0.5)) * turns;
-        if (!best.parts || cost < least) {
+        const double turns = !k.per_round ? up(tasks) + k.wait
+                                          : (double)(tasks / slots) * ((double)slots / (double)simds + k.wait) +
+                                                (rest ? up(rest) + k.wait : 0.);
+        double cost = ((double)iters + k.startup) * turns;
+        if (parts > 1)
+            cost += k.join * (double)((nb + k.join_batches - 1) / k.join_batches);
+        if (!best.parts || cost < least * (best.parts == 1 ? k.gain : 1.)) {
             least = cost;
             // a wavefront that takes several parts keeps its place in the batch
             best = Split{(uint32_t)parts, run, (int)std::min(tasks, slots / parts * parts)};
         }
     }
-    if (!best.parts) // batches of more than 64 * 157 events, in more parts than are resident
+    if (!best.parts) // no split within the limits
         best = Split{1, (n + 63) / 64, (int)std::min(nb, slots)};
     return best;
+}
+inline Split split_for(const Ctx *c, int source, int precision, uint64_t nb, uint32_t n)
+{
+    return split_for((uint64_t)c->cus, (uint64_t)c->blocks_per_cu[source][precision], nb, n, source == 0,
+                     event_part_cost(source));
+}
+inline Split split_for_f32(const Ctx *c, int source, uint64_t nb, uint32_t n)
+{
+    return split_for((uint64_t)c->cus, (uint64_t)c->f32_blocks[source], nb, n, source == 0, f32_part_cost(source));
+}
+
+// The jump of a wavefront that strides over parts of the one RANF stream.
+inline void set_ranf_jump(tpk::RanfSource &R, const Split &s, uint64_t nb, uint32_t batch_size, uint32_t n)
+{
+    R.jump_rounds = 0;
+    if (R.origin || nb * s.parts <= (uint64_t)s.grid)
+        return;
+    // the least number of rounds from the last one of a part to the first of
+    // the wavefront's next (a part of whole runs: that or one more)
+    const uint64_t stride = 12ull * batch_size * (s.grid / s.parts), part = 12ull * std::min<uint64_t>(64ull * s.run, n);
+    R.jump_rounds = (stride - part + 1) / 55;
+    const tp::RanfPoly q = tp::ranf_poly_rounds(R.jump_rounds);
+    std::copy(q.begin(), q.end(), R.jump);
+}
+
+// The lane table of a run length, or null if there is none (split_for picks a
+// run of XO_RUNS for every batch of up to 64 * 157 * the resident wavefronts).
+inline const uint32_t *xo_lane_table(const uint32_t *lanes, size_t words, uint32_t run)
+{
+    for (int i = 0; i < tpk::XO_NRUNS; ++i)
+        if (tpk::XO_RUNS[i] == run)
+            return lanes + i * words;
+    return nullptr;
 }
 
 // The event loop on a.nb batches of n events, split as split_for says, with
 // the batches' sums in a.out.
-inline void launch_event_loop(const Ctx *c, tpk::FusedArgs &a, int source, uint32_t n)
+inline int launch_event_loop(Ctx *c, tpk::FusedArgs &a, int source, uint32_t n)
 {
     const Split s = split_for(c, source, a.precision, a.nb, n);
     a.parts = s.parts;
     a.run = s.run;
     a.part_out = c->parts.p;
-    if (source == 0) {
-        a.lanes = nullptr;
-        for (int i = 0; i < tpk::XO_NRUNS; ++i)
-            if (tpk::XO_RUNS[i] == s.run)
-                a.lanes = c->xo->lanes + (size_t)i * tpk::XO_LANE_WORDS;
-    }
-    a.rjump_rounds = 0;
-    const uint64_t stride = 12ull * a.batch_size * (s.grid / s.parts), part = 12ull * std::min<uint64_t>(64ull * s.run, n);
-    if (source == 1 && !a.rorigin && a.nb * s.parts > (uint64_t)s.grid) {
-        // the least number of rounds from the last one of a part to the first
-        // of the wavefront's next (a part of whole runs: that or one more)
-        a.rjump_rounds = (stride - part + 1) / 55;
-        const tp::RanfPoly q = tp::ranf_poly_rounds(a.rjump_rounds);
-        std::copy(q.begin(), q.end(), a.rjump);
-    }
+    if (source == 0)
+        a.lanes = reinterpret_cast<const uint64_t *>(
+            xo_lane_table(reinterpret_cast<const uint32_t *>(c->xo->lanes), 2 * tpk::XO_LANE_WORDS, s.run));
+    if (source == 0 && !a.lanes)
+        return fail(c, TP_ERR_INTERNAL, "no lane table for this batch size");
+    if (source == 1)
+        set_ranf_jump(a.ranf, s, a.nb, a.batch_size, n);
     tpk::launch_fused(a, source, s.grid, c->stream);
-    if (s.parts > 1)
+    HIPCHK(c, hipGetLastError());
+    if (s.parts > 1) {
         tpk::launch_batch_sums(a, c->stream);
+        HIPCHK(c, hipGetLastError());
+    }
+    return TP_OK;
+}
+
+// The same in the all-f32 mode, with the sums in event order.
+inline int launch_f32_batches(Ctx *c, tpk::F32Args &a, uint32_t n)
+{
+    const Split s = split_for_f32(c, a.source, a.nb, n);
+    a.parts = s.parts;
+    a.run = s.run;
+    if (a.source == 0)
+        a.lanes = xo_lane_table(c->xo->lanes128, tpk::XO128_LANE_WORDS, s.run);
+    if (a.source == 0 && !a.lanes)
+        return fail(c, TP_ERR_INTERNAL, "no lane table for this batch size");
+    if (a.source == 1)
+        set_ranf_jump(a.ranf, s, a.nb, a.batch_size, n);
+    if (!tpk::f32_sums_in_kernel(a)) {
+        a.ev_stride = a.nb * a.batch_size;
+        int rc = ensure(c, c->f32ev, a.ev_stride * (a.source == 0 ? 6 : 5) * sizeof(float));
+        if (!rc)
+            rc = ensure(c, c->f32cnt, a.nb * a.parts * sizeof(uint32_t));
+        if (rc)
+            return rc;
+        a.ev = static_cast<float *>(c->f32ev.p);
+        a.counts = static_cast<uint32_t *>(c->f32cnt.p);
+    }
+    tpk::launch_f32_events(a, s.grid, c->stream);
+    HIPCHK(c, hipGetLastError());
+    if (!tpk::f32_sums_in_kernel(a)) {
+        tpk::launch_f32_accumulate(a, c->stream);
+        HIPCHK(c, hipGetLastError());
+    }
+    return TP_OK;
 }
 
 // Device-side constants of a run, computed exactly as the reference does on

@@ -129,25 +129,6 @@ using namespace tpe;
 
 int bits_for(uint64_t n);
 
-// xoshiro128+ skip-ahead tables for the all-f32 mode: M^(2^k) (k < KM128:
-// a lane's draw offset inside its batch, below 12 * batch_size) and B^(2^k)
-// with B = M^(12 batch_size) or the 2^64 jump.  The largest batch is one
-// tp_simulate_batch call of 640 000 events: offsets below 7 680 000 < 2^23.
-constexpr int KM128 = 24;
-static_assert(12ull * 64 * TP_BATCH_SIZE < (1ull << KM128), "xoshiro128+ offset table too short");
-
-int ensure_mt128(Ctx *c)
-{
-    if (!c->mt128.p) {
-        const std::vector<tp::Gf2Mat128> &t = tp::xoshiro128_step_pow2();
-        int rc = ensure(c, c->mt128, KM128 * sizeof(tp::Gf2Mat128));
-        if (rc)
-            return rc;
-        HIPCHK(c, hipMemcpy(c->mt128.p, t.data(), KM128 * sizeof(tp::Gf2Mat128), hipMemcpyHostToDevice));
-    }
-    return TP_OK;
-}
-
 // B^(2^k), k < kb, of the xoshiro128+ piece matrix B (the 2^64 jump, or
 // M^piece_len for pieces tiling one stream), into c->xo128_pt.
 int ensure_xo128_piece_table(Ctx *c, bool jump, uint64_t piece_len, uint64_t max_piece)
@@ -172,73 +153,27 @@ int ensure_xo128_piece_table(Ctx *c, bool jump, uint64_t piece_len, uint64_t max
     return TP_OK;
 }
 
-int ensure_tables128(Ctx *c, int seeding, uint32_t batch_size, uint64_t nb, int grid, DevBuf **bt_out, int *kb_out)
-{
-    int rc0 = ensure_mt128(c);
-    if (rc0)
-        return rc0;
-    const int kb = std::max(1, bits_for(nb));
-    const std::string key = std::to_string(seeding) + ":" + std::to_string(batch_size);
-    if (c->bt128_key != key || c->bt128_kb < kb) {
-        tp::Gf2Mat128 B;
-        if (seeding == TP_SEED_JUMP)
-            tp::gf2_128_jump64(B);
-        else
-            tp::gf2_128_pow_from_table(tp::xoshiro128_step_pow2(), 12ull * batch_size, B);
-        const std::vector<tp::Gf2Mat128> bt = tp::gf2_128_pow2_table(B, kb);
-        int rc = ensure(c, c->bt128, bt.size() * sizeof(tp::Gf2Mat128));
-        if (rc)
-            return rc;
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        HIPCHK(c, hipMemcpy(c->bt128.p, bt.data(), bt.size() * sizeof(tp::Gf2Mat128), hipMemcpyHostToDevice));
-        c->bt128_key = key;
-        c->bt128_kb = kb;
-    }
-    const std::string skey = key + ":" + std::to_string(grid);
-    if (c->st128_key != skey) {
-        tp::Gf2Mat128 B, S;
-        if (seeding == TP_SEED_JUMP)
-            tp::gf2_128_jump64(B);
-        else
-            tp::gf2_128_pow_from_table(tp::xoshiro128_step_pow2(), 12ull * batch_size, B);
-        tp::gf2_128_pow_from_table(tp::gf2_128_pow2_table(B, std::max(1, bits_for((uint64_t)grid))), (uint64_t)grid, S);
-        int rc = ensure(c, c->st128, sizeof S);
-        if (rc)
-            return rc;
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        HIPCHK(c, hipMemcpy(c->st128.p, &S, sizeof S, hipMemcpyHostToDevice));
-        c->st128_key = skey;
-    }
-    *bt_out = &c->bt128;
-    *kb_out = c->bt128_kb;
-    return TP_OK;
-}
-
-// 24576 * 10000 events * 24 B = 5.9 GB of per-event values.  The grid is 24
-// workgroups per CU (6 waves per SIMD, the occupancy the kernel's register
-// budget allows), so each lane steps through 4 batches of a full chunk by the
-// grid-stride matrix instead of a full skip-ahead per batch.
+// Batches per launch of the xoshiro128+ events in registers:
+// 24576 * 10000 events * 24 B = 5.9 GB of per-event values.
 constexpr uint64_t F32_CHUNK_BATCHES = 24576;
 
-int f32_grid(const Ctx *c, uint64_t nb) { return (int)std::max<uint64_t>(1, std::min<uint64_t>(nb, 24ull * c->cus)); }
+int xo_tables(Ctx *c)
+{
+    if (!c->xo || c->xo->rc != TP_OK)
+        return fail(c, c->xo ? c->xo->rc : TP_ERR_UNSUPPORTED,
+                    "xoshiro table set-up failed: " + (c->xo ? c->xo->err : std::string("device ordinal above 63")));
+    return TP_OK;
+}
 
 // All-f32 run with the xoshiro128+ stream.
 int enqueue_xo128_f32(Ctx *c, const tp_params *params, int seeding, const tp_xoshiro128_state *x,
                       uint64_t num_events, uint32_t batch_size, void *per_batch_dev)
 {
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
-    if (12ull * batch_size >= (1ull << KM128))
-        return fail(c, TP_ERR_ARG, "all-f32 batch exceeds the xoshiro128+ offset range");
-    DevBuf *bt = nullptr;
-    int kb = 0;
-    const int sgrid = f32_grid(c, F32_CHUNK_BATCHES);
-    int rc = ensure_tables128(c, seeding, batch_size, nb, sgrid, &bt, &kb);
+    int rc = xo_tables(c);
     if (rc)
         return rc;
     const uint64_t chunk = std::min<uint64_t>(nb, F32_CHUNK_BATCHES);
-    rc = ensure(c, c->f32ev, chunk * batch_size * 6 * sizeof(float));
-    if (rc)
-        return rc;
     tpk::F32Args a;
     std::memset(&a, 0, sizeof a);
     a.P = make_fparams(params);
@@ -246,27 +181,20 @@ int enqueue_xo128_f32(Ctx *c, const tp_params *params, int seeding, const tp_xos
     a.batch_size = batch_size;
     a.source = 0;
     std::memcpy(a.s0, x->s, sizeof a.s0);
-    a.mt = static_cast<const uint32_t *>(c->mt128.p);
-    a.km = KM128;
-    a.bt = static_cast<const uint32_t *>(bt->p);
-    a.kb = kb;
-    a.stride = static_cast<const uint32_t *>(c->st128.p);
-    a.stride_grid = sgrid;
-    a.ev = static_cast<float *>(c->f32ev.p);
+    a.m16 = c->xo->m16_128;
+    a.b16 = c->xo->b16_128[seeding];
     HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
     for (uint64_t b0 = 0; b0 < nb; b0 += chunk) {
         a.nb = std::min(nb, b0 + chunk) - b0;
         a.b_first = b0;
         a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-        tpk::launch_f32_events(a, f32_grid(c, a.nb), c->stream);
-        HIPCHK(c, hipGetLastError());
-        tpk::launch_f32_accumulate(a, f32_grid(c, a.nb), c->stream);
-        HIPCHK(c, hipGetLastError());
+        rc = launch_f32_batches(c, a, (uint32_t)std::min<uint64_t>(num_events, batch_size));
+        if (rc)
+            return rc;
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     return TP_OK;
 }
-
 
 int upload_mats(Ctx *c, DevBuf &b, const std::vector<tp::Gf2Mat> &mats)
 {
@@ -503,7 +431,6 @@ int xo128_expand(Ctx *c, const uint32_t s0[4], uint64_t b_first, uint64_t np)
     p.xbuf = static_cast<float *>(c->xo128_draws.p);
     p.acc1 = static_cast<uint32_t *>(c->xo_acc.p);
     p.acc3 = p.acc1 + c->xo_acc_words;
-    static_assert(FE_XO_PIECE < (1ull << KM128), "in-piece offsets within the step table");
     tpk::launch_xo128_expand(p, c->stream);
     HIPCHK(c, hipGetLastError());
     return TP_OK;
@@ -684,12 +611,6 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     c->fe_host_chunks = 0;
-    if (fa) {
-        int rc = ensure(c, c->f32ev, chunk * batch_size * 6 * sizeof(float));
-        if (rc)
-            return rc;
-        fa->ev = static_cast<float *>(c->f32ev.p);
-    }
     const int source = fs.kind == 2 ? 4 : 3;
     bool first = true;
     for (uint64_t b0 = 0; b0 < nb; b0 += chunk) {
@@ -736,10 +657,9 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
             fa->bstride = 0;
             fa->evq = static_cast<const uint64_t *>(c->evq.p);
             fa->out = static_cast<tp_acc *>(per_batch_dev) + b0;
-            tpk::launch_f32_events(*fa, f32_grid(c, fa->nb), c->stream);
-            HIPCHK(c, hipGetLastError());
-            tpk::launch_f32_accumulate(*fa, f32_grid(c, fa->nb), c->stream);
-            HIPCHK(c, hipGetLastError());
+            const int rc = launch_f32_batches(c, *fa, (uint32_t)std::min<uint64_t>(num_events, batch_size));
+            if (rc)
+                return rc;
         } else {
             a.nb = b1 - b0;
             a.b_first = b0;
@@ -752,8 +672,8 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
             a.bstride = 0;
             a.evq = static_cast<const uint64_t *>(c->evq.p);
             a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-            launch_event_loop(c, a, source, (uint32_t)std::min<uint64_t>(num_events, batch_size));
-            HIPCHK(c, hipGetLastError());
+            if (const int e = launch_event_loop(c, a, source, (uint32_t)std::min<uint64_t>(num_events, batch_size)))
+                return e;
         }
         if (!ok) // fe_starts is staged for the copy above
             HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -887,8 +807,6 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         rc = ensure(c, c->evq, chunk * batch_size * sizeof(uint64_t));
     if (!rc)
         rc = ensure(c, c->fe_flag, sizeof(uint32_t));
-    if (!rc && f32)
-        rc = ensure(c, c->f32ev, chunk * batch_size * 6 * sizeof(float));
     if (!rc) // each piece's bits: its segments' words, the last one cut at the piece's end
         rc = ensure_acc_words(c, (chunk + 1) * (PS / 32) + RANF_SEG_WORDS);
     if (rc)
@@ -900,7 +818,6 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         fa.num_events = num_events;
         fa.batch_size = batch_size;
         fa.source = 2;
-        fa.ev = static_cast<float *>(c->f32ev.p);
     }
     HIPCHK(c, hipStreamSynchronize(c->stream)); // previous users of the staging copies are done
     std::memcpy(c->origin0, rs->numbers, sizeof c->origin0);
@@ -984,10 +901,9 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
             fa.bstride = PS;
             fa.evq = static_cast<const uint64_t *>(c->evq.p);
             fa.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-            tpk::launch_f32_events(fa, f32_grid(c, cnb), c->stream);
-            HIPCHK(c, hipGetLastError());
-            tpk::launch_f32_accumulate(fa, f32_grid(c, cnb), c->stream);
-            HIPCHK(c, hipGetLastError());
+            rc = launch_f32_batches(c, fa, (uint32_t)std::min<uint64_t>(num_events, batch_size));
+            if (rc)
+                return rc;
             continue;
         }
         a.nb = cnb;
@@ -999,8 +915,8 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         a.bstride = PS;
         a.evq = static_cast<const uint64_t *>(c->evq.p);
         a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-        launch_event_loop(c, a, 3, (uint32_t)std::min<uint64_t>(num_events, batch_size));
-        HIPCHK(c, hipGetLastError());
+        if (const int e = launch_event_loop(c, a, 3, (uint32_t)std::min<uint64_t>(num_events, batch_size)))
+            return e;
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     HIPCHK(c, hipMemcpyAsync(&c->fe_flag_host, c->fe_flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
@@ -1096,8 +1012,8 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
             HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
             first = false;
         }
-        launch_event_loop(c, a, 4, (uint32_t)std::min<uint64_t>(num_events, batch_size));
-        HIPCHK(c, hipGetLastError());
+        if (const int e = launch_event_loop(c, a, 4, (uint32_t)std::min<uint64_t>(num_events, batch_size)))
+            return e;
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     HIPCHK(c, hipMemcpyAsync(&c->fe_flag_host, c->fe_flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
@@ -1149,11 +1065,8 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         rc = ensure(c, c->evq, chunk * batch_size * sizeof(uint64_t));
     if (!rc)
         rc = ensure(c, c->fe_flag, sizeof(uint32_t));
-    if (!rc)
-        rc = ensure(c, c->f32ev, chunk * batch_size * 6 * sizeof(float));
     if (rc)
         return rc;
-    fa.ev = static_cast<float *>(c->f32ev.p);
     c->fe_flag_host = 0;
     HIPCHK(c, hipMemcpyAsync(c->fe_flag.p, &c->fe_flag_host, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
     tpk::FeBatchWalkArgs w;
@@ -1194,10 +1107,9 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         fa.bstride = FE_XO_PIECE;
         fa.evq = w.evq;
         fa.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-        tpk::launch_f32_events(fa, f32_grid(c, cnb), c->stream);
-        HIPCHK(c, hipGetLastError());
-        tpk::launch_f32_accumulate(fa, f32_grid(c, cnb), c->stream);
-        HIPCHK(c, hipGetLastError());
+        rc = launch_f32_batches(c, fa, (uint32_t)std::min<uint64_t>(num_events, batch_size));
+        if (rc)
+            return rc;
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     HIPCHK(c, hipMemcpyAsync(&c->fe_flag_host, c->fe_flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
@@ -1212,9 +1124,9 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
 // size is one batch and uses none.)
 int xo_event_args(Ctx *c, tpk::FusedArgs &a, int seeding, uint64_t nb)
 {
-    if (!c->xo || c->xo->rc != TP_OK)
-        return fail(c, c->xo ? c->xo->rc : TP_ERR_UNSUPPORTED,
-                    "xoshiro256+ table set-up failed: " + (c->xo ? c->xo->err : std::string("device ordinal above 63")));
+    const int rc = xo_tables(c);
+    if (rc)
+        return rc;
     a.m16 = c->xo->m16;
     a.b16 = c->xo->b16[seeding];
     a.nb = nb;
@@ -1252,10 +1164,6 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         fa.num_events = num_events;
         fa.batch_size = batch_size;
         fa.source = 1;
-        rc = ensure(c, c->f32ev, std::min<uint64_t>(nb, RANF_CHUNK_BATCHES) * batch_size * 6 * sizeof(float));
-        if (rc)
-            return rc;
-        fa.ev = static_cast<float *>(c->f32ev.p);
     }
     if (rng_kind == TP_RNG_XOSHIRO && params->faster_evgen) {
         if (seeding == TP_SEED_JUMP)
@@ -1272,8 +1180,8 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
             return rc;
         a.out = per_batch_dev;
         HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-        launch_event_loop(c, a, 0, (uint32_t)std::min<uint64_t>(num_events, batch_size));
-        HIPCHK(c, hipGetLastError());
+        if (const int e = launch_event_loop(c, a, 0, (uint32_t)std::min<uint64_t>(num_events, batch_size)))
+            return e;
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         return TP_OK;
     }
@@ -1290,111 +1198,38 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     rc = ensure_r16(c);
     if (rc)
         return rc;
-    if (!f32) { // the event loop makes its draws itself
-        std::memcpy(a.rround, rs->numbers, sizeof a.rround);
-        a.rp0 = 55u - rs->index;
-        a.r16 = static_cast<const uint32_t *>(c->r16.p);
-        a.nb = nb;
-        a.b_first = 0;
-        a.out = per_batch_dev;
-        HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-        if (seeding == TP_SEED_JUMP) {
-            rc = ensure(c, c->origin, nb * 56 * sizeof(int32_t));
-            if (!rc)
-                rc = ensure(c, c->p0, nb * sizeof(int32_t));
-            if (rc)
-                return rc;
-            tpk::launch_ranf_seed(rs->seed, 0, nb, static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p),
-                                  c->stream);
-            HIPCHK(c, hipGetLastError());
-            a.rorigin = static_cast<const int32_t *>(c->origin.p);
-        }
-        HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-        launch_event_loop(c, a, 1, (uint32_t)std::min<uint64_t>(num_events, batch_size));
+    // the event loop makes its draws itself
+    tpk::RanfSource &R = f32 ? fa.ranf : a.ranf;
+    std::memcpy(R.round, rs->numbers, sizeof R.round);
+    R.p0 = 55u - rs->index;
+    R.r16 = static_cast<const uint32_t *>(c->r16.p);
+    HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+    if (seeding == TP_SEED_JUMP) {
+        rc = ensure(c, c->origin, nb * 56 * sizeof(int32_t));
+        if (!rc)
+            rc = ensure(c, c->p0, nb * sizeof(int32_t));
+        if (rc)
+            return rc;
+        tpk::launch_ranf_seed(rs->seed, 0, nb, static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p),
+                              c->stream);
         HIPCHK(c, hipGetLastError());
-        HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
-        return TP_OK;
+        R.origin = static_cast<const int32_t *>(c->origin.p);
     }
-    // All-f32 mode: the stream of a chunk of batches expanded into HBM, then
-    // its events.
-    const uint64_t chunk = std::min<uint64_t>(nb, RANF_CHUNK_BATCHES);
-    const size_t per_batch_draws = 12ull * batch_size;
-    rc = ensure(c, c->draws, chunk * per_batch_draws * sizeof(int32_t));
-    if (rc)
-        return rc;
-    rc = ensure(c, c->origin, chunk * 56 * sizeof(int32_t));
-    if (rc)
-        return rc;
-    rc = ensure(c, c->p0, chunk * sizeof(int32_t));
-    if (rc)
-        return rc;
-    // Segments needed to cover one chunk: every segment spans R rounds.
-    const uint64_t total_draws = 12ull * num_events;
-    const uint64_t p0_master = 55u - rs->index;
-    uint64_t max_rounds = (seeding == TP_SEED_JUMP) ? (per_batch_draws + 54) / 55 + 1
-                                                    : (p0_master + total_draws + 54) / 55 + 1;
-    HIPCHK(c, hipStreamSynchronize(c->stream)); // previous users of the staging copy are done
-    int32_t *origin0 = c->origin0;
-    std::memcpy(origin0, rs->numbers, sizeof c->origin0);
-    c->p00 = static_cast<int32_t>(p0_master);
-    int32_t &p00 = c->p00;
-    bool first_kernel = true;
-    for (uint64_t b0 = 0; b0 < nb; b0 += chunk) {
-        const uint64_t b1 = std::min(nb, b0 + chunk);
-        const uint64_t cnb = b1 - b0;
-        tpk::RanfArgs r;
-        std::memset(&r, 0, sizeof r);
-        r.origin = static_cast<const int32_t *>(c->origin.p);
-        r.p0 = static_cast<const int32_t *>(c->p0.p);
-        r.r16 = static_cast<const uint32_t *>(c->r16.p);
-        r.R = RANF_R;
-        r.out = static_cast<int32_t *>(c->draws.p);
-        uint64_t npieces;
-        if (seeding == TP_SEED_JUMP) {
-            tpk::launch_ranf_seed(rs->seed, b0, cnb, static_cast<int32_t *>(c->origin.p),
-                                  static_cast<int32_t *>(c->p0.p), c->stream);
-            HIPCHK(c, hipGetLastError());
-            if (b0 == 0) { // batch 0 runs on the caller's state itself
-                HIPCHK(c, hipMemcpyAsync(c->origin.p, origin0, sizeof c->origin0, hipMemcpyHostToDevice, c->stream));
-                HIPCHK(c, hipMemcpyAsync(c->p0.p, &p00, sizeof p00, hipMemcpyHostToDevice, c->stream));
-            }
-            npieces = cnb;
-            r.d_begin = 0;
-            r.d_end = per_batch_draws;
-            r.seg_first = 0;
-            r.piece_stride = per_batch_draws;
-            r.nsegs = ((uint64_t)(max_rounds) + RANF_R - 1) / RANF_R + 1;
-        } else {
-            if (b0 == 0) {
-                HIPCHK(c, hipMemcpyAsync(c->origin.p, origin0, sizeof c->origin0, hipMemcpyHostToDevice, c->stream));
-                HIPCHK(c, hipMemcpyAsync(c->p0.p, &p00, sizeof p00, hipMemcpyHostToDevice, c->stream));
-            }
-            npieces = 1;
-            r.d_begin = b0 * per_batch_draws;
-            r.d_end = std::min<uint64_t>(b1 * per_batch_draws, total_draws);
-            const uint64_t q_begin = p0_master + r.d_begin, q_end = p0_master + r.d_end;
-            r.seg_first = q_begin / 55 / RANF_R;
-            const uint64_t seg_last = (q_end - 1) / 55 / RANF_R;
-            r.nsegs = seg_last - r.seg_first + 1;
-            r.piece_stride = 0;
-        }
-        if (first_kernel) {
-            HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-        }
-        tpk::launch_ranf_expand(r, npieces, c->stream);
-        HIPCHK(c, hipGetLastError());
-        if (first_kernel) {
-            HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-            first_kernel = false;
-        }
-        fa.nb = cnb;
-        fa.b_first = b0;
-        fa.draws = static_cast<const int32_t *>(c->draws.p);
-        fa.out = static_cast<tp_acc *>(per_batch_dev) + b0;
-        tpk::launch_f32_events(fa, f32_grid(c, cnb), c->stream);
-        HIPCHK(c, hipGetLastError());
-        tpk::launch_f32_accumulate(fa, f32_grid(c, cnb), c->stream);
-        HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+    const uint32_t n = (uint32_t)std::min<uint64_t>(num_events, batch_size);
+    if (f32) {
+        // (a run whose batches are split has at most MAX_PARTS of them: its
+        // per-event values stay below 13.2 GB)
+        fa.nb = nb;
+        fa.out = per_batch_dev;
+        rc = launch_f32_batches(c, fa, n);
+        if (rc)
+            return rc;
+    } else {
+        a.nb = nb;
+        a.out = per_batch_dev;
+        if (const int e = launch_event_loop(c, a, 1, n))
+            return e;
     }
     HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
     return TP_OK;
@@ -1410,8 +1245,8 @@ float elapsed(hipEvent_t a, hipEvent_t b)
 
 } // namespace
 
-// ---- xoshiro256+ skip tables ---------------------------------------------------
-// The GF(2) tables the xoshiro256+ event loop reads live in `scratch`, a
+// ---- xoshiro skip tables -------------------------------------------------------
+// The GF(2) tables the xoshiro event loops read live in `scratch`, a
 // file-scope device array, so that tp_run_device_noalloc needs no allocation.
 // It is filled once per device at set-up (tp_create) and only read after that,
 // so calls on one device that overlap do not race on it.  Each device holds
@@ -1421,7 +1256,11 @@ float elapsed(hipEvent_t a, hipEvent_t b)
 constexpr size_t NS_M = 0;                                             // M^(v 16^j)
 constexpr size_t NS_B = NS_M + 15 * tpk::XO_M_DIGITS * tpk::XO_MAT_WORDS; // B^(v 16^j), skip-ahead then jump
 constexpr size_t NS_LANES = NS_B + 2 * 15 * tpk::XO_B_DIGITS * tpk::XO_MAT_WORDS;
-constexpr size_t NS_WORDS = NS_LANES + tpk::XO_NRUNS * tpk::XO_LANE_WORDS; // 24 MiB
+constexpr size_t NS_128 = NS_LANES + tpk::XO_NRUNS * tpk::XO_LANE_WORDS;  // xoshiro128+ (u32 words), as above
+constexpr size_t NS128_B = 15 * tpk::XO_M_DIGITS * tpk::XO128_MAT_WORDS;
+constexpr size_t NS128_LANES = NS128_B + 2 * 15 * tpk::XO_B_DIGITS * tpk::XO128_MAT_WORDS;
+constexpr size_t NS_WORDS = NS_128 + (NS128_LANES + tpk::XO_NRUNS * tpk::XO128_LANE_WORDS) / 2; // 30 MiB
+static_assert(sizeof(tp::Gf2Mat128) == tpk::XO128_MAT_WORDS * sizeof(uint32_t), "matrix layout");
 static_assert(sizeof(tp::Gf2Mat) == tpk::XO_MAT_WORDS * sizeof(uint64_t), "matrix layout");
 static __device__ __align__(256) uint64_t scratch[NS_WORDS];
 
@@ -1459,11 +1298,33 @@ void xo_setup(XoTables &T, hipStream_t st)
         const std::vector<tp::Gf2Mat> bt = tp::gf2_pow2_table(B, 4 * digits[1 + sd]);
         mats.insert(mats.end(), bt.begin(), bt.end());
     }
+    const std::vector<tp::Gf2Mat128> &mt128 = tp::xoshiro128_step_pow2();
+    std::vector<tp::Gf2Mat128> mats128(mt128.begin(), mt128.begin() + 4 * digits[0]);
+    for (int sd = 0; sd < 2; ++sd) {
+        tp::Gf2Mat128 B;
+        if (sd == TP_SEED_JUMP)
+            tp::gf2_128_jump64(B);
+        else
+            tp::gf2_128_pow_from_table(mt128, 12ull * TP_BATCH_SIZE, B);
+        const std::vector<tp::Gf2Mat128> bt = tp::gf2_128_pow2_table(B, 4 * digits[1 + sd]);
+        mats128.insert(mats128.end(), bt.begin(), bt.end());
+    }
     uint64_t *t = static_cast<uint64_t *>(ptr);
-    const size_t bytes = mats.size() * sizeof(tp::Gf2Mat);
-    bool ok = check(hipMalloc(&pow2, bytes), "hipMalloc of the powers") &&
-              check(hipMemcpy(pow2, mats.data(), bytes, hipMemcpyHostToDevice), "upload of the powers");
+    uint32_t *t128 = reinterpret_cast<uint32_t *>(t + NS_128);
+    const size_t bytes = mats.size() * sizeof(tp::Gf2Mat), bytes128 = mats128.size() * sizeof(tp::Gf2Mat128);
+    bool ok = check(hipMalloc(&pow2, bytes + bytes128), "hipMalloc of the powers") &&
+              check(hipMemcpy(pow2, mats.data(), bytes, hipMemcpyHostToDevice), "upload of the powers") &&
+              check(hipMemcpy(static_cast<char *>(pow2) + bytes, mats128.data(), bytes128, hipMemcpyHostToDevice),
+                    "upload of the powers");
     if (ok) {
+        const uint32_t *p128 = reinterpret_cast<const uint32_t *>(static_cast<const char *>(pow2) + bytes);
+        uint32_t *o128 = t128;
+        for (int d : digits) {
+            tpk::launch_xo128_digit_table(p128, d, o128, st);
+            p128 += 4 * d * tpk::XO128_MAT_WORDS;
+            o128 += 15 * d * tpk::XO128_MAT_WORDS;
+        }
+        tpk::launch_xo128_lane_tables(t128, t128 + NS128_LANES, st);
         const uint64_t *p = static_cast<const uint64_t *>(pow2);
         uint64_t *o = t + NS_M;
         for (int d : digits) {
@@ -1482,6 +1343,10 @@ void xo_setup(XoTables &T, hipStream_t st)
     T.b16[TP_SEED_SKIPAHEAD] = t + NS_B;
     T.b16[TP_SEED_JUMP] = t + NS_B + 15 * tpk::XO_B_DIGITS * tpk::XO_MAT_WORDS;
     T.lanes = t + NS_LANES;
+    T.m16_128 = t128;
+    T.b16_128[TP_SEED_SKIPAHEAD] = t128 + NS128_B;
+    T.b16_128[TP_SEED_JUMP] = t128 + NS128_B + 15 * tpk::XO_B_DIGITS * tpk::XO128_MAT_WORDS;
+    T.lanes128 = t128 + NS128_LANES;
     T.rc = TP_OK;
 }
 } // namespace
@@ -1516,7 +1381,9 @@ extern "C" int tp_create(int device, void **ctx_out)
         for (int src = 0; src < 5; ++src)
             for (int prec = 0; prec < 2; ++prec)
                 c->blocks_per_cu[src][prec] = tpk::fused_blocks_per_cu(src, prec);
-        if (device < NS_MAX_DEVICES) { // xoshiro256+ tables (device current)
+        for (int src = 0; src < 4; ++src)
+            c->f32_blocks[src] = tpk::f32_blocks_per_cu(src);
+        if (device < NS_MAX_DEVICES) { // xoshiro tables (device current)
             std::call_once(g_xo[device].once, [&] { xo_setup(g_xo[device].t, c->stream); });
             c->xo = &g_xo[device].t;
         }
@@ -1539,7 +1406,7 @@ extern "C" int tp_destroy(void *ctx)
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
         for (DevBuf *b : {&c->parts, &c->mt, &c->r16, &c->draws, &c->origin, &c->p0, &c->per_batch, &c->merged, &c->evq,
-                          &c->mt128, &c->bt128, &c->st128, &c->f32ev, &c->fe_lists, &c->fe_meta, &c->fe_piece,
+                          &c->f32ev, &c->f32cnt, &c->fe_lists, &c->fe_meta, &c->fe_piece,
                           &c->fe_flag, &c->fe_seq, &c->xo_states, &c->xo_draws, &c->xo128_states,
                           &c->xo128_draws, &c->xo128_pt, &c->xo_acc, &c->xo_lt, &c->xo128_lt, &c->fe_stat, &c->adj_u})
             if (b->p)
@@ -1984,8 +1851,8 @@ extern "C" int tp_run_device_noalloc(void *ctx, const tp_params *params, int rng
         a.out = per_batch_dev;
         HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
         HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-        launch_event_loop(c, a, 0, (uint32_t)std::min<uint64_t>(num_events, TP_BATCH_SIZE));
-        HIPCHK(c, hipGetLastError());
+        if (const int e = launch_event_loop(c, a, 0, (uint32_t)std::min<uint64_t>(num_events, TP_BATCH_SIZE)))
+            return e;
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         if (merged_dev) {
             tpk::launch_merge(per_batch_dev, nb, merged_dev, c->stream, 0);

@@ -624,8 +624,8 @@ extern "C" int tp_flow_run_device(void *flow, const tp_params *params, double al
             fa.nb = b1 - b0;
             fa.b_first = b0;
             fa.out = per_batch_dev + b0;
-            launch_event_loop(c, fa, 2, (uint32_t)std::min<uint64_t>(num_events, bs));
-            FHIP(f, hipGetLastError());
+            if (const int e = launch_event_loop(c, fa, 2, (uint32_t)std::min<uint64_t>(num_events, bs)))
+                return e;
         }
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         if (merged_dev) {

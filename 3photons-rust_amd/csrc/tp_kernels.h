@@ -11,6 +11,20 @@
 namespace tpk {
 
 
+// The RANF stream of a run.  Batch b's events draw from position p0 + 12
+// batch_size b on of the stream whose round 0 is `round` (X[1..55]); with jump
+// seeding (origin non-null) batch b > 0 has a stream of its own, round 0 at
+// origin[56 b] and positions from 0.
+struct RanfSource {
+    int32_t round[56];
+    uint32_t p0;
+    const int32_t *origin;
+    const uint32_t *r16;  // x^(55 v 16^j) mod the recurrence's polynomial, 55 coefficients each, v = 1..15,
+                          // for the digits of a number of rounds
+    uint32_t jump[55];    // x^(55 jump_rounds): from the end of a wavefront's part to near its next one
+    uint64_t jump_rounds; // (0: none)
+};
+
 // Arguments of the fused event-loop kernel.
 struct FusedArgs {
     tpd::Params P;
@@ -34,18 +48,7 @@ struct FusedArgs {
     // tp_events: M^(2^k), k < km, each 256x4 words
     const uint64_t *mt;
     int32_t km;
-    // RANF source: batch b's events draw from position rp0 + 12 batch_size b
-    // on of the stream whose round 0 is rround (X[1..55]); with jump seeding
-    // (rorigin non-null) batch b > 0 has a stream of its own, round 0 at
-    // rorigin[56 b] and positions from 0.  r16: x^(55 v 16^j) mod the
-    // recurrence's polynomial, 55 coefficients each, v = 1..15, for the digits
-    // of a number of rounds.
-    int32_t rround[56];
-    uint32_t rp0;
-    const int32_t *rorigin;
-    const uint32_t *r16;
-    uint32_t rjump[55];    // x^(55 rjump_rounds): from the end of a wavefront's part to near its next one
-    uint64_t rjump_rounds; // (0: none)
+    RanfSource ranf;       // RANF source
     // expanded RANF values: faster-evgen (below), tp_events
     const int32_t *draws;
     // weighted source (importance sampling): uniforms (f64) and weight 1/q(u)
@@ -132,32 +135,52 @@ void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, int32_t *ori
 // In-order fold of nb accumulators; f32 = 1 adds in float (all-f32 mode).
 void launch_merge(const void *per_batch, uint64_t nb, void *merged, hipStream_t st, int f32 = 0);
 
-// ---- all-f32 mode: events, then per-batch sums in event order --------------
+// ---- all-f32 mode: events and per-batch sums in event order -----------------
+// Batches are split over wavefronts as in FusedArgs.  A wavefront that has a
+// whole batch forms its sums in event order itself (no per-event values reach
+// memory), except with the xoshiro128+ stream in registers, whose lanes take
+// runs of events; otherwise launch_f32_accumulate forms them from the events'
+// values.
 struct F32Args {
     tpd::FParams P;
     uint64_t nb, b_first, num_events;
     uint32_t batch_size;
-    int32_t source;        // 0 xoshiro128+ in registers, 1 RANF values from draws, 2 faster-evgen on
+    int32_t source;        // 0 xoshiro128+ in registers, 1 RANF, 2 faster-evgen on
                            // RANF draws, 3 faster-evgen on xoshiro128+ uniforms (x32draws)
-    uint32_t s0[4];        // xoshiro128+ state of the run
-    const uint32_t *mt;    // M^(2^k) of xoshiro128+, k < km (128 columns x 4 words)
-    const uint32_t *bt;    // B^(2^k), k < kb: B = M^(12 batch_size) or the 2^64 jump
-    const uint32_t *stride;// B^stride_grid: a lane's next batch of a grid-stride loop
-    int32_t km, kb;
-    int32_t stride_grid;
-    const int32_t *draws;  // RANF values of this launch's batches, 12 per event, batch-major
+    uint32_t parts, run;
+    uint32_t s0[4];        // xoshiro128+ state of the run, and its skip tables as in FusedArgs
+    const uint32_t *m16, *b16;
+    const uint32_t *lanes;
+    RanfSource ranf;       // source 1
     // faster-evgen (source 2, RANF): event starts evq[batch_size*(b - b_first) + e]
     // in draws from position qbase, as FusedArgs
+    const int32_t *draws;
     const uint64_t *evq;
     uint64_t qbase;
     const float *x32draws; // faster-evgen (source 3): xoshiro128+ uniforms from position qbase
     const uint32_t *acc1;  // faster-evgen: accept bits, as FusedArgs
     uint64_t bbase, blimit, bstride;
-    float *ev;             // per event m[5] and keep (0/1), at batch_size*(b - b_first) + e
+    // Events' values.  Source 0: m[5] and keep (0/1) of event e of batch
+    // b - b_first at ev[6 * (batch_size*(b - b_first) + e)].  Others: the
+    // accepted events of a part in event order, m[c] of the i-th at
+    // ev[c * ev_stride + batch_size*(b - b_first) + the part's first event + i],
+    // their number at counts[(b - b_first) * parts + part].
+    float *ev;
+    uint64_t ev_stride;
+    uint32_t *counts;
     void *out;             // tp_acc per batch, index b - b_first (f32 values)
 };
+constexpr uint32_t F32_MAX_PARTS = 256; // parts that launch_f32_accumulate joins (source 0: any number)
+inline bool f32_sums_in_kernel(const F32Args &a) { return a.source != 0 && a.parts == 1; }
+int f32_blocks_per_cu(int source); // resident wavefronts per CU
 void launch_f32_events(const F32Args &a, int grid, hipStream_t st);
-void launch_f32_accumulate(const F32Args &a, int grid, hipStream_t st);
+void launch_f32_accumulate(const F32Args &a, hipStream_t st); // not after f32_sums_in_kernel
+
+// xoshiro128+ skip tables, as launch_xo_digit_table and launch_xo_lane_tables.
+constexpr size_t XO128_MAT_WORDS = 512;                  // 128 columns of 4 words
+constexpr size_t XO128_LANE_WORDS = 32 * 16 * 64 * 4;    // per run length: 512 KiB
+void launch_xo128_digit_table(const uint32_t *pow2, int digits, uint32_t *tab16, hipStream_t st);
+void launch_xo128_lane_tables(const uint32_t *m16, uint32_t *lanes, hipStream_t st);
 
 // ---- faster-evgen stream walk on the device ----------------------------------
 // Event starts of the faster-evgen draws (evgen.rs:209-255, random_array's

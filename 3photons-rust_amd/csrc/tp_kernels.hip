@@ -215,25 +215,56 @@ __device__ __forceinline__ int32_t ranf_advance(int32_t x, const uint32_t *__res
 // again: 1e9 events 43.4 -> 28.3 ms with the event loop's own gains, the
 // expansion having been 10.4 ms of them; 1e7 events 586 -> 414 us.
 //
-// The next `need` (at most 768) values of the stream into ring[0 ..] in
-// stream order: lane l holds X[l + 1] of the current round in x, whose next
-// unread value is its o-th (X[55 - o], o up to 55).  Rounds are written whole,
-// values past `need` (below ring[need + 54]) and lanes with nothing to write
-// (to ring[dump]) included.
-__device__ __forceinline__ void ranf_fill(int32_t &x, uint32_t &o, uint32_t need, int32_t *ring, uint32_t dump,
-                                          const RanfLanes &l)
-{
-    const int lane = (int)(threadIdx.x & 63u), at = 54 - lane - (int)o;
-    ring[lane < 55 && at >= 0 ? (uint32_t)at : dump] = x;
-    uint32_t p = lane < 55 ? (uint32_t)(at + 55) : dump;
-    const uint32_t step = lane < 55 ? 55u : 0u, rounds = (o + need + 54) / 55 - 1;
-    for (uint32_t r = 0; r < rounds; ++r) {
-        x = ranf_next_round(x, l);
-        ring[p] = x;
-        p += step;
+struct RanfPart {
+    int32_t x = 0;        // lane l: X[l + 1] of the current round
+    uint32_t o = 0;       // the place of the next unread value in it: X[55 - o], o up to 55
+    uint64_t round = 0;   // the number of the last round the part reads
+    bool have = false;
+    RanfLanes l = ranf_lanes();
+
+    // To the first draw of n > 0 events from event `first` of batch b on.  win:
+    // 110 ints of LDS, free before and after.
+    __device__ __forceinline__ void start(const RanfSource &R, uint64_t b, uint32_t batch_size, uint32_t first,
+                                          uint32_t n, int32_t *win)
+    {
+        const bool own = R.origin && b > 0;
+        const uint64_t q = (own ? 0 : R.p0) + 12ull * (first + (R.origin ? 0 : b * batch_size));
+        uint64_t skip = q / 55;
+        if (have && R.jump_rounds && round + R.jump_rounds <= skip) { // on from the previous part
+            x = ranf_jump(x, R.jump, win);
+            skip -= round + R.jump_rounds;
+        } else {
+            const uint32_t lane = threadIdx.x & 63u;
+            x = lane < 55 ? (own ? R.origin[56 * b + lane + 1] : R.round[lane + 1]) : 0;
+        }
+        if (skip < 4) // (a round costs a twentieth of a jump)
+            for (; skip; --skip)
+                x = ranf_next_round(x, l);
+        x = ranf_advance(x, R.r16, skip, win);
+        o = (uint32_t)(q % 55);
+        round = (q + 12ull * n - 1) / 55;
+        have = true;
     }
-    o = o + need - 55 * rounds;
-}
+    // The next `need` (12 .. 768) values into lds[base ..] in stream order.
+    // Lanes with nothing to write do so to lds[dump].
+    __device__ __forceinline__ void fill(uint32_t need, int32_t *lds, uint32_t base, uint32_t dump)
+    {
+        const int lane = (int)(threadIdx.x & 63u), at = 54 - lane - (int)o;
+        lds[lane < 55 && at >= 0 ? base + (uint32_t)at : dump] = x;
+        uint32_t p = lane < 55 ? base + (uint32_t)(at + 55) : dump;
+        const uint32_t step = lane < 55 ? 55u : 0u, rounds = (o + need + 54) / 55 - 1;
+        for (uint32_t r = 1; r < rounds; ++r) {
+            x = ranf_next_round(x, l);
+            lds[p] = x;
+            p += step;
+        }
+        if (rounds) { // the last one may reach past `need`
+            x = ranf_next_round(x, l);
+            lds[p < base + need ? p : dump] = x;
+        }
+        o = o + need - 55 * rounds;
+    }
+};
 
 // ---- the fused event loop ------------------------------------------------
 //
@@ -250,7 +281,7 @@ __device__ __forceinline__ void ranf_fill(int32_t &x, uint32_t &o, uint32_t need
 // Event assignment inside the part: with the in-register xoshiro stream each
 // lane owns a contiguous run (one skip-ahead per run); the others take events
 // l, l+64, ... in lane l.  The RANF stream is made by the wavefront as a whole,
-// 55 values a round, into LDS (ranf_fill), where each lane picks its event's 12
+// 55 values a round, into LDS (RanfPart), where each lane picks its event's 12
 // values; values read from HBM then lie side by side across the lanes.
 //
 // What bounds it: VALU issue, at the measured issue times (f64 fma 4.9 cycles,
@@ -289,16 +320,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
     // half holds an iteration's draws until its events are pushed
     __shared__ __align__(16) double queue[2][12][64];
     auto slot_of = [&](uint32_t s) -> double * { return &queue[0][0][0] + (s >> 6) * (12 * 64) + (s & 63u); };
-    int32_t *ring = reinterpret_cast<int32_t *>(&queue[1][0][0]);
-    constexpr uint32_t RING_DUMP = 1400; // past the 768 + 54 values written, below the half's 1536
+    int32_t *const qints = reinterpret_cast<int32_t *>(&queue[0][0][0]);
+    constexpr uint32_t RING = 2 * 12 * 64, RING_DUMP = RING + 768; // of the upper half's 1536 ints
     __shared__ uint32_t qev[SOURCE == 2 ? QCAP : 1]; // weighted source: the event's index in the chunk
     __shared__ double red[1][13];
     const uint32_t lane = threadIdx.x;
     const uint64_t lanemask_lt = (1ull << lane) - 1ull;
     uint64_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}; // xoshiro state at the part's first draw (uniform)
-    int32_t rx = 0;      // RANF: X[lane + 1] of the current round,
-    uint32_t ro = 0;     // the place of the next unread value in it,
-    uint64_t rround = 0; // and the round's number at the end of the part
+    RanfPart ranf;
     bool have = false;
     for (uint64_t t = blockIdx.x; t < a.nb * a.parts; t += gridDim.x) {
         const uint64_t lb = a.parts == 1 ? t : t / a.parts;
@@ -323,26 +352,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
             len = n / 64 + (lane < n % 64 ? 1u : 0u); // events lane, lane+64, ...
             iters = (n + 63) / 64;
         }
-        const RanfLanes rl = ranf_lanes();
-        if (SOURCE == 1 && n) {
-            const bool own = a.rorigin && b > 0;
-            const uint64_t q = (own ? 0 : a.rp0) + 12ull * (first + (a.rorigin ? 0 : b * a.batch_size));
-            uint64_t skip = q / 55;
-            if (have && a.rjump_rounds && rround + a.rjump_rounds <= skip) { // on from the previous part
-                rx = ranf_jump(rx, a.rjump, ring);
-                skip -= rround + a.rjump_rounds;
-            } else {
-                rx = lane < 55 ? (own ? a.rorigin[56 * b + lane + 1] : a.rround[lane + 1]) : 0;
-            }
-            if (skip < 4) // (a round costs a twentieth of a jump)
-                for (; skip; --skip)
-                    rx = ranf_next_round(rx, rl);
-            rx = ranf_advance(rx, a.r16, skip, ring);
-            ro = (uint32_t)(q % 55);
-            // the round the part leaves in rx (ranf_fill stops at the last one it reads)
-            rround = (q + 12ull * n - 1) / 55;
-            have = true;
-        }
+        if (SOURCE == 1 && n)
+            ranf.start(a.ranf, b, a.batch_size, first, n, qints + RING);
         const size_t wbase = (size_t)lb * a.batch_size + first;
         const RerollBits rb{a.acc1, a.bbase, a.bstride ? (lb + 1) * a.bstride : a.blimit};
         Acc<PREC> A;
@@ -359,11 +370,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                 qnext = a.evq[wbase + (size_t)((k + 1) * 64 + lane)];
             int4 rd[3]; // RANF: the lane's 12 draws
             if (SOURCE == 1) {
-                ranf_fill(rx, ro, 12 * min(64u, n - 64 * k), ring, RING_DUMP, rl);
+                ranf.fill(12 * min(64u, n - 64 * k), qints, RING, RING_DUMP);
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < 3; ++j)
-                    rd[j] = reinterpret_cast<const int4 *>(ring)[3 * lane + j];
+                    rd[j] = reinterpret_cast<const int4 *>(qints + RING)[3 * lane + j];
                 __syncthreads(); // read before the events are pushed
             }
             if (k < len && SOURCE == 3) {
@@ -544,6 +555,66 @@ void launch_xo_lane_tables(const uint64_t *m16, uint64_t *lanes, hipStream_t st)
     for (int i = 0; i < XO_NRUNS; ++i)
         r.n[i] = XO_RUNS[i];
     hipLaunchKernelGGL(xo_lane_table_kernel, dim3(64, XO_NRUNS), dim3(64), 0, st, m16, lanes, r);
+}
+
+// The xoshiro128+ tables: lane c < 64 takes columns c and c + 64; one lane per
+// (nibble, half) of the state.
+__global__ __launch_bounds__(64) void xo128_digit_table_kernel(const uint32_t *pow2, uint32_t *tab16)
+{
+    const uint32_t j = blockIdx.x / 15, v = blockIdx.x % 15 + 1, col = 64 * blockIdx.y + threadIdx.x;
+    uint32_t s[4];
+#pragma unroll
+    for (uint32_t w = 0; w < 4; ++w)
+        s[w] = w == col / 32 ? 1u << (col % 32) : 0;
+    for (uint32_t k = 0; k < 4; ++k)
+        if ((v >> k) & 1u)
+            gf2_apply128(pow2 + XO128_MAT_WORDS * (4 * j + k), s);
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+        tab16[XO128_MAT_WORDS * blockIdx.x + 4 * col + w] = s[w];
+}
+
+void launch_xo128_digit_table(const uint32_t *pow2, int digits, uint32_t *tab16, hipStream_t st)
+{
+    hipLaunchKernelGGL(xo128_digit_table_kernel, dim3(15 * digits, 2), dim3(64), 0, st, pow2, tab16);
+}
+
+__global__ __launch_bounds__(64) void xo128_lane_table_kernel(const uint32_t *m16, uint32_t *lanes, XoRuns runs)
+{
+    const uint32_t l = blockIdx.x, ch = threadIdx.x & 31u;
+    uint32_t img[4][4]; // of the nibble's four bits
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w)
+            img[k][w] = w == ch / 8 ? 1u << (4 * (ch % 8) + k) : 0;
+        const uint32_t *tab = m16;
+        for (uint32_t e = 12 * runs.n[blockIdx.y] * l; e; e >>= 4, tab += 15 * XO128_MAT_WORDS)
+            if (e & 15u)
+                gf2_apply128(tab + ((e & 15u) - 1) * XO128_MAT_WORDS, img[k]);
+    }
+    uint32_t *out = lanes + XO128_LANE_WORDS * blockIdx.y + 256 * (size_t)(16 * ch) + 4 * l;
+    const uint32_t v0 = threadIdx.x < 32 ? 0 : 8; // half of the nibble's values per lane
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t v = v0 + i;
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) {
+            uint32_t x = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                x ^= (v >> k) & 1u ? img[k][w] : 0;
+            out[256 * v + w] = x;
+        }
+    }
+}
+
+void launch_xo128_lane_tables(const uint32_t *m16, uint32_t *lanes, hipStream_t st)
+{
+    XoRuns r;
+    for (int i = 0; i < XO_NRUNS; ++i)
+        r.n[i] = XO_RUNS[i];
+    hipLaunchKernelGGL(xo128_lane_table_kernel, dim3(64, XO_NRUNS), dim3(64), 0, st, m16, lanes, r);
 }
 
 template <int SOURCE, int PREC> int blocks_per_cu()
@@ -786,6 +857,9 @@ template <int BITS> __global__ __launch_bounds__(64) void ranf_expand_kernel(Ran
         return; // whole workgroup
     int32_t x = lane < 55 ? a.origin[56 * piece + lane + 1] : 0;
     x = ranf_advance(x, a.r16, seg * (uint64_t)a.R, win);
+    // (the empty asm makes the wait for a load of x come here: in the rounds'
+    // loop, where the compiler would place it, it waits for each round's store)
+    asm volatile("" : "+v"(x));
     int32_t *out = a.out + piece * a.piece_stride;
     const RanfLanes l = ranf_lanes();
     __shared__ uint64_t bm[2][BITS ? 32 : 1];
@@ -1822,104 +1896,156 @@ void launch_merge(const void *per_batch, uint64_t nb, void *merged, hipStream_t 
 }
 
 // ---- all-f32 mode --------------------------------------------------------------
-// One wavefront per batch (grid-stride).  Each lane takes a contiguous run of
-// the batch's events (one skip-ahead of the xoshiro128+ stream per run; with
-// faster-evgen every 64th event instead) and writes each event's m[5] and
-// cut decision; the batch sums are then formed
-// in event order, as the reference's sequential loop does in f32
-// (resacc.rs:121-129), where a tree sum would round differently.
-// Events that pass the cuts are queued in LDS (momenta and event index) and
-// their helicity sums computed 64 at a time on dense lanes, as in the f64
-// event loop; each event's m[5] and cut flag go to its own slot of a.ev.
-template <int SOURCE>
+// One wavefront per part of a batch (grid-stride), as in the f64 event loop:
+// events that pass the cuts are queued in LDS and their helicity sums computed
+// 64 at a time on dense lanes.  The batch sums are formed in event order, as
+// the reference's sequential loop does in f32 (resacc.rs:121-129), where a tree
+// sum would round differently.  So the queue is first in, first out: the
+// oldest 64 events fill the half at `head`, and with sources whose lane l
+// takes events l, l + 64, ... they leave in event order.  A wavefront with a
+// whole batch (SUMS) puts the 12 summands of the 64 into the half just emptied
+// and 12 lanes add them in turn: 64 dependent adds of 9 cycles that the
+// other five wavefronts of the SIMD hide, against 24 bytes per event written
+// and read again (7.5 of 50 ms per 1e9 events, and as much again in the
+// writes).  A part of a batch hands its accepted events on in order
+// (f32_accumulate_kernel).  With the xoshiro128+ stream in registers (SOURCE 0)
+// a lane takes a run of events, and each event's values go to its own slot.
+static_assert(offsetof(F32Args, P) == 0, "FParams first in F32Args");
+typedef const __attribute__((address_space(4))) FParams KFParams;
+__device__ __forceinline__ const FParams &fresh_fparams() // as fresh_params
+{
+    KFParams *k = (KFParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    return *(const FParams *)k;
+}
+
+template <int SOURCE, bool SUMS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void f32_events_kernel(F32Args a)
 {
-    __shared__ float queue[12][QCAP];
-    __shared__ uint32_t qidx[QCAP];
+    constexpr uint32_t HALF = 12 * 64, DUMP = 2 * HALF;
+    __shared__ __align__(16) float queue[2 * HALF + 4];
+    __shared__ uint32_t qidx[SOURCE == 0 ? QCAP : 1];
+    int32_t *const qints = reinterpret_cast<int32_t *>(queue);
     const uint32_t lane = threadIdx.x;
     const uint64_t lanemask_lt = (1ull << lane) - 1ull;
-    // helicity sums of the queued event in `slot`, stored to its output slot
-    auto flush_one = [&](uint32_t slot) {
-        float pq[3][4], m[5];
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                pq[i][j] = queue[4 * i + j][slot];
-        const uint32_t idx = qidx[slot];
-        matrix_elements_f32(a.P, pq, m);
-        float *o = a.ev + 6 * (size_t)idx;
-#pragma unroll
-        for (int c = 0; c < 5; ++c)
-            o[c] = m[c];
-        o[5] = 1.f;
-    };
-    uint32_t st[4] = {0, 0, 0, 0}; // xoshiro128+ state at this lane's chunk of the previous batch
+    uint32_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}; // xoshiro128+ state at the part's first draw (uniform)
+    RanfPart ranf;
     bool have = false;
-    for (uint64_t lb = blockIdx.x; lb < a.nb; lb += gridDim.x) {
+    for (uint64_t t = blockIdx.x; t < a.nb * a.parts; t += gridDim.x) {
+        const uint64_t lb = a.parts == 1 ? t : t / a.parts;
+        const uint32_t first = (uint32_t)(t - lb * a.parts) * 64u * a.run; // the part's first event in the batch
         const uint64_t b = a.b_first + lb;
         const uint64_t left = a.num_events - b * a.batch_size;
-        const uint32_t n = left < a.batch_size ? (uint32_t)left : a.batch_size;
-        const uint32_t q = n / 64, r = n % 64;
-        const uint32_t len = q + (lane < r ? 1u : 0u);
-        // a contiguous run of events per lane (one skip-ahead of the stream
-        // per run) for the sources that draw 12 values per event; with
-        // faster-evgen the events lane, lane + 64, ... (their draws lie side
-        // by side across the wavefront)
+        const uint32_t nbatch = left < a.batch_size ? (uint32_t)left : a.batch_size;
+        const uint32_t n = first < nbatch ? min(nbatch - first, 64u * a.run) : 0u;
         constexpr bool FE = SOURCE == 2 || SOURCE == 3;
-        const uint32_t e0 = FE ? lane : lane * q + (lane < r ? lane : r);
-        const uint32_t estep = FE ? 64u : 1u;
-        uint32_t s[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]};
+        uint32_t len, iters;
+        uint32_t s[4] = {0, 0, 0, 0};
         if (SOURCE == 0) {
-            // M^(12 e0) B^b s0; the next batch of the grid-stride loop is B^grid
-            // times the same (all factors are powers of the step matrix, so
-            // they commute), unless its event split differs (the last batch)
-            if (have && n == a.batch_size && (int)gridDim.x == a.stride_grid) {
-                gf2_apply128(a.stride, st);
-            } else {
-                st[0] = a.s0[0];
-                st[1] = a.s0[1];
-                st[2] = a.s0[2];
-                st[3] = a.s0[3];
-                for (int k = 0; k < a.kb; ++k)
-                    if ((b >> k) & 1ull) // uniform across the wavefront
-                        gf2_apply128(a.bt + 512 * k, st);
-                const uint64_t off = 12ull * e0;
-                for (int k = 0; k < a.km; ++k)
-                    if ((off >> k) & 1ull)
-                        gf2_apply128(a.mt + 512 * k, st);
-            }
-            have = n == a.batch_size;
-            s[0] = st[0];
-            s[1] = st[1];
-            s[2] = st[2];
-            s[3] = st[3];
+            len = lane * a.run < n ? min(n - lane * a.run, a.run) : 0u;
+            iters = min(n, a.run);
+            xo128_advance_uniform(a.b16, have ? gridDim.x / a.parts : b, sw);
+            if (!have)
+                xo128_advance_uniform(a.m16, 12ull * first, sw);
+            have = true;
+            xo128_lane_states(a.lanes, sw, s);
+        } else {
+            len = n / 64 + (lane < n % 64 ? 1u : 0u);
+            iters = (n + 63) / 64;
         }
-        const uint32_t iters = q + (r ? 1u : 0u);
-        uint32_t qn = 0; // queued events (uniform)
+        if (SOURCE == 1 && n)
+            ranf.start(a.ranf, b, a.batch_size, first, n, qints);
+        const uint64_t base = lb * a.batch_size + first; // the part's first slot
+        uint32_t qn = 0, head = 0, done = 0; // queued events, their first slot (0 or 64), events that left (uniform)
+        float sum = 0.f;                     // SUMS: lane j < 12: sum j of (spm2[5], vars[5], sigma, variance)
+        // the oldest `cnt` (64, or at the part's end all) queued events
+        auto flush = [&](uint32_t cnt) {
+            __syncthreads();
+            float *const half = queue + (head ? HALF : 0);
+            auto sums = [&](float m[5]) {
+                float pq[3][4];
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        pq[i][j] = half[64 * (4 * i + j) + lane];
+                matrix_elements_f32(fresh_fparams(), pq, m);
+            };
+            if (SUMS) {
+                // summand j of event e at column (e + 4 j) % 64 of row j: the 12
+                // lanes' 16-byte reads hit distinct banks.  -0.0 past the last
+                // event: x + (-0.0) = x for every x.
+                float m[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+                const bool in = lane < cnt;
+                if (in)
+                    sums(m);
+                const float w = weight_f32(fresh_fparams(), m), z = -0.f;
+                __syncthreads();
+#pragma unroll
+                for (uint32_t j = 0; j < 12; ++j) {
+                    const float x = j < 5 ? m[j] : j < 10 ? m[j - 5] * m[j - 5] : j == 10 ? w : w * w;
+                    half[64 * j + ((lane + 4 * j) & 63u)] = in ? x : z;
+                }
+                __syncthreads();
+                if (lane < 12) {
+                    const float4 *row = reinterpret_cast<const float4 *>(half + 64 * lane);
+#pragma unroll 4
+                    for (uint32_t g = 0; g < 16; ++g) {
+                        const float4 x = row[(g + lane) & 15u];
+                        sum = sum + x.x;
+                        sum = sum + x.y;
+                        sum = sum + x.z;
+                        sum = sum + x.w;
+                    }
+                }
+            } else if (lane < cnt) {
+                float m[5];
+                sums(m);
+                if (SOURCE == 0) {
+                    float *o = a.ev + 6 * (size_t)qidx[head + lane];
+#pragma unroll
+                    for (int c = 0; c < 5; ++c)
+                        o[c] = m[c];
+                    o[5] = 1.f;
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 5; ++c) {
+                        float *row = a.ev + (c * a.ev_stride + base + done); // uniform
+                        row[lane] = m[c];
+                    }
+                }
+            }
+            __syncthreads();
+            done += cnt;
+            qn -= cnt;
+            head ^= 64u;
+        };
         // faster-evgen: the lane's next event start, loaded an event ahead
-        uint64_t qnext = FE && len > 0 ? a.evq[lb * a.batch_size + e0] : 0;
+        uint64_t qnext = FE && len > 0 ? a.evq[base + lane] : 0;
         for (uint32_t i = 0; i < iters; ++i) {
-            const uint64_t e = lb * a.batch_size + e0 + (uint64_t)i * estep;
             bool pass = false;
             float p[3][4];
             const uint64_t qk = qnext;
             if (FE && i + 1 < len)
-                qnext = a.evq[e + estep];
+                qnext = a.evq[base + 64 * (i + 1) + lane];
+            int4 rd[3]; // RANF: the lane's 12 draws, through the half that is free
+            if (SOURCE == 1) {
+                const uint32_t ring = head ? 0 : HALF;
+                ranf.fill(12 * min(64u, n - 64 * i), qints, ring, DUMP);
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    rd[j] = reinterpret_cast<const int4 *>(qints + ring)[3 * lane + j];
+                __syncthreads(); // read before the events are pushed
+            }
             if (i < len && FE) {
                 const RerollBits rb{a.acc1, a.bbase, a.bstride ? (lb + 1) * a.bstride : a.blimit};
                 if constexpr (SOURCE == 2) {
                     RanfWalkF32 w{a.draws, a.qbase, qk, rb};
-                    pass = generate_faster_f32(a.P, w, p);
+                    pass = generate_faster_f32(fresh_fparams(), w, p);
                 } else {
                     Xo128WalkF32 w{a.x32draws, a.qbase, qk, rb};
-                    pass = generate_faster_f32(a.P, w, p);
-                }
-                if (!pass) {
-                    float *o = a.ev + 6 * e;
-#pragma unroll
-                    for (int c = 0; c < 6; ++c)
-                        o[c] = 0.f;
+                    pass = generate_faster_f32(fresh_fparams(), w, p);
                 }
             } else if (i < len) {
                 float u[12];
@@ -1928,126 +2054,218 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
                     for (int j = 0; j < 12; ++j)
                         u[j] = xo128_uniform(s);
                 } else {
-                    const int32_t *d = a.draws + 12 * e;
 #pragma unroll
-                    for (int j = 0; j < 12; ++j)
-                        u[j] = (float)d[j] * 1e-9f; // (n as f32) * INV_MODULO (ranf.rs:99)
+                    for (int j = 0; j < 3; ++j) { // (n as f32) * INV_MODULO (ranf.rs:99)
+                        u[4 * j] = (float)rd[j].x * 1e-9f;
+                        u[4 * j + 1] = (float)rd[j].y * 1e-9f;
+                        u[4 * j + 2] = (float)rd[j].z * 1e-9f;
+                        u[4 * j + 3] = (float)rd[j].w * 1e-9f;
+                    }
                 }
-                pass = generate_f32(a.P, u, p);
-                if (!pass) {
-                    float *o = a.ev + 6 * e;
+                pass = generate_f32(fresh_fparams(), u, p);
+            }
+            if (SOURCE == 0 && i < len && !pass) {
+                float *o = a.ev + 6 * (size_t)(base + lane * a.run + i);
 #pragma unroll
-                    for (int c = 0; c < 6; ++c)
-                        o[c] = 0.f;
-                }
+                for (int c = 0; c < 6; ++c)
+                    o[c] = 0.f;
             }
             const uint64_t mask = __ballot(pass);
             if (pass) {
-                const uint32_t slot = qn + (uint32_t)__popcll(mask & lanemask_lt);
+                const uint32_t slot = (head + qn + (uint32_t)__popcll(mask & lanemask_lt)) & 127u;
+                float *q = queue + (slot >> 6) * HALF + (slot & 63u);
 #pragma unroll
                 for (int k = 0; k < 3; ++k)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        queue[4 * k + j][slot] = p[k][j];
-                qidx[slot] = (uint32_t)e;
+                        q[64 * (4 * k + j)] = p[k][j];
+                if (SOURCE == 0)
+                    qidx[slot] = (uint32_t)(base + lane * a.run + i);
             }
             qn += (uint32_t)__popcll(mask);
-            if (qn >= 64) {
-                __syncthreads();
-                flush_one(qn - 64 + lane);
-                __syncthreads();
-                qn -= 64;
-            }
+            if (qn >= 64)
+                flush(64);
         }
-        if (qn > 0) { // partial flush
-            __syncthreads();
-            if (lane < qn)
-                flush_one(lane);
+        if (qn > 0)
+            flush(qn);
+        if (SUMS) {
+            DevAcc *out = reinterpret_cast<DevAcc *>(a.out) + lb;
+            if (lane < 12)
+                reinterpret_cast<double *>(out)[1 + lane] = (double)sum;
+            if (lane == 0)
+                out->selected = done;
+        } else if (SOURCE != 0 && lane == 0) {
+            a.counts[t] = done;
         }
         __syncthreads();
     }
 }
 
-constexpr int F32_TILE = 256;
+// In-order f32 batch sums (resacc.rs:121-129 with Float = f32) from the
+// events' values, four wavefronts per batch: lanes 0..11 of the first add a
+// tile's summands (m_c, m_c^2, w, w^2) in event order, the order that fixes the
+// f32 rounding, while the other three, tile about, load the next tiles' events
+// and write their summands to LDS.  SLOTS: every event has a slot and a flag
+// (source 0), a rejected one's summands being -0.0 (x + (-0.0) == x for every
+// x, so it changes no sum, as when the reference skips it); otherwise the
+// accepted events of the batch's parts in order, tiles running on from part to
+// part.  What bounds it: the chain of adds, 9 cycles an accepted event (26 us a
+// batch, 1536 batches at once), or for long runs the bytes of the events.  A
+// tile's loads have three tiles' time to arrive: with one loading wavefront a
+// closure call of 10 000 events spent 160 us here on their latency.
+constexpr int F32_TILE = 128, F32_ROW = F32_TILE + 4; // rows 4 banks apart for the chains' 16-byte reads
+constexpr int F32_BUFS = 4;                           // tiles in LDS: one being added, three being made
 
-// In-order f32 batch sums (resacc.rs:121-129 with Float = f32).  For each
-// tile of events all 64 lanes form the 12 summands (m_c, m_c^2, w, w^2) in
-// parallel, writing -0.0 for a rejected event (x + (-0.0) == x for every x,
-// so a rejected event changes no sum, as when the reference skips it); then
-// lanes 0..11 add their summand column in event order, which is the order
-// that fixes the f32 rounding.  Selected events are counted with ballots.
-__global__ __launch_bounds__(64) void f32_accumulate_kernel(F32Args a)
+template <bool SLOTS> __global__ __launch_bounds__(256) void f32_accumulate_kernel(F32Args a)
 {
-    __shared__ float terms[12][F32_TILE + 1];
-    const uint32_t lane = threadIdx.x;
-    DevAcc *out = reinterpret_cast<DevAcc *>(a.out);
-    for (uint64_t lb = blockIdx.x; lb < a.nb; lb += gridDim.x) {
-        const uint64_t b = a.b_first + lb;
-        const uint64_t left = a.num_events - b * a.batch_size;
-        const uint32_t n = left < a.batch_size ? (uint32_t)left : a.batch_size;
-        const float *ev = a.ev + 6 * lb * a.batch_size;
-        float t = 0.f; // lane j < 12: sum j of (spm2[5], vars[5], sigma, variance)
-        uint32_t cnt = 0;
-        for (uint32_t base = 0; base < n; base += F32_TILE) {
-            const uint32_t mm = n - base < (uint32_t)F32_TILE ? n - base : (uint32_t)F32_TILE;
-            __syncthreads(); // the previous tile has been summed
-            for (uint32_t e = lane; e < mm; e += 64) {
-                const float *x = ev + 6 * (size_t)(base + e);
-                float m[5];
+    __shared__ __align__(16) float terms[F32_BUFS][12][F32_ROW];
+    __shared__ uint32_t before[F32_MAX_PARTS + 1]; // accepted events of the parts before each
+    __shared__ uint32_t kept;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint64_t lb = blockIdx.x;
+    const uint64_t left = a.num_events - (a.b_first + lb) * a.batch_size;
+    const uint64_t base = lb * a.batch_size;
+    const uint32_t nparts = SLOTS ? 1u : a.parts; // at most F32_MAX_PARTS
+    uint32_t n = left < a.batch_size ? (uint32_t)left : a.batch_size;
+    if (threadIdx.x == 0)
+        kept = 0;
+    if (!SLOTS) {
+        if (threadIdx.x < nparts)
+            before[threadIdx.x + 1] = a.counts[lb * nparts + threadIdx.x];
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            before[0] = 0;
+            for (uint32_t s = 0; s < nparts; ++s)
+                before[s + 1] += before[s];
+        }
+        __syncthreads();
+        n = before[nparts];
+    } else {
+        __syncthreads();
+    }
+    const uint32_t tiles = (n + F32_TILE - 1) / F32_TILE;
+    constexpr int PER = F32_TILE / 64;
+    float m[PER][5];
+    bool keep[PER];
+    uint32_t cnt = 0;
+    auto load = [&](uint32_t k) {
 #pragma unroll
-                for (int c = 0; c < 5; ++c)
-                    m[c] = x[c];
-                const bool keep = x[5] != 0.f;
-                cnt += (uint32_t)__popcll(__ballot(keep));
-                const float w = weight_f32(a.P, m);
-                const float z = -0.f;
-#pragma unroll
-                for (int c = 0; c < 5; ++c) {
-                    terms[c][e] = keep ? m[c] : z;
-                    terms[5 + c][e] = keep ? m[c] * m[c] : z;
+        for (int i = 0; i < PER; ++i) {
+            const uint32_t e = k * F32_TILE + 64 * i + lane;
+            keep[i] = e < n;
+            uint64_t at = base + e;
+            if (!SLOTS && keep[i]) {
+                uint32_t lo = 0, hi = nparts; // before[lo] <= e < before[hi]
+                while (hi - lo > 1) {
+                    const uint32_t mid = (lo + hi) / 2;
+                    if (before[mid] <= e)
+                        lo = mid;
+                    else
+                        hi = mid;
                 }
-                terms[10][e] = keep ? w : z;
-                terms[11][e] = keep ? w * w : z;
+                at = base + (uint64_t)lo * 64u * a.run + (e - before[lo]);
             }
-            __syncthreads();
-            if (lane < 12) {
-                const float *row = terms[lane];
-                uint32_t e = 0;
-                for (; e + 16 <= mm; e += 16) {
-                    float v[16];
 #pragma unroll
-                    for (int u = 0; u < 16; ++u)
-                        v[u] = row[e + u];
+            for (int c = 0; c < 5; ++c)
+                m[i][c] = !keep[i] ? 0.f : SLOTS ? a.ev[6 * at + c] : a.ev[c * a.ev_stride + at];
+            if (SLOTS && keep[i])
+                keep[i] = a.ev[6 * at + 5] != 0.f;
+        }
+    };
+    auto write = [&](uint32_t k) {
+        float(*row)[F32_ROW] = terms[k % F32_BUFS];
 #pragma unroll
-                    for (int u = 0; u < 16; ++u)
-                        t = t + v[u];
-                }
-                for (; e < mm; ++e)
-                    t = t + row[e];
+        for (int i = 0; i < PER; ++i) {
+            const float w = weight_f32(a.P, m[i]), z = -0.f;
+            cnt += (uint32_t)__popcll(__ballot(keep[i]));
+#pragma unroll
+            for (int j = 0; j < 12; ++j) {
+                const float x = j < 5 ? m[i][j] : j < 10 ? m[i][j - 5] * m[i][j - 5] : j == 10 ? w : w * w;
+                row[j][64 * i + lane] = keep[i] ? x : z;
             }
         }
-        if (lane < 12)
-            reinterpret_cast<double *>(out + lb)[1 + lane] = (double)t;
-        if (lane == 0) // lane 0 runs every pass of the tile loop, so its count is complete
-            out[lb].selected = cnt;
+    };
+    // tile j is loaded at step j - 3, after its buffer's previous tile j - 4,
+    // and written at step j - 1
+    float t = 0.f; // lane j < 12 of the first wavefront: sum j of (spm2[5], vars[5], sigma, variance)
+    const uint32_t p = wave - 1;
+    if (wave && p < tiles)
+        load(p);
+    if (wave == 1 && tiles)
+        write(0);
+    __syncthreads();
+    for (uint32_t i = 0; i < tiles; ++i) {
+        if (wave) {
+            if ((i + 1) % 3 == p && i + 1 < tiles)
+                write(i + 1);
+            if (i % 3 == p && i + 3 < tiles)
+                load(i + 3);
+        } else if (lane < 12) {
+            const float4 *row = reinterpret_cast<const float4 *>(terms[i % F32_BUFS][lane]);
+#pragma unroll 2
+            for (int g = 0; g < F32_TILE / 16; ++g) {
+                float4 x[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    x[u] = row[4 * g + u];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    t = t + x[u].x;
+                    t = t + x[u].y;
+                    t = t + x[u].z;
+                    t = t + x[u].w;
+                }
+            }
+        }
+        __syncthreads();
     }
+    if (wave && lane == 0)
+        atomicAdd(&kept, cnt);
+    __syncthreads();
+    DevAcc *out = reinterpret_cast<DevAcc *>(a.out) + lb;
+    if (threadIdx.x < 12)
+        reinterpret_cast<double *>(out)[1 + lane] = (double)t;
+    if (threadIdx.x == 0)
+        out->selected = kept;
+}
+
+template <int SOURCE> static int f32_blocks()
+{
+    int n = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f32_events_kernel<SOURCE, SOURCE != 0>, 64, 0);
+    return (e == hipSuccess && n > 0) ? n : 1;
+}
+int f32_blocks_per_cu(int source)
+{
+    return source == 0 ? f32_blocks<0>() : source == 1 ? f32_blocks<1>() : source == 2 ? f32_blocks<2>() : f32_blocks<3>();
+}
+
+template <int SOURCE> static void launch_f32_source(const F32Args &a, int grid, hipStream_t st)
+{
+    if (f32_sums_in_kernel(a))
+        hipLaunchKernelGGL((f32_events_kernel<SOURCE, true>), dim3(grid), dim3(64), 0, st, a);
+    else
+        hipLaunchKernelGGL((f32_events_kernel<SOURCE, false>), dim3(grid), dim3(64), 0, st, a);
 }
 
 void launch_f32_events(const F32Args &a, int grid, hipStream_t st)
 {
     if (a.source == 0)
-        hipLaunchKernelGGL(f32_events_kernel<0>, dim3(grid), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((f32_events_kernel<0, false>), dim3(grid), dim3(64), 0, st, a);
     else if (a.source == 1)
-        hipLaunchKernelGGL(f32_events_kernel<1>, dim3(grid), dim3(64), 0, st, a);
+        launch_f32_source<1>(a, grid, st);
     else if (a.source == 2)
-        hipLaunchKernelGGL(f32_events_kernel<2>, dim3(grid), dim3(64), 0, st, a);
+        launch_f32_source<2>(a, grid, st);
     else
-        hipLaunchKernelGGL(f32_events_kernel<3>, dim3(grid), dim3(64), 0, st, a);
+        launch_f32_source<3>(a, grid, st);
 }
 
-void launch_f32_accumulate(const F32Args &a, int grid, hipStream_t st)
+void launch_f32_accumulate(const F32Args &a, hipStream_t st)
 {
-    hipLaunchKernelGGL(f32_accumulate_kernel, dim3(grid), dim3(64), 0, st, a);
+    if (a.source == 0)
+        hipLaunchKernelGGL(f32_accumulate_kernel<true>, dim3((unsigned)a.nb), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(f32_accumulate_kernel<false>, dim3((unsigned)a.nb), dim3(256), 0, st, a);
 }
 
 } // namespace tpk

@@ -213,4 +213,40 @@ __device__ __forceinline__ void gf2_apply128(const uint32_t *__restrict__ mg, ui
     s[3] = r3;
 }
 
+// The same for 128x128 matrices: lane l takes columns l and l + 64.
+__device__ __forceinline__ void gf2_uniform128(const uint32_t *__restrict__ m, uint32_t s[4])
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint4 *c = reinterpret_cast<const uint4 *>(m) + lane;
+    const uint4 a = c[0], b = c[64];
+    const uint32_t ka = 0u - ((uint32_t)(pack64(s[0], s[1]) >> lane) & 1u);
+    const uint32_t kb = 0u - ((uint32_t)(pack64(s[2], s[3]) >> lane) & 1u);
+    s[0] = wave_xor((a.x & ka) ^ (b.x & kb));
+    s[1] = wave_xor((a.y & ka) ^ (b.y & kb));
+    s[2] = wave_xor((a.z & ka) ^ (b.z & kb));
+    s[3] = wave_xor((a.w & ka) ^ (b.w & kb));
+}
+__device__ __forceinline__ void xo128_advance_uniform(const uint32_t *__restrict__ tab, uint64_t e, uint32_t s[4])
+{
+    for (; e; e >>= 4, tab += 15 * 512)
+        if (e & 15u)
+            gf2_uniform128(tab + ((e & 15u) - 1) * 512, s);
+}
+// Entry [ch][v][lane][4 words] of the lane table.
+__device__ __forceinline__ void xo128_lane_states(const uint32_t *__restrict__ tab, const uint32_t s[4], uint32_t st[4])
+{
+    const uint4 *t = reinterpret_cast<const uint4 *>(tab) + (threadIdx.x & 63u);
+    st[0] = st[1] = st[2] = st[3] = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll 4
+        for (int k = 0; k < 8; ++k) {
+            const uint4 e = t[64 * (16 * (8 * w + k) + ((s[w] >> (4 * k)) & 15u))];
+            st[0] ^= e.x;
+            st[1] ^= e.y;
+            st[2] ^= e.z;
+            st[3] ^= e.w;
+        }
+}
+
 } // namespace tpd
