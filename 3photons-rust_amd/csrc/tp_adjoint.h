@@ -610,6 +610,182 @@ __device__ __forceinline__ bool event_adjoint_sweeps(const AdjParams<T> &P, cons
     return keep;
 }
 
+// The five sums of one event and all their derivatives in f64: what
+// event_adjoint_sweeps<double, 0, 5> gives, from one evaluation of the closed
+// forms' gradients (helicity_gradients) instead of five sweeps back through the
+// amplitudes.  The five go on through the conformal map and the generation,
+// whose divisions are taken once.  Momenta and cuts are the same bits; the sums
+// are symmetric in the photons, so only dF/dp needs their order.
+//
+// row: this lane's 60 doubles of staging, 16-byte aligned.  They hold
+// w dF_c / dp, [c][place][X, Y, Z, E], when dp_ready(F) is called, and
+// w dF_c / du, [c][12], at the end; all zero, F too, for a cut event.  Every
+// lane calls dp_ready, which may let the other lanes read the row.
+template <class Ready>
+__device__ __forceinline__ void event_jacobian(const Params &P, const HelicityK &K, double w, const double u[12],
+                                               double *row, bool want_du, Ready &&dp_ready)
+{
+    using tpm::fma_;
+    const double two_pi = 2. * 3.14159265358979323846, tiny = 2.2250738585072014e-308;
+    double ct[3], sp[3], cp[3], st[3], en[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) { // evgen.rs:174-207
+        ct[i] = 2. * u[4 * i] - 1.;
+        tpm::sincos_f64(two_pi * u[4 * i + 1], sp[i], cp[i]);
+        st[i] = sq(1. - ct[i] * ct[i]);
+        en[i] = -tpm::log_pos(u[4 * i + 2] * u[4 * i + 3] + tiny);
+    }
+    double q[3][4], R[4], rn2, alpha, rn, beta, rq[3], b[3], p[3][4];
+    auto conformal = [&]() { // evgen.rs:93-106
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            q[i][0] = en[i] * (st[i] * sp[i]);
+            q[i][1] = en[i] * (st[i] * cp[i]);
+            q[i][2] = en[i] * ct[i];
+            q[i][3] = en[i];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            R[k] = (q[0][k] + q[1][k]) + q[2][k];
+        rn2 = R[3] * R[3] - ((R[0] * R[0] + R[1] * R[1]) + R[2] * R[2]);
+        alpha = dv(P.e_total, rn2);
+        rn = sq(rn2);
+        beta = dv(1., rn + R[3]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            rq[i] = (q[i][0] * R[0] + q[i][1] * R[1]) + q[i][2] * R[2];
+            p[i][3] = alpha * (R[3] * q[i][3] - rq[i]);
+            b[i] = beta * rq[i] - q[i][3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                p[i][k] = alpha * (rn * q[i][k] + b[i] * R[k]);
+        }
+    };
+    conformal();
+    int pos[3] = {0, 1, 2};
+    if (P.sort) { // evgen.rs:109-118: the photon at each place, then the places
+        double e0 = p[0][3], e1 = p[1][3], e2 = p[2][3];
+        int k0 = 0, k1 = 1, k2 = 2;
+        if (e1 > e0) { double t = e0; e0 = e1; e1 = t; k0 = 1; k1 = 0; }
+        if (e2 > e0) { double t = e0; e0 = e2; e2 = t; k2 = k0; k0 = 2; }
+        if (e2 > e1) { int k = k1; k1 = k2; k2 = k; }
+        pos[0] = k0 == 0 ? 0 : k1 == 0 ? 1 : 2;
+        pos[1] = k0 == 1 ? 0 : k1 == 1 ? 1 : 2;
+        pos[2] = k0 == 2 ? 0 : k1 == 2 ? 1 : 2;
+    }
+    // evcut.rs:42-96.  Only the plane cut looks at the order, and at the normal
+    // of the first two photons, so it takes them sorted.
+    bool keep = !(fmin(fmin(p[0][3], p[1][3]), p[2][3]) < P.e_min);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        keep = keep && !(fabs(p[i][0] * P.el_x) > P.cut_beam * (p[i][3] * P.el_e));
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = i + 1; j < 3; ++j)
+            keep = keep && !(((p[i][0] * p[j][0] + p[i][1] * p[j][1]) + p[i][2] * p[j][2]) > P.cut_pp * (p[i][3] * p[j][3]));
+    if (P.cut_plane > 0.) {
+        double f[3], g[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            f[k] = pos[0] == 0 ? p[0][k] : pos[1] == 0 ? p[1][k] : p[2][k];
+            g[k] = pos[0] == 1 ? p[0][k] : pos[1] == 1 ? p[1][k] : p[2][k];
+        }
+        const double n0 = f[1] * g[2] - f[2] * g[1], n1 = f[2] * g[0] - f[0] * g[2], n2 = f[0] * g[1] - f[1] * g[0];
+        keep = keep && !(fabs(P.el_x * n0) < P.cut_plane * (P.el_e * sqrt((n0 * n0 + n1 * n1) + n2 * n2)));
+    }
+    {
+        double m[5], g[5][3][3], F[5] = {0., 0., 0., 0., 0.};
+        int along = 0;
+        if (keep)
+            helicity_gradients(K, p, m, g, along);
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            if (keep)
+                F[c] = w * m[c];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                double x = 0., y = 0., z = 0., e = 0.;
+                if (keep) {
+                    x = w * g[c][i][0];
+                    y = w * g[c][i][1];
+                    e = w * g[c][i][2];
+                    z = along >> i & 1 ? 0. : e;
+                }
+                double *o = row + 12 * c + 4 * pos[i];
+                *reinterpret_cast<double2 *>(o) = double2{x, y};
+                *reinterpret_cast<double2 *>(o + 2) = double2{z, e};
+            }
+        }
+        dp_ready(F);
+    }
+    if (!want_du)
+        return;
+    // The map back to the uniforms; the divisions are the same for all sums.
+    // The map itself is computed again: kept over the gradients, its 40 values
+    // would go to scratch memory.
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        asm("" : "+v"(en[i]), "+v"(ct[i]));
+    conformal();
+    const double ir2 = tpm::rcp_n(rn2), irn = 0.5 * tpm::rcp_n(rn);
+    double cot[3], c0[3], c1[3], c2[3], c3[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        cot[i] = st[i] > 0. ? dv(ct[i], st[i]) : 0.; // no derivative of the sine along the axis
+        c0[i] = 2. * en[i];
+        c1[i] = (two_pi * en[i]) * st[i];
+        const double iem = -tpm::rcp_n(u[4 * i + 2] * u[4 * i + 3] + tiny);
+        c2[i] = iem * u[4 * i + 3];
+        c3[i] = iem * u[4 * i + 2];
+    }
+#pragma unroll 1
+    for (int c = 0; c < 5; ++c, row += 12) {
+        double qb[3][4], Rb[4] = {0., 0., 0., 0.}, ap = 0., rnb = 0., beb = 0.;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double2 xy = *reinterpret_cast<const double2 *>(row + 4 * pos[i]);
+            const double2 ze = *reinterpret_cast<const double2 *>(row + 4 * pos[i] + 2);
+            const double dp[4] = {xy.x, xy.y, ze.x, ze.y};
+            double bb = 0.;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                ap = fma_(dp[k], p[i][k], ap); // alpha d/d alpha: the momenta are alpha times the rest
+                const double t = alpha * dp[k];
+                rnb = fma_(t, q[i][k], rnb);
+                qb[i][k] = t * rn;
+                bb = fma_(t, R[k], bb);
+                Rb[k] = fma_(t, b[i], Rb[k]);
+            }
+            ap = fma_(dp[3], p[i][3], ap);
+            const double t = alpha * dp[3], rqb = fma_(beta, bb, -t);
+            Rb[3] = fma_(t, q[i][3], Rb[3]);
+            qb[i][3] = fma_(t, R[3], -bb);
+            beb = fma_(bb, rq[i], beb);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                qb[i][k] = fma_(rqb, R[k], qb[i][k]);
+                Rb[k] = fma_(rqb, q[i][k], Rb[k]);
+            }
+        }
+        const double db = -(beb * beta) * beta;
+        const double r2 = 2. * fma_(rnb + db, irn, -(ap * ir2));
+        Rb[3] = fma_(r2, R[3], Rb[3] + db);
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            Rb[k] = fma_(-r2, R[k], Rb[k]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const double x = qb[i][0] + Rb[0], y = qb[i][1] + Rb[1], z = qb[i][2] + Rb[2], e = qb[i][3] + Rb[3];
+            const double s = fma_(x, sp[i], y * cp[i]), r = fma_(x, cp[i], -(y * sp[i]));
+            const double enb = fma_(s, st[i], fma_(z, ct[i], e));
+            double2 *o = reinterpret_cast<double2 *>(row + 4 * i);
+            o[0] = keep ? double2{c0[i] * fma_(-cot[i], s, z), c1[i] * r} : double2{0., 0.};
+            o[1] = keep ? double2{c2[i] * enb, c3[i] * enb} : double2{0., 0.};
+        }
+    }
+}
+
 template <class T, int SOFT = 0>
 __device__ __forceinline__ bool event_adjoint(const AdjParams<T> &P, const T u[12], const T lam[5], T m[5], T du[12],
                                               T dp[12], T tau = (T)0, T fcap = (T)INFINITY)

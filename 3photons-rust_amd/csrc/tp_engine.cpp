@@ -1622,6 +1622,17 @@ extern "C" int tp_events(void *ctx, const tp_params *params, int rng_kind, const
     });
 }
 
+// Points per lane of the kernel that expands tp_adjoint's stream: the longest
+// run that still gives each SIMD a wavefront (whole calls at 2^20 points: 295 us
+// in runs of 10 or 20, 309 of 5, 349 of 1; at 1001: 30 us of 1, 35 of 10).
+static uint32_t adjoint_run(const Ctx *c, uint64_t n)
+{
+    for (uint32_t run : tpk::XO_RUNS)
+        if (64ull * run * 4 * c->cus <= n)
+            return run;
+    return 1;
+}
+
 extern "C" int tp_adjoint(void *ctx, const tp_params *params, int rng_kind, const void *rng_state, const void *u_in,
                           uint64_t n, int precision, int on_device, void *F, void *dF_du, void *dF_dp)
 {
@@ -1642,22 +1653,25 @@ extern "C" int tp_adjoint(void *ctx, const tp_params *params, int rng_kind, cons
         if (!u_in && 12 * n >= (1ull << KM))
             return fail(c, TP_ERR_ARG, "tp_adjoint: n exceeds the stream offset range");
         HIPCHK(c, hipSetDevice(c->device));
-        int rc = ensure_mt(c);
-        if (rc)
-            return rc;
+        int rc = TP_OK;
         tpk::AdjArgs a;
         std::memset(&a, 0, sizeof a);
         a.P = make_params(params);
+        a.hk = tpd::helicity_constants(params->e_total, params->g_a, params->g_beta_p, params->g_beta_m, 1.);
         a.w = params->ev_weight;
         a.n = n;
-        a.mt = static_cast<const uint64_t *>(c->mt.p);
-        a.km = c->km;
         if (!u_in) {
             std::memcpy(a.s0, static_cast<const tp_xoshiro_state *>(rng_state)->s, sizeof a.s0);
-            rc = ensure(c, c->adj_u, 12 * n * sizeof(double)); // the stream's points, expanded first
+            rc = xo_tables(c);
+            if (!rc)
+                rc = ensure(c, c->adj_u, 12 * n * sizeof(double)); // the stream's points, expanded first
             if (rc)
                 return rc;
             a.u_gen = static_cast<double *>(c->adj_u.p);
+            a.m16 = c->xo->m16;
+            a.run = adjoint_run(c, n);
+            a.lanes = reinterpret_cast<const uint64_t *>(
+                xo_lane_table(reinterpret_cast<const uint32_t *>(c->xo->lanes), 2 * tpk::XO_LANE_WORDS, a.run));
         }
         const size_t es = precision == TP_PREC_F32 ? sizeof(float) : sizeof(double);
         const size_t bytes[3] = {5 * n * es, 60 * n * es, 60 * n * es};
@@ -1707,7 +1721,6 @@ extern "C" int tp_adjoint(void *ctx, const tp_params *params, int rng_kind, cons
             c->last.events = n;
             c->last.batches = 0;
             c->last.host_walk_chunks = 0;
-        c->last.chunks = 0;
             c->last.chunks = 0;
         }
         return rc;

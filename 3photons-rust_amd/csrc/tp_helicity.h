@@ -121,6 +121,179 @@ TPM_FN void helicity_sums_closed(const HelicityK &K, const double p[3][4], doubl
     m[4] = x * sI;
 }
 
+// The sums and their derivatives.  With zeta = c / ez the sums separate: for
+// photon k let n0 = |1 + zeta|^2, n1 = |1 - zeta|^2, s = |zeta|^2,
+//   u = ez^2 (n0^2 + n1^2) = ez^2 (2 (1 + s)^2 + 8 Re(zeta)^2),
+//   v = ez^2 (n0^2 - n1^2) = 8 ez^2 (1 + s) Re(zeta),
+//   rho = 1 / (ez^2 n0 n1),  f = 1 / (1 - zeta^2),
+// and for the pair (a, b) beside it d = zeta_a - zeta_b, S = ez_a ez_b |d|^2 and
+// tau = d^2 f_a f_b; with Z as above
+//   sum |A|^2  = K.a sum_k u rho_a rho_b,     sum |B+|^2 = K.p sum_k u S^2,
+//   sum 2 A B* = K.x sum_k (u Re tau + i v Im tau),
+//   sum |B-|^2 = K.m Z (|sum_k (1 + zeta^2) d^2|^2 + 4 |sum_k zeta d^2|^2),
+// where tau and the two sums of the last line are analytic in the zetas.  The
+// derivatives by (ez, Re zeta, Im zeta) go over to (X, Y, ez) at the end; by
+// E and by Z are the one by ez.
+//
+// m[5]: the sums; g[c][k] = d m_c / d (X, Y, ez) of photon k.  `along`: bit k is
+// set for a photon with the spinor (0, sqrt(2 E)), which depends on E alone; its
+// X and Y derivatives are 0 and g[c][k][2] is the one by E (a photon with E
+// below -Z counts as one too, and its sums and derivatives are NaN).
+TPM_FN void helicity_gradients(const HelicityK &K, const double p[3][4], double m[5], double g[5][3][3], int &along)
+{
+    using tpm::fma_;
+    double ez[3], px[3], py[3];
+    along = 0;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        ez[k] = p[k][3] + p[k][2];
+        px[k] = p[k][0];
+        py[k] = p[k][1];
+    }
+    if (!(ez[0] > 0. && ez[1] > 0. && ez[2] > 0.)) { // as in helicity_sums_closed
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (!(ez[k] > 0.))
+                along |= 1 << k;
+            if (ez[k] == 0.) {
+                ez[k] = p[k][3] * 0x1.0p-120;
+                px[k] = tpm::sqrt_n(2. * p[k][3] * ez[k]);
+                py[k] = 0.;
+            }
+            if (!(ez[k] > 0.))
+                ez[k] = __builtin_nan("");
+        }
+    }
+    double iz[3], zr[3], zi[3], u[3], v[3], rho[3], fr[3], fi[3], Gr[3], Gi[3], ur[3], ui[3], vr[3], vi[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        iz[k] = tpm::rcp_n(ez[k]);
+        zr[k] = px[k] * iz[k];
+        zr[k] = fma_(fma_(-zr[k], ez[k], px[k]), iz[k], zr[k]);
+        zi[k] = py[k] * iz[k];
+        zi[k] = fma_(fma_(-zi[k], ez[k], py[k]), iz[k], zi[k]);
+        const double a = 1. + zr[k], b = 1. - zr[k], y2 = zi[k] * zi[k], x2 = zr[k] * zr[k];
+        const double n0 = fma_(a, a, y2), n1 = fma_(b, b, y2), in = tpm::rcp_n(n0 * n1);
+        fr[k] = fma_(a, b, y2) * in;
+        fi[k] = ((zr[k] + zr[k]) * zi[k]) * in;
+        Gr[k] = fma_(zr[k], fr[k], -(zi[k] * fi[k])); // zeta f: d f / d zeta = 2 zeta f^2
+        Gi[k] = fma_(zr[k], fi[k], zi[k] * fr[k]);
+        rho[k] = (iz[k] * iz[k]) * in;
+        const double s = x2 + y2, h = 1. + s, e2 = ez[k] * ez[k], e8 = 8. * e2;
+        u[k] = fma_(e8, x2, (2. * e2) * (h * h));
+        v[k] = (e8 * h) * zr[k];
+        ur[k] = (e8 * (3. + s)) * zr[k];
+        ui[k] = (e8 * h) * zi[k];
+        vr[k] = e8 * fma_(2., x2, h);
+        vi[k] = (2. * e8) * (zr[k] * zi[k]);
+    }
+    // derivatives by (Re zeta, Im zeta), and ez times the one by ez
+    double wr[5][3], wi[5][3], we[5][3];
+    double dr[3], di[3], Dr[3], Di[3];
+    // Pair k is (a, b) = (1, 2), (0, 2), (0, 1): photon j is its first member if
+    // j < k or (j, k) = (1, 0), else its second, where d counts negative.
+    double tr[3], ti[3], Pr = 0., Pi = 0., Tr = 0., Ti = 0.;
+    double tAr[3][3], tAi[3][3]; // d tau_k / d zeta_j
+    double cS[3];                // 2 K.p u S ez_a ez_b of the pair, twice
+    m[1] = 0.;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int a = k == 0 ? 1 : 0, b = k == 2 ? 1 : 2;
+        dr[k] = zr[a] - zr[b];
+        di[k] = zi[a] - zi[b];
+        const double di2 = di[k] * di[k], ab = ez[a] * ez[b];
+        Dr[k] = fma_(dr[k], dr[k], -di2);
+        Di[k] = (dr[k] + dr[k]) * di[k];
+        const double S = ab * fma_(dr[k], dr[k], di2), KS = K.p * S;
+        cS[k] = (4. * u[k]) * (KS * ab);
+        const double aS = KS * S;
+        wr[1][k] = aS * ur[k];
+        wi[1][k] = aS * ui[k];
+        m[1] = fma_(aS, u[k], m[1]);
+        const double hr = fma_(fr[a], fr[b], -(fi[a] * fi[b])), hi = fma_(fr[a], fi[b], fi[a] * fr[b]);
+        tr[k] = fma_(Dr[k], hr, -(Di[k] * hi));
+        ti[k] = fma_(Dr[k], hi, Di[k] * hr);
+        const double d2r = dr[k] + dr[k], d2i = di[k] + di[k], t2r = tr[k] + tr[k], t2i = ti[k] + ti[k];
+        const double er = fma_(d2r, hr, -(d2i * hi)), ei = fma_(d2r, hi, d2i * hr);
+        tAr[k][a] = fma_(t2r, Gr[a], fma_(-t2i, Gi[a], er));
+        tAi[k][a] = fma_(t2r, Gi[a], fma_(t2i, Gr[a], ei));
+        tAr[k][b] = fma_(t2r, Gr[b], fma_(-t2i, Gi[b], -er));
+        tAi[k][b] = fma_(t2r, Gi[b], fma_(t2i, Gr[b], -ei));
+        Tr = fma_(zr[k], Dr[k], fma_(-zi[k], Di[k], Tr));
+        Ti = fma_(zr[k], Di[k], fma_(zi[k], Dr[k], Ti));
+        const double qr = fma_(zr[k], zr[k], fma_(-zi[k], zi[k], 1.)), qi = (zr[k] + zr[k]) * zi[k];
+        Pr = fma_(qr, Dr[k], fma_(-qi, Di[k], Pr));
+        Pi = fma_(qr, Di[k], fma_(qi, Dr[k], Pi));
+    }
+    // sum |A|^2 and the interference
+    double A[3], AU[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int a = k == 0 ? 1 : 0, b = k == 2 ? 1 : 2;
+        A[k] = (K.a * rho[a]) * rho[b];
+        AU[k] = A[k] * u[k];
+    }
+    m[0] = (AU[0] + AU[1]) + AU[2];
+    m[3] = K.x * fma_(u[0], tr[0], fma_(u[1], tr[1], u[2] * tr[2]));
+    m[4] = K.x * fma_(v[0], ti[0], fma_(v[1], ti[1], v[2] * ti[2]));
+    const double Z = (ez[0] * ez[1]) * ez[2], KZ = (K.m * Z) * Z;
+    m[2] = KZ * fma_(4., fma_(Tr, Tr, Ti * Ti), fma_(Pr, Pr, Pi * Pi));
+    const double K2 = KZ + KZ, Kx2 = K.x + K.x;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int a = k == 0 ? 1 : 0, b = k == 2 ? 1 : 2;
+        const double bk = 4. * (AU[a] + AU[b]); // 4 rho d / d rho
+        wr[0][k] = fma_(bk, Gr[k], A[k] * ur[k]);
+        wi[0][k] = fma_(-bk, Gi[k], A[k] * ui[k]);
+        we[0][k] = fma_(-0.5, bk, AU[k] + AU[k]);
+        // pair a is (k, b) or (b, k), pair b is (k, a) or (a, k)
+        const double sa = k < b ? cS[a] : -cS[a], sb = k < a ? cS[b] : -cS[b];
+        wr[1][k] = fma_(sa, dr[a], fma_(sb, dr[b], wr[1][k]));
+        wi[1][k] = fma_(sa, di[a], fma_(sb, di[b], wi[1][k]));
+        we[1][k] = m[1] + m[1];
+        const double Rr = fma_(u[a], tAr[a][k], u[b] * tAr[b][k]), Ri = fma_(u[a], tAi[a][k], u[b] * tAi[b][k]);
+        const double Ir = fma_(v[a], tAr[a][k], v[b] * tAr[b][k]), Ii = fma_(v[a], tAi[a][k], v[b] * tAi[b][k]);
+        wr[3][k] = K.x * fma_(ur[k], tr[k], Rr);
+        wi[3][k] = K.x * fma_(ui[k], tr[k], -Ri);
+        we[3][k] = Kx2 * (u[k] * tr[k]);
+        wr[4][k] = K.x * fma_(vr[k], ti[k], Ii);
+        wi[4][k] = K.x * fma_(vi[k], ti[k], Ir);
+        we[4][k] = Kx2 * (v[k] * ti[k]);
+        // d/d zeta_k of sum zeta d^2 and, halved, of sum (1 + zeta^2) d^2
+        const double ga = k < b ? 1. : -1., gb = k < a ? 1. : -1.;
+        const double Yar = fma_(zr[a], dr[a], -(zi[a] * di[a])), Yai = fma_(zr[a], di[a], zi[a] * dr[a]);
+        const double Ybr = fma_(zr[b], dr[b], -(zi[b] * di[b])), Ybi = fma_(zr[b], di[b], zi[b] * dr[b]);
+        const double T1r = fma_(2., fma_(ga, Yar, gb * Ybr), Dr[k]), T1i = fma_(2., fma_(ga, Yai, gb * Ybi), Di[k]);
+        const double Wr = fma_(ga, fma_(zr[a], Yar, fma_(-zi[a], Yai, dr[a])), gb * fma_(zr[b], Ybr, fma_(-zi[b], Ybi, dr[b])));
+        const double Wi = fma_(ga, fma_(zr[a], Yai, fma_(zi[a], Yar, di[a])), gb * fma_(zr[b], Ybi, fma_(zi[b], Ybr, di[b])));
+        const double P1r = fma_(zr[k], Dr[k], fma_(-zi[k], Di[k], Wr)), P1i = fma_(zr[k], Di[k], fma_(zi[k], Dr[k], Wi));
+        // 2 conj(P) P1 + 4 conj(T) T1
+        const double hr = fma_(4., fma_(Tr, T1r, Ti * T1i), 2. * fma_(Pr, P1r, Pi * P1i));
+        const double hi = fma_(4., fma_(Tr, T1i, -(Ti * T1r)), 2. * fma_(Pr, P1i, -(Pi * P1r)));
+        wr[2][k] = K2 * hr;
+        wi[2][k] = -(K2 * hi);
+        we[2][k] = m[2] + m[2];
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            g[c][k][0] = wr[c][k] * iz[k];
+            g[c][k][1] = wi[c][k] * iz[k];
+            g[c][k][2] = fma_(-zr[k], wr[c][k], fma_(-zi[k], wi[c][k], we[c][k])) * iz[k];
+        }
+    if (along) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (along >> k & 1) // X = sqrt(ez) sqrt(2 E): d/dE = d/dX ez / X
+#pragma unroll
+                for (int c = 0; c < 5; ++c) {
+                    g[c][k][2] = g[c][k][0] / zr[k];
+                    g[c][k][0] = g[c][k][1] = 0.;
+                }
+    }
+}
+
 // The power of two that takes e_total into [64, 128) (1 for the shipped
 // 91.187 GeV): momenta and energies scaled by it keep every bit.
 inline double energy_unit(double e_total)

@@ -305,26 +305,22 @@ namespace tpk {
 
 // Arguments of the adjoint kernel (tp_adjoint).
 // The adjoint kernels run one 64-lane workgroup per 64 consecutive points,
-// one point per lane; the f32 kernel stores the rows through LDS
-// (tp_adjstore.h), the f64 kernel straight from registers.  Points of the
-// xoshiro stream (u_in null) are first expanded into u_gen by a kernel whose
-// threads each step through ADJ_GEN_POINTS consecutive points from one
-// skip-ahead.
+// one point per lane, and store the rows through LDS.  Points of the
+// xoshiro stream (u_in null) are first expanded into u_gen.
 struct AdjArgs {
     tpd::Params P;
+    tpd::HelicityK hk;     // f64: the sums in the caller's units
     double w;              // RAMBO event weight
     uint64_t n;            // points
-    // uniforms: u_in (n x 12 doubles) if non-null, else xoshiro from s0 via mt,
-    // expanded into u_gen (n x 12 doubles)
+    // uniforms: u_in (n x 12 doubles) if non-null, else xoshiro from s0,
+    // expanded into u_gen (n x 12 doubles) `run` points per lane
     const double *u_in;
     double *u_gen;
     uint64_t s0[4];
-    const uint64_t *mt;
-    int32_t km;
+    const uint64_t *m16, *lanes; // as FusedArgs
+    uint32_t run;          // one of XO_RUNS
     void *F, *dF_du, *dF_dp; // [n][5], [n][5][12], [n][5][12] of double or float
 };
-constexpr uint32_t ADJ_GEN_POINTS = 256;
-
 void launch_adjoint(const AdjArgs &a, int precision /*TP_PREC_F64 or TP_PREC_F32*/, hipStream_t st);
 
 } // namespace tpk

@@ -2276,7 +2276,7 @@ void launch_f32_accumulate(const F32Args &a, hipStream_t st)
 
 namespace tpk {
 
-// One 64-lane workgroup per 64 consecutive points.  The sweeps run
+// One 64-lane workgroup per 64 consecutive points.  In f32 the sweeps run
 // convergently (a cut point's lane runs them too and hands zeros on), so the
 // sink can synchronise the workgroup: it stages F and dF/du in LDS for the
 // whole pass and dF/dp one sweep at a time, and the stores go out with
@@ -2292,36 +2292,68 @@ template <int K, class T, class Put> __device__ __forceinline__ void flush_full(
         put(lane + tpa::LANES * k, stage[lane + tpa::LANES * k]);
 }
 
-// One point per lane, each sweep's values stored straight from registers:
-// a store instruction writes 64 rows 480 B apart (f64), so lines reach HBM
-// partly written (WRITE_SIZE 1.28x the output bytes), but nothing waits on
-// them.  The f64 kernel, at one wavefront per SIMD, is fastest this way.
-template <class T> __device__ __forceinline__ void adjoint_direct(const AdjArgs &a)
+// Pairs of doubles, for pointers a caller has aligned to one.
+typedef double pair8 __attribute__((ext_vector_type(2), aligned(8)));
+
+// f64: one point per lane, all derivatives from one evaluation of the closed
+// forms (event_jacobian), rows staged in LDS and stored 1 KiB per instruction.
+// Bound by the 1000 bytes a point writes (1.05 GB per 2^20 points: 153 us at
+// the rate of a fill); its 1600 f64 instructions a point take 80 us of issue.
+// One row at a time in LDS, dF/dp and then dF/du in its place: five workgroups
+// per CU and 256 VGPRs.  2^20 points: 210 us; with five sweeps back through the
+// amplitudes 487 (one wavefront per SIMD); with rows stored straight from
+// registers, 96 B of each per sweep and lane, 620.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void adjoint_kernel_f64(AdjArgs a)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.n)
+    constexpr uint32_t ROW = 62; // doubles: an odd number of 16-byte units, so lanes fall on different banks
+    __shared__ __attribute__((aligned(16))) double rows[ROW * tpa::LANES];
+    const uint32_t lane = threadIdx.x;
+    const uint64_t base = (uint64_t)blockIdx.x * tpa::LANES;
+    if (base >= a.n) // whole workgroup
         return;
-    const AdjParams<T> P = adj_params<T>(a.P, a.w);
-    T *F = reinterpret_cast<T *>(a.F), *Gu = reinterpret_cast<T *>(a.dF_du), *Gp = reinterpret_cast<T *>(a.dF_dp);
-    T u[12];
+    const uint32_t np = tpa::points(a.n, base);
+    double *F = reinterpret_cast<double *>(a.F), *Gu = reinterpret_cast<double *>(a.dF_du), *Gp = reinterpret_cast<double *>(a.dF_dp);
+    const double *uu = a.u_in + 12 * (base + (lane < np ? lane : 0)); // lanes past n: a copy of point base, never stored
+    double u[12];
 #pragma unroll
-    for (int j = 0; j < 12; ++j)
-        u[j] = (T)a.u_in[12 * i + j];
-    // one forward pass, then one reverse sweep per coupling component
-    T m[5], du[12], dp[12];
-    event_adjoint_sweeps<T, 0, 5>(P, u, nullptr, m, du, dp, (T)0, (T)INFINITY,
-                                  [&](int c, const T *mc, const T *duc, const T *dpc) {
-                                      if (F)
-                                          F[5 * i + c] = P.w * (c == 0 ? mc[0] : c == 1 ? mc[1] : c == 2 ? mc[2] : c == 3 ? mc[3] : mc[4]);
-                                      if (Gu)
+    for (int j = 0; j < 6; ++j) {
+        const pair8 x = *reinterpret_cast<const pair8 *>(uu + 2 * j);
+        u[2 * j] = x.x;
+        u[2 * j + 1] = x.y;
+    }
+    // 16-byte element e of the workgroup's rows, e < 30 np: row e / 30
+    auto flush = [&](double *out) {
+        double *o = out + 60 * base;
+        uint32_t pt = lane / 30, r = lane % 30;
+        auto put = [&](uint32_t e) {
+            const double2 x = *reinterpret_cast<const double2 *>(rows + ROW * pt + 2 * r);
+            *reinterpret_cast<pair8 *>(o + 2 * e) = pair8{x.x, x.y};
+            r += 4; // 64 = 2 * 30 + 4
+            pt += r >= 30 ? 3 : 2;
+            r -= r >= 30 ? 30 : 0;
+        };
+        if (np == tpa::LANES)
+#pragma unroll 10
+            for (uint32_t k = 0; k < 30; ++k)
+                put(lane + 64 * k);
+        else
+            for (uint32_t e = lane; e < 30 * np; e += 64)
+                put(e);
+    };
+    event_jacobian(a.P, a.hk, a.w, u, rows + ROW * lane, Gu != nullptr, [&](const double *Fc) {
+        if (F && lane < np)
 #pragma unroll
-                                          for (int j = 0; j < 12; ++j)
-                                              Gu[60 * i + 12 * c + j] = duc[j];
-                                      if (Gp)
-#pragma unroll
-                                          for (int j = 0; j < 12; ++j)
-                                              Gp[60 * i + 12 * c + j] = dpc[j];
-                                  });
+            for (int c = 0; c < 5; ++c)
+                F[5 * (base + lane) + c] = Fc[c];
+        __syncthreads();
+        if (Gp)
+            flush(Gp);
+        __syncthreads();
+    });
+    if (Gu) {
+        __syncthreads();
+        flush(Gu);
+    }
 }
 
 // One point per lane, rows staged in LDS and stored with consecutive lanes
@@ -2383,31 +2415,29 @@ template <class T> __device__ __forceinline__ void adjoint_staged(const AdjArgs 
     }
 }
 
-// The stream's points, ADJ_GEN_POINTS consecutive ones per thread from one
-// skip-ahead (12 draws per point, rand's Standard f64).
+// The stream's points (12 draws each, rand's Standard f64): a wavefront skips
+// to its first draw, its lanes take `run` consecutive points each from there.
+// Bound by latency, of the skip and of stores 96 B per lane: 46 us per 2^20
+// points, 540 with one skip per thread and 256 points each.
 __global__ __launch_bounds__(64) void adjoint_points_kernel(AdjArgs a)
 {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t first = t * ADJ_GEN_POINTS;
-    if (first >= a.n)
-        return;
-    uint64_t s[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]};
-    const uint64_t off = 12ull * first;
-    for (int k = 0; k < a.km; ++k)
-        if ((off >> k) & 1ull)
-            gf2_apply(a.mt + 1024 * k, s);
-    const uint64_t last = first + ADJ_GEN_POINTS < a.n ? first + ADJ_GEN_POINTS : a.n;
-    double *out = a.u_gen + 12 * first;
-    for (uint64_t k = 0; k < 12 * (last - first); ++k)
-        out[k] = xo_uniform(s);
+    const uint64_t base = 64ull * a.run * blockIdx.x;
+    uint64_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}, s[4];
+    xo_advance_uniform(a.m16, 12 * base, sw);
+    xo_lane_states(a.lanes, sw, s);
+    const uint64_t first = base + (uint64_t)a.run * threadIdx.x, last = min(first + a.run, a.n);
+    for (uint64_t k = first; k < last; ++k) {
+        pair8 *out = reinterpret_cast<pair8 *>(a.u_gen + 12 * k);
+#pragma unroll
+        for (int j = 0; j < 6; ++j) {
+            const double x = xo_uniform(s);
+            out[j] = pair8{x, xo_uniform(s)};
+        }
+    }
 }
 
-// f64: 256 VGPRs + 218 AGPRs, one wavefront per SIMD (two would spill
-// hundreds of bytes per lane); with the staged store (39.4 KB of LDS) it ran
-// 2.5 % slower than with direct stores, so it stores directly.
 // f32: 255 VGPRs, two wavefronts per SIMD (waves_per_eu(2, 2)), no spill;
 // 19.7 KB of stage, eight workgroups per CU.
-__global__ __launch_bounds__(64) void adjoint_kernel_f64(AdjArgs a) { adjoint_direct<double>(a); }
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2))) void adjoint_kernel_f32(AdjArgs a)
 {
     __shared__ float sF[5 * tpa::LANES], sU[60 * tpa::LANES], sP[12 * tpa::LANES];
@@ -2418,8 +2448,8 @@ void launch_adjoint(const AdjArgs &a0, int precision, hipStream_t st)
 {
     AdjArgs a = a0;
     if (!a.u_in) {
-        const uint64_t threads = (a.n + ADJ_GEN_POINTS - 1) / ADJ_GEN_POINTS;
-        hipLaunchKernelGGL(adjoint_points_kernel, dim3((unsigned)((threads + 63) / 64)), dim3(64), 0, st, a);
+        const uint64_t wave = 64ull * a.run;
+        hipLaunchKernelGGL(adjoint_points_kernel, dim3((unsigned)((a.n + wave - 1) / wave)), dim3(64), 0, st, a);
         a.u_in = a.u_gen;
     }
     const dim3 g((unsigned)((a.n + tpa::LANES - 1) / tpa::LANES)), b(tpa::LANES);
