@@ -103,7 +103,20 @@ struct Ctx {
 };
 
 constexpr int KM = 32;              // intra-call offsets < 2^32 draws
-constexpr int RANF_R = 2048;        // RANF rounds per expansion segment (one jump per segment)
+// RANF rounds per segment of an expansion (one wavefront and one jump each), of
+// `rounds` in all: the most, up to 512, that give each SIMD six wavefronts, as a
+// round waits on its LDS permutes for several times its issue.  Whole runs with
+// segments of 2048, 512, 256, 128 and 64 rounds (faster-evgen): 1e7 events 1412,
+// 1074, 1061, 1137, 1298 us; 1.2e6 events 987, 558, 480, 464, 470 us; 5e7 with
+// jump seeding 5170, 4423, 4436, 4552, 4997 us; 1e8 8442, 8326, 8721, 9833 us.
+constexpr int RANF_R_MIN = 64, RANF_R_MAX = 512;
+inline int ranf_seg_rounds(const Ctx *c, uint64_t rounds)
+{
+    int r = RANF_R_MAX;
+    while (r > RANF_R_MIN && rounds / r < 24ull * c->cus)
+        r /= 2;
+    return r;
+}
 // Where tp_guard stores an exception's message for tp_last_error.
 inline std::string *ctx_err(void *ctx) { return ctx ? &static_cast<Ctx *>(ctx)->err : nullptr; }
 

@@ -317,8 +317,7 @@ constexpr uint64_t FE_XO_WORDS = FE_XO_PIECE / 32; // accept-bit words per piece
 static_assert(FE_XO_PER_THREAD % 128 == 0, "whole groups of 4 bit words per lane");
 // Accept-bit words per RANF expansion segment (each segment's bits start on
 // a word of their own).
-constexpr uint64_t RANF_SEG_WORDS = 55ull * RANF_R / 32;
-static_assert(55ull * RANF_R % 32 == 0, "RANF segments of whole bit words");
+static_assert(RANF_R_MIN % 32 == 0, "RANF segments of whole bit words");
 
 namespace {
 
@@ -344,10 +343,11 @@ int ensure_acc(Ctx *c, uint64_t np) { return ensure_acc_words(c, np * FE_XO_WORD
 // from *bbase, the first position of the first expansion segment, on.
 int fe_expand(Ctx *c, uint64_t p0_master, uint64_t q_first, uint64_t q_last, int kind, uint64_t *bbase)
 {
-    const uint64_t seg_first = q_first / 55 / RANF_R, nsegs = (q_last - 1) / 55 / RANF_R - seg_first + 1;
+    const uint64_t R = ranf_seg_rounds(c, (q_last - q_first) / 55);
+    const uint64_t seg_first = q_first / 55 / R, nsegs = (q_last - 1) / 55 / R - seg_first + 1;
     int rc = ensure(c, c->draws, (q_last - q_first) * sizeof(int32_t));
     if (!rc)
-        rc = ensure_acc_words(c, nsegs * RANF_SEG_WORDS);
+        rc = ensure_acc_words(c, nsegs * (55 * R / 32));
     if (rc)
         return rc;
     tpk::RanfArgs r;
@@ -355,7 +355,7 @@ int fe_expand(Ctx *c, uint64_t p0_master, uint64_t q_first, uint64_t q_last, int
     r.origin = static_cast<const int32_t *>(c->origin.p);
     r.p0 = static_cast<const int32_t *>(c->p0.p);
     r.r16 = static_cast<const uint32_t *>(c->r16.p);
-    r.R = RANF_R;
+    r.R = (int32_t)R;
     r.out = static_cast<int32_t *>(c->draws.p);
     r.d_begin = q_first - p0_master;
     r.d_end = q_last - p0_master;
@@ -367,7 +367,7 @@ int fe_expand(Ctx *c, uint64_t p0_master, uint64_t q_first, uint64_t q_last, int
     r.acc3 = r.acc1 + c->xo_acc_words;
     tpk::launch_ranf_expand(r, 1, c->stream);
     HIPCHK(c, hipGetLastError());
-    *bbase = seg_first * 55 * RANF_R;
+    *bbase = seg_first * 55 * R;
     return TP_OK;
 }
 
@@ -795,7 +795,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     const uint64_t PS = FE_JUMP_PIECE * ((batch_size + TP_BATCH_SIZE - 1) / TP_BATCH_SIZE);
-    const uint64_t max_rounds = PS / 55 + 2;
+    const uint64_t max_rounds = PS / 55 + 2, R = ranf_seg_rounds(c, chunk * max_rounds);
     int rc = ensure_r16(c);
     if (!rc)
         rc = ensure(c, c->draws, chunk * PS * sizeof(int32_t));
@@ -808,7 +808,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
     if (!rc)
         rc = ensure(c, c->fe_flag, sizeof(uint32_t));
     if (!rc) // each piece's bits: its segments' words, the last one cut at the piece's end
-        rc = ensure_acc_words(c, (chunk + 1) * (PS / 32) + RANF_SEG_WORDS);
+        rc = ensure_acc_words(c, (chunk + 1) * (PS / 32) + 55 * R / 32);
     if (rc)
         return rc;
     tpk::F32Args fa;
@@ -830,12 +830,12 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         r.origin = static_cast<const int32_t *>(c->origin.p) + 56 * first_piece;
         r.p0 = static_cast<const int32_t *>(c->p0.p) + first_piece;
         r.r16 = static_cast<const uint32_t *>(c->r16.p);
-        r.R = RANF_R;
+        r.R = (int32_t)R;
         r.out = static_cast<int32_t *>(c->draws.p) + first_piece * PS;
         r.d_begin = d_begin;
         r.d_end = d_end;
         r.seg_first = 0;
-        r.nsegs = (max_rounds + RANF_R - 1) / RANF_R + 1;
+        r.nsegs = (max_rounds + R - 1) / R + 1;
         r.piece_stride = PS;
         r.bits = f32 ? 2 : 1;
         r.bits_piece_words = PS / 32;
@@ -1574,12 +1574,12 @@ extern "C" int tp_events(void *ctx, const tp_params *params, int rng_kind, const
             r.origin = static_cast<const int32_t *>(c->origin.p);
             r.p0 = static_cast<const int32_t *>(c->p0.p);
             r.r16 = static_cast<const uint32_t *>(c->r16.p);
-            r.R = RANF_R;
+            r.R = ranf_seg_rounds(c, D / 55);
             r.out = static_cast<int32_t *>(c->draws.p);
             r.d_begin = 0;
             r.d_end = D;
             r.seg_first = 0;
-            r.nsegs = (c->p00 + D - 1) / 55 / RANF_R + 1;
+            r.nsegs = (c->p00 + D - 1) / 55 / r.R + 1;
             tpk::launch_ranf_expand(r, 1, c->stream);
             HIPCHK(c, hipGetLastError());
             a.draws = static_cast<const int32_t *>(c->draws.p);
