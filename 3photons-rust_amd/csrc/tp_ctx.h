@@ -7,7 +7,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <map>
 #include <memory>
 #include <string>
 #include <vector>
@@ -39,11 +38,6 @@ template <int N> struct ScopedBufs {
     }
 };
 
-struct Tables { // device copy of the powers 2^k of a GF(2) matrix
-    DevBuf bt;
-    int kb = 0;
-};
-
 // xoshiro skip tables of one device, filled once by the first tp_create on
 // it and only read afterwards (tp_kernels.h).
 struct XoTables {
@@ -51,7 +45,7 @@ struct XoTables {
     std::string err;
     const uint64_t *m16 = nullptr;     // M^(v 16^j), M one draw
     const uint64_t *b16[2] = {nullptr, nullptr}; // B^(v 16^j): M^(12 * 10 000), the 2^128 jump (by seeding)
-    const uint64_t *lanes = nullptr;   // lane tables of every run length
+    const uint64_t *lanes = nullptr;   // lane tables of every run length, then of the pieces of a stream
     const uint32_t *m16_128 = nullptr, *b16_128[2] = {nullptr, nullptr}, *lanes128 = nullptr; // the same of xoshiro128+
 };
 
@@ -66,7 +60,6 @@ struct Ctx {
     std::string err;
     DevBuf mt;       // M^(2^k)
     int km = 0;
-    std::map<std::string, std::unique_ptr<Tables>> tables;
     DevBuf r16;             // RANF: jump polynomials of the digits of a number of rounds
     bool r16_ready = false;
     DevBuf draws, origin, p0, per_batch, merged, evq;
@@ -87,13 +80,9 @@ struct Ctx {
     DevBuf fe_stat;  // the device walk's stitch status: failed, start n
     uint64_t *fe_stat_host = nullptr; // its pinned host copy (hipHostMalloc)
     DevBuf fe_seq;   // jump seeding: batches left to the one-thread walk
-    DevBuf xo_states, xo_draws; // faster-evgen on xoshiro256+: piece states and uniforms
-    DevBuf xo128_states, xo128_draws, xo128_pt; // the same on xoshiro128+ (f32), and the piece matrix powers
+    DevBuf xo_draws, xo128_draws; // faster-evgen on xoshiro256+, on xoshiro128+ (f32): the pieces' uniforms
     DevBuf xo_acc;              // accept bits of the expanded xoshiro pieces: acc1, then acc3
-    DevBuf xo_lt, xo128_lt;     // the expanding lanes' skip matrices (xoshiro256+, xoshiro128+)
     uint64_t xo_acc_words = 0;  // words per array in xo_acc
-    std::string xo128_pt_key;
-    int xo128_pt_kb = 0;
     DevBuf adj_u;               // tp_adjoint: the stream's points, expanded
     uint32_t fe_flag_host = 0;
     uint64_t fe_qnext = 0;  // the device walk's start n: where the next chunk begins

@@ -127,32 +127,6 @@ namespace {
 
 using namespace tpe;
 
-int bits_for(uint64_t n);
-
-// B^(2^k), k < kb, of the xoshiro128+ piece matrix B (the 2^64 jump, or
-// M^piece_len for pieces tiling one stream), into c->xo128_pt.
-int ensure_xo128_piece_table(Ctx *c, bool jump, uint64_t piece_len, uint64_t max_piece)
-{
-    const int kb = std::max(1, bits_for(max_piece + 1));
-    const std::string key = jump ? std::string("jump") : "piece:" + std::to_string(piece_len);
-    if (c->xo128_pt_key == key && c->xo128_pt_kb >= kb)
-        return TP_OK;
-    tp::Gf2Mat128 B;
-    if (jump)
-        tp::gf2_128_jump64(B);
-    else
-        tp::gf2_128_pow_from_table(tp::xoshiro128_step_pow2(), piece_len, B);
-    const std::vector<tp::Gf2Mat128> bt = tp::gf2_128_pow2_table(B, kb);
-    int rc = ensure(c, c->xo128_pt, bt.size() * sizeof(tp::Gf2Mat128));
-    if (rc)
-        return rc;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(c->xo128_pt.p, bt.data(), bt.size() * sizeof(tp::Gf2Mat128), hipMemcpyHostToDevice));
-    c->xo128_pt_key = key;
-    c->xo128_pt_kb = kb;
-    return TP_OK;
-}
-
 // Batches per launch of the xoshiro128+ events in registers:
 // 24576 * 10000 events * 24 B = 5.9 GB of per-event values.
 constexpr uint64_t F32_CHUNK_BATCHES = 24576;
@@ -220,37 +194,6 @@ int ensure_mt(Ctx *c)
     return TP_OK;
 }
 
-int bits_for(uint64_t n)
-{
-    int k = 0;
-    while (k < 64 && (n >> k))
-        ++k;
-    return k;
-}
-
-// The 2^128 jump as a table of its powers 2^k up to nb (faster-evgen with jump
-// seeding).
-int ensure_jump_table(Ctx *c, uint64_t nb, Tables **out)
-{
-    const int kb = std::max(1, bits_for(nb));
-    const std::string key = "jump";
-    auto it = c->tables.find(key);
-    if (it != c->tables.end() && it->second->kb >= kb) {
-        *out = it->second.get();
-        return TP_OK;
-    }
-    tp::Gf2Mat B;
-    tp::gf2_jump128(B);
-    std::unique_ptr<Tables> t(new Tables);
-    int rc = upload_mats(c, t->bt, tp::gf2_pow2_table(B, kb));
-    if (rc)
-        return rc;
-    t->kb = kb;
-    *out = t.get();
-    c->tables[key] = std::move(t);
-    return TP_OK;
-}
-
 // The jump polynomials of the digits of a number of RANF rounds, into c->r16
 // (once per context).
 int ensure_r16(Ctx *c)
@@ -288,35 +231,38 @@ int check_common(Ctx *c, const tp_params *params, int rng_kind, const void *stat
 // them with its stream expanded into HBM.  Runs of FE_DEVICE_WALK_MIN events
 // or more walk the stream on the device (fe_walk_kernel: segment walkers
 // joined where they meet); shorter runs, and any chunk whose device walkers
-// do not all join, take the host walk.
-constexpr uint64_t FE_DEVICE_WALK_MIN = 1u << 20;
+// do not all join, take the host walk, 20 to 90 ns an event.  The device's takes
+// its launches and a segment's length at least.  Closures of 2000, 8000, 32 000
+// and 300 000 events on the host and on the device: RANF 120, 190, 706, 5900 us
+// and 175, 175, 178, 221; xoshiro256+ 153, 363, 1149, 9880 us and about 800 (a
+// segment has 1024 events there).
+constexpr uint64_t FE_DEVICE_WALK_MIN = 8192, FE_XO_DEVICE_WALK_MIN = 16384;
 constexpr uint64_t FE_WALK_BATCHES = 12288; // batches per chunk: four strides of the event-loop grid
 constexpr double FE_POSITIONS_PER_EVENT = 18.5; // stream positions allowed for per event (mean 17.9)
-constexpr uint64_t FE_EVENTS_PER_WALKER = 256, FE_MAX_WALKERS = 1u << 18;
+constexpr uint64_t FE_MAX_WALKERS = 1u << 18;
 static_assert(FE_MAX_WALKERS <= 256ull * tpk::FE_STITCH_THREADS, "the device stitch's block sums fit one workgroup");
-// Positions a walker goes past its segment's end: 24 rounds, ~74 events; a
-// walker meets the true walk within 49 events in the runs checked.
-constexpr uint64_t FE_OVERLAP = 24 * 55;
+// A walker's segment, and how far past its end it goes at most to meet the
+// next one: 24 rounds, ~74 events; a walker meets the true walk within 49
+// events in the runs checked.
+constexpr uint64_t FE_SEG = 24 * 55, FE_OVERLAP = 24 * 55;
 // The xoshiro256+ stream has no rounds whose discards bring walkers together:
 // a walker meets the true walk only where both happen to start an event, after
 // a median of 22 events but a long tail (at most 832 over 176 447 walkers of a
-// simulated 1.5e9-draw stream, 12 of them past 512).  Its walkers therefore
-// take 1024 events each and go 1024 events (17 500 positions) past their
-// segment; 16.64 positions per event on average, 17.0 allowed for.
+// simulated 1.5e9-draw stream, 12 of them past 512).  On one stream its
+// walkers, which have to meet the next one within its segment, therefore take
+// 1024 events each; a batch's own stream is walked by chains of walkers that
+// may leave some out, 256 events each, going up to 1024 events (17 500
+// positions) past their segment; 16.64 positions per event on average, 17.0
+// allowed for.
 constexpr double FE_XO_POSITIONS_PER_EVENT = 17.0;
-constexpr uint64_t FE_XO_EVENTS_PER_WALKER = 1024, FE_XO_OVERLAP = 17500;
-// xoshiro streams are expanded in pieces of FE_XO_PIECE uniforms, one
-// wavefront per piece and FE_XO_PER_THREAD consecutive draws per lane from one
-// skip-ahead (a multiple of 128: the lanes' accept-bit words go out 4 at a
-// time).  With jump seeding a piece is a batch's stream; with skip-ahead
-// seeding the pieces tile the run's one stream (piece p starts FE_XO_PIECE p
-// draws after the run's state).
-constexpr uint32_t FE_XO_PER_THREAD = 2688;
-constexpr uint64_t FE_XO_PIECE = 64 * FE_XO_PER_THREAD;
+constexpr uint64_t FE_XO_EVENTS_PER_WALKER = 1024, FE_XO_BATCH_EVENTS_PER_WALKER = 1024, FE_XO_OVERLAP = 17500;
+// xoshiro streams are expanded in pieces of FE_XO_PIECE uniforms, seven
+// wavefronts each.  With jump seeding a piece is a batch's stream; with
+// skip-ahead seeding the pieces tile the run's one stream (piece p starts
+// FE_XO_PIECE p draws after the run's state).
+constexpr uint64_t FE_XO_PIECE = 7 * 64 * 12 * tpk::XO_EXPAND_RUN;
+static_assert(FE_XO_PIECE == 172032);
 constexpr uint64_t FE_XO_WORDS = FE_XO_PIECE / 32; // accept-bit words per piece and test
-static_assert(FE_XO_PER_THREAD % 128 == 0, "whole groups of 4 bit words per lane");
-// Accept-bit words per RANF expansion segment (each segment's bits start on
-// a word of their own).
 static_assert(RANF_R_MIN % 32 == 0, "RANF segments of whole bit words");
 
 namespace {
@@ -326,7 +272,7 @@ namespace {
 // stays put while the buffer is reused).
 int ensure_acc_words(Ctx *c, uint64_t need)
 {
-    const uint64_t words = std::max(need, c->xo_acc_words);
+    const uint64_t words = std::max<uint64_t>((need + 3) & ~3ull, c->xo_acc_words); // acc3 starts at whole 16 bytes
     int rc = ensure(c, c->xo_acc, 2 * words * sizeof(uint32_t));
     if (rc)
         return rc;
@@ -380,37 +326,12 @@ struct FeStream {
 };
 
 
-// M^(FE_XO_PER_THREAD 2^j), j < 6, of both xoshiro generators: the expanding
-// lanes' skips (lane l skips l * FE_XO_PER_THREAD draws into its piece).
-int ensure_lane_tables(Ctx *c)
+// Expands xoshiro128+ pieces b_first .. b_first + np - 1 of FE_XO_PIECE f32
+// uniforms into c->xo128_draws: the batches' streams (jump) or pieces of the one
+// that starts at s0.
+int xo128_expand(Ctx *c, const uint32_t s0[4], bool jump, uint64_t b_first, uint64_t np)
 {
-    if (!c->xo_lt.p) {
-        tp::Gf2Mat m;
-        tp::gf2_pow_from_table(tp::xoshiro_step_pow2(), FE_XO_PER_THREAD, m);
-        int rc = upload_mats(c, c->xo_lt, tp::gf2_pow2_table(m, 6));
-        if (rc)
-            return rc;
-    }
-    if (!c->xo128_lt.p) {
-        tp::Gf2Mat128 m;
-        tp::gf2_128_pow_from_table(tp::xoshiro128_step_pow2(), FE_XO_PER_THREAD, m);
-        const std::vector<tp::Gf2Mat128> t = tp::gf2_128_pow2_table(m, 6);
-        int rc = ensure(c, c->xo128_lt, t.size() * sizeof(tp::Gf2Mat128));
-        if (rc)
-            return rc;
-        HIPCHK(c, hipMemcpy(c->xo128_lt.p, t.data(), t.size() * sizeof(tp::Gf2Mat128), hipMemcpyHostToDevice));
-    }
-    return TP_OK;
-}
-
-// Expands xoshiro128+ pieces b_first .. b_first + np - 1 of piece_len f32
-// uniforms into c->xo128_draws (piece k from B^(b_first + k) s0, B as
-// ensure_xo128_piece_table made it).
-int xo128_expand(Ctx *c, const uint32_t s0[4], uint64_t b_first, uint64_t np)
-{
-    int rc = ensure_lane_tables(c);
-    if (!rc)
-        rc = ensure(c, c->xo128_states, np * 4 * sizeof(uint32_t));
+    int rc = xo_tables(c);
     if (!rc)
         rc = ensure(c, c->xo128_draws, np * FE_XO_PIECE * sizeof(float));
     if (!rc)
@@ -420,14 +341,12 @@ int xo128_expand(Ctx *c, const uint32_t s0[4], uint64_t b_first, uint64_t np)
     tpk::Xo128PieceArgs p;
     std::memset(&p, 0, sizeof p);
     std::memcpy(p.s0, s0, sizeof p.s0);
-    p.bt = static_cast<const uint32_t *>(c->xo128_pt.p);
-    p.kb = c->xo128_pt_kb;
-    p.lt = static_cast<const uint32_t *>(c->xo128_lt.p);
+    p.m16 = c->xo->m16_128;
+    p.b16 = jump ? c->xo->b16_128[TP_SEED_JUMP] : nullptr;
+    p.lanes = c->xo->lanes128 + tpk::XO_NRUNS * tpk::XO128_LANE_WORDS;
     p.nb = np;
     p.b_first = b_first;
-    p.states = static_cast<uint32_t *>(c->xo128_states.p);
     p.piece_len = FE_XO_PIECE;
-    p.per_thread = FE_XO_PER_THREAD;
     p.xbuf = static_cast<float *>(c->xo128_draws.p);
     p.acc1 = static_cast<uint32_t *>(c->xo_acc.p);
     p.acc3 = p.acc1 + c->xo_acc_words;
@@ -436,25 +355,30 @@ int xo128_expand(Ctx *c, const uint32_t s0[4], uint64_t b_first, uint64_t np)
     return TP_OK;
 }
 
-// (M^FE_XO_PIECE)^(2^k), k < kb, on the device: the states of the pieces.
-int ensure_xo_piece_table(Ctx *c, uint64_t max_piece, Tables **out)
+// The same for xoshiro256+ pieces of doubles, into c->xo_draws.
+int xo256_expand(Ctx *c, const uint64_t s0[4], bool jump, uint64_t b_first, uint64_t np)
 {
-    const int kb = std::max(1, bits_for(max_piece + 1));
-    const std::string key = "xo-piece:" + std::to_string(FE_XO_PIECE);
-    auto it = c->tables.find(key);
-    if (it != c->tables.end() && it->second->kb >= kb) {
-        *out = it->second.get();
-        return TP_OK;
-    }
-    tp::Gf2Mat B;
-    tp::gf2_pow_from_table(tp::xoshiro_step_pow2(), FE_XO_PIECE, B);
-    std::unique_ptr<Tables> t(new Tables);
-    int rc = upload_mats(c, t->bt, tp::gf2_pow2_table(B, kb));
+    int rc = xo_tables(c);
+    if (!rc)
+        rc = ensure(c, c->xo_draws, np * FE_XO_PIECE * sizeof(double));
+    if (!rc)
+        rc = ensure_acc(c, np);
     if (rc)
         return rc;
-    t->kb = kb;
-    *out = t.get();
-    c->tables[key] = std::move(t);
+    tpk::XoPieceArgs p;
+    std::memset(&p, 0, sizeof p);
+    std::memcpy(p.s0, s0, sizeof p.s0);
+    p.m16 = c->xo->m16;
+    p.b16 = jump ? c->xo->b16[TP_SEED_JUMP] : nullptr;
+    p.lanes = c->xo->lanes + tpk::XO_NRUNS * tpk::XO_LANE_WORDS;
+    p.nb = np;
+    p.b_first = b_first;
+    p.piece_len = FE_XO_PIECE;
+    p.xbuf = static_cast<double *>(c->xo_draws.p);
+    p.acc1 = static_cast<uint32_t *>(c->xo_acc.p);
+    p.acc3 = p.acc1 + c->xo_acc_words;
+    tpk::launch_xo_expand(p, c->stream);
+    HIPCHK(c, hipGetLastError());
     return TP_OK;
 }
 
@@ -471,45 +395,8 @@ int fe_stream_expand(Ctx *c, const FeStream &fs, uint64_t q_first, uint64_t q_la
     }
     const uint64_t p_first = q_first / FE_XO_PIECE, p_end = (q_last + FE_XO_PIECE - 1) / FE_XO_PIECE;
     const uint64_t np = p_end - p_first;
-    if (fs.kind == 3) {
-        int rc = ensure_xo128_piece_table(c, false, FE_XO_PIECE, p_end);
-        if (!rc)
-            rc = xo128_expand(c, fs.s0_128, p_first, np);
-        if (rc)
-            return rc;
-        *qbase = *bbase = p_first * FE_XO_PIECE;
-        return TP_OK;
-    }
-    Tables *t = nullptr;
-    int rc = ensure_xo_piece_table(c, p_end, &t);
-    if (!rc)
-        rc = ensure_lane_tables(c);
-    if (!rc)
-        rc = ensure(c, c->xo_states, np * 4 * sizeof(uint64_t));
-    if (!rc)
-        rc = ensure(c, c->xo_draws, np * FE_XO_PIECE * sizeof(double));
-    if (!rc)
-        rc = ensure_acc(c, np);
-    if (rc)
-        return rc;
-    tpk::XoPieceArgs p;
-    std::memset(&p, 0, sizeof p);
-    std::memcpy(p.s0, fs.s0, sizeof p.s0);
-    p.bt = static_cast<const uint64_t *>(t->bt.p);
-    p.kb = t->kb;
-    p.lt = static_cast<const uint64_t *>(c->xo_lt.p);
-    p.nb = np;
-    p.b_first = p_first;
-    p.states = static_cast<uint64_t *>(c->xo_states.p);
-    p.piece_len = FE_XO_PIECE;
-    p.per_thread = FE_XO_PER_THREAD;
-    p.xbuf = static_cast<double *>(c->xo_draws.p);
-    p.acc1 = static_cast<uint32_t *>(c->xo_acc.p);
-    p.acc3 = p.acc1 + c->xo_acc_words;
-    tpk::launch_xo_expand(p, c->stream);
-    HIPCHK(c, hipGetLastError());
     *qbase = *bbase = p_first * FE_XO_PIECE;
-    return TP_OK;
+    return fs.kind == 3 ? xo128_expand(c, fs.s0_128, false, p_first, np) : xo256_expand(c, fs.s0, false, p_first, np);
 }
 
 // Device walk of n + 1 event starts from the true start q_start into c->evq,
@@ -535,7 +422,7 @@ int fe_device_walk(Ctx *c, const FeStream &fs, uint64_t q_start, uint64_t n, boo
         w.overlap = FE_XO_OVERLAP;
     } else {
         const uint64_t span = (uint64_t)std::ceil((double)(n + 1) * FE_POSITIONS_PER_EVENT) + 55;
-        w.nwalkers = (uint32_t)std::min<uint64_t>(FE_MAX_WALKERS, std::max<uint64_t>(64, n / FE_EVENTS_PER_WALKER));
+        w.nwalkers = (uint32_t)std::min<uint64_t>(FE_MAX_WALKERS, span / FE_SEG + 1);
         w.seg_origin = q_start / 55 * 55;
         w.seg = ((q_start - w.seg_origin + span) / w.nwalkers / 55 + 1) * 55;
         w.overlap = FE_OVERLAP;
@@ -546,9 +433,9 @@ int fe_device_walk(Ctx *c, const FeStream &fs, uint64_t q_start, uint64_t n, boo
     w.qlimit = w.seg_origin + (uint64_t)T * w.seg + w.overlap + 128;
     int rc = fe_stream_expand(c, fs, q_start, w.qlimit, &w.qbase, &w.bbase);
     if (!rc)
-        rc = ensure(c, c->fe_lists, (size_t)T * w.cap * sizeof(uint64_t));
+        rc = ensure(c, c->fe_lists, (size_t)T * w.cap * sizeof(uint32_t));
     if (!rc)
-        rc = ensure(c, c->fe_meta, (size_t)T * 3 * sizeof(uint32_t));
+        rc = ensure(c, c->fe_meta, (size_t)T * 5 * sizeof(uint32_t));
     if (!rc)
         rc = ensure(c, c->fe_piece, (size_t)T * (2 * sizeof(uint32_t) + sizeof(uint64_t)));
     if (!rc)
@@ -564,8 +451,10 @@ int fe_device_walk(Ctx *c, const FeStream &fs, uint64_t q_start, uint64_t n, boo
     w.buf = static_cast<const int32_t *>(c->draws.p);
     w.acc1 = static_cast<const uint32_t *>(c->xo_acc.p);
     w.acc3 = w.acc1 + c->xo_acc_words;
-    w.lists = static_cast<uint64_t *>(c->fe_lists.p);
-    w.counts = static_cast<uint32_t *>(c->fe_meta.p);
+    w.lists = static_cast<uint32_t *>(c->fe_lists.p);
+    w.len = static_cast<uint32_t *>(c->fe_meta.p);
+    w.tail = w.len + T;
+    w.counts = w.tail + T;
     w.join_prev = reinterpret_cast<int32_t *>(w.counts + T);
     w.join_next = w.join_prev + T;
     tpk::launch_fe_walk(w, c->stream);
@@ -607,7 +496,7 @@ using FeHostWalk = std::function<void(uint64_t q, uint64_t n, uint64_t *starts, 
 int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, tpk::FusedArgs &a, tpk::F32Args *fa,
                       uint64_t q_start, uint64_t num_events, uint32_t batch_size, void *per_batch_dev, uint64_t *q_end)
 {
-    const bool device_walk = num_events >= FE_DEVICE_WALK_MIN;
+    const bool device_walk = num_events >= (fs.kind < 2 ? FE_DEVICE_WALK_MIN : FE_XO_DEVICE_WALK_MIN);
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     c->fe_host_chunks = 0;
@@ -761,27 +650,29 @@ static_assert(FE_JUMP_PIECE % 32 == 0, "pieces of whole accept-bit words");
 int fe_batch_walk_setup(Ctx *c, tpk::FeBatchWalkArgs &w, int kind, uint64_t max_batches, uint32_t batch_size)
 {
     const bool xo = kind >= 2; // the xoshiro streams: no rounds
-    const uint64_t per_walker = xo ? FE_XO_EVENTS_PER_WALKER : FE_EVENTS_PER_WALKER;
     w.kind = kind;
-    w.S = (uint32_t)std::max<uint64_t>(1, (batch_size + per_walker - 1) / per_walker);
     const uint64_t span =
         (uint64_t)std::ceil((double)batch_size * (xo ? FE_XO_POSITIONS_PER_EVENT : FE_POSITIONS_PER_EVENT)) + 128;
+    w.S = (uint32_t)(xo ? std::max<uint64_t>(1, (batch_size + FE_XO_BATCH_EVENTS_PER_WALKER - 1) / FE_XO_BATCH_EVENTS_PER_WALKER)
+                        : span / FE_SEG + 1);
     w.seg = xo ? span / w.S + 1 : (span / w.S / 55 + 1) * 55; // > 55: past every piece's first position
     w.overlap = xo ? FE_XO_OVERLAP : FE_OVERLAP;
     // every event takes at least 15 positions: no walk holds more starts
     w.cap = (uint32_t)((w.seg + w.overlap + 63) / 15 + 2);
     const uint64_t walkers = max_batches * w.S;
-    int rc = ensure(c, c->fe_lists, walkers * w.cap * sizeof(uint64_t));
+    int rc = ensure(c, c->fe_lists, walkers * w.cap * sizeof(uint32_t));
     if (!rc)
-        rc = ensure(c, c->fe_meta, walkers * 3 * sizeof(uint32_t));
+        rc = ensure(c, c->fe_meta, walkers * 5 * sizeof(uint32_t));
     if (!rc)
         rc = ensure(c, c->fe_seq, max_batches * sizeof(uint32_t));
     if (rc)
         return rc;
-    w.lists = static_cast<uint64_t *>(c->fe_lists.p);
-    w.counts = static_cast<uint32_t *>(c->fe_meta.p);
-    w.join_prev = reinterpret_cast<int32_t *>(w.counts + walkers);
-    w.join_next = w.join_prev + walkers;
+    w.lists = static_cast<uint32_t *>(c->fe_lists.p);
+    w.len = static_cast<uint32_t *>(c->fe_meta.p);
+    w.tail = w.len + walkers;
+    w.counts = w.tail + walkers;
+    w.next = reinterpret_cast<int32_t *>(w.counts + walkers);
+    w.met = w.counts + 2 * walkers;
     w.seq = static_cast<uint32_t *>(c->fe_seq.p);
     return TP_OK;
 }
@@ -942,14 +833,7 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
         return fail(c, TP_ERR_ARG, "faster-evgen with jump seeding runs batches of at most 10 000 events");
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
-    Tables *t = nullptr;
-    int rc = ensure_jump_table(c, nb, &t);
-    if (!rc)
-        rc = ensure_lane_tables(c);
-    if (!rc)
-        rc = ensure(c, c->xo_states, chunk * 4 * sizeof(uint64_t));
-    if (!rc)
-        rc = ensure(c, c->xo_draws, chunk * FE_XO_PIECE * sizeof(double));
+    int rc = ensure(c, c->xo_draws, chunk * FE_XO_PIECE * sizeof(double));
     if (!rc)
         rc = ensure_acc(c, chunk);
     if (!rc)
@@ -961,25 +845,13 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->fe_flag_host = 0;
     HIPCHK(c, hipMemcpyAsync(c->fe_flag.p, &c->fe_flag_host, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    tpk::XoPieceArgs p;
-    std::memset(&p, 0, sizeof p);
-    std::memcpy(p.s0, x->s, sizeof p.s0);
-    p.bt = static_cast<const uint64_t *>(t->bt.p);
-    p.kb = t->kb;
-    p.lt = static_cast<const uint64_t *>(c->xo_lt.p);
-    p.states = static_cast<uint64_t *>(c->xo_states.p);
-    p.piece_len = FE_XO_PIECE;
-    p.per_thread = FE_XO_PER_THREAD;
-    p.xbuf = static_cast<double *>(c->xo_draws.p);
-    p.acc1 = static_cast<uint32_t *>(c->xo_acc.p);
-    p.acc3 = p.acc1 + c->xo_acc_words;
     tpk::FeBatchWalkArgs w;
     std::memset(&w, 0, sizeof w);
     rc = fe_batch_walk_setup(c, w, 2, chunk, batch_size);
     if (rc)
         return rc;
-    w.acc1 = p.acc1;
-    w.acc3 = p.acc3;
+    w.acc1 = static_cast<const uint32_t *>(c->xo_acc.p);
+    w.acc3 = w.acc1 + c->xo_acc_words;
     w.piece_stride = FE_XO_PIECE;
     w.num_events = num_events;
     w.batch_size = batch_size;
@@ -991,17 +863,16 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
         const uint64_t cnb = std::min(nb, b0 + chunk) - b0;
         if (first)
             HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-        p.nb = cnb;
-        p.b_first = b0;
-        tpk::launch_xo_expand(p, c->stream);
-        HIPCHK(c, hipGetLastError());
+        rc = xo256_expand(c, x->s, true, b0, cnb);
+        if (rc)
+            return rc;
         w.nb = cnb;
         w.b_first = b0;
         tpk::launch_fe_walk_batches(w, c->stream);
         HIPCHK(c, hipGetLastError());
         a.nb = cnb;
         a.b_first = b0;
-        a.xdraws = p.xbuf;
+        a.xdraws = static_cast<const double *>(c->xo_draws.p);
         a.qbase = 0;
         a.acc1 = w.acc1;
         a.bbase = 0;
@@ -1060,9 +931,7 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         return fail(c, TP_ERR_ARG, "faster-evgen with jump seeding runs batches of at most 10 000 events");
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
-    int rc = ensure_xo128_piece_table(c, true, FE_XO_PIECE, nb);
-    if (!rc)
-        rc = ensure(c, c->evq, chunk * batch_size * sizeof(uint64_t));
+    int rc = ensure(c, c->evq, chunk * batch_size * sizeof(uint64_t));
     if (!rc)
         rc = ensure(c, c->fe_flag, sizeof(uint32_t));
     if (rc)
@@ -1085,7 +954,7 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         const uint64_t cnb = std::min(nb, b0 + chunk) - b0;
         if (first)
             HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-        rc = xo128_expand(c, s0, b0, cnb);
+        rc = xo128_expand(c, s0, true, b0, cnb);
         if (rc)
             return rc;
         w.acc1 = static_cast<const uint32_t *>(c->xo_acc.p);
@@ -1256,10 +1125,10 @@ float elapsed(hipEvent_t a, hipEvent_t b)
 constexpr size_t NS_M = 0;                                             // M^(v 16^j)
 constexpr size_t NS_B = NS_M + 15 * tpk::XO_M_DIGITS * tpk::XO_MAT_WORDS; // B^(v 16^j), skip-ahead then jump
 constexpr size_t NS_LANES = NS_B + 2 * 15 * tpk::XO_B_DIGITS * tpk::XO_MAT_WORDS;
-constexpr size_t NS_128 = NS_LANES + tpk::XO_NRUNS * tpk::XO_LANE_WORDS;  // xoshiro128+ (u32 words), as above
+constexpr size_t NS_128 = NS_LANES + tpk::XO_NTABLES * tpk::XO_LANE_WORDS;  // xoshiro128+ (u32 words), as above
 constexpr size_t NS128_B = 15 * tpk::XO_M_DIGITS * tpk::XO128_MAT_WORDS;
 constexpr size_t NS128_LANES = NS128_B + 2 * 15 * tpk::XO_B_DIGITS * tpk::XO128_MAT_WORDS;
-constexpr size_t NS_WORDS = NS_128 + (NS128_LANES + tpk::XO_NRUNS * tpk::XO128_LANE_WORDS) / 2; // 30 MiB
+constexpr size_t NS_WORDS = NS_128 + (NS128_LANES + tpk::XO_NTABLES * tpk::XO128_LANE_WORDS) / 2; // 33 MiB
 static_assert(sizeof(tp::Gf2Mat128) == tpk::XO128_MAT_WORDS * sizeof(uint32_t), "matrix layout");
 static_assert(sizeof(tp::Gf2Mat) == tpk::XO_MAT_WORDS * sizeof(uint64_t), "matrix layout");
 static __device__ __align__(256) uint64_t scratch[NS_WORDS];
@@ -1407,14 +1276,10 @@ extern "C" int tp_destroy(void *ctx)
         (void)hipStreamSynchronize(c->stream);
         for (DevBuf *b : {&c->parts, &c->mt, &c->r16, &c->draws, &c->origin, &c->p0, &c->per_batch, &c->merged, &c->evq,
                           &c->f32ev, &c->f32cnt, &c->fe_lists, &c->fe_meta, &c->fe_piece,
-                          &c->fe_flag, &c->fe_seq, &c->xo_states, &c->xo_draws, &c->xo128_states,
-                          &c->xo128_draws, &c->xo128_pt, &c->xo_acc, &c->xo_lt, &c->xo128_lt, &c->fe_stat, &c->adj_u})
+                          &c->fe_flag, &c->fe_seq, &c->xo_draws, &c->xo128_draws, &c->xo_acc,
+                          &c->fe_stat, &c->adj_u})
             if (b->p)
                 (void)hipFree(b->p);
-        for (auto &kv : c->tables) {
-            if (kv.second->bt.p)
-                (void)hipFree(kv.second->bt.p);
-        }
         for (auto &e : c->ev)
             if (e)
                 (void)hipEventDestroy(e);

@@ -111,12 +111,16 @@ void launch_batch_sums(const FusedArgs &a, hipStream_t st);
 // 79 and 157 parts.
 constexpr uint32_t XO_RUNS[] = {157, 79, 53, 40, 20, 10, 5, 4, 2, 1};
 constexpr int XO_NRUNS = sizeof XO_RUNS / sizeof XO_RUNS[0];
+// Lane tables: of every run length, and of the lanes that expand the stream for
+// faster-evgen, 12 * XO_EXPAND_RUN draws each.
+constexpr uint32_t XO_EXPAND_RUN = 32;
+constexpr int XO_NTABLES = XO_NRUNS + 1;
 constexpr int XO_M_DIGITS = 12, XO_B_DIGITS = 8;         // exponents below 2^48 draws, 2^32 batches
 constexpr size_t XO_MAT_WORDS = 1024;                    // 256 columns of 4 words
 constexpr size_t XO_LANE_WORDS = 64 * 16 * 64 * 4;       // per run length: 2 MiB
 // tab16[(15 j + v - 1) * 1024 ..] = B^(v 16^j) from pow2[k * 1024 ..] = B^(2^k), k < 4 digits.
 void launch_xo_digit_table(const uint64_t *pow2, int digits, uint64_t *tab16, hipStream_t st);
-// The lane tables of every run length of XO_RUNS, in that order.
+// The lane tables of every run length of XO_RUNS, in that order, and XO_EXPAND_RUN's.
 void launch_xo_lane_tables(const uint64_t *m16, uint64_t *lanes, hipStream_t st);
 // Per-event diagnostics: one thread per event, same device code as the loop.
 // Event e draws from offset 12*e (xoshiro: a.s0 with a.mt; buffer: a.draws).
@@ -186,9 +190,10 @@ void launch_xo128_lane_tables(const uint32_t *m16, uint32_t *lanes, hipStream_t 
 // Event starts of the faster-evgen draws (evgen.rs:209-255, random_array's
 // discarded round leftovers ranf.rs:89-92), split like the host walk: walker
 // k starts at seg_origin + k*seg (walker 0 at the true start q_start), as if
-// an event started there, and records its event starts until it passes the
-// next segment's start by `overlap` positions.  Positions are counted from
-// the start of the master state's round; buf holds positions [qbase, qlimit).
+// an event started there, and records its event starts up to the next segment,
+// then on to where it meets that segment's walker, at most `overlap` positions
+// past the segment's end.  Positions are counted from the start of the master
+// state's round; buf holds positions [qbase, qlimit).
 struct FeWalkArgs {
     const int32_t *buf;    // RANF values of positions qbase .. qlimit - 1 (kinds 0, 1)
     int32_t kind;          // 0: RANF, unit-disc test in f64; 1: RANF, in f32; 2: xoshiro256+; 3: xoshiro128+ (f32)
@@ -204,8 +209,9 @@ struct FeWalkArgs {
     uint64_t seg_origin, seg, overlap;
     uint32_t nwalkers;
     uint32_t cap;          // list capacity per walker (>= its longest possible walk)
-    uint64_t *lists;       // [nwalkers][cap] event starts, ascending
-    uint32_t *counts;      // [nwalkers]
+    uint32_t *lists;       // [nwalkers][cap] event starts, ascending, from the segment's start
+    uint32_t *len, *tail;  // [nwalkers] starts in the own segment; where the walk enters the next one
+    uint32_t *counts;      // [nwalkers] starts in all
     int32_t *join_prev;    // [nwalkers] for k >= 1: index in list k-1 of the first start >= the
     int32_t *join_next;    //   start of segment k that list k also holds, and its index there (-1: none)
 };
@@ -239,9 +245,9 @@ void launch_fe_scatter(const FeWalkArgs &a, const uint32_t *begin, const uint32_
 //
 // Each batch is walked by S segment walkers, as the one-stream walk is
 // (walker s of batch k starts at k * piece_stride + s * seg, walker 0 at the
-// batch's first position, and walks overlap positions past its segment),
-// joined where they meet; a batch whose walkers do not all meet before its
-// events are covered is walked by one thread from its first position.
+// batch's first position), each on to where it meets a later one, not always
+// the next; a batch whose chain of walkers ends before its events are covered
+// is walked by one thread from its first position.
 struct FeBatchWalkArgs {
     const int32_t *buf;    // RANF pieces (kinds 0, 1)
     int32_t kind;          // 0: RANF, unit-disc test in f64; 1: in f32 (all-f32 mode); 2: xoshiro256+;
@@ -256,46 +262,41 @@ struct FeBatchWalkArgs {
     uint32_t S;            // walkers per batch
     uint64_t seg, overlap; // segment length (a multiple of 55 for RANF) and overlap
     uint32_t cap;          // list capacity per walker
-    uint64_t *lists;       // [nb * S][cap]
-    uint32_t *counts;      // [nb * S]
-    int32_t *join_prev, *join_next; // [nb * S] as FeWalkArgs, within each batch
+    uint32_t *lists;       // [nb * S][cap], len, tail and counts [nb * S] as FeWalkArgs
+    uint32_t *len, *tail, *counts;
+    int32_t *next;         // [nb * S] the walker of the batch it meets (-1: none)
+    uint32_t *met;         // [nb * S] and the index in that one's list
     uint32_t *seq;         // [nb] 1: walk the batch with one thread
 };
 void launch_fe_walk_batches(const FeBatchWalkArgs &a, hipStream_t st);
 
-// Pieces of the xoshiro256+ stream: piece k starts from B^(b_first + k) s0
-// (B the 2^128 jump with jump seeding, each piece a batch's stream; or
-// M^piece_len, the pieces tiling one stream) and holds its first piece_len
-// uniforms at xbuf[k * piece_len ..], and the accept bits of those positions
-// at acc1 / acc3 (the last three positions' bits from the draws that follow
-// the piece: the next piece's first ones when the pieces tile one stream).
+// Pieces of the xoshiro256+ stream: piece k starts from J^(b_first + k) s0
+// (J the 2^128 jump with jump seeding, each piece a batch's stream) or, with no
+// b16, (b_first + k) * piece_len draws after s0 (the pieces tiling one stream)
+// and holds its first piece_len uniforms at xbuf[k * piece_len ..], and the
+// accept bits of those positions at acc1 / acc3 (the last three positions' bits
+// from the draws that follow the piece: the next piece's first ones when the
+// pieces tile one stream).
 struct XoPieceArgs {
     uint64_t s0[4];
-    const uint64_t *bt;    // B^(2^k), k < kb
-    int32_t kb;
-    const uint64_t *lt;    // M^(per_thread 2^j), j < 6: lane l's skip of l * per_thread draws
+    const uint64_t *m16, *b16; // as FusedArgs
+    const uint64_t *lanes;     // XO_EXPAND_RUN's table
     uint64_t nb, b_first;
-    uint64_t *states;      // [nb][4] scratch: each piece's first state
-    uint64_t piece_len;    // uniforms expanded per piece: 64 * per_thread
-    uint32_t per_thread;   // uniforms per lane, a multiple of 128
-    double *xbuf;          // [nb][piece_len]
-    uint32_t *acc1, *acc3; // [nb][piece_len / 32] accept bits of the positions, as FeWalkArgs
+    uint64_t piece_len;        // uniforms per piece: a multiple of 64 * 12 * XO_EXPAND_RUN, one wavefront's
+    double *xbuf;              // [nb][piece_len]
+    uint32_t *acc1, *acc3;     // [nb][piece_len / 32] accept bits of the positions, as FeWalkArgs
 };
-void launch_xo_expand(const XoPieceArgs &a, hipStream_t st); // piece states and expansion
+void launch_xo_expand(const XoPieceArgs &a, hipStream_t st);
 
-// The same for the xoshiro128+ stream of the all-f32 mode (B the 2^64 jump
-// or M^piece_len; f32 uniforms).
+// The same for the xoshiro128+ stream of the all-f32 mode (J the 2^64 jump; f32
+// uniforms, and the unit-disc test in f32).
 struct Xo128PieceArgs {
     uint32_t s0[4];
-    const uint32_t *bt;    // B^(2^k), k < kb (128 columns x 4 words each)
-    int32_t kb;
-    const uint32_t *lt;    // M^(per_thread 2^j), j < 6
+    const uint32_t *m16, *b16, *lanes;
     uint64_t nb, b_first;
-    uint32_t *states;      // [nb][4] scratch: each piece's first state
-    uint64_t piece_len;    // 64 * per_thread
-    uint32_t per_thread;   // a multiple of 128
-    float *xbuf;           // [nb][piece_len]
-    uint32_t *acc1, *acc3; // [nb][piece_len / 32] accept bits (the unit-disc test in f32)
+    uint64_t piece_len;
+    float *xbuf;
+    uint32_t *acc1, *acc3;
 };
 void launch_xo128_expand(const Xo128PieceArgs &a, hipStream_t st);
 

@@ -516,7 +516,7 @@ void launch_xo_digit_table(const uint64_t *pow2, int digits, uint64_t *tab16, hi
 }
 
 struct XoRuns {
-    uint32_t n[XO_NRUNS];
+    uint32_t n[XO_NTABLES];
 };
 // Lane l's images of every value of nibble `threadIdx.x` of the state, for run
 // length runs.n[blockIdx.y] (l = blockIdx.x, so the skip matrices are uniform).
@@ -554,7 +554,8 @@ void launch_xo_lane_tables(const uint64_t *m16, uint64_t *lanes, hipStream_t st)
     XoRuns r;
     for (int i = 0; i < XO_NRUNS; ++i)
         r.n[i] = XO_RUNS[i];
-    hipLaunchKernelGGL(xo_lane_table_kernel, dim3(64, XO_NRUNS), dim3(64), 0, st, m16, lanes, r);
+    r.n[XO_NRUNS] = XO_EXPAND_RUN;
+    hipLaunchKernelGGL(xo_lane_table_kernel, dim3(64, XO_NTABLES), dim3(64), 0, st, m16, lanes, r);
 }
 
 // The xoshiro128+ tables: lane c < 64 takes columns c and c + 64; one lane per
@@ -614,7 +615,8 @@ void launch_xo128_lane_tables(const uint32_t *m16, uint32_t *lanes, hipStream_t 
     XoRuns r;
     for (int i = 0; i < XO_NRUNS; ++i)
         r.n[i] = XO_RUNS[i];
-    hipLaunchKernelGGL(xo128_lane_table_kernel, dim3(64, XO_NRUNS), dim3(64), 0, st, m16, lanes, r);
+    r.n[XO_NRUNS] = XO_EXPAND_RUN;
+    hipLaunchKernelGGL(xo128_lane_table_kernel, dim3(64, XO_NTABLES), dim3(64), 0, st, m16, lanes, r);
 }
 
 template <int SOURCE, int PREC> int blocks_per_cu()
@@ -762,18 +764,19 @@ template <class T> __device__ __forceinline__ T ranf_sq(int32_t v)
 
 // Lane moves within the wavefront (DPP, no LDS): DPP_WAVE_ROR1 gives lane i
 // the value of lane i - 1 (lane 0: lane 63); DPP_ROW_SHR9 gives lane i of each
-// row of 16 the value of lane i - 9 of the row (lanes 61..63: lanes 52..54).
+// row of 16 the value of lane i - 9 of the row (lanes 61..63: lanes 52..54), 0
+// to its first nine lanes.
 constexpr int DPP_WAVE_ROR1 = 0x13C, DPP_ROW_SHR9 = 0x119;
 template <int CTRL> __device__ __forceinline__ double lanes_dpp(double v)
 {
     const uint64_t b = (uint64_t)__double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, false);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, false);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 template <int CTRL> __device__ __forceinline__ float lanes_dpp(float v)
 {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 
 // Accept bits of a segment's rounds.  Lane i holds the square of position
@@ -1090,130 +1093,143 @@ __device__ __forceinline__ bool ranf_walk_event(const uint32_t *acc1, const uint
 
 // The walkers' accept bits through LDS.  Bits read straight from HBM cost
 // each event several scattered loads, and a compute unit's walkers touch
-// more lines than its L1 holds.  So each walking lane keeps BW_WORDS words of
-// acc1 and acc3 (BW_WORDS * 32 positions) from the word of its next event's
+// more lines than its L1 holds.  So each walking lane keeps W words of
+// acc1 and acc3 (32 W positions) from the word of its next event's
 // first test on in rows of its own, and takes its events' tests from there;
 // the wavefront refills every lane's rows (16-byte loads) when some lane's
 // next event could leave its window.  No lane reads another's rows.
-constexpr int BW_WORDS = 32, BW_ROW = BW_WORDS + 4, BW_THREADS = 128;
+constexpr int BW_THREADS = 128;
+constexpr int BW_WALK = 32, BW_JOIN = 16;   // words per row of the two kernels
+constexpr int bw_lds(int words) { return 2 * BW_THREADS * (words + 4); }
 
-struct BitWin {
-    uint32_t *w1, *w3; // the lane's rows
-    uint64_t wb;       // first word held (counted from bbase)
-    uint64_t end;      // stream position where the held bits end
+constexpr uint32_t FE_STUCK = 0xffffffffu; // the place of a walk that left the stored range
+
+// The candidate pairs of an event's re-rolls by the place in the round where
+// the event starts (RANF), a table in LDS of every block that walks.
+struct FeLds {
+    uint64_t pairs[55];
 };
-
-// Words from the one holding position q + 9 on, in whole groups of 4 below
-// qlimit.
-__device__ __forceinline__ void bit_win_fill(BitWin &v, const uint32_t *acc1, const uint32_t *acc3, uint64_t bbase,
-                                             uint64_t qlimit, uint64_t q)
+// Where an event that starts at place a of its round goes on after its takes of
+// 9 and 6, and the positions it discards before them.
+__device__ __forceinline__ void ranf_takes(uint32_t a, uint32_t &d, uint32_t &a1)
 {
-    const uint64_t lim4 = ((qlimit - bbase) >> 5) & ~3ull;
-    const uint64_t wb = ((q + 9 - bbase) >> 5) & ~3ull;
-    uint64_t have = 0;
+    d = a >= 47 ? 55 - a : a >= 41 ? 46 - a : 0;
+    a1 = a >= 47 ? 15 : a >= 41 ? 6 : a == 40 ? 0 : a + 15;
+}
+__device__ __forceinline__ void fe_lds_fill(FeLds &t)
+{
+    if (threadIdx.x < 55) {
+        uint32_t d, a1;
+        ranf_takes(threadIdx.x, d, a1);
+        t.pairs[threadIdx.x] = ranf_pair_starts(55u - a1);
+    }
+    __syncthreads();
+}
+
+// A walk of the RANF stream or of a xoshiro one from its walker's segment
+// start, positions counted from there (p).
+template <bool RANF, int W> struct FeWalker {
+    // Positions past p that an event's tests may read: the 15 values, 64
+    // positions of re-rolls and the rest of their last word, and on the RANF
+    // stream up to 13 discarded leftovers.
+    static constexpr uint32_t REACH = RANF ? 128 : 111;
+    const uint32_t *acc1, *acc3;
+    const FeLds *lds;
+    uint64_t origin;     // bit of p = 0
+    uint64_t lim;        // bits stored
+    uint32_t *w1, *w3;   // the lane's rows
+    uint32_t p;          // the next event's start
+    uint32_t a;          // RANF: its place in the round
+    uint32_t win;        // p of the rows' first bit (modulo 2^32)
+    uint32_t pmax, plim; // the last p whose event's tests lie in the rows, in the stored range (+ 1)
+
+    __device__ __forceinline__ void start(const uint32_t *b1, const uint32_t *b3, uint32_t *rows, const FeLds *t, uint64_t bit0,
+                                          uint64_t limit, uint64_t q0, uint32_t p0)
+    {
+        acc1 = b1;
+        acc3 = b3;
+        lds = t;
+        w1 = rows + threadIdx.x * (W + 4);
+        w3 = rows + (BW_THREADS + threadIdx.x) * (W + 4);
+        origin = bit0;
+        lim = limit;
+        p = p0;
+        a = RANF ? (uint32_t)((q0 + p0) % 55u) : 0u;
+        win = p0;
+        pmax = 0;
+        plim = limit < bit0 + REACH ? 0u : (uint32_t)min<uint64_t>(limit - bit0 - REACH + 1, 0x7fffffffu);
+    }
+    // Rows from the word holding position p + 9 on, in whole groups of 4
+    // words below the stored range's end (past it, copies of the last group).
+    // All loads go out before the first one is waited for.
+    __device__ __forceinline__ void fill()
+    {
+        const uint64_t lim4 = (lim >> 5) & ~3ull, wb = ((origin + p + 9) >> 5) & ~3ull;
+        uint4 b1[W / 4], b3[W / 4];
 #pragma unroll
-    for (int i = 0; i < BW_WORDS / 4; ++i) {
-        const uint64_t w = wb + 4 * i;
-        if (w < lim4) {
-            *reinterpret_cast<uint4 *>(v.w1 + 4 * i) = *reinterpret_cast<const uint4 *>(acc1 + w);
-            *reinterpret_cast<uint4 *>(v.w3 + 4 * i) = *reinterpret_cast<const uint4 *>(acc3 + w);
-            have = 4 * i + 4;
+        for (int i = 0; i < W / 4; ++i) {
+            const uint64_t w = min(wb + 4 * i, lim4 - 4);
+            b1[i] = *reinterpret_cast<const uint4 *>(acc1 + w);
+            b3[i] = *reinterpret_cast<const uint4 *>(acc3 + w);
+        }
+#pragma unroll
+        for (int i = 0; i < W / 4; ++i) {
+            *reinterpret_cast<uint4 *>(w1 + 4 * i) = b1[i];
+            *reinterpret_cast<uint4 *>(w3 + 4 * i) = b3[i];
+        }
+        const uint32_t have = wb < lim4 ? 32u * (uint32_t)min<uint64_t>(lim4 - wb, W) : 0u;
+        win = (uint32_t)(32 * wb - origin);
+        pmax = (uint32_t)max((int32_t)(win + have - REACH + 1), 0); // (win is at most 127 below 0)
+    }
+    // On past one event, to FE_STUCK when the stored range ends inside it.
+    // With the tests in the rows: the takes of 9 and 6 by position arithmetic,
+    // the re-rolls as the F-th accepted pair past them, all as straight code
+    // (a lane waits for each of its steps, and the other lanes' branches add to
+    // them).
+    __device__ __forceinline__ void event()
+    {
+        if (__any(p >= pmax && p < plim))
+            fill();
+        uint32_t d = 0, a1 = 0;
+        if (RANF)
+            ranf_takes(a, d, a1);
+        // (clamped for a lane whose tests lie elsewhere)
+        const uint32_t x3 = min(p + 9 - win, 32u * W - REACH + 9) + d, x1 = x3 + 6;
+        const uint32_t *p3 = w3 + (x3 >> 5), *p1 = w1 + (x1 >> 5);
+        const uint32_t ok3 = __builtin_amdgcn_alignbit(p3[1], p3[0], x3 & 31) & 7u;
+        const uint32_t lo = __builtin_amdgcn_alignbit(p1[1], p1[0], x1 & 31), hi = __builtin_amdgcn_alignbit(p1[2], p1[1], x1 & 31);
+        const uint64_t y0 = (((uint64_t)hi << 32) | lo) & (RANF ? lds->pairs[a] : 0x5555555555555555ull);
+        const uint64_t y1 = y0 & (y0 - 1), y2 = y1 & (y1 - 1);
+        const uint32_t good3 = (uint32_t)__popc(ok3);
+        const uint64_t y = good3 == 2 ? y0 : good3 == 1 ? y1 : y2;
+        const uint32_t k = good3 == 3 ? 0u : (uint32_t)__builtin_ctzll(y | 1ull << 63) + 2; // past the accepted pair
+        const bool good = p < pmax && (good3 == 3 || y);
+        if (__any(!good)) {
+            if (!good) {
+                uint64_t q = origin + p;
+                const bool ok = RANF ? ranf_walk_event(acc1, acc3, 0, lim, q, a) : xo_walk_event(acc1, acc3, 0, lim, q);
+                p = ok ? (uint32_t)(q - origin) : FE_STUCK;
+            }
+        }
+        p = good ? p + d + 15 + k : p;
+        if (RANF) {
+            a1 += k;
+            a1 = a1 >= 110u ? a1 - 110u : a1;
+            a = good ? (a1 >= 55u ? a1 - 55u : a1) : a;
         }
     }
-    v.wb = wb;
-    v.end = bbase + 32 * (wb + have);
-}
-
-// xo_walk_event with the tests from the lane's window when the event's bits
-// (as far as position q + 110) lie in it.
-struct XoBitWalk {
-    static constexpr uint64_t REACH = 111;
-    const uint32_t *acc1, *acc3;
-    uint64_t bbase, qlimit;
-    __device__ __forceinline__ void start(uint64_t) {}
-    __device__ __forceinline__ bool event(const BitWin &v, uint64_t &q)
+    // Records the starts below stop into list (every event takes at least 15
+    // positions, so the loop ends and the list's capacity holds them).
+    __device__ __forceinline__ void run(uint32_t stop, uint32_t *list, uint32_t &n)
     {
-        if (q + REACH <= v.end) {
-            const uint64_t r3 = q + 9 - bbase, r1 = q + 15 - bbase;
-            const uint32_t *p3 = v.w3 + ((r3 >> 5) - v.wb);
-            const uint32_t ok3 = (uint32_t)((((uint64_t)p3[1] << 32) | p3[0]) >> (r3 & 31)) & 7u;
-            const uint32_t fails = 3u - (uint32_t)__popc(ok3);
-            if (fails == 0) {
-                q += 15;
-                return true;
-            }
-            const uint64_t y = nth_accept(bits64(v.w1 + ((r1 >> 5) - v.wb), r1) & 0x5555555555555555ull, fails);
-            if (y) {
-                q += 17 + (uint64_t)__builtin_ctzll(y);
-                return true;
-            }
+        uint32_t *o = list + n;
+        while (p < stop) {
+            *o++ = p;
+            event();
         }
-        return xo_walk_event(acc1, acc3, bbase, qlimit, q);
+        n = (uint32_t)(o - list);
     }
 };
-
-// ranf_walk_event with the tests from the lane's window when the event's
-// bits (as far as position q + 123: up to 13 discarded leftovers, the 15
-// values, 64 positions of re-rolls and the rest of their last word) lie in
-// it: the 9 and 6 takes by position arithmetic, the re-rolls as the F-th
-// accepted pair among ranf_pair_starts.
-struct RanfBitWalk {
-    static constexpr uint64_t REACH = 128;
-    const uint32_t *acc1, *acc3;
-    uint64_t bbase, qlimit;
-    uint32_t a; // q % 55
-    __device__ __forceinline__ void start(uint64_t q) { a = (uint32_t)(q % 55u); }
-    __device__ __forceinline__ bool event(const BitWin &v, uint64_t &q)
-    {
-        if (q + REACH <= v.end) {
-            uint64_t q1 = q;
-            uint32_t a1 = a;
-            ranf_skip(q1, a1, 9);
-            ranf_step(q1, a1, 9);
-            ranf_skip(q1, a1, 6);
-            const uint64_t r3 = q1 - bbase;
-            ranf_step(q1, a1, 6);
-            const uint32_t *p3 = v.w3 + ((r3 >> 5) - v.wb);
-            const uint32_t ok3 = (uint32_t)((((uint64_t)p3[1] << 32) | p3[0]) >> (r3 & 31)) & 7u;
-            const uint32_t fails = 3u - (uint32_t)__popc(ok3);
-            if (fails == 0) {
-                q = q1;
-                a = a1;
-                return true;
-            }
-            const uint64_t r1 = q1 - bbase;
-            const uint64_t y = nth_accept(bits64(v.w1 + ((r1 >> 5) - v.wb), r1) & ranf_pair_starts(55u - a1), fails);
-            if (y) {
-                const uint32_t k = (uint32_t)__builtin_ctzll(y) + 2; // past the accepted pair
-                q = q1 + k;
-                a = a1 + k;
-                a = a >= 110u ? a - 110u : a >= 55u ? a - 55u : a;
-                return true;
-            }
-        }
-        return ranf_walk_event(acc1, acc3, bbase, qlimit, q, a);
-    }
-};
-
-// Records starts from q while q < stop and the list has room (each event
-// consumes at least 15 positions, so the loop ends); returns the count.
-template <class W>
-__device__ __forceinline__ uint32_t bit_walk_run(W w, BitWin &v, uint64_t q, uint64_t stop, uint64_t *list,
-                                                 uint32_t cap)
-{
-    v.wb = 0;
-    v.end = 0;
-    w.start(q);
-    uint32_t n = 0;
-    while (q < stop && n < cap) {
-        list[n++] = q;
-        if (__any(q + W::REACH > v.end && q + W::REACH <= w.qlimit))
-            bit_win_fill(v, w.acc1, w.acc3, w.bbase, w.qlimit, q);
-        if (!w.event(v, q))
-            break;
-    }
-    return n;
-}
 
 // One event of the walk of kind a.kind: RANF with the unit-disc test in f64
 // (0) or f32 (1), the xoshiro256+ stream (2) or the xoshiro128+ one (3).
@@ -1224,71 +1240,124 @@ __device__ __forceinline__ bool fe_walk_any(const FeWalkArgs &a, uint64_t &q)
     return a.kind == 1 ? fe_walk_event<float>(a, q) : fe_walk_event<double>(a, q);
 }
 
-// One thread per walker.  Every step records a start and then consumes at
-// least 15 positions, and the loop stops at the segment end, the list
-// capacity or the stored range, so it always ends.  The tests come from the
-// accept bits through LDS windows (every kind).
-__global__ __launch_bounds__(BW_THREADS) void fe_bit_walk_kernel(FeWalkArgs a)
+// One thread per walker, over its own segment: its list, its length and where
+// the walk enters the next segment.  Bound by latency: an event is a chain of an
+// LDS read and some 40 dependent integer steps, so segments are as short as the
+// walks' meeting allows and a walker goes no further than that needs.  1e7 RANF
+// events in 140 000 segments: 90 us here and 43 in fe_join_kernel; in 39 000
+// with a fixed overlap of 24 rounds, branches and one load at a time to fill the
+// rows 238 and 22.  5e7 xoshiro128+ events in 50 000: 345 and 420 us, before
+// 1078 and 318.
+template <bool RANF> __device__ __forceinline__ void fe_walk_segment(const FeWalkArgs &a, uint32_t *win, const FeLds *t0, uint32_t k)
 {
-    __shared__ uint32_t win[2 * BW_THREADS * BW_ROW];
+    FeWalker<RANF, BW_WALK> w;
+    const uint64_t q0 = a.seg_origin + (uint64_t)k * a.seg;
+    w.start(a.acc1, a.acc3, win, t0, q0 - a.bbase, a.qlimit - a.bbase, q0, k == 0 ? (uint32_t)(a.q_start - q0) : 0u);
+    uint32_t n = 0;
+    w.run((uint32_t)a.seg, a.lists + (size_t)k * a.cap, n);
+    a.len[k] = n;
+    a.tail[k] = w.p;
+}
+__global__ __launch_bounds__(BW_THREADS) void fe_walk_kernel(FeWalkArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t win[bw_lds(BW_WALK)];
+    __shared__ FeLds t0;
+    fe_lds_fill(t0);
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= a.nwalkers)
         return;
-    BitWin v;
-    v.w1 = win + threadIdx.x * BW_ROW;
-    v.w3 = win + (BW_THREADS + threadIdx.x) * BW_ROW;
-    const uint64_t q = k == 0 ? a.q_start : a.seg_origin + (uint64_t)k * a.seg;
-    const uint64_t stop = a.seg_origin + (uint64_t)(k + 1) * a.seg + a.overlap;
-    uint64_t *list = a.lists + (size_t)k * a.cap;
-    a.counts[k] = a.kind >= 2 ? bit_walk_run(XoBitWalk{a.acc1, a.acc3, a.bbase, a.qlimit}, v, q, stop, list, a.cap)
-                              : bit_walk_run(RanfBitWalk{a.acc1, a.acc3, a.bbase, a.qlimit, 0}, v, q, stop, list, a.cap);
+    if (a.kind >= 2)
+        fe_walk_segment<false>(a, win, &t0, k);
+    else
+        fe_walk_segment<true>(a, win, &t0, k);
 }
 
-// Walker k's first start that walker k-1 also reached past segment k's start:
-// from there on both walks agree.
-__global__ __launch_bounds__(256) void fe_join_kernel(FeWalkArgs a)
+// A walk goes on past its segment until it starts an event where a later
+// segment's walker does (from there on both agree), at most to `stop`: list and
+// n grow by its starts; true when they met, with j the index in that walker's
+// list.  That walk, from `from` up to its segment's end `to`, is taken again
+// beside this one, always the one that is behind, so that nothing waits for a
+// list in memory.
+template <class W>
+__device__ __forceinline__ bool fe_walk_on(W &w, uint32_t from, uint32_t to, uint32_t stop, uint32_t *list, uint32_t &n,
+                                           uint32_t &j)
 {
+    uint32_t o = from, oa = 0, p = w.p, pa = w.a; // segments start at the start of a round
+    uint32_t *at = list + n;
+    j = 0;
+    while (p != o && o < to && p < stop) {
+        const bool behind = p < o;
+        if (behind)
+            *at++ = p;
+        w.p = behind ? p : o;
+        w.a = behind ? pa : oa;
+        w.event();
+        p = behind ? w.p : p;
+        pa = behind ? w.a : pa;
+        o = behind ? o : w.p;
+        oa = behind ? oa : w.a;
+        j += behind ? 0u : 1u;
+    }
+    w.p = p;
+    w.a = pa;
+    n = (uint32_t)(at - list);
+    return p == o && o < to;
+}
+
+// One thread per walker: on to where it meets the next one (the last one:
+// `overlap` positions on).  They met within 58 events in 1.2e7 starts on the RANF
+// stream, whose discards bring walkers together (each 8 events more leave an
+// eighth of the walkers apart); on xoshiro streams only starting an event at the
+// same place does, after a median of 22 events but at most 832 over 176 447
+// walkers, and the last walker to meet is what this kernel takes its time for.
+template <bool RANF> __device__ __forceinline__ void fe_join_segment(const FeWalkArgs &a, uint32_t *win, const FeLds *t0, uint32_t k)
+{
+    uint32_t n = a.len[k];
+    const uint32_t at = a.tail[k];
+    int32_t ji = -1, jj = -1;
+    if (at != FE_STUCK) {
+        FeWalker<RANF, BW_JOIN> w;
+        const uint64_t q0 = a.seg_origin + (uint64_t)k * a.seg;
+        w.start(a.acc1, a.acc3, win, t0, q0 - a.bbase, a.qlimit - a.bbase, q0, at);
+        uint32_t *list = a.lists + (size_t)k * a.cap;
+        const uint32_t stop = (uint32_t)(a.seg + a.overlap);
+        if (k + 1 == a.nwalkers) {
+            w.run(stop, list, n);
+        } else {
+            uint32_t j = 0;
+            if (fe_walk_on(w, (uint32_t)a.seg, (uint32_t)(2 * a.seg), stop, list, n, j)) {
+                ji = (int32_t)n;
+                jj = (int32_t)j;
+            }
+        }
+    }
+    a.counts[k] = n;
+    if (k == 0)
+        a.join_prev[0] = a.join_next[0] = 0;
+    if (k + 1 < a.nwalkers) {
+        a.join_prev[k + 1] = ji;
+        a.join_next[k + 1] = jj;
+    }
+}
+__global__ __launch_bounds__(BW_THREADS) void fe_join_kernel(FeWalkArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t win[bw_lds(BW_JOIN)];
+    __shared__ FeLds t0;
+    fe_lds_fill(t0);
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= a.nwalkers)
         return;
-    if (k == 0) {
-        a.join_prev[0] = a.join_next[0] = 0;
-        return;
-    }
-    const uint64_t *pa = a.lists + (size_t)(k - 1) * a.cap, *pb = a.lists + (size_t)k * a.cap;
-    const uint32_t na = a.counts[k - 1], nb = a.counts[k];
-    const uint64_t qs = a.seg_origin + (uint64_t)k * a.seg;
-    uint32_t lo = 0, hi = na; // first index of list k-1 with a start >= qs
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) / 2;
-        if (pa[mid] < qs)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    uint32_t i = lo, j = 0;
-    int32_t ji = -1, jj = -1;
-    while (i < na && j < nb) {
-        if (pa[i] == pb[j]) {
-            ji = (int32_t)i;
-            jj = (int32_t)j;
-            break;
-        }
-        if (pa[i] < pb[j])
-            ++i;
-        else
-            ++j;
-    }
-    a.join_prev[k] = ji;
-    a.join_next[k] = jj;
+    if (a.kind >= 2)
+        fe_join_segment<false>(a, win, &t0, k);
+    else
+        fe_join_segment<true>(a, win, &t0, k);
 }
 
 void launch_fe_walk(const FeWalkArgs &a, hipStream_t st)
 {
-    const unsigned blocks = (a.nwalkers + 255) / 256;
-    hipLaunchKernelGGL(fe_bit_walk_kernel, dim3((a.nwalkers + BW_THREADS - 1) / BW_THREADS), dim3(BW_THREADS), 0, st,
-                       a);
-    hipLaunchKernelGGL(fe_join_kernel, dim3(blocks), dim3(256), 0, st, a);
+    const dim3 blocks((a.nwalkers + BW_THREADS - 1) / BW_THREADS);
+    hipLaunchKernelGGL(fe_walk_kernel, blocks, dim3(BW_THREADS), 0, st, a);
+    hipLaunchKernelGGL(fe_join_kernel, blocks, dim3(BW_THREADS), 0, st, a);
 }
 
 // Walker k's piece of the true walk is its list from where walker k - 1 met
@@ -1379,7 +1448,7 @@ __global__ __launch_bounds__(FE_STITCH_BLOCK) void fe_stitch_cut_kernel(FeWalkAr
     const uint64_t o = min(status[2 + blockIdx.x] + s[t] - l, need);
     const uint32_t cut = (uint32_t)min<uint64_t>(l, need - o);
     if (o < need && need - 1 < o + cut) // this piece holds start need - 1
-        status[1] = a.lists[(size_t)k * a.cap + beg[k] + (need - 1 - o)];
+        status[1] = a.seg_origin + (uint64_t)k * a.seg + a.lists[(size_t)k * a.cap + beg[k] + (need - 1 - o)];
     off[k] = o;
     len[k] = cut;
 }
@@ -1394,21 +1463,26 @@ void launch_fe_stitch(const FeWalkArgs &a, uint64_t need, uint32_t *begin, uint3
                        status);
 }
 
-// One block per piece.
+// Sixteen lanes per piece.
 __global__ __launch_bounds__(256) void fe_scatter_kernel(FeWalkArgs a, const uint32_t *begin, const uint32_t *len,
                                                          const uint64_t *off, uint64_t *out)
 {
-    const uint32_t k = blockIdx.x;
-    const uint64_t *src = a.lists + (size_t)k * a.cap + begin[k];
+    const uint32_t k = 16 * blockIdx.x + threadIdx.x / 16;
+    if (k >= a.nwalkers)
+        return;
+    const uint32_t *src = a.lists + (size_t)k * a.cap + begin[k];
+    const uint64_t q0 = a.seg_origin + (uint64_t)k * a.seg;
     uint64_t *dst = out + off[k];
-    for (uint32_t i = threadIdx.x; i < len[k]; i += blockDim.x)
-        dst[i] = src[i];
+    const uint32_t n = len[k];
+#pragma unroll 4
+    for (uint32_t i = threadIdx.x % 16; i < n; i += 16)
+        dst[i] = q0 + src[i];
 }
 
 void launch_fe_scatter(const FeWalkArgs &a, const uint32_t *begin, const uint32_t *len, const uint64_t *off,
                        uint64_t *out, hipStream_t st)
 {
-    hipLaunchKernelGGL(fe_scatter_kernel, dim3(a.nwalkers), dim3(256), 0, st, a, begin, len, off, out);
+    hipLaunchKernelGGL(fe_scatter_kernel, dim3((a.nwalkers + 15) / 16), dim3(256), 0, st, a, begin, len, off, out);
 }
 
 // Events of batch b_first + k.
@@ -1432,120 +1506,131 @@ __device__ __forceinline__ FeWalkArgs fe_batch_view(const FeBatchWalkArgs &a, ui
     return w;
 }
 
-// Walker s of batch k (thread k * S + s).  Every step records a start and
-// then consumes at least 15 positions, and the loop stops at the segment end
-// plus the overlap, the piece's end or the list capacity, so it always ends.
-// The tests come from the accept bits through LDS windows (every kind).
-__global__ __launch_bounds__(BW_THREADS) void fe_seg_bit_walk_kernel(FeBatchWalkArgs a)
+// Walker s of batch k (thread k * S + s), as fe_walk_kernel.
+template <bool RANF> __device__ __forceinline__ void fe_seg_walk(const FeBatchWalkArgs &a, uint32_t *win, const FeLds *t0, uint64_t t)
 {
-    __shared__ uint32_t win[2 * BW_THREADS * BW_ROW];
+    const uint64_t k = t / a.S, q0 = k * a.piece_stride + (t - k * a.S) * a.seg;
+    FeWalker<RANF, BW_WALK> w;
+    w.start(a.acc1, a.acc3, win, t0, q0, (k + 1) * a.piece_stride, q0, t == k * a.S && a.p0 ? (uint32_t)a.p0[k] : 0u);
+    uint32_t n = 0;
+    w.run((uint32_t)a.seg, a.lists + t * a.cap, n);
+    a.len[t] = n;
+    a.tail[t] = w.p;
+}
+__global__ __launch_bounds__(BW_THREADS) void fe_seg_walk_kernel(FeBatchWalkArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t win[bw_lds(BW_WALK)];
+    __shared__ FeLds t0;
+    fe_lds_fill(t0);
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= a.nb * a.S)
         return;
-    const uint64_t k = t / a.S;
-    const uint32_t s = (uint32_t)(t % a.S);
-    const uint64_t base = k * a.piece_stride, end = base + a.piece_stride;
-    const uint64_t q = s == 0 ? base + (a.p0 ? (uint64_t)a.p0[k] : 0) : base + (uint64_t)s * a.seg;
-    const uint64_t stop = min(base + (uint64_t)(s + 1) * a.seg + a.overlap, end);
-    BitWin v;
-    v.w1 = win + threadIdx.x * BW_ROW;
-    v.w3 = win + (BW_THREADS + threadIdx.x) * BW_ROW;
-    uint64_t *list = a.lists + t * a.cap;
-    a.counts[t] = a.kind >= 2 ? bit_walk_run(XoBitWalk{a.acc1, a.acc3, 0, end}, v, q, stop, list, a.cap)
-                              : bit_walk_run(RanfBitWalk{a.acc1, a.acc3, 0, end, 0}, v, q, stop, list, a.cap);
+    if (a.kind >= 2)
+        fe_seg_walk<false>(a, win, &t0, t);
+    else
+        fe_seg_walk<true>(a, win, &t0, t);
 }
 
-// Walker s's first start that walker s - 1 of the same batch also reached
-// past segment s's start, as fe_join_kernel.
-__global__ __launch_bounds__(256) void fe_seg_join_kernel(FeBatchWalkArgs a)
+// On to where the walker meets a later one of its batch, not always the next:
+// next[t] that walker's number in the batch (-1: none, or the last one), met[t]
+// the index in its list, counts[t] the starts of its own list up to there.
+template <bool RANF> __device__ __forceinline__ void fe_seg_join(const FeBatchWalkArgs &a, uint32_t *win, const FeLds *t0, uint64_t t)
 {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.nb * a.S)
-        return;
-    const uint64_t k = t / a.S;
-    const uint32_t s = (uint32_t)(t % a.S);
-    if (s == 0) {
-        a.join_prev[t] = a.join_next[t] = 0;
-        return;
-    }
-    const uint64_t *pa = a.lists + (t - 1) * a.cap, *pb = a.lists + t * a.cap;
-    const uint32_t na = a.counts[t - 1], nb = a.counts[t];
-    const uint64_t qs = k * a.piece_stride + (uint64_t)s * a.seg;
-    uint32_t lo = 0, hi = na; // first index of list s - 1 with a start >= qs
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) / 2;
-        if (pa[mid] < qs)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    uint32_t i = lo, j = 0;
-    int32_t ji = -1, jj = -1;
-    while (i < na && j < nb) {
-        if (pa[i] == pb[j]) {
-            ji = (int32_t)i;
-            jj = (int32_t)j;
-            break;
+    const uint64_t k = t / a.S, q0 = k * a.piece_stride + (t - k * a.S) * a.seg;
+    const uint32_t s = (uint32_t)(t - k * a.S), at = a.tail[t];
+    uint32_t n = a.len[t], j = 0;
+    int32_t next = -1;
+    if (at != FE_STUCK) {
+        FeWalker<RANF, BW_JOIN> w;
+        w.start(a.acc1, a.acc3, win, t0, q0, (k + 1) * a.piece_stride, q0, at);
+        uint32_t *list = a.lists + t * a.cap;
+        const uint32_t seg = (uint32_t)a.seg, stop = (uint32_t)(a.seg + a.overlap);
+        if (s + 1 == a.S)
+            w.run(stop, list, n);
+        for (uint32_t o = 1; s + o < a.S; ++o) {
+            if (fe_walk_on(w, o * seg, (o + 1) * seg, stop, list, n, j)) {
+                next = (int32_t)(s + o);
+                break;
+            }
+            // past that list's end, within its segment: the walk goes on alone to the next one
+            w.run(min(stop, (o + 1) * seg), list, n);
+            if (w.p >= stop)
+                break;
         }
-        if (pa[i] < pb[j])
-            ++i;
-        else
-            ++j;
     }
-    a.join_prev[t] = ji;
-    a.join_next[t] = jj;
+    a.counts[t] = n;
+    a.next[t] = next;
+    a.met[t] = j;
+}
+__global__ __launch_bounds__(BW_THREADS) void fe_seg_join_kernel(FeBatchWalkArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint32_t win[bw_lds(BW_JOIN)];
+    __shared__ FeLds t0;
+    fe_lds_fill(t0);
+    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= a.nb * a.S)
+        return;
+    if (a.kind >= 2)
+        fe_seg_join<false>(a, win, &t0, t);
+    else
+        fe_seg_join<true>(a, win, &t0, t);
 }
 
-// One wavefront per batch: the true walk is walker 0's list from its first
-// start, then each walker's from where its predecessor met it.  Its first n
-// starts go to the batch's slots of evq, each piece copied by the 64 lanes
-// together; seq[k] = 1 (nothing written) when the true walk leaves a list
-// before meeting the next one, or the lists end, before n starts.  The piece
-// bounds are the same in every lane (uniform loads), so the loops are too.
+// One wavefront per batch: the true walk is walker 0's list, then each walker's
+// from where its predecessor met it.  Its first n starts go to the batch's
+// slots of evq; seq[k] = 1 (nothing written) when the true walk meets no later
+// walker, or the lists end, before n starts.  The chain is followed 64 walkers
+// at a time, from their values in the lanes' registers, first to see whether
+// it covers the batch and then to copy its pieces, 16 lanes each.
 __global__ __launch_bounds__(64) void fe_seg_assemble_kernel(FeBatchWalkArgs a)
 {
     const uint64_t k = blockIdx.x;
     const uint32_t lane = threadIdx.x;
     if (k >= a.nb)
         return;
-    const uint32_t n = fe_batch_events(a, k);
-    // check first, so that a batch left to the one-thread walk gets no partial starts
-    uint32_t begin = 0;
-    uint64_t have = 0;
-    bool ok = false;
-    for (uint32_t s = 0; s < a.S; ++s) {
-        const uint64_t w = k * a.S + s;
-        const int32_t jp = s + 1 < a.S ? a.join_prev[w + 1] : -1;
-        const bool meets = jp >= 0 && (uint32_t)jp >= begin;
-        const uint32_t end = meets ? (uint32_t)jp : a.counts[w];
-        have += end > begin ? end - begin : 0;
-        if (have >= n) {
-            ok = true;
-            break;
-        }
-        if (!meets)
-            break;
-        begin = (uint32_t)a.join_next[w + 1];
-    }
-    if (lane == 0)
-        a.seq[k] = ok ? 0u : 1u;
-    if (!ok)
-        return;
+    const uint32_t n = fe_batch_events(a, k), S = a.S;
     uint64_t *out = a.evq + k * a.batch_size;
-    uint64_t off = 0;
-    begin = 0;
-    for (uint32_t s = 0; s < a.S && off < n; ++s) {
-        const uint64_t w = k * a.S + s;
-        const int32_t jp = s + 1 < a.S ? a.join_prev[w + 1] : -1;
-        const bool meets = jp >= 0 && (uint32_t)jp >= begin;
-        const uint32_t end = meets ? (uint32_t)jp : a.counts[w];
-        const uint64_t *list = a.lists + w * a.cap;
-        const uint32_t cnt = end > begin ? (uint32_t)min<uint64_t>(end - begin, n - off) : 0u;
-        for (uint32_t i = lane; i < cnt; i += 64)
-            out[off + i] = list[begin + i];
-        off += cnt;
-        if (meets)
-            begin = (uint32_t)a.join_next[w + 1];
+    for (int pass = 0; pass < 2; ++pass) {
+        uint32_t total = 0, s = 0, from = 0; // the chain's starts so far, its walker and where it enters that list
+        for (uint32_t g = 0; g < S && s < S && total < n; g += 64) {
+            const uint64_t t = k * S + min(g + lane, S - 1);
+            const uint32_t cnt = a.counts[t];
+            const int32_t next = a.next[t];
+            const uint32_t met = a.met[t];
+            uint32_t begin = 0, len = 0, off = 0; // this lane's walker's piece
+            while (s < S && s < g + 64 && total < n) { // uniform
+                const int l = (int)(s - g);
+                const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cnt, l);
+                const uint32_t piece = c > from ? c - from : 0u;
+                if ((int)lane == l) {
+                    begin = from;
+                    len = min(piece, n - total);
+                    off = total;
+                }
+                total += piece;
+                const int32_t to = __builtin_amdgcn_readlane(next, l);
+                from = (uint32_t)__builtin_amdgcn_readlane((int)met, l);
+                s = to < 0 ? S : (uint32_t)to;
+            }
+            if (pass == 0)
+                continue;
+            for (uint32_t w0 = 0; w0 < 64; w0 += 4) {
+                const uint32_t w = w0 + lane / 16, i0 = lane % 16;
+                const uint32_t wb = (uint32_t)__shfl((int)begin, (int)w), wl = (uint32_t)__shfl((int)len, (int)w);
+                const uint32_t wo = (uint32_t)__shfl((int)off, (int)w);
+                const uint32_t *src = a.lists + (k * S + g + w) * a.cap + wb;
+                const uint64_t q0 = k * a.piece_stride + (uint64_t)(g + w) * a.seg;
+#pragma unroll 4
+                for (uint32_t i = i0; i < wl; i += 16)
+                    out[wo + i] = q0 + src[i];
+            }
+        }
+        if (pass == 0) {
+            if (lane == 0)
+                a.seq[k] = total >= n ? 0u : 1u;
+            if (total < n)
+                return;
+        }
     }
 }
 
@@ -1579,32 +1664,14 @@ __global__ __launch_bounds__(64) void fe_seq_walk_kernel(FeBatchWalkArgs a)
 void launch_fe_walk_batches(const FeBatchWalkArgs &a, hipStream_t st)
 {
     const uint64_t walkers = a.nb * a.S;
-    const unsigned wb = (unsigned)((walkers + 255) / 256), bb = (unsigned)((a.nb + 63) / 64);
-    hipLaunchKernelGGL(fe_seg_bit_walk_kernel, dim3((unsigned)((walkers + BW_THREADS - 1) / BW_THREADS)),
-                       dim3(BW_THREADS), 0, st, a);
-    hipLaunchKernelGGL(fe_seg_join_kernel, dim3(wb), dim3(256), 0, st, a);
+    const unsigned wb = (unsigned)((walkers + BW_THREADS - 1) / BW_THREADS), bb = (unsigned)((a.nb + 63) / 64);
+    hipLaunchKernelGGL(fe_seg_walk_kernel, dim3(wb), dim3(BW_THREADS), 0, st, a);
+    hipLaunchKernelGGL(fe_seg_join_kernel, dim3(wb), dim3(BW_THREADS), 0, st, a);
     hipLaunchKernelGGL(fe_seg_assemble_kernel, dim3((unsigned)a.nb), dim3(64), 0, st, a);
     hipLaunchKernelGGL(fe_seq_walk_kernel, dim3(bb), dim3(64), 0, st, a);
 }
 
-// ---- faster-evgen on the xoshiro256+ stream, jump seeding --------------------
-// Each piece's first state J^b s0, one thread per piece (divergent bit tests;
-// the matrix columns still come in with uniform scalar loads).
-__global__ __launch_bounds__(64) void xo_piece_state_kernel(XoPieceArgs a)
-{
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= a.nb)
-        return;
-    const uint64_t b = a.b_first + k;
-    uint64_t s[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]};
-    for (int j = 0; j < a.kb; ++j)
-        if ((b >> j) & 1ull)
-            gf2_apply(a.bt + 1024 * j, s);
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-        a.states[4 * k + w] = s[w];
-}
-
+// ---- expansion of the xoshiro streams for faster-evgen ------------------------
 struct Xo256Gen {
     uint64_t s[4];
     __device__ __forceinline__ double next() { return xo_uniform(s); }
@@ -1614,8 +1681,8 @@ struct Xo128Gen {
     __device__ __forceinline__ float next() { return xo128_uniform(s); }
 };
 
-// One wavefront per piece.  Lane l expands positions [l * pt, (l + 1) * pt)
-// of the piece from its state skipped l * pt draws, one 128-byte line of
+// Lane l of a wavefront expands positions [l * pt, (l + 1) * pt)
+// of its range from its state skipped l * pt draws, one 128-byte line of
 // values (16 f64 or 32 f32) at a time, with the draws of positions
 // p + 1 .. p + 3 in hand when position p is stored, so that p's accept bits
 // (with p + 1 and with p + 3) are known; 3 draws past the lane's range
@@ -1624,8 +1691,10 @@ struct Xo128Gen {
 // scattered values.  The bit words go out 4 at a time (128 positions) per
 // lane.
 template <class T, class Gen>
-__device__ __forceinline__ void xo_expand_piece(Gen g, T *piece, uint32_t *acc1, uint32_t *acc3, uint32_t pt)
+__device__ __forceinline__ void xo_expand_piece(Gen g, T *piece, uint32_t *acc1, uint32_t *acc3)
 {
+    constexpr uint32_t pt = 12 * XO_EXPAND_RUN; // positions per lane
+    static_assert(pt % 128 == 0, "whole groups of 4 bit words per lane");
     constexpr int B = 128 / sizeof(T), ROW = B + 1; // values per block (a 128-byte line), padded LDS rows
     constexpr int NB = 128 / B;        // blocks per group of 4 bit words
     __shared__ T st[64 * ROW];
@@ -1669,64 +1738,47 @@ __device__ __forceinline__ void xo_expand_piece(Gen g, T *piece, uint32_t *acc1,
     }
 }
 
-// Skip of the lane's state to its first draw: M^(lane * pt) as the product
-// of M^(pt 2^j) over the set bits j of the lane index, six matrices that every
-// lane reads alike.
+// One wavefront per XO_EXPAND draws of a piece: it skips to the piece's first
+// draw, on to its own and then to its lanes' states.  Bound by the stores and,
+// for few pieces, by one wavefront's draws: 5000 pieces of xoshiro128+ 750 us
+// (3.65 GB), 1060 with a wavefront per piece and the skips of pieces and lanes
+// thread by thread; 484 of xoshiro256+ 177 us, before 640.
+constexpr uint64_t XO_EXPAND = 64 * 12 * XO_EXPAND_RUN;
 __global__ __launch_bounds__(64) void xo_expand_kernel(XoPieceArgs a)
 {
-    const uint64_t k = blockIdx.x;
+    const uint32_t split = (uint32_t)(a.piece_len / XO_EXPAND);
+    const uint64_t k = blockIdx.x / split, b = a.b_first + k, at = XO_EXPAND * (blockIdx.x % split);
+    uint64_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]};
+    if (a.b16)
+        xo_advance_uniform(a.b16, b, sw);
+    xo_advance_uniform(a.m16, a.b16 ? at : b * a.piece_len + at, sw);
     Xo256Gen g;
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-        g.s[w] = a.states[4 * k + w];
-#pragma unroll 1
-    for (int j = 0; j < 6; ++j)
-        if ((threadIdx.x >> j) & 1u)
-            gf2_apply(a.lt + 1024 * j, g.s);
-    const uint64_t words = a.piece_len / 32;
-    xo_expand_piece<double>(g, a.xbuf + k * a.piece_len, a.acc1 + k * words, a.acc3 + k * words, a.per_thread);
+    xo_lane_states(a.lanes, sw, g.s);
+    const uint64_t o = k * a.piece_len + at;
+    xo_expand_piece<double>(g, a.xbuf + o, a.acc1 + o / 32, a.acc3 + o / 32);
 }
-// xoshiro128+ pieces, as the xoshiro256+ ones above.
-__global__ __launch_bounds__(64) void xo128_piece_state_kernel(Xo128PieceArgs a)
-{
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= a.nb)
-        return;
-    const uint64_t b = a.b_first + k;
-    uint32_t s[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]};
-    for (int j = 0; j < a.kb; ++j)
-        if ((b >> j) & 1ull)
-            gf2_apply128(a.bt + 512 * j, s);
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-        a.states[4 * k + w] = s[w];
-}
-
 __global__ __launch_bounds__(64) void xo128_expand_kernel(Xo128PieceArgs a)
 {
-    const uint64_t k = blockIdx.x;
+    const uint32_t split = (uint32_t)(a.piece_len / XO_EXPAND);
+    const uint64_t k = blockIdx.x / split, b = a.b_first + k, at = XO_EXPAND * (blockIdx.x % split);
+    uint32_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]};
+    if (a.b16)
+        xo128_advance_uniform(a.b16, b, sw);
+    xo128_advance_uniform(a.m16, a.b16 ? at : b * a.piece_len + at, sw);
     Xo128Gen g;
-#pragma unroll
-    for (int w = 0; w < 4; ++w)
-        g.s[w] = a.states[4 * k + w];
-#pragma unroll 1
-    for (int j = 0; j < 6; ++j)
-        if ((threadIdx.x >> j) & 1u)
-            gf2_apply128(a.lt + 512 * j, g.s);
-    const uint64_t words = a.piece_len / 32;
-    xo_expand_piece<float>(g, a.xbuf + k * a.piece_len, a.acc1 + k * words, a.acc3 + k * words, a.per_thread);
+    xo128_lane_states(a.lanes, sw, g.s);
+    const uint64_t o = k * a.piece_len + at;
+    xo_expand_piece<float>(g, a.xbuf + o, a.acc1 + o / 32, a.acc3 + o / 32);
 }
 
 void launch_xo128_expand(const Xo128PieceArgs &a, hipStream_t st)
 {
-    hipLaunchKernelGGL(xo128_piece_state_kernel, dim3((unsigned)((a.nb + 63) / 64)), dim3(64), 0, st, a);
-    hipLaunchKernelGGL(xo128_expand_kernel, dim3((unsigned)a.nb), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(xo128_expand_kernel, dim3((unsigned)(a.nb * (a.piece_len / XO_EXPAND))), dim3(64), 0, st, a);
 }
 
 void launch_xo_expand(const XoPieceArgs &a, hipStream_t st)
 {
-    hipLaunchKernelGGL(xo_piece_state_kernel, dim3((unsigned)((a.nb + 63) / 64)), dim3(64), 0, st, a);
-    hipLaunchKernelGGL(xo_expand_kernel, dim3((unsigned)a.nb), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(xo_expand_kernel, dim3((unsigned)(a.nb * (a.piece_len / XO_EXPAND))), dim3(64), 0, st, a);
 }
 
 
