@@ -38,8 +38,11 @@ constexpr uint32_t COND_MASK[L] = {0x03Fu, 0xFC0u, 0x555u, 0xAAAu, 0x1C7u, 0xE38
 // and sample: a(16) h1(64) h2(64) obar(32) h2bar(64) h1bar(64).
 constexpr int SAVE_A = 0, SAVE_H1 = 16, SAVE_H2 = 80, SAVE_OB = 144, SAVE_H2B = 176, SAVE_H1B = 240, SAVE_F = 304;
 
+// The bf16 weights as the kernels take them into LDS, one image per layer.
+constexpr int WIMG_BYTES = 32512;
+
 struct FlowKernelArgs {
-    const uint16_t *wbf; // bf16 parameters [L][LP]
+    const void *wimg;    // [L] images
     uint64_t n;          // samples
     // Input of the forward pass: explicit v (n x 16 f32, device) when v_in is
     // set, else the counter stream: v_ij from draw 12 (sample0 + i) + j of key.
@@ -62,11 +65,11 @@ struct FlowKernelArgs {
 };
 
 struct FlowBackArgs {
-    const uint16_t *wbf;
+    const void *wimg;
     uint64_t n;
     const float *zsave;  // [L][n][16]
     const float *gz;     // [n][16] dloss/dz at the flow output
-    uint16_t *save;      // [L][SAVE_F][n] bf16, feature-major
+    uint16_t *save;      // [L][n / 16][SAVE_F / 16][16 samples][16 rows] bf16 (n a multiple of 16)
     float *gv;           // [n][16] dloss/dz at the flow input (may be null)
 };
 
@@ -75,14 +78,26 @@ void launch_flow_forward(const FlowKernelArgs &a, hipStream_t st);
 // log q (and 1/q_mix) of given or uniformly drawn points.
 void launch_flow_inverse(const FlowKernelArgs &a, hipStream_t st);
 void launch_flow_backward(const FlowBackArgs &a, hipStream_t st);
+// The mean of logq - logf over the batch's samples.
+struct FlowLossArgs {
+    const float *logq, *logf;
+    float *out;
+};
+// An Adam step of all parameters: weights, moments, images.
+struct FlowAdamArgs {
+    float *w, *m, *v;
+    void *wimg;
+    int step;
+    float lr, beta1, beta2, eps;
+};
 // Weight and bias gradients over the batch (n a multiple of 16):
 // grad[L][LP] = inv_n sum_n ..., through a partial-sum buffer `part` of
-// flow_wgrad_part_bytes(n) bytes.
+// flow_wgrad_part_bytes(n) bytes; with them the batch's loss and the Adam step
+// that takes the gradient, if given.
 size_t flow_wgrad_part_bytes(uint64_t n);
-void launch_flow_wgrad(const uint16_t *save, uint64_t n, float inv_n, float *part, float *grad, hipStream_t st);
-void launch_flow_adam(float *w, uint16_t *wbf, float *m, float *v, const float *g, int step, float lr, float beta1,
-                      float beta2, float eps, hipStream_t st);
-void launch_flow_to_bf16(const float *w, uint16_t *wbf, hipStream_t st);
+void launch_flow_wgrad(const uint16_t *save, uint64_t n, float inv_n, float *part, float *grad, const FlowLossArgs *loss,
+                       const FlowAdamArgs *adam, hipStream_t st);
+void launch_flow_to_bf16(const float *w, void *wimg, hipStream_t st);
 
 } // namespace tpf
 
@@ -100,6 +115,4 @@ namespace tpf {
 void launch_flow_integrand(const tpd::Params &P, const double lam[5], uint64_t n, const double *u, double eps,
                            double tau, double fcap, int target, float clip, float *gz, float *logf, double *f_out,
                            hipStream_t st);
-// *out = mean(logq - logf) over n samples.
-void launch_flow_loss(const float *logq, const float *logf, uint64_t n, float *out, hipStream_t st);
 } // namespace tpf

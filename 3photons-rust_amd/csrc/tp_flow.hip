@@ -82,49 +82,46 @@ __host__ __device__ constexpr int k32_pos(int k) // stored position of original 
     return 32 * (k / 32) + 8 * ((k % 16) / 4) + (k % 4) + 4 * ((k % 32) / 16);
 }
 constexpr int L_W1 = 0, L_W2 = L_W1 + H * S_W1, L_W3 = L_W2 + H * S_W2, L_FWD = L_W3 + O * S_W3;
-constexpr int L_W1T = L_FWD, L_W2T = L_W1T + DP * S_W1T, L_W3T = L_W2T + H * S_W2T, L_ALL = L_W3T + H * S_W3T;
+constexpr int L_W1T = 0, L_W2T = L_W1T + DP * S_W1T, L_W3T = L_W2T + H * S_W2T, L_T = L_W3T + H * S_W3T;
 
-struct LdsLayer {
-    uint16_t w[L_ALL];
-    float b[H + H + O];
-};
-
-// Forward weights only (W1, W2, W3 and the biases, same offsets as LdsLayer):
-// the forward and inverse kernels keep all L layers of them resident.
+// Forward weights only (W1, W2, W3 and the biases): the forward and inverse
+// kernels keep all L layers of them resident.
 struct LdsFwd {
     uint16_t w[L_FWD];
     float b[H + H + O];
 };
 
-// One layer's weights and biases into LDS; TRANSPOSED (backward pass, an
-// LdsLayer) also writes W1^T, W2^T, W3^T.
-template <bool TRANSPOSED, class Lds> __device__ __forceinline__ void load_layer(Lds &s, const uint16_t *wl)
+// With W1^T, W2^T, W3^T (backward pass).
+struct LdsLayer : LdsFwd {
+    uint16_t wt[L_T];
+};
+static_assert(sizeof(LdsLayer) == WIMG_BYTES && sizeof(LdsFwd) % 16 == 0, "the weights' images are copied by 16 bytes");
+
+// Parameter i of a layer, in bf16, into the layer's image: the kernels that
+// write the weights lay them out once, so that a workgroup takes them into LDS
+// as they are, 16 bytes a lane (from the parameters' own order, 2 bytes a lane
+// with their places worked out, it took 10 us of the forward kernel's 31).
+__device__ __forceinline__ void put_weight(LdsLayer &s, int i, uint16_t v)
 {
-    static_assert(!TRANSPOSED || sizeof(s.w) == sizeof(uint16_t) * L_ALL, "the transposed copies need an LdsLayer");
-    for (int i = threadIdx.x; i < H * DP; i += blockDim.x) {
+    if (i < OFF_B1) {
         const int r = i / DP, c = i % DP;
-        s.w[L_W1 + r * S_W1 + c] = wl[OFF_W1 + i];
-        if constexpr (TRANSPOSED)
-            s.w[L_W1T + c * S_W1T + r] = wl[OFF_W1 + i];
+        s.w[L_W1 + r * S_W1 + c] = v;
+        s.wt[L_W1T + c * S_W1T + r] = v;
+    } else if (i < OFF_W2) {
+        s.b[i - OFF_B1] = bf2f(v);
+    } else if (i < OFF_B2) {
+        const int r = (i - OFF_W2) / H, c = (i - OFF_W2) % H;
+        s.w[L_W2 + r * S_W2 + k32_pos(c)] = v;
+        s.wt[L_W2T + c * S_W2T + r] = v;
+    } else if (i < OFF_W3) {
+        s.b[H + i - OFF_B2] = bf2f(v);
+    } else if (i < OFF_B3) {
+        const int r = (i - OFF_W3) / H, c = (i - OFF_W3) % H;
+        s.w[L_W3 + r * S_W3 + k32_pos(c)] = v;
+        s.wt[L_W3T + c * S_W3T + r] = v;
+    } else {
+        s.b[2 * H + i - OFF_B3] = bf2f(v);
     }
-    for (int i = threadIdx.x; i < H * H; i += blockDim.x) {
-        const int r = i / H, c = i % H;
-        s.w[L_W2 + r * S_W2 + k32_pos(c)] = wl[OFF_W2 + i];
-        if constexpr (TRANSPOSED)
-            s.w[L_W2T + c * S_W2T + r] = wl[OFF_W2 + i];
-    }
-    for (int i = threadIdx.x; i < O * H; i += blockDim.x) {
-        const int r = i / H, c = i % H;
-        s.w[L_W3 + r * S_W3 + k32_pos(c)] = wl[OFF_W3 + i];
-        if constexpr (TRANSPOSED)
-            s.w[L_W3T + c * S_W3T + r] = wl[OFF_W3 + i];
-    }
-    for (int i = threadIdx.x; i < H; i += blockDim.x) {
-        s.b[i] = bf2f(wl[OFF_B1 + i]);
-        s.b[H + i] = bf2f(wl[OFF_B2 + i]);
-    }
-    for (int i = threadIdx.x; i < O; i += blockDim.x)
-        s.b[2 * H + i] = bf2f(wl[OFF_B3 + i]);
 }
 
 // A operand of a 16x16 tile of a row-major LDS matrix: rows 16 mb .., cols 16 kb ..
@@ -217,6 +214,16 @@ __device__ __forceinline__ f4 masked(f4 z, uint32_t cond)
     return a;
 }
 
+// x, computed in every lane: a select between x and another value then stays
+// one, where the compiler would branch around x (the lane groups differ in what
+// they transform, so such a branch is never skipped, and it keeps the features'
+// exponentials from running beside each other).
+__device__ __forceinline__ float always(float x)
+{
+    asm("" : "+v"(x));
+    return x;
+}
+
 // Sum over the four lane groups of one sample (lanes l, l^16, l^32, l^48).
 __device__ __forceinline__ float sample_sum(float x)
 {
@@ -259,26 +266,42 @@ __device__ __forceinline__ double sigmoid_u(float z)
 // ---- forward ----------------------------------------------------------------
 // The forward and inverse kernels load the forward weights of all L layers
 // into LDS once (97.5 KB, one block per CU) and then stride over the samples
-// with no further barrier: one 512-thread block (8 wavefronts, two per SIMD)
-// takes 8 waves x TILES tiles x 16 samples per pass.  Tiles per wavefront: 4
-// for long runs; batches below FWD_SMALL_N samples take FWD_TILES_SMALL so
-// that the grid still covers every CU.
-constexpr int FWD_WAVES = 8, FWD_TILES = 4, FWD_TILES_SMALL = 2, BWD_TILES = 4;
+// with no further barrier: a block takes waves x tiles x 16 samples per pass.
+// Bound by VALU issue (some 120 instructions per tile, layer and wavefront next
+// to 16 matrix instructions) where the wavefronts cover each other's latencies,
+// so three wavefronts per SIMD with two tiles each take the long runs and four
+// with one tile the batches that would leave CUs idle otherwise.  1.4e7 samples
+// drawn and 6e6 inverted, with the weighted event loop: 4.05 ms; 4.11 at two
+// wavefronts of four tiles, 4.14 at four of one; a training batch of 65 536: 20
+// us, 31 at two of two with the weights read by 2 bytes.
+constexpr int FWD_WAVES = 12, FWD_TILES = 2, FWD_WAVES_SMALL = 16, FWD_TILES_SMALL = 1;
 constexpr uint64_t FWD_SMALL_N = 1u << 20;
 
-__device__ __forceinline__ void load_resident(LdsFwd (&s)[L], const uint16_t *wbf)
+template <int WAVES> __device__ __forceinline__ void load_resident(LdsFwd (&s)[L], const void *wimg)
 {
+    constexpr int THREADS = 64 * WAVES;
+    constexpr int N = sizeof(LdsFwd) / 16, PER = (N + THREADS - 1) / (THREADS);
+    uint4 v[L][PER];
+#pragma unroll
     for (int l = 0; l < L; ++l)
-        load_layer<false>(s[l], wbf + (size_t)l * LP);
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+            v[l][k] = static_cast<const uint4 *>(wimg)[l * (WIMG_BYTES / 16) + min((int)threadIdx.x + THREADS * k, N - 1)];
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+            if ((int)threadIdx.x + THREADS * k < N)
+                reinterpret_cast<uint4 *>(&s[l])[threadIdx.x + THREADS * k] = v[l][k];
     __syncthreads();
 }
 
-template <int TILES>
-__global__ __launch_bounds__(64 * FWD_WAVES) void flow_forward_kernel(FlowKernelArgs a)
+template <int TILES, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void flow_forward_kernel(FlowKernelArgs a)
 {
-    constexpr int CHUNK = FWD_WAVES * TILES * 16;
-    __shared__ LdsFwd s[L];
-    load_resident(s, a.wbf);
+    constexpr int CHUNK = WAVES * TILES * 16;
+    __shared__ __attribute__((aligned(16))) LdsFwd s[L];
+    load_resident<WAVES>(s, a.wimg);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
     for (uint64_t base = (uint64_t)blockIdx.x * CHUNK; base < a.n; base += (uint64_t)gridDim.x * CHUNK) {
         f4 z[TILES];
@@ -304,10 +327,12 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void flow_forward_kernel(FlowKernel
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float x = 4 * g + i < D ? vv[i] : 0.5f;
-                const float lx = flog(x), l1x = flog(1.f - x);
-                z[t][i] = lx - l1x;
+                // (the multiply-adds are written out: which product the compiler
+                // contracts would depend on the kernel's other choices)
+                const float lx = __builtin_amdgcn_logf(x), l1x = flog(1.f - x);
+                z[t][i] = fmaf(lx, LN2, -l1x);
                 if (4 * g + i < D)
-                    l += lx + l1x; // log v (1 - v)
+                    l += fmaf(lx, LN2, l1x); // log v (1 - v)
             }
             ld[t] = l;
         }
@@ -322,7 +347,7 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void flow_forward_kernel(FlowKernel
 #pragma unroll
                 for (int i = 0; i < 4; ++i) { // branch-free: exp(0) = 1 exactly
                     const bool tr = transformed(cond, 4 * g + i);
-                    const float sc = tr ? FLOW_SCALE * ftanh(r.o0[i]) : 0.f;
+                    const float sc = tr ? always(FLOW_SCALE * ftanh(r.o0[i])) : 0.f;
                     z[t][i] = z[t][i] * fexp(sc) + (tr ? r.o1[i] : 0.f);
                     ld[t] -= sc;
                 }
@@ -360,12 +385,12 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void flow_forward_kernel(FlowKernel
 }
 
 // ---- inverse: density of given or uniformly drawn points --------------------
-template <int TILES>
-__global__ __launch_bounds__(64 * FWD_WAVES) void flow_inverse_kernel(FlowKernelArgs a)
+template <int TILES, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void flow_inverse_kernel(FlowKernelArgs a)
 {
-    constexpr int CHUNK = FWD_WAVES * TILES * 16;
-    __shared__ LdsFwd s[L];
-    load_resident(s, a.wbf);
+    constexpr int CHUNK = WAVES * TILES * 16;
+    __shared__ __attribute__((aligned(16))) LdsFwd s[L];
+    load_resident<WAVES>(s, a.wimg);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
     for (uint64_t base = (uint64_t)blockIdx.x * CHUNK; base < a.n; base += (uint64_t)gridDim.x * CHUNK) {
         f4 z[TILES];
@@ -391,10 +416,10 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void flow_inverse_kernel(FlowKernel
                     }
                 }
                 // u and 1 - u formed in f64, logs in f32
-                const float lu = flog((float)u), l1u = flog((float)(1. - u));
-                z[t][i] = lu - l1u;
+                const float lu = __builtin_amdgcn_logf((float)u), l1u = flog((float)(1. - u));
+                z[t][i] = fmaf(lu, LN2, -l1u);
                 if (j < D)
-                    l -= lu + l1u; // - log u (1 - u)
+                    l -= fmaf(lu, LN2, l1u); // - log u (1 - u)
             }
             ld[t] = l;
         }
@@ -407,7 +432,7 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void flow_inverse_kernel(FlowKernel
 #pragma unroll
                 for (int i = 0; i < 4; ++i) { // branch-free: exp(0) = 1 exactly
                     const bool tr = transformed(cond, 4 * g + i);
-                    const float sc = tr ? FLOW_SCALE * ftanh(r.o0[i]) : 0.f;
+                    const float sc = tr ? always(FLOW_SCALE * ftanh(r.o0[i])) : 0.f;
                     z[t][i] = (z[t][i] - (tr ? r.o1[i] : 0.f)) * fexp(-sc);
                     ld[t] -= sc;
                 }
@@ -434,18 +459,35 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void flow_inverse_kernel(FlowKernel
 // ---- backward (training) -----------------------------------------------------
 // loss per sample: log q(u) - log(f(u) + eps); gz = dloss/dz at the flow
 // output.  Walks the layers top-down, recomputing each MLP from the saved
-// layer input, and stores the bf16 activations and deltas (feature-major) for
-// the batch weight-gradient products.
+// layer input, and stores the bf16 activations and deltas for the batch
+// weight-gradient products, by tiles of 16 samples: [layer][tile][19 row
+// blocks][16 samples][16 rows], so that a wavefront stores a row block's 512
+// bytes as its lanes hold them.  Bound by those stores (239 MB for a batch of
+// 65 536, 35 us at the rate of a fill) and the latency of a layer's products,
+// which four wavefronts per SIMD of one tile each share: 51 us; at two of two
+// tiles 74; at one of four, with 2-byte stores row by row and the weights read
+// and transposed by 2 bytes, 150.
+//
+constexpr int BWD_TILES = 1, BWD_WAVES = 16, SAVE_BLOCKS = SAVE_F / 16;
 template <int TILES>
-__global__ __launch_bounds__(256) void flow_backward_kernel(FlowBackArgs a)
+__global__ __launch_bounds__(64 * BWD_WAVES) __attribute__((amdgpu_waves_per_eu(4, 4))) void flow_backward_kernel(FlowBackArgs a)
 {
-    constexpr int CHUNK = 4 * TILES * 16;
-    __shared__ LdsLayer s;
+    constexpr int THREADS = 64 * BWD_WAVES, CHUNK = BWD_WAVES * TILES * 16;
+    constexpr int N = sizeof(LdsLayer) / 16, PER = (N + THREADS - 1) / THREADS;
+    __shared__ __attribute__((aligned(16))) LdsLayer s;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
+    const uint4 *img = static_cast<const uint4 *>(a.wimg);
     for (uint64_t base = (uint64_t)blockIdx.x * CHUNK; base < a.n; base += (uint64_t)gridDim.x * CHUNK) {
         f4 gz[TILES];
         bool valid[TILES];
         uint64_t idx[TILES];
+        uint4 next[PER]; // the next layer's weights, loaded beside the products of this one
+        auto fetch = [&](int l) {
+#pragma unroll
+            for (int k = 0; k < PER; ++k)
+                next[k] = img[l * N + min((int)threadIdx.x + THREADS * k, N - 1)];
+        };
+        fetch(L - 1);
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             idx[t] = base + (uint64_t)(wave * TILES + t) * 16 + (lane & 15);
@@ -454,23 +496,27 @@ __global__ __launch_bounds__(256) void flow_backward_kernel(FlowBackArgs a)
         }
         for (int l = L - 1; l >= 0; --l) {
             __syncthreads();
-            load_layer<true>(s, a.wbf + (size_t)l * LP);
+#pragma unroll
+            for (int k = 0; k < PER; ++k)
+                if ((int)threadIdx.x + THREADS * k < N)
+                    reinterpret_cast<uint4 *>(&s)[threadIdx.x + THREADS * k] = next[k];
             __syncthreads();
+            if (l > 0)
+                fetch(l - 1);
             const uint32_t cond = COND_MASK[l];
-            uint16_t *sv = a.save + (size_t)l * SAVE_F * a.n;
 #pragma unroll 1
             for (int t = 0; t < TILES; ++t) {
+                asm volatile("" ::: "memory"); // weights come from LDS for each tile: kept over them they spill
                 f4 zin = valid[t] ? *reinterpret_cast<const f4 *>(a.zsave + ((size_t)l * a.n + idx[t]) * 16 + 4 * g)
                                   : (f4){0.f, 0.f, 0.f, 0.f};
                 // rows row0 + 4g .. + 3 of this lane's sample, stored as soon as
                 // they are formed (short live ranges)
                 const bool ok = valid[t];
-                const uint64_t n = idx[t], N = a.n;
+                s4 *sv = reinterpret_cast<s4 *>(a.save) +
+                         ((size_t)l * (a.n / 16) + idx[t] / 16) * (SAVE_BLOCKS * 64) + 4 * (lane & 15) + g;
                 auto put = [&](int row0, s4 v) {
                     if (ok)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            sv[(size_t)(row0 + 4 * g + i) * N + n] = (uint16_t)v[i];
+                        sv[row0 * 4] = v;
                 };
                 MlpFwd r;
                 mlp_forward(s, masked(zin, cond), r);
@@ -484,18 +530,13 @@ __global__ __launch_bounds__(256) void flow_backward_kernel(FlowBackArgs a)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int j = 4 * g + i;
-                    if (transformed(cond, j)) {
-                        const float th = ftanh(r.o0[i]);
-                        const float es = fexp(FLOW_SCALE * th);
-                        const float sbar = gz[t][i] * zin[i] * es - 1.f; // the -sum s term of log q
-                        ob0[i] = sbar * FLOW_SCALE * (1.f - th * th);
-                        ob1[i] = gz[t][i];
-                        zb[i] = gz[t][i] * es;
-                    } else {
-                        ob0[i] = 0.f;
-                        ob1[i] = 0.f;
-                        zb[i] = j < D ? gz[t][i] : 0.f;
-                    }
+                    const bool tr = transformed(cond, j);
+                    const float th = ftanh(r.o0[i]);
+                    const float es = fexp(FLOW_SCALE * th);
+                    const float sbar = gz[t][i] * zin[i] * es - 1.f; // the -sum s term of log q
+                    ob0[i] = tr ? always(sbar * FLOW_SCALE * (1.f - th * th)) : 0.f;
+                    ob1[i] = tr ? gz[t][i] : 0.f;
+                    zb[i] = tr ? always(gz[t][i] * es) : j < D ? gz[t][i] : 0.f;
                 }
                 const s4 obb0 = pack4(ob0), obb1 = pack4(ob1);
                 put(SAVE_OB, obb0);
@@ -504,8 +545,8 @@ __global__ __launch_bounds__(256) void flow_backward_kernel(FlowBackArgs a)
                 s4 h2b[4], h1b[4];
 #pragma unroll
                 for (int mb = 0; mb < 4; ++mb) {
-                    f4 c = mfma(atile(s.w + L_W3T, S_W3T, mb, 0), obb0, zero);
-                    c = mfma(atile(s.w + L_W3T, S_W3T, mb, 1), obb1, c);
+                    f4 c = mfma(atile(s.wt + L_W3T, S_W3T, mb, 0), obb0, zero);
+                    c = mfma(atile(s.wt + L_W3T, S_W3T, mb, 1), obb1, c);
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         c[i] *= r.h2d[mb][i];
@@ -517,7 +558,7 @@ __global__ __launch_bounds__(256) void flow_backward_kernel(FlowBackArgs a)
                     f4 c = zero;
 #pragma unroll
                     for (int kb = 0; kb < 4; ++kb)
-                        c = mfma(atile(s.w + L_W2T, S_W2T, mb, kb), h2b[kb], c);
+                        c = mfma(atile(s.wt + L_W2T, S_W2T, mb, kb), h2b[kb], c);
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         c[i] *= r.h1d[mb][i];
@@ -527,7 +568,7 @@ __global__ __launch_bounds__(256) void flow_backward_kernel(FlowBackArgs a)
                 f4 ab = zero;
 #pragma unroll
                 for (int kb = 0; kb < 4; ++kb)
-                    ab = mfma(atile(s.w + L_W1T, S_W1T, 0, kb), h1b[kb], ab);
+                    ab = mfma(atile(s.wt + L_W1T, S_W1T, 0, kb), h1b[kb], ab);
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if (conditioning(cond, 4 * g + i))
@@ -548,40 +589,20 @@ __global__ __launch_bounds__(256) void flow_backward_kernel(FlowBackArgs a)
 // on MFMA, with the sample index as the reduction dimension.  One 256-thread
 // block per (layer, sample range): chunks of 64 samples of all 304 saved rows
 // are staged through LDS (the next chunk is loaded into registers while the
-// current one is multiplied), so every saved value is read from HBM once.
+// current one is multiplied), so every saved value is read from HBM once, and
+// that read is what bounds the kernel (48 us for 65 536 samples, 4.9 TB/s).  A row block of 16 samples lies there
+// sample by sample; the transposing LDS read gives lane 16 g + r row r's
+// samples 4g .. 4g + 3, the operand layout of the products.
 // The layer's 38 output tiles -- 28 weight tiles and 10 bias tiles, whose
-// B operand is a column of ones -- are spread over the four wavefronts.  Each
+// B operand is a column of ones -- are spread over the four wavefronts by the
+// row blocks of their deltas, so that a wavefront reads three of those and
+// seven row blocks of activations for its ten products.  Each
 // block writes partial sums for all of its layer's parameters, and
 // flow_grad_reduce_kernel adds the partials of each parameter in block order,
 // so the result does not depend on scheduling.
-constexpr int GR_CHUNK = 64, GR_STRIDE = 68, GR_TILES = 38, GR_PER_WAVE = 10;
-constexpr int GR_PIECES = SAVE_F * (GR_CHUNK / 8), GR_LOADS = (GR_PIECES + 255) / 256;
+constexpr int GR_CHUNK = 64, GR_TILE_BYTES = SAVE_BLOCKS * 512;
+constexpr int GR_PIECES = GR_CHUNK / 16 * GR_TILE_BYTES / 16, GR_LOADS = (GR_PIECES + 255) / 256;
 constexpr int GR_MIN_CHUNKS = 8, GR_MAX_SPLIT = 128;
-
-struct GTile {
-    int delta_row, act_row, param_off, ld; // act_row < 0: bias tile (ones operand)
-};
-
-// Tiles of one layer: W1 4 row blocks, W2 4 x 4, W3 2 x 4, then b1 4, b2 4,
-// b3 2 row blocks.  param_off is the parameter of the tile's element (0, 0).
-__device__ __forceinline__ GTile gtile(int t)
-{
-    if (t < 4)
-        return {SAVE_H1B + 16 * t, SAVE_A, OFF_W1 + 16 * t * DP, DP};
-    if (t < 20) {
-        const int mb = (t - 4) / 4, kb = (t - 4) % 4;
-        return {SAVE_H2B + 16 * mb, SAVE_H1 + 16 * kb, OFF_W2 + 16 * mb * H + 16 * kb, H};
-    }
-    if (t < 28) {
-        const int mb = (t - 20) / 4, kb = (t - 20) % 4;
-        return {SAVE_OB + 16 * mb, SAVE_H2 + 16 * kb, OFF_W3 + 16 * mb * H + 16 * kb, H};
-    }
-    if (t < 32)
-        return {SAVE_H1B + 16 * (t - 28), -1, OFF_B1 + 16 * (t - 28), 0};
-    if (t < 36)
-        return {SAVE_H2B + 16 * (t - 32), -1, OFF_B2 + 16 * (t - 32), 0};
-    return {SAVE_OB + 16 * (t - 36), -1, OFF_B3 + 16 * (t - 36), 0};
-}
 
 // Sample-range blocks per layer for n samples.
 static int wgrad_split(uint64_t n)
@@ -591,33 +612,69 @@ static int wgrad_split(uint64_t n)
     return (int)(s < 1 ? 1 : s > GR_MAX_SPLIT ? GR_MAX_SPLIT : s);
 }
 
-__global__ __launch_bounds__(256) void flow_wgrad_kernel(const uint16_t *save, uint64_t n, int split, float *part)
+// Mean over the batch of log q - log(f + eps) by one workgroup of 256 threads,
+// in a fixed order: 1024 strided sums of 4-wide loads, then a tree.
+__device__ __forceinline__ void batch_loss(const FlowLossArgs &a, uint64_t n, double *red)
 {
-    __shared__ uint16_t lds[SAVE_F * GR_STRIDE];
+    const uint64_t n4 = n / 4;
+    const float4 *q4 = reinterpret_cast<const float4 *>(a.logq), *f4p = reinterpret_cast<const float4 *>(a.logf);
+    for (uint32_t v = threadIdx.x; v < 1024; v += 256) {
+        double acc = 0.;
+#pragma unroll 8
+        for (uint64_t i = v; i < n4; i += 1024) {
+            const float4 q = q4[i], f = f4p[i];
+            acc += (((double)q.x - (double)f.x) + ((double)q.y - (double)f.y)) +
+                   (((double)q.z - (double)f.z) + ((double)q.w - (double)f.w));
+        }
+        for (uint64_t i = 4 * n4 + v; i < n; i += 1024)
+            acc += (double)a.logq[i] - (double)a.logf[i];
+        red[v] = acc;
+    }
+    __syncthreads();
+    for (uint32_t o = 512; o > 0; o >>= 1) {
+        for (uint32_t v = threadIdx.x; v < o; v += 256)
+            red[v] += red[v + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0)
+        *a.out = (float)(red[0] / (double)n);
+}
+
+__global__ __launch_bounds__(256) void flow_wgrad_kernel(const uint16_t *save, uint64_t n, int split, float *part,
+                                                         FlowLossArgs loss)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t lds[GR_CHUNK / 16 * GR_TILE_BYTES / 2];
     const int layer = blockIdx.x / split, ks = blockIdx.x % split;
+    if (layer == L) { // one block more where the training step's loss is wanted
+        batch_loss(loss, n, reinterpret_cast<double *>(lds));
+        return;
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r16 = lane & 15;
     const uint64_t chunks = (n + GR_CHUNK - 1) / GR_CHUNK, per = (chunks + split - 1) / split;
     const uint64_t c0 = (uint64_t)ks * per, c1 = c0 + per < chunks ? c0 + per : chunks;
-    const uint16_t *sv = save + (size_t)layer * SAVE_F * n;
-    // piece p = 8 samples (16 B) of row p / 8; n is a multiple of 16, so a
-    // piece lies wholly inside or wholly past the batch
+    // n is a multiple of 16: whole tiles
+    const uint64_t pieces = n / 16 * (GR_TILE_BYTES / 16);
+    const uint4 *sv = reinterpret_cast<const uint4 *>(save) + (size_t)layer * pieces;
     uint4 buf[GR_LOADS];
     auto load = [&](uint64_t c) {
 #pragma unroll
         for (int k = 0; k < GR_LOADS; ++k) {
             const int p = threadIdx.x + 256 * k;
-            const uint64_t smp = c * GR_CHUNK + 8 * (p & 7);
+            const uint64_t at = c * GR_PIECES + p;
             buf[k] = make_uint4(0u, 0u, 0u, 0u);
-            if (p < GR_PIECES && smp < n)
-                buf[k] = *reinterpret_cast<const uint4 *>(sv + (size_t)(p >> 3) * n + smp);
+            if (p < GR_PIECES && at < pieces)
+                buf[k] = sv[at];
         }
     };
-    f4 acc[GR_PER_WAVE];
+    // The wavefront's products: b1, W1 (with a) of row block H1B + wave, b2, W2
+    // (with h1's four) of H2B + wave, b3 and W3 (with two of h2's) of OB.
+    f4 acc[10];
 #pragma unroll
-    for (int j = 0; j < GR_PER_WAVE; ++j)
+    for (int j = 0; j < 10; ++j)
         acc[j] = (f4){0.f, 0.f, 0.f, 0.f};
     const short one = (short)0x3F80; // bf16 1.0
     const s4 ones = {one, one, one, one};
+    const int ob = wave & 1, h2 = 2 * (wave >> 1);
     if (c0 < c1)
         load(c0);
     for (uint64_t c = c0; c < c1; ++c) {
@@ -625,100 +682,105 @@ __global__ __launch_bounds__(256) void flow_wgrad_kernel(const uint16_t *save, u
 #pragma unroll
         for (int k = 0; k < GR_LOADS; ++k) {
             const int p = threadIdx.x + 256 * k;
-            if (p < GR_PIECES) {
-                uint2 *d = reinterpret_cast<uint2 *>(lds + (p >> 3) * GR_STRIDE + 8 * (p & 7));
-                d[0] = make_uint2(buf[k].x, buf[k].y);
-                d[1] = make_uint2(buf[k].z, buf[k].w);
-            }
+            if (p < GR_PIECES)
+                reinterpret_cast<uint4 *>(lds)[p] = buf[k];
         }
         __syncthreads();
         if (c + 1 < c1)
             load(c + 1);
 #pragma unroll
-        for (int kk = 0; kk < GR_CHUNK / 16; ++kk)
+        for (int kk = 0; kk < GR_CHUNK / 16; ++kk) {
+            typedef __attribute__((address_space(3))) s4 lds_s4;
+            uint16_t *tile = lds + kk * (GR_TILE_BYTES / 2) + 4 * lane;
+            auto rows = [&](int row0) { // row block row0 / 16
+                return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)(tile + 16 * row0));
+            };
+            const s4 d1 = rows(SAVE_H1B + 16 * wave), d2 = rows(SAVE_H2B + 16 * wave), d3 = rows(SAVE_OB + 16 * ob);
+            acc[0] = mfma(d1, ones, acc[0]);
+            acc[1] = mfma(d1, rows(SAVE_A), acc[1]);
+            acc[2] = mfma(d2, ones, acc[2]);
 #pragma unroll
-            for (int j = 0; j < GR_PER_WAVE; ++j) {
-                const int t = wave + 4 * j;
-                if (t < GR_TILES) {
-                    const GTile w = gtile(t);
-                    const int col = 16 * kk + 4 * g;
-                    const s4 A = *reinterpret_cast<const s4 *>(lds + (w.delta_row + r16) * GR_STRIDE + col);
-                    const s4 B =
-                        w.act_row < 0 ? ones : *reinterpret_cast<const s4 *>(lds + (w.act_row + r16) * GR_STRIDE + col);
-                    acc[j] = mfma(A, B, acc[j]);
-                }
-            }
-    }
-    float *pl = part + ((size_t)ks * L + layer) * LP;
+            for (int kb = 0; kb < 4; ++kb)
+                acc[3 + kb] = mfma(d2, rows(SAVE_H1 + 16 * kb), acc[3 + kb]);
+            acc[7] = mfma(d3, ones, acc[7]);
 #pragma unroll
-    for (int j = 0; j < GR_PER_WAVE; ++j) {
-        const int t = wave + 4 * j;
-        if (t >= GR_TILES)
-            continue;
-        const GTile w = gtile(t);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = 4 * g + i; // C layout: lane holds rows 4g.. of column r16
-            if (w.act_row >= 0)
-                pl[w.param_off + row * w.ld + r16] = acc[j][i];
-            else if (r16 == 0)
-                pl[w.param_off + row] = acc[j][i];
+            for (int kb = 0; kb < 2; ++kb)
+                acc[8 + kb] = mfma(d3, rows(SAVE_H2 + 16 * (h2 + kb)), acc[8 + kb]);
         }
     }
+    float *pl = part + ((size_t)ks * L + layer) * LP;
+    auto weights = [&](int off, int ld, f4 v) { // C layout: lane holds rows 4g.. of column r16
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            pl[off + (4 * g + i) * ld + r16] = v[i];
+    };
+    auto bias = [&](int off, f4 v) {
+        if (r16 == 0)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                pl[off + 4 * g + i] = v[i];
+    };
+    bias(OFF_B1 + 16 * wave, acc[0]);
+    weights(OFF_W1 + 16 * wave * DP, DP, acc[1]);
+    bias(OFF_B2 + 16 * wave, acc[2]);
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+        weights(OFF_W2 + 16 * wave * H + 16 * kb, H, acc[3 + kb]);
+    if (wave < 2)
+        bias(OFF_B3 + 16 * ob, acc[7]);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+        weights(OFF_W3 + 16 * ob * H + 16 * (h2 + kb), H, acc[8 + kb]);
 }
 
 // grad[i] = inv_n sum over the sample-range blocks, in block order (loads
-// in groups of 16 so that they are in flight together).
-__global__ __launch_bounds__(256) void flow_grad_reduce_kernel(const float *part, int split, float inv_n, float *grad)
+// in groups of 32 so that they are in flight together), and in training the
+// parameter's Adam step from it.
+__device__ __forceinline__ LdsLayer &weight_image(void *wimg, int i) { return static_cast<LdsLayer *>(wimg)[i / LP]; }
+template <bool ADAM>
+__global__ __launch_bounds__(256) void flow_grad_reduce_kernel(const float *part, int split, float inv_n, float *grad,
+                                                               FlowAdamArgs a)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= NPARAM)
         return;
     float sum = 0.f;
-    for (int k0 = 0; k0 < split; k0 += 16) {
-        float v[16];
+    for (int k0 = 0; k0 < split; k0 += 32) {
+        float v[32];
 #pragma unroll
-        for (int j = 0; j < 16; ++j)
+        for (int j = 0; j < 32; ++j)
             v[j] = k0 + j < split ? part[(size_t)(k0 + j) * NPARAM + i] : 0.f;
 #pragma unroll
-        for (int j = 0; j < 16; ++j)
+        for (int j = 0; j < 32; ++j)
             sum += v[j];
     }
-    grad[i] = sum * inv_n;
+    const float gi = sum * inv_n;
+    grad[i] = gi;
+    if constexpr (ADAM) {
+        const float mi = a.beta1 * a.m[i] + (1.f - a.beta1) * gi;
+        const float vi = a.beta2 * a.v[i] + (1.f - a.beta2) * gi * gi;
+        a.m[i] = mi;
+        a.v[i] = vi;
+        const float mh = mi / (1.f - powf(a.beta1, (float)a.step)), vh = vi / (1.f - powf(a.beta2, (float)a.step));
+        const float wi = a.w[i] - a.lr * mh / (sqrtf(vh) + a.eps);
+        a.w[i] = wi;
+        put_weight(weight_image(a.wimg, i), i % LP, f2bf(wi));
+    }
 }
 
-__global__ void flow_adam_kernel(float *w, uint16_t *wbf, float *m, float *v, const float *g, int step, float lr,
-                                 float b1, float b2, float eps)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= NPARAM)
-        return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float mh = mi / (1.f - powf(b1, (float)step)), vh = vi / (1.f - powf(b2, (float)step));
-    const float wi = w[i] - lr * mh / (sqrtf(vh) + eps);
-    w[i] = wi;
-    wbf[i] = f2bf(wi);
-}
-
-__global__ void flow_to_bf16_kernel(const float *w, uint16_t *wbf)
+__global__ void flow_to_bf16_kernel(const float *w, void *wimg)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < NPARAM)
-        wbf[i] = f2bf(w[i]);
+        put_weight(weight_image(wimg, i), i % LP, f2bf(w[i]));
 }
 
 // ---- launchers ---------------------------------------------------------------
-template <int TILES> static unsigned grid_for(uint64_t n) { return (unsigned)((n + 64 * TILES - 1) / (64 * TILES)); }
-
 // Resident-weight kernels: one pass per block covers FWD_WAVES * TILES * 16
 // samples; at most max_blocks blocks (one per CU), striding over the rest.
-template <int TILES> static unsigned grid_resident(const FlowKernelArgs &a)
+template <int TILES, int WAVES> static unsigned grid_resident(const FlowKernelArgs &a)
 {
-    const uint64_t chunk = (uint64_t)FWD_WAVES * TILES * 16, need = (a.n + chunk - 1) / chunk;
+    const uint64_t chunk = (uint64_t)WAVES * TILES * 16, need = (a.n + chunk - 1) / chunk;
     const uint64_t cap = a.max_blocks ? a.max_blocks : need;
     return (unsigned)std::max<uint64_t>(1, std::min(need, cap));
 }
@@ -726,48 +788,49 @@ template <int TILES> static unsigned grid_resident(const FlowKernelArgs &a)
 void launch_flow_forward(const FlowKernelArgs &a, hipStream_t st)
 {
     if (a.n < FWD_SMALL_N)
-        hipLaunchKernelGGL(flow_forward_kernel<FWD_TILES_SMALL>, dim3(grid_resident<FWD_TILES_SMALL>(a)),
-                           dim3(64 * FWD_WAVES), 0, st, a);
+        hipLaunchKernelGGL((flow_forward_kernel<FWD_TILES_SMALL, FWD_WAVES_SMALL>),
+                           dim3(grid_resident<FWD_TILES_SMALL, FWD_WAVES_SMALL>(a)), dim3(64 * FWD_WAVES_SMALL), 0, st, a);
     else
-        hipLaunchKernelGGL(flow_forward_kernel<FWD_TILES>, dim3(grid_resident<FWD_TILES>(a)), dim3(64 * FWD_WAVES), 0,
-                           st, a);
+        hipLaunchKernelGGL((flow_forward_kernel<FWD_TILES, FWD_WAVES>), dim3(grid_resident<FWD_TILES, FWD_WAVES>(a)),
+                           dim3(64 * FWD_WAVES), 0, st, a);
 }
 
 void launch_flow_inverse(const FlowKernelArgs &a, hipStream_t st)
 {
     if (a.n < FWD_SMALL_N)
-        hipLaunchKernelGGL(flow_inverse_kernel<FWD_TILES_SMALL>, dim3(grid_resident<FWD_TILES_SMALL>(a)),
-                           dim3(64 * FWD_WAVES), 0, st, a);
+        hipLaunchKernelGGL((flow_inverse_kernel<FWD_TILES_SMALL, FWD_WAVES_SMALL>),
+                           dim3(grid_resident<FWD_TILES_SMALL, FWD_WAVES_SMALL>(a)), dim3(64 * FWD_WAVES_SMALL), 0, st, a);
     else
-        hipLaunchKernelGGL(flow_inverse_kernel<FWD_TILES>, dim3(grid_resident<FWD_TILES>(a)), dim3(64 * FWD_WAVES), 0,
-                           st, a);
+        hipLaunchKernelGGL((flow_inverse_kernel<FWD_TILES, FWD_WAVES>), dim3(grid_resident<FWD_TILES, FWD_WAVES>(a)),
+                           dim3(64 * FWD_WAVES), 0, st, a);
 }
 
 void launch_flow_backward(const FlowBackArgs &a, hipStream_t st)
 {
-    hipLaunchKernelGGL(flow_backward_kernel<BWD_TILES>, dim3(grid_for<BWD_TILES>(a.n)), dim3(256), 0, st, a);
+    constexpr uint64_t chunk = BWD_WAVES * BWD_TILES * 16;
+    hipLaunchKernelGGL(flow_backward_kernel<BWD_TILES>, dim3((unsigned)((a.n + chunk - 1) / chunk)), dim3(64 * BWD_WAVES), 0,
+                       st, a);
 }
 
 size_t flow_wgrad_part_bytes(uint64_t n) { return (size_t)wgrad_split(n) * NPARAM * sizeof(float); }
 
-void launch_flow_wgrad(const uint16_t *save, uint64_t n, float inv_n, float *part, float *grad, hipStream_t st)
+void launch_flow_wgrad(const uint16_t *save, uint64_t n, float inv_n, float *part, float *grad, const FlowLossArgs *loss,
+                       const FlowAdamArgs *adam, hipStream_t st)
 {
     const int split = wgrad_split(n);
-    hipLaunchKernelGGL(flow_wgrad_kernel, dim3(L * split), dim3(256), 0, st, save, n, split, part);
-    hipLaunchKernelGGL(flow_grad_reduce_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, st, part, split, inv_n,
-                       grad);
+    hipLaunchKernelGGL(flow_wgrad_kernel, dim3(L * split + (loss ? 1 : 0)), dim3(256), 0, st, save, n, split, part,
+                       loss ? *loss : FlowLossArgs{});
+    if (adam)
+        hipLaunchKernelGGL(flow_grad_reduce_kernel<true>, dim3((NPARAM + 255) / 256), dim3(256), 0, st, part, split, inv_n,
+                           grad, *adam);
+    else
+        hipLaunchKernelGGL(flow_grad_reduce_kernel<false>, dim3((NPARAM + 255) / 256), dim3(256), 0, st, part, split, inv_n,
+                           grad, FlowAdamArgs{});
 }
 
-void launch_flow_adam(float *w, uint16_t *wbf, float *m, float *v, const float *g, int step, float lr, float beta1,
-                      float beta2, float eps, hipStream_t st)
+void launch_flow_to_bf16(const float *w, void *wimg, hipStream_t st)
 {
-    hipLaunchKernelGGL(flow_adam_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, st, w, wbf, m, v, g, step, lr,
-                       beta1, beta2, eps);
-}
-
-void launch_flow_to_bf16(const float *w, uint16_t *wbf, hipStream_t st)
-{
-    hipLaunchKernelGGL(flow_to_bf16_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, st, w, wbf);
+    hipLaunchKernelGGL(flow_to_bf16_kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, st, w, wimg);
 }
 
 // ---- integrand and its gradient for training --------------------------------
@@ -825,38 +888,6 @@ void launch_flow_integrand(const tpd::Params &P, const double lam[5], uint64_t n
 {
     hipLaunchKernelGGL(flow_integrand_kernel, dim3((unsigned)((n + 127) / 128)), dim3(128), 0, st, P, lam[0], lam[1],
                        lam[2], lam[3], lam[4], n, u, eps, tau, fcap, target, clip, gz, logf, f_out);
-}
-
-// Mean over the batch of log q - log(f + eps), one 1024-thread block, fixed
-// summation order (per-thread strided sums of 4-wide loads, then a tree).
-__global__ __launch_bounds__(1024) void flow_loss_kernel(const float *logq, const float *logf, uint64_t n, float *out)
-{
-    __shared__ double red[1024];
-    double acc = 0.;
-    const uint64_t n4 = n / 4;
-    const float4 *q4 = reinterpret_cast<const float4 *>(logq), *f4p = reinterpret_cast<const float4 *>(logf);
-#pragma unroll 4
-    for (uint64_t i = threadIdx.x; i < n4; i += 1024) {
-        const float4 q = q4[i], f = f4p[i];
-        acc += (((double)q.x - (double)f.x) + ((double)q.y - (double)f.y)) +
-               (((double)q.z - (double)f.z) + ((double)q.w - (double)f.w));
-    }
-    for (uint64_t i = 4 * n4 + threadIdx.x; i < n; i += 1024)
-        acc += (double)logq[i] - (double)logf[i];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int o = 512; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o)
-            red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
-        *out = (float)(red[0] / (double)n);
-}
-
-void launch_flow_loss(const float *logq, const float *logf, uint64_t n, float *out, hipStream_t st)
-{
-    hipLaunchKernelGGL(flow_loss_kernel, dim3(1), dim3(1024), 0, st, logq, logf, n, out);
 }
 
 } // namespace tpf

@@ -21,7 +21,7 @@ using namespace tpe;
 
 struct Flow {
     Ctx *c = nullptr;
-    DevBuf w, wbf, m, v, grad;            // parameters, bf16 copy, Adam moments, gradient
+    DevBuf w, wimg, m, v, grad;           // parameters, their bf16 images, Adam moments, gradient
     DevBuf zsave, save, u, logq, gz, logf; // training batch
     DevBuf gpart;                         // per-block partial weight gradients
     DevBuf f, loss, vin, io;              // integrand values, per-step loss, staging
@@ -102,7 +102,7 @@ int upload_params(Flow *f, std::vector<float> w)
     const size_t bytes = (size_t)tpf::NPARAM * sizeof(float);
     int rc = ensure(f->c, f->w, bytes);
     if (!rc)
-        rc = ensure(f->c, f->wbf, (size_t)tpf::NPARAM * sizeof(uint16_t));
+        rc = ensure(f->c, f->wimg, (size_t)tpf::L * tpf::WIMG_BYTES);
     if (!rc)
         rc = ensure(f->c, f->m, bytes);
     if (!rc)
@@ -114,7 +114,7 @@ int upload_params(Flow *f, std::vector<float> w)
     FHIP(f, hipMemcpyAsync(f->w.p, w.data(), bytes, hipMemcpyHostToDevice, f->c->stream));
     FHIP(f, hipMemsetAsync(f->m.p, 0, bytes, f->c->stream));
     FHIP(f, hipMemsetAsync(f->v.p, 0, bytes, f->c->stream));
-    tpf::launch_flow_to_bf16(static_cast<const float *>(f->w.p), static_cast<uint16_t *>(f->wbf.p), f->c->stream);
+    tpf::launch_flow_to_bf16(static_cast<const float *>(f->w.p), f->wimg.p, f->c->stream);
     FHIP(f, hipGetLastError());
     FHIP(f, hipStreamSynchronize(f->c->stream)); // w is a host temporary
     f->step = 0;
@@ -125,7 +125,7 @@ tpf::FlowKernelArgs base_args(const Flow *f, uint64_t n)
 {
     tpf::FlowKernelArgs a;
     std::memset(&a, 0, sizeof a);
-    a.wbf = static_cast<const uint16_t *>(f->wbf.p);
+    a.wimg = f->wimg.p;
     a.n = n;
     a.alpha = 1.;
     a.max_blocks = (uint32_t)f->c->cus;
@@ -223,7 +223,7 @@ extern "C" int tp_flow_destroy(void *flow)
             return TP_ERR_ARG;
         (void)hipSetDevice(f->c->device);
         (void)hipStreamSynchronize(f->c->stream);
-        for (DevBuf *b : {&f->w, &f->wbf, &f->m, &f->v, &f->grad, &f->zsave, &f->save, &f->u, &f->logq, &f->gz, &f->logf,
+        for (DevBuf *b : {&f->w, &f->wimg, &f->m, &f->v, &f->grad, &f->zsave, &f->save, &f->u, &f->logq, &f->gz, &f->logf,
                           &f->gpart, &f->f, &f->loss, &f->vin, &f->io, &f->ru, &f->rinvq})
             if (b->p)
                 (void)hipFree(b->p);
@@ -347,12 +347,13 @@ int ensure_train(Flow *f, uint64_t n)
 }
 
 // Backward pass and batch weight gradients for zsave (filled by a forward
-// pass with zsave set) and gz in f->gz.
-int enqueue_grad(Flow *f, uint64_t n, float *gv)
+// pass with zsave set) and gz in f->gz; with the loss and the Adam step, if given.
+int enqueue_grad(Flow *f, uint64_t n, float *gv, const tpf::FlowLossArgs *loss = nullptr,
+                 const tpf::FlowAdamArgs *adam = nullptr)
 {
     tpf::FlowBackArgs b;
     std::memset(&b, 0, sizeof b);
-    b.wbf = static_cast<const uint16_t *>(f->wbf.p);
+    b.wimg = f->wimg.p;
     b.n = n;
     b.zsave = static_cast<const float *>(f->zsave.p);
     b.gz = static_cast<const float *>(f->gz.p);
@@ -361,7 +362,7 @@ int enqueue_grad(Flow *f, uint64_t n, float *gv)
     tpf::launch_flow_backward(b, f->c->stream);
     FHIP(f, hipGetLastError());
     tpf::launch_flow_wgrad(static_cast<const uint16_t *>(f->save.p), n, 1.f / (float)n, static_cast<float *>(f->gpart.p),
-                           static_cast<float *>(f->grad.p), f->c->stream);
+                           static_cast<float *>(f->grad.p), loss, adam, f->c->stream);
     FHIP(f, hipGetLastError());
     return TP_OK;
 }
@@ -517,18 +518,14 @@ extern "C" int tp_flow_train(void *flow, const tp_params *params, const tp_flow_
                                        o->cut_width, o->cap_rel * mean_f, o->target, o->grad_clip, static_cast<float *>(f->gz.p), static_cast<float *>(f->logf.p),
                                        nullptr, c->stream);
             FHIP(f, hipGetLastError());
-            tpf::launch_flow_loss(static_cast<const float *>(f->logq.p), static_cast<const float *>(f->logf.p), n,
-                                  static_cast<float *>(f->loss.p) + s, c->stream);
-            FHIP(f, hipGetLastError());
-            rc = enqueue_grad(f, n, nullptr);
+            ++f->step;
+            const tpf::FlowLossArgs la{static_cast<const float *>(f->logq.p), static_cast<const float *>(f->logf.p),
+                                       static_cast<float *>(f->loss.p) + s};
+            const tpf::FlowAdamArgs aa{static_cast<float *>(f->w.p), static_cast<float *>(f->m.p), static_cast<float *>(f->v.p),
+                                       f->wimg.p, f->step, o->lr, o->beta1, o->beta2, o->adam_eps};
+            rc = enqueue_grad(f, n, nullptr, &la, &aa);
             if (rc)
                 return rc;
-            ++f->step;
-            tpf::launch_flow_adam(static_cast<float *>(f->w.p), static_cast<uint16_t *>(f->wbf.p),
-                                  static_cast<float *>(f->m.p), static_cast<float *>(f->v.p),
-                                  static_cast<const float *>(f->grad.p), f->step, o->lr, o->beta1, o->beta2, o->adam_eps,
-                                  c->stream);
-            FHIP(f, hipGetLastError());
         }
         HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         HIPCHK(c, hipEventRecord(c->ev[3], c->stream));
