@@ -67,6 +67,8 @@ struct Ctx {
     DevBuf f32ev, f32cnt;       // all-f32 mode: per-event values, accepted events of the parts
     tp_stats last{};
     bool timed = false;
+    bool marking = true;        // whether mark() records its events (closure calls report no times)
+    tp_acc *host_acc = nullptr; // HOST_ACCS accumulators of host memory that kernels write
     // Host staging of the RANF origin: must outlive the asynchronous copies.
     int32_t origin0[56];
     int32_t p00 = 0;
@@ -122,6 +124,28 @@ inline int fail(Ctx *c, int code, const std::string &msg)
         if (e_ != hipSuccess)                                                                          \
             return fail((ctx), TP_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));         \
     } while (0)
+
+// Records event i of the call's times.
+inline int mark(Ctx *c, int i)
+{
+    if (c->marking)
+        HIPCHK(c, hipEventRecord(c->ev[i], c->stream));
+    return TP_OK;
+}
+
+// No event is recorded while one of these lives.
+struct Unmarked {
+    Ctx *c;
+    explicit Unmarked(Ctx *ctx) : c(ctx) { c->marking = false; }
+    ~Unmarked() { c->marking = true; }
+    Unmarked(const Unmarked &) = delete;
+    Unmarked &operator=(const Unmarked &) = delete;
+};
+
+// Results that go to the host in the end, up to this many accumulators, are
+// written there by the kernels: a copy of its own waits for the last kernel and
+// takes some 10 us of the 40 of a small call.
+constexpr uint64_t HOST_ACCS = 4096;
 
 inline int ensure(Ctx *c, DevBuf &b, size_t bytes)
 {

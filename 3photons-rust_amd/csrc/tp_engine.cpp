@@ -157,7 +157,8 @@ int enqueue_xo128_f32(Ctx *c, const tp_params *params, int seeding, const tp_xos
     std::memcpy(a.s0, x->s, sizeof a.s0);
     a.m16 = c->xo->m16_128;
     a.b16 = c->xo->b16_128[seeding];
-    HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+    if (const int e = mark(c, 1))
+        return e;
     for (uint64_t b0 = 0; b0 < nb; b0 += chunk) {
         a.nb = std::min(nb, b0 + chunk) - b0;
         a.b_first = b0;
@@ -166,7 +167,8 @@ int enqueue_xo128_f32(Ctx *c, const tp_params *params, int seeding, const tp_xos
         if (rc)
             return rc;
     }
-    HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+    if (const int e = mark(c, 2))
+        return e;
     return TP_OK;
 }
 
@@ -508,7 +510,8 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
         const uint64_t e0 = b0 * batch_size, e1 = std::min<uint64_t>(b1 * batch_size, num_events);
         const uint64_t n = e1 - e0;
         if (first)
-            HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+            if (const int e = mark(c, 0))
+                return e;
         bool ok = false;
         uint64_t q_next = 0, qbase = 0, bbase = 0, blimit = 0;
         if (device_walk) {
@@ -531,7 +534,8 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
                                      c->stream));
         }
         if (first) {
-            HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+            if (const int e = mark(c, 1))
+                return e;
             first = false;
         }
         if (fa) {
@@ -568,7 +572,8 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
             HIPCHK(c, hipStreamSynchronize(c->stream));
         q_start = q_next;
     }
-    HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+    if (const int e = mark(c, 2))
+        return e;
     *q_end = q_start;
     return TP_OK;
 }
@@ -741,7 +746,8 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         ++c->fe_chunks;
         const uint64_t cnb = std::min(nb, b0 + chunk) - b0;
         if (first)
-            HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+            if (const int e = mark(c, 0))
+                return e;
         tpk::launch_ranf_seed(rs->seed, b0, cnb, static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p),
                               c->stream);
         HIPCHK(c, hipGetLastError());
@@ -779,7 +785,8 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         tpk::launch_fe_walk_batches(w, c->stream);
         HIPCHK(c, hipGetLastError());
         if (first) {
-            HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+            if (const int e = mark(c, 1))
+                return e;
             first = false;
         }
         if (f32) {
@@ -809,7 +816,8 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         if (const int e = launch_event_loop(c, a, 3, (uint32_t)std::min<uint64_t>(num_events, batch_size)))
             return e;
     }
-    HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+    if (const int e = mark(c, 2))
+        return e;
     HIPCHK(c, hipMemcpyAsync(&c->fe_flag_host, c->fe_flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->fe_flag_host)
@@ -862,7 +870,8 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
         ++c->fe_chunks;
         const uint64_t cnb = std::min(nb, b0 + chunk) - b0;
         if (first)
-            HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+            if (const int e = mark(c, 0))
+                return e;
         rc = xo256_expand(c, x->s, true, b0, cnb);
         if (rc)
             return rc;
@@ -880,13 +889,15 @@ int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_sta
         a.evq = w.evq;
         a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
         if (first) {
-            HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+            if (const int e = mark(c, 1))
+                return e;
             first = false;
         }
         if (const int e = launch_event_loop(c, a, 4, (uint32_t)std::min<uint64_t>(num_events, batch_size)))
             return e;
     }
-    HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+    if (const int e = mark(c, 2))
+        return e;
     HIPCHK(c, hipMemcpyAsync(&c->fe_flag_host, c->fe_flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->fe_flag_host)
@@ -953,7 +964,8 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         ++c->fe_chunks;
         const uint64_t cnb = std::min(nb, b0 + chunk) - b0;
         if (first)
-            HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+            if (const int e = mark(c, 0))
+                return e;
         rc = xo128_expand(c, s0, true, b0, cnb);
         if (rc)
             return rc;
@@ -964,7 +976,8 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         tpk::launch_fe_walk_batches(w, c->stream);
         HIPCHK(c, hipGetLastError());
         if (first) {
-            HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+            if (const int e = mark(c, 1))
+                return e;
             first = false;
         }
         fa.nb = cnb;
@@ -980,7 +993,8 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         if (rc)
             return rc;
     }
-    HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+    if (const int e = mark(c, 2))
+        return e;
     HIPCHK(c, hipMemcpyAsync(&c->fe_flag_host, c->fe_flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (c->fe_flag_host)
@@ -1048,10 +1062,12 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         if (rc)
             return rc;
         a.out = per_batch_dev;
-        HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+        if (const int e = mark(c, 1))
+            return e;
         if (const int e = launch_event_loop(c, a, 0, (uint32_t)std::min<uint64_t>(num_events, batch_size)))
             return e;
-        HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+        if (const int e = mark(c, 2))
+            return e;
         return TP_OK;
     }
     const tp_ranf_state *rs = static_cast<const tp_ranf_state *>(state0);
@@ -1072,7 +1088,6 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     std::memcpy(R.round, rs->numbers, sizeof R.round);
     R.p0 = 55u - rs->index;
     R.r16 = static_cast<const uint32_t *>(c->r16.p);
-    HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
     if (seeding == TP_SEED_JUMP) {
         rc = ensure(c, c->origin, nb * 56 * sizeof(int32_t));
         if (!rc)
@@ -1084,7 +1099,8 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         HIPCHK(c, hipGetLastError());
         R.origin = static_cast<const int32_t *>(c->origin.p);
     }
-    HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+    if (const int e = mark(c, 1))
+        return e;
     const uint32_t n = (uint32_t)std::min<uint64_t>(num_events, batch_size);
     if (f32) {
         // (a run whose batches are split has at most MAX_PARTS of them: its
@@ -1100,7 +1116,8 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         if (const int e = launch_event_loop(c, a, 1, n))
             return e;
     }
-    HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
+    if (const int e = mark(c, 2))
+        return e;
     return TP_OK;
 }
 
@@ -1256,7 +1273,12 @@ extern "C" int tp_create(int device, void **ctx_out)
             std::call_once(g_xo[device].once, [&] { xo_setup(g_xo[device].t, c->stream); });
             c->xo = &g_xo[device].t;
         }
-        const int rc = ensure(c, c->parts, MAX_PARTS * sizeof(tp_acc));
+        int rc = ensure(c, c->parts, MAX_PARTS * sizeof(tp_acc));
+        if (!rc && hipHostMalloc(reinterpret_cast<void **>(&c->host_acc), HOST_ACCS * sizeof(tp_acc), hipHostMallocMapped | hipHostMallocCoherent) !=
+                       hipSuccess) {
+            c->host_acc = nullptr;
+            rc = TP_ERR_NOMEM;
+        }
         if (rc) {
             tp_destroy(c);
             return rc;
@@ -1285,6 +1307,8 @@ extern "C" int tp_destroy(void *ctx)
                 (void)hipEventDestroy(e);
         if (c->fe_stat_host)
             (void)hipHostFree(c->fe_stat_host);
+        if (c->host_acc)
+            (void)hipHostFree(c->host_acc);
         (void)hipStreamDestroy(c->stream);
         delete c;
         return TP_OK;
@@ -1611,13 +1635,12 @@ extern "C" int tp_simulate_batch(void *ctx, const tp_params *params, int rng_kin
             std::memset(out, 0, sizeof *out);
             return TP_OK;
         }
-        rc = ensure(c, c->per_batch, sizeof(tp_acc));
+        {
+            const Unmarked quiet(c);
+            rc = enqueue_run(c, params, rng_kind, TP_SEED_SKIPAHEAD, rng_state, n, n, c->host_acc);
+        }
         if (rc)
             return rc;
-        rc = enqueue_run(c, params, rng_kind, TP_SEED_SKIPAHEAD, rng_state, n, n, c->per_batch.p);
-        if (rc)
-            return rc;
-        HIPCHK(c, hipMemcpyAsync(out, c->per_batch.p, sizeof(tp_acc), hipMemcpyDeviceToHost, c->stream));
         // `&mut rng` side effect: 12 draws per event (evgen.rs:182-187), or the
         // walk of the faster-evgen draws.  The new state is formed while the
         // device works, and handed over once it is done.
@@ -1646,6 +1669,7 @@ extern "C" int tp_simulate_batch(void *ctx, const tp_params *params, int rng_kin
             HIPCHK(c, hipStreamSynchronize(c->stream));
             *static_cast<tp_xoshiro128_state *>(rng_state) = s;
         }
+        *out = *c->host_acc;
         return TP_OK;
     });
 }
@@ -1778,17 +1802,21 @@ extern "C" int tp_run(void *ctx, const tp_params *params, int rng_kind, int seed
         if (num_events == 0)
             return fail(c, TP_ERR_ARG, "Must simulate at least one event");
         const uint64_t nb = (num_events + TP_BATCH_SIZE - 1) / TP_BATCH_SIZE;
-        int rc = ensure(c, c->per_batch, nb * sizeof(tp_acc));
+        const bool direct = nb <= HOST_ACCS;
+        int rc = direct ? TP_OK : ensure(c, c->per_batch, nb * sizeof(tp_acc));
         if (rc)
             return rc;
-        rc = tp_run_device(ctx, params, rng_kind, seeding, rng_state0, num_events, static_cast<tp_acc *>(c->per_batch.p),
-                           nullptr, nullptr);
+        rc = tp_run_device(ctx, params, rng_kind, seeding, rng_state0, num_events,
+                           direct ? c->host_acc : static_cast<tp_acc *>(c->per_batch.p), nullptr, nullptr);
         if (rc)
             return rc;
-        HIPCHK(c, hipMemcpyAsync(per_batch_out, c->per_batch.p, nb * sizeof(tp_acc), hipMemcpyDeviceToHost, c->stream));
+        if (!direct)
+            HIPCHK(c, hipMemcpyAsync(per_batch_out, c->per_batch.p, nb * sizeof(tp_acc), hipMemcpyDeviceToHost, c->stream));
         rc = tp_sync(ctx, stats);
         if (rc)
             return rc;
+        if (direct)
+            std::memcpy(per_batch_out, c->host_acc, nb * sizeof(tp_acc));
         if (merged_out && params->precision == TP_PREC_F32) {
             tp_acc m = per_batch_out[0];
             for (uint64_t b = 1; b < nb; ++b)
