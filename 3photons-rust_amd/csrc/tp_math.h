@@ -124,6 +124,27 @@ TPM_FN double sqrt_nonneg(double x)
     d = __builtin_fma(-g, g, x);
     return __builtin_fma(d, h, g);
 }
+// a / b and sqrt(x) in f32, the values of '/' and sqrtf(): their sequences
+// without the scaling that only acts where an exponent (of b, of a below -103, of
+// the quotient, of x below -96) comes near the ends of the range, which the
+// all-f32 event loop's values stay away from; zeros, infinities and NaN come out
+// as in those.  8 and 9 instructions instead of 11 and 16, and quotients by one
+// divisor share its reciprocal.
+TPM_FN float div_f(float a, float b)
+{
+    float y = __builtin_amdgcn_rcpf(b);
+    y = __builtin_fmaf(__builtin_fmaf(-b, y, 1.f), y, y);
+    float q = a * y;
+    q = __builtin_fmaf(__builtin_fmaf(-b, q, a), y, q);
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), y, q), b, a);
+}
+TPM_FN float sqrt_f(float x)
+{
+    const float s = __builtin_amdgcn_sqrtf(x); // within an ulp: the neighbours' residuals decide
+    const float lo = __uint_as_float(__float_as_uint(s) - 1u), hi = __uint_as_float(__float_as_uint(s) + 1u);
+    const float r = __builtin_fmaf(-lo, s, x) <= 0.f ? lo : s;
+    return __builtin_fmaf(-hi, s, x) > 0.f ? hi : r;
+}
 #else
 TPM_FN double div_n(double a, double b) { return a / b; }
 TPM_FN double rcp_n(double b) { return 1. / b; }

@@ -63,20 +63,20 @@ template <class T> __device__ __forceinline__ C<T> cmul(C<T> a, C<T> b)
 }
 // IEEE division and square root: in f64 through tpm::div_n / tpm::sqrt_n
 // (the same correctly rounded results in the event loop's range, fewer
-// instructions), in f32 the plain operations.
+// instructions), in f32 through tpm::div_f / tpm::sqrt_f.
 template <class T> __device__ __forceinline__ T dv(T a, T b)
 {
     if constexpr (std::is_same<T, double>::value)
         return tpm::div_n(a, b);
     else
-        return a / b;
+        return tpm::div_f(a, b);
 }
 template <class T> __device__ __forceinline__ T sq(T x)
 {
     if constexpr (std::is_same<T, double>::value)
         return tpm::sqrt_n(x);
     else
-        return sqrt(x);
+        return tpm::sqrt_f(x);
 }
 // num-complex naive division (spinor.rs divides with it).
 template <class T> __device__ __forceinline__ C<T> cdiv(C<T> a, C<T> b)
@@ -822,7 +822,7 @@ __device__ __forceinline__ void raw_photon_f32(float uc, float uphi, float ue1, 
     double sd, cd;
     tpm::sincos_f64((double)phi, sd, cd);
     const float sphi = (float)sd, cphi = (float)cd;
-    float st = sqrtf(1.f - cos_t * cos_t);
+    float st = tpm::sqrt_f(1.f - cos_t * cos_t);
     float en = -(float)tpm::log_pos((double)(em + 1.17549435e-38f));
     q[0] = en * (st * sphi);
     q[1] = en * (st * cphi);
@@ -837,9 +837,9 @@ __device__ __forceinline__ void conformal_f32(const FParams &P, const float q[3]
     for (int k = 0; k < 4; ++k)
         r[k] = (q[0][k] + q[1][k]) + q[2][k];
     float rn2 = r[3] * r[3] - ((r[0] * r[0] + r[1] * r[1]) + r[2] * r[2]);
-    float alpha = P.e_total / rn2;
-    float rn = sqrtf(rn2);
-    float beta = 1.f / (rn + r[3]);
+    float alpha = tpm::div_f(P.e_total, rn2);
+    float rn = tpm::sqrt_f(rn2);
+    float beta = tpm::div_f(1.f, rn + r[3]);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         float rq = q[i][0] * r[0];
