@@ -66,8 +66,13 @@ __device__ __forceinline__ void hswish_d(float c, float &y, float &d)
     y = c * fminf(fmaxf(fmaf(c, 1.f / 6.f, 0.5f), 0.f), 1.f);
     d = c < -3.f ? 0.f : (c > 3.f ? 1.f : fmaf(c, 1.f / 3.f, 0.5f));
 }
-__device__ __forceinline__ float ftanh(float x) { return 1.f - 2.f * frcp(fexp(2.f * x) + 1.f); }
-__device__ __forceinline__ float softplus(float x) { return fmaxf(x, 0.f) + flog(1.f + fexp(-fabsf(x))); }
+__device__ __forceinline__ float ftanh(float x) { return 1.f - 2.f * frcp(__builtin_amdgcn_exp2f(x * (2.f * LOG2E)) + 1.f); }
+// softplus(-x) + softplus(x) with softplus(x) = max(x, 0) + log(1 + exp(-|x|))
+__device__ __forceinline__ float softplus2(float x)
+{
+    const float lg = __builtin_amdgcn_logf(1.f + fexp(-fabsf(x)));
+    return fmaf(lg, LN2, fabsf(x)) + fmaf(lg, LN2, 0.f); // (each rounded: a product would be contracted into the sum)
+}
 
 // ---- LDS image of one layer (bf16, padded row strides against bank conflicts)
 // W2 and W3 (K = 64) feed K = 32 products: their columns are stored in the
@@ -155,10 +160,10 @@ struct MlpFwd {
     f4 o0, o1;     // s raw (rows 0..15), t raw (rows 16..31)
 };
 
-template <class Lds> __device__ __forceinline__ void mlp_forward(const Lds &s, f4 a_in, MlpFwd &r)
+template <class Lds> __device__ __forceinline__ void mlp_forward(const Lds &s, s4 a_in, MlpFwd &r)
 {
     const int g = (threadIdx.x & 63) >> 4;
-    r.a = pack4(a_in);
+    r.a = a_in;
 #pragma unroll
     for (int mb = 0; mb < 4; ++mb) {
         const f4 c = mfma(atile(s.w + L_W1, S_W1, mb, 0), r.a, bias4(s, 16 * mb + 4 * g));
@@ -204,24 +209,19 @@ template <class Lds> __device__ __forceinline__ void mlp_forward(const Lds &s, f
 __device__ __forceinline__ bool transformed(uint32_t cond, int j) { return j < D && !((cond >> j) & 1u); }
 __device__ __forceinline__ bool conditioning(uint32_t cond, int j) { return j < D && ((cond >> j) & 1u); }
 
-__device__ __forceinline__ f4 masked(f4 z, uint32_t cond)
+// The layer's input in bf16: the lane's conditioning features, the others 0.
+struct CondMask { // all ones in the halves that stay
+    uint32_t lo, hi;
+};
+__device__ __forceinline__ CondMask cond_mask(uint32_t cond)
 {
-    const int g = (threadIdx.x & 63) >> 4;
-    f4 a;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        a[i] = conditioning(cond, 4 * g + i) ? z[i] : 0.f;
-    return a;
+    const uint32_t c = cond >> (4 * ((threadIdx.x & 63) >> 4)); // (no bits from D on)
+    return {(c & 1u ? 0xffffu : 0u) | (c & 2u ? 0xffff0000u : 0u), (c & 4u ? 0xffffu : 0u) | (c & 8u ? 0xffff0000u : 0u)};
 }
-
-// x, computed in every lane: a select between x and another value then stays
-// one, where the compiler would branch around x (the lane groups differ in what
-// they transform, so such a branch is never skipped, and it keeps the features'
-// exponentials from running beside each other).
-__device__ __forceinline__ float always(float x)
+__device__ __forceinline__ s4 masked(f4 z, CondMask m)
 {
-    asm("" : "+v"(x));
-    return x;
+    const uint2 v = __builtin_bit_cast(uint2, pack4(z));
+    return __builtin_bit_cast(s4, make_uint2(v.x & m.lo, v.y & m.hi));
 }
 
 // Sum over the four lane groups of one sample (lanes l, l^16, l^32, l^48).
@@ -239,21 +239,24 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z)
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     return z ^ (z >> 31);
 }
-__device__ __forceinline__ uint64_t stream_u64(uint64_t key, uint64_t k)
+// The Weyl sequence of draw k; the draws after it are GOLDEN apart.
+constexpr uint64_t GOLDEN = 0x9E3779B97F4A7C15ull;
+__device__ __forceinline__ uint64_t stream_at(uint64_t key, uint64_t k)
 {
-    return mix64(key + (k + 1) * 0x9E3779B97F4A7C15ull);
+    uint64_t w = key + (k + 1) * GOLDEN;
+    asm("" : "+v"(w)); // (one product, not one for each of the draws that follow)
+    return w;
 }
 // (2 m + 1) 2^-24 with m the top 23 bits: strictly inside (0, 1), so logit(v)
 // is finite.
-__device__ __forceinline__ float stream_v(uint64_t key, uint64_t k)
+__device__ __forceinline__ float stream_v(uint64_t w)
 {
-    return (float)(uint32_t)(stream_u64(key, k) >> 41) * 0x1.0p-23f + 0x1.0p-24f;
+    uint32_t hi = (uint32_t)(mix64(w) >> 32);
+    asm("" : "+v"(hi)); // (a 32-bit conversion: the compiler would make it a 64-bit one)
+    return (float)(hi >> 9) * 0x1.0p-23f + 0x1.0p-24f;
 }
 // (2 m + 1) 2^-53 with m the top 52 bits: strictly inside (0, 1).
-__device__ __forceinline__ double stream_u(uint64_t key, uint64_t k)
-{
-    return (double)(stream_u64(key, k) >> 12) * 0x1.0p-52 + 0x1.0p-53;
-}
+__device__ __forceinline__ double stream_u(uint64_t w) { return (double)(mix64(w) >> 12) * 0x1.0p-52 + 0x1.0p-53; }
 // u = sigmoid(z), evaluated in f32 (the density is that of the f32 network;
 // the point moves by at most an f32 rounding), stored as f64 and kept inside
 // (0, 1): at most 1 - 2^-53 where the f32 value rounds to 1.
@@ -303,6 +306,7 @@ __global__ __launch_bounds__(64 * WAVES) void flow_forward_kernel(FlowKernelArgs
     __shared__ __attribute__((aligned(16))) LdsFwd s[L];
     load_resident<WAVES>(s, a.wimg);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
+    const bool feat = g < D / 4; // lane group 3 holds padding
     for (uint64_t base = (uint64_t)blockIdx.x * CHUNK; base < a.n; base += (uint64_t)gridDim.x * CHUNK) {
         f4 z[TILES];
         float ld[TILES];
@@ -313,41 +317,44 @@ __global__ __launch_bounds__(64 * WAVES) void flow_forward_kernel(FlowKernelArgs
             idx[t] = base + (uint64_t)(wave * TILES + t) * 16 + (lane & 15);
             valid[t] = idx[t] < a.n;
             f4 vv = {0.5f, 0.5f, 0.5f, 0.5f};
-            if (valid[t]) {
-                if (a.v_in) {
+            if (a.v_in) {
+                if (valid[t])
                     vv = *reinterpret_cast<const f4 *>(a.v_in + 16 * idx[t] + 4 * g);
-                } else {
+            } else if (feat) {
+                const uint64_t w = stream_at(a.key, 12ull * (a.sample0 + idx[t]) + 4 * g);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (4 * g + i < D)
-                            vv[i] = stream_v(a.key, 12ull * (a.sample0 + idx[t]) + 4 * g + i);
-                }
+                for (int i = 0; i < 4; ++i)
+                    vv[i] = stream_v(w + i * GOLDEN);
             }
             float l = 0.f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float x = 4 * g + i < D ? vv[i] : 0.5f;
+                const float x = feat ? vv[i] : 0.5f;
                 // (the multiply-adds are written out: which product the compiler
                 // contracts would depend on the kernel's other choices)
                 const float lx = __builtin_amdgcn_logf(x), l1x = flog(1.f - x);
                 z[t][i] = fmaf(lx, LN2, -l1x);
-                if (4 * g + i < D)
+                if (feat)
                     l += fmaf(lx, LN2, l1x); // log v (1 - v)
             }
             ld[t] = l;
         }
         for (int l = 0; l < L; ++l) {
             const uint32_t cond = COND_MASK[l];
+            const CondMask cm = cond_mask(cond);
 #pragma unroll
             for (int t = 0; t < TILES; ++t) {
                 if (a.zsave && valid[t])
                     *reinterpret_cast<f4 *>(a.zsave + ((size_t)l * a.n + idx[t]) * 16 + 4 * g) = z[t];
                 MlpFwd r;
-                mlp_forward(s[l], masked(z[t], cond), r);
+                mlp_forward(s[l], masked(z[t], cm), r);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) { // branch-free: exp(0) = 1 exactly
+                for (int i = 0; i < 4; ++i) { // exp(0) = 1 exactly
+                    // (sv before the select: the lane groups differ in what they
+                    // transform, so a branch around it is never skipped, and it
+                    // keeps the features' exponentials from running side by side)
                     const bool tr = transformed(cond, 4 * g + i);
-                    const float sc = tr ? always(FLOW_SCALE * ftanh(r.o0[i])) : 0.f;
+                    const float sv = FLOW_SCALE * ftanh(r.o0[i]), sc = tr ? sv : 0.f;
                     z[t][i] = z[t][i] * fexp(sc) + (tr ? r.o1[i] : 0.f);
                     ld[t] -= sc;
                 }
@@ -356,24 +363,32 @@ __global__ __launch_bounds__(64 * WAVES) void flow_forward_kernel(FlowKernelArgs
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             float l = ld[t];
+            if (feat)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (4 * g + i < D) // - log u (1 - u) = softplus(-z) + softplus(z)
-                    l += softplus(-z[t][i]) + softplus(z[t][i]);
+                for (int i = 0; i < 4; ++i) // - log u (1 - u) = softplus(-z) + softplus(z)
+                    l += softplus2(z[t][i]);
             l = sample_sum(l);
             if (!valid[t])
                 continue;
+            if (feat && a.u_out) {
+                double u[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int j = 4 * g + i;
-                if (j < D) {
-                    const double u = sigmoid_u(z[t][i]);
-                    if (a.u_out)
-                        a.u_out[a.u_stride ? j * a.u_stride + idx[t] : 12 * idx[t] + j] = u;
-                    if (a.z_out)
-                        a.z_out[12 * idx[t] + j] = z[t][i];
+                for (int i = 0; i < 4; ++i)
+                    u[i] = sigmoid_u(z[t][i]);
+                if (a.u_stride) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        a.u_out[(4 * g + i) * a.u_stride + idx[t]] = u[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        a.u_out[12 * idx[t] + 4 * g + i] = u[i];
                 }
             }
+            if (feat && a.z_out)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    a.z_out[12 * idx[t] + 4 * g + i] = z[t][i];
             if (g == 0) {
                 if (a.logq_out)
                     a.logq_out[idx[t]] = l;
@@ -392,6 +407,7 @@ __global__ __launch_bounds__(64 * WAVES) void flow_inverse_kernel(FlowKernelArgs
     __shared__ __attribute__((aligned(16))) LdsFwd s[L];
     load_resident<WAVES>(s, a.wimg);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4;
+    const bool feat = g < D / 4; // lane group 3 holds padding
     for (uint64_t base = (uint64_t)blockIdx.x * CHUNK; base < a.n; base += (uint64_t)gridDim.x * CHUNK) {
         f4 z[TILES];
         float ld[TILES];
@@ -401,38 +417,54 @@ __global__ __launch_bounds__(64 * WAVES) void flow_inverse_kernel(FlowKernelArgs
         for (int t = 0; t < TILES; ++t) {
             idx[t] = base + (uint64_t)(wave * TILES + t) * 16 + (lane & 15);
             valid[t] = idx[t] < a.n;
+            double u[4] = {0.5, 0.5, 0.5, 0.5};
+            if (feat && a.u_in) {
+                if (valid[t])
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        u[i] = fmin(fmax(a.u_in[12 * idx[t] + 4 * g + i], 0x1.0p-126), 0x1.fffffffffffffp-1);
+            } else if (feat) {
+                const uint64_t w = stream_at(a.key, 12ull * (a.sample0 + idx[t]) + 4 * g);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    u[i] = stream_u(w + i * GOLDEN);
+                if (a.u_out && valid[t]) {
+                    if (a.u_stride) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            a.u_out[(4 * g + i) * a.u_stride + idx[t]] = u[i];
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            a.u_out[12 * idx[t] + 4 * g + i] = u[i];
+                    }
+                }
+            }
             float l = 0.f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int j = 4 * g + i;
-                double u = 0.5;
-                if (valid[t] && j < D) {
-                    if (a.u_in) {
-                        u = fmin(fmax(a.u_in[12 * idx[t] + j], 0x1.0p-126), 0x1.fffffffffffffp-1);
-                    } else {
-                        u = stream_u(a.key, 12ull * (a.sample0 + idx[t]) + j);
-                        if (a.u_out)
-                            a.u_out[a.u_stride ? j * a.u_stride + idx[t] : 12 * idx[t] + j] = u;
-                    }
-                }
                 // u and 1 - u formed in f64, logs in f32
-                const float lu = __builtin_amdgcn_logf((float)u), l1u = flog((float)(1. - u));
+                const float lu = __builtin_amdgcn_logf((float)u[i]), l1u = flog((float)(1. - u[i]));
                 z[t][i] = fmaf(lu, LN2, -l1u);
-                if (j < D)
+                if (feat)
                     l -= fmaf(lu, LN2, l1u); // - log u (1 - u)
             }
             ld[t] = l;
         }
         for (int l = L - 1; l >= 0; --l) {
             const uint32_t cond = COND_MASK[l];
+            const CondMask cm = cond_mask(cond);
 #pragma unroll
             for (int t = 0; t < TILES; ++t) {
                 MlpFwd r;
-                mlp_forward(s[l], masked(z[t], cond), r);
+                mlp_forward(s[l], masked(z[t], cm), r);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) { // branch-free: exp(0) = 1 exactly
+                for (int i = 0; i < 4; ++i) { // exp(0) = 1 exactly
+                    // (sv before the select: the lane groups differ in what they
+                    // transform, so a branch around it is never skipped, and it
+                    // keeps the features' exponentials from running side by side)
                     const bool tr = transformed(cond, 4 * g + i);
-                    const float sc = tr ? always(FLOW_SCALE * ftanh(r.o0[i])) : 0.f;
+                    const float sv = FLOW_SCALE * ftanh(r.o0[i]), sc = tr ? sv : 0.f;
                     z[t][i] = (z[t][i] - (tr ? r.o1[i] : 0.f)) * fexp(-sc);
                     ld[t] -= sc;
                 }
@@ -441,10 +473,10 @@ __global__ __launch_bounds__(64 * WAVES) void flow_inverse_kernel(FlowKernelArgs
 #pragma unroll
         for (int t = 0; t < TILES; ++t) {
             float l = ld[t];
+            if (feat)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (4 * g + i < D) // log v (1 - v) = -softplus(-z) - softplus(z)
-                    l -= softplus(-z[t][i]) + softplus(z[t][i]);
+                for (int i = 0; i < 4; ++i) // log v (1 - v) = -softplus(-z) - softplus(z)
+                    l -= softplus2(z[t][i]);
             l = sample_sum(l);
             if (valid[t] && g == 0) {
                 if (a.logq_out)
@@ -504,6 +536,7 @@ __global__ __launch_bounds__(64 * BWD_WAVES) __attribute__((amdgpu_waves_per_eu(
             if (l > 0)
                 fetch(l - 1);
             const uint32_t cond = COND_MASK[l];
+            const CondMask cm = cond_mask(cond);
 #pragma unroll 1
             for (int t = 0; t < TILES; ++t) {
                 asm volatile("" ::: "memory"); // weights come from LDS for each tile: kept over them they spill
@@ -519,7 +552,7 @@ __global__ __launch_bounds__(64 * BWD_WAVES) __attribute__((amdgpu_waves_per_eu(
                         sv[row0 * 4] = v;
                 };
                 MlpFwd r;
-                mlp_forward(s, masked(zin, cond), r);
+                mlp_forward(s, masked(zin, cm), r);
                 put(SAVE_A, r.a);
 #pragma unroll
                 for (int mb = 0; mb < 4; ++mb) {
@@ -534,9 +567,10 @@ __global__ __launch_bounds__(64 * BWD_WAVES) __attribute__((amdgpu_waves_per_eu(
                     const float th = ftanh(r.o0[i]);
                     const float es = fexp(FLOW_SCALE * th);
                     const float sbar = gz[t][i] * zin[i] * es - 1.f; // the -sum s term of log q
-                    ob0[i] = tr ? always(sbar * FLOW_SCALE * (1.f - th * th)) : 0.f;
+                    const float o = sbar * FLOW_SCALE * (1.f - th * th), z = gz[t][i] * es;
+                    ob0[i] = tr ? o : 0.f;
                     ob1[i] = tr ? gz[t][i] : 0.f;
-                    zb[i] = tr ? always(gz[t][i] * es) : j < D ? gz[t][i] : 0.f;
+                    zb[i] = tr ? z : j < D ? gz[t][i] : 0.f;
                 }
                 const s4 obb0 = pack4(ob0), obb1 = pack4(ob1);
                 put(SAVE_OB, obb0);
