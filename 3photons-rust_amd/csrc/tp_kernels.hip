@@ -174,37 +174,60 @@ __device__ __forceinline__ int32_t ranf_next_round(int32_t x, const RanfLanes &l
 }
 
 // X_{r+m} from X_r with c = x^(55 m) mod P: X_{r+m}[i] = sum_k c_k Y[i-1+k]
-// over the window Y = (X_r, X_{r+1}).
-__device__ __forceinline__ int32_t ranf_jump(int32_t x, const uint32_t *__restrict__ c, int32_t *win)
+// over the window Y = (X_r, X_{r+1}).  Lane k holds c_k, so that a term waits
+// for no memory but its LDS read, and those are in flight together: a part's
+// start in the event loop takes some 3 us less than with the coefficients read
+// term by term (closure of 10 000 events 35 -> 26 us, 1e7 events 330 -> 307).
+__device__ __forceinline__ uint32_t ranf_jump_lane(const uint32_t *c) { return (threadIdx.x & 63u) < 55 ? c[threadIdx.x & 63u] : 0u; }
+__device__ __forceinline__ int32_t ranf_jump(int32_t x, uint32_t ck, int32_t *win)
 {
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
     int32_t nx = ranf_next_round(x, ranf_lanes());
     if (lane < 55) {
         win[lane] = x;
         win[55 + lane] = nx;
     }
     __syncthreads();
+    const int32_t *w = win + (lane < 55 ? lane : 0);
     uint64_t acc = 0;
-    if (lane < 55) {
-#pragma unroll 5
-        for (int k = 0; k < 55; ++k) {
-            acc += (uint64_t)c[k] * (uint64_t)(uint32_t)win[lane + k];
-            if ((k & 15) == 15)
-                acc %= (uint64_t)MODULO;
-        }
-        acc %= (uint64_t)MODULO;
+#pragma unroll
+    for (int k0 = 0; k0 < 55; k0 += 14) {
+        uint32_t y[14];
+#pragma unroll
+        for (int k = 0; k < 14; ++k)
+            y[k] = k0 + k < 55 ? (uint32_t)w[k0 + k] : 0u;
+#pragma unroll
+        for (int k = 0; k < 14; ++k)
+            if (k0 + k < 55)
+                acc += (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ck, k0 + k) * y[k];
+        acc %= (uint64_t)MODULO; // 14 products and a rest stay below 2^64
     }
     __syncthreads();
     return lane < 55 ? (int32_t)acc : 0;
 }
 
 // X_{r+e} from X_r for a number of rounds e all lanes hold alike.  win: 110
-// ints of LDS, free before and after.
+// ints of LDS, free before and after.  A digit's coefficients are loaded beside
+// the jump before it.
 __device__ __forceinline__ int32_t ranf_advance(int32_t x, const uint32_t *__restrict__ r16, uint64_t e, int32_t *win)
 {
-    for (; e; e >>= 4, r16 += 15 * 55)
-        if (e & 15u)
-            x = ranf_jump(x, r16 + 55 * ((uint32_t)(e & 15u) - 1), win);
+    auto seek = [&]() { // to the next digit that is not 0
+        while (e && !(e & 15u)) {
+            e >>= 4;
+            r16 += 15 * 55;
+        }
+    };
+    auto coefficients = [&]() { return e ? ranf_jump_lane(r16 + 55 * ((uint32_t)(e & 15u) - 1)) : 0u; };
+    seek();
+    uint32_t ck = coefficients();
+    while (e) {
+        const uint32_t now = ck;
+        e >>= 4;
+        r16 += 15 * 55;
+        seek();
+        ck = coefficients();
+        x = ranf_jump(x, now, win);
+    }
     return x;
 }
 
@@ -231,7 +254,7 @@ struct RanfPart {
         const uint64_t q = (own ? 0 : R.p0) + 12ull * (first + (R.origin ? 0 : b * batch_size));
         uint64_t skip = q / 55;
         if (have && R.jump_rounds && round + R.jump_rounds <= skip) { // on from the previous part
-            x = ranf_jump(x, R.jump, win);
+            x = ranf_jump(x, ranf_jump_lane(R.jump), win);
             skip -= round + R.jump_rounds;
         } else {
             const uint32_t lane = threadIdx.x & 63u;

@@ -156,7 +156,7 @@ __device__ __forceinline__ void xo_lane_states(const uint64_t *__restrict__ tab,
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         const uint64_t x = s[w];
-#pragma unroll 4
+#pragma unroll 8
         for (int k = 0; k < 16; ++k) {
             const ulonglong2 *e = t + 128 * (16 * (16 * w + k) + (uint32_t)((x >> (4 * k)) & 15u));
             const ulonglong2 a = e[0], b = e[64];
