@@ -2180,14 +2180,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
 // events' values, four wavefronts per batch: lanes 0..11 of the first add a
 // tile's summands (m_c, m_c^2, w, w^2) in event order, the order that fixes the
 // f32 rounding, while the other three, tile about, load the next tiles' events
-// and write their summands to LDS.  SLOTS: every event has a slot and a flag
-// (source 0), a rejected one's summands being -0.0 (x + (-0.0) == x for every
-// x, so it changes no sum, as when the reference skips it); otherwise the
-// accepted events of the batch's parts in order, tiles running on from part to
-// part.  What bounds it: the chain of adds, 9 cycles an accepted event (26 us a
-// batch, 1536 batches at once), or for long runs the bytes of the events.  A
-// tile's loads have three tiles' time to arrive: with one loading wavefront a
-// closure call of 10 000 events spent 160 us here on their latency.
+// and write the accepted ones' summands to LDS side by side.  SLOTS: every event
+// has a slot and a flag (source 0); otherwise the values are the accepted events
+// of the batch's parts in order, tiles running on from part to part.  What bounds
+// it: the chain of adds, 9 cycles an accepted event (26 us a batch, 1536 batches
+// at once), or for long runs the bytes of the events.  A tile's loads have three
+// tiles' time to arrive: with one loading wavefront a closure call of 10 000
+// events spent 160 us here on their latency, and 54 with a rejected event's slot
+// added as -0.0; 41 now (10 000 batches with slots 745 -> 445 us).
 constexpr int F32_TILE = 128, F32_ROW = F32_TILE + 4; // rows 4 banks apart for the chains' 16-byte reads
 constexpr int F32_BUFS = 4;                           // tiles in LDS: one being added, three being made
 
@@ -2195,7 +2195,7 @@ template <bool SLOTS> __global__ __launch_bounds__(256) void f32_accumulate_kern
 {
     __shared__ __align__(16) float terms[F32_BUFS][12][F32_ROW];
     __shared__ uint32_t before[F32_MAX_PARTS + 1]; // accepted events of the parts before each
-    __shared__ uint32_t kept;
+    __shared__ uint32_t kept, filled[SLOTS ? F32_BUFS : 1]; // accepted events in all, in the tiles
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint64_t lb = blockIdx.x;
     const uint64_t left = a.num_events - (a.b_first + lb) * a.batch_size;
@@ -2220,10 +2220,10 @@ template <bool SLOTS> __global__ __launch_bounds__(256) void f32_accumulate_kern
     }
     const uint32_t tiles = (n + F32_TILE - 1) / F32_TILE;
     constexpr int PER = F32_TILE / 64;
-    float m[PER][5];
+    float m[PER][5], flag[PER];
     bool keep[PER];
     uint32_t cnt = 0;
-    auto load = [&](uint32_t k) {
+    auto load = [&](uint32_t k) { // (nothing in it waits for what it loads)
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const uint32_t e = k * F32_TILE + 64 * i + lane;
@@ -2243,20 +2243,42 @@ template <bool SLOTS> __global__ __launch_bounds__(256) void f32_accumulate_kern
 #pragma unroll
             for (int c = 0; c < 5; ++c)
                 m[i][c] = !keep[i] ? 0.f : SLOTS ? a.ev[6 * at + c] : a.ev[c * a.ev_stride + at];
-            if (SLOTS && keep[i])
-                keep[i] = a.ev[6 * at + 5] != 0.f;
+            flag[i] = SLOTS && keep[i] ? a.ev[6 * at + 5] : 1.f;
         }
     };
     auto write = [&](uint32_t k) {
         float(*row)[F32_ROW] = terms[k % F32_BUFS];
+        if constexpr (SLOTS) { // the accepted ones side by side, in whole groups of 16
+            uint32_t c = 0;
 #pragma unroll
-        for (int i = 0; i < PER; ++i) {
-            const float w = weight_f32(a.P, m[i]), z = -0.f;
-            cnt += (uint32_t)__popcll(__ballot(keep[i]));
+            for (int i = 0; i < PER; ++i) {
+                const float w = weight_f32(a.P, m[i]);
+                const bool in = keep[i] && flag[i] != 0.f;
+                const uint64_t ins = __ballot(in);
+                const uint32_t at = c + (uint32_t)__popcll(ins & ((1ull << lane) - 1ull));
+                c += (uint32_t)__popcll(ins);
+                if (in)
 #pragma unroll
-            for (int j = 0; j < 12; ++j) {
-                const float x = j < 5 ? m[i][j] : j < 10 ? m[i][j - 5] * m[i][j - 5] : j == 10 ? w : w * w;
-                row[j][64 * i + lane] = keep[i] ? x : z;
+                    for (int j = 0; j < 12; ++j)
+                        row[j][at] = j < 5 ? m[i][j] : j < 10 ? m[i][j - 5] * m[i][j - 5] : j == 10 ? w : w * w;
+            }
+            cnt += c;
+            if (lane < (16u - c) % 16u) // x + (-0.0) = x for every x
+#pragma unroll
+                for (int j = 0; j < 12; ++j)
+                    row[j][c + lane] = -0.f;
+            if (lane == 0)
+                filled[k % F32_BUFS] = c;
+        } else {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const float w = weight_f32(a.P, m[i]), z = -0.f;
+                cnt += (uint32_t)__popcll(__ballot(keep[i]));
+#pragma unroll
+                for (int j = 0; j < 12; ++j) {
+                    const float x = j < 5 ? m[i][j] : j < 10 ? m[i][j - 5] * m[i][j - 5] : j == 10 ? w : w * w;
+                    row[j][64 * i + lane] = keep[i] ? x : z;
+                }
             }
         }
     };
@@ -2277,8 +2299,9 @@ template <bool SLOTS> __global__ __launch_bounds__(256) void f32_accumulate_kern
                 load(i + 3);
         } else if (lane < 12) {
             const float4 *row = reinterpret_cast<const float4 *>(terms[i % F32_BUFS][lane]);
+            const int groups = SLOTS ? (__builtin_amdgcn_readfirstlane((int)filled[i % F32_BUFS]) + 15) / 16 : F32_TILE / 16;
 #pragma unroll 2
-            for (int g = 0; g < F32_TILE / 16; ++g) {
+            for (int g = 0; g < groups; ++g) {
                 float4 x[4];
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
