@@ -696,7 +696,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
     if (!rc)
         rc = ensure(c, c->draws, chunk * PS * sizeof(int32_t));
     if (!rc)
-        rc = ensure(c, c->origin, chunk * 56 * sizeof(int32_t));
+        rc = ensure(c, c->origin, 2 * chunk * 56 * sizeof(int32_t)); // origins, then their rounds RANF_LATE
     if (!rc)
         rc = ensure(c, c->p0, chunk * sizeof(int32_t));
     if (!rc)
@@ -720,10 +720,12 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
     c->p00 = static_cast<int32_t>(55u - rs->index);
     c->fe_flag_host = 0;
     HIPCHK(c, hipMemcpyAsync(c->fe_flag.p, &c->fe_flag_host, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    auto expand = [&](uint64_t first_piece, uint64_t npieces, uint64_t d_begin, uint64_t d_end) -> int {
+    int32_t *const later = static_cast<int32_t *>(c->origin.p) + 56 * chunk;
+    auto expand = [&](uint64_t first_piece, uint64_t npieces, uint64_t d_begin, uint64_t d_end, bool own) -> int {
         tpk::RanfArgs r;
         std::memset(&r, 0, sizeof r);
         r.origin = static_cast<const int32_t *>(c->origin.p) + 56 * first_piece;
+        r.later = own && batch_size <= TP_BATCH_SIZE ? later + 56 * first_piece : nullptr;
         r.p0 = static_cast<const int32_t *>(c->p0.p) + first_piece;
         r.r16 = static_cast<const uint32_t *>(c->r16.p);
         r.R = (int32_t)R;
@@ -748,8 +750,8 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
         if (first)
             if (const int e = mark(c, 0))
                 return e;
-        tpk::launch_ranf_seed(rs->seed, b0, cnb, static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p),
-                              c->stream);
+        tpk::launch_ranf_seed(rs->seed, b0, cnb, static_cast<const uint32_t *>(c->r16.p),
+                              static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p), later, c->stream);
         HIPCHK(c, hipGetLastError());
         if (b0 == 0) {
             // batch 0 runs on the caller's state, which may be inside its
@@ -758,11 +760,11 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
             HIPCHK(c, hipMemcpyAsync(c->origin.p, c->origin0, sizeof c->origin0, hipMemcpyHostToDevice, c->stream));
             HIPCHK(c, hipMemcpyAsync(c->p0.p, &c->p00, sizeof c->p00, hipMemcpyHostToDevice, c->stream));
             const uint64_t p00 = (uint64_t)c->p00;
-            rc = expand(0, 1, 0ull - p00, PS - p00);
+            rc = expand(0, 1, 0ull - p00, PS - p00, false);
             if (!rc && cnb > 1)
-                rc = expand(1, cnb - 1, 0, PS);
+                rc = expand(1, cnb - 1, 0, PS, true);
         } else {
-            rc = expand(0, cnb, 0, PS);
+            rc = expand(0, cnb, 0, PS, true);
         }
         if (rc)
             return rc;
@@ -1089,15 +1091,16 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     R.p0 = 55u - rs->index;
     R.r16 = static_cast<const uint32_t *>(c->r16.p);
     if (seeding == TP_SEED_JUMP) {
-        rc = ensure(c, c->origin, nb * 56 * sizeof(int32_t));
+        rc = ensure(c, c->origin, 2 * nb * 56 * sizeof(int32_t)); // origins, then their rounds RANF_LATE
         if (!rc)
             rc = ensure(c, c->p0, nb * sizeof(int32_t));
         if (rc)
             return rc;
-        tpk::launch_ranf_seed(rs->seed, 0, nb, static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p),
-                              c->stream);
+        int32_t *const origin = static_cast<int32_t *>(c->origin.p);
+        tpk::launch_ranf_seed(rs->seed, 0, nb, R.r16, origin, static_cast<int32_t *>(c->p0.p), origin + 56 * nb, c->stream);
         HIPCHK(c, hipGetLastError());
-        R.origin = static_cast<const int32_t *>(c->origin.p);
+        R.origin = origin;
+        R.later = origin + 56 * nb;
     }
     if (const int e = mark(c, 1))
         return e;

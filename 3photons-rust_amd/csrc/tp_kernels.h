@@ -14,11 +14,13 @@ namespace tpk {
 // The RANF stream of a run.  Batch b's events draw from position p0 + 12
 // batch_size b on of the stream whose round 0 is `round` (X[1..55]); with jump
 // seeding (origin non-null) batch b > 0 has a stream of its own, round 0 at
-// origin[56 b] and positions from 0.
+// origin[56 b] and positions from 0.  A batch whose origin holds values outside
+// [0, 1e9) goes on from later[56 b] at round RANF_LATE.
+constexpr uint32_t RANF_LATE = 2048, RANF_LATE_R16 = 2 * 15 + 7; // 8 * 16^2: its place in r16
 struct RanfSource {
     int32_t round[56];
     uint32_t p0;
-    const int32_t *origin;
+    const int32_t *origin, *later;
     const uint32_t *r16;  // x^(55 v 16^j) mod the recurrence's polynomial, 55 coefficients each, v = 1..15,
                           // for the digits of a number of rounds
     uint32_t jump[55];    // x^(55 jump_rounds): from the end of a wavefront's part to near its next one
@@ -81,6 +83,7 @@ struct FusedArgs {
 // skip-ahead mode, or one reseeded batch stream in jump mode.
 struct RanfArgs {
     const int32_t *origin; // [npieces][56] round X[1..55] at [1..55]
+    const int32_t *later;  // the same for round RANF_LATE of reseeded streams, as RanfSource; may be null
     const int32_t *p0;     // [npieces] values of the origin round already consumed
     uint64_t d_begin, d_end; // window of draws (piece-relative) to write
     uint64_t seg_first;    // first segment index of the window
@@ -133,8 +136,8 @@ struct EventOut {
 void launch_events(const FusedArgs &a, int source, uint32_t n, const EventOut &o, hipStream_t st);
 void launch_ranf_expand(const RanfArgs &a, uint64_t npieces, hipStream_t st);
 // Per-batch RANF origins of jump mode: seeded_new(seed0 + 123456*b).
-void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, int32_t *origin, int32_t *p0,
-                      hipStream_t st);
+void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16, int32_t *origin, int32_t *p0,
+                      int32_t *later, hipStream_t st);
 // In-order left fold of nb accumulators (resacc.rs:133-139) into *merged.
 // In-order fold of nb accumulators; f32 = 1 adds in float (all-f32 mode).
 void launch_merge(const void *per_batch, uint64_t nb, void *merged, hipStream_t st, int f32 = 0);

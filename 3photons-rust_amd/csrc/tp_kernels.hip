@@ -191,16 +191,16 @@ __device__ __forceinline__ int32_t ranf_jump(int32_t x, uint32_t ck, int32_t *wi
     const int32_t *w = win + (lane < 55 ? lane : 0);
     uint64_t acc = 0;
 #pragma unroll
-    for (int k0 = 0; k0 < 55; k0 += 14) {
-        uint32_t y[14];
+    for (int k0 = 0; k0 < 55; k0 += 16) {
+        uint32_t y[16];
 #pragma unroll
-        for (int k = 0; k < 14; ++k)
+        for (int k = 0; k < 16; ++k)
             y[k] = k0 + k < 55 ? (uint32_t)w[k0 + k] : 0u;
 #pragma unroll
-        for (int k = 0; k < 14; ++k)
+        for (int k = 0; k < 16; ++k)
             if (k0 + k < 55)
                 acc += (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ck, k0 + k) * y[k];
-        acc %= (uint64_t)MODULO; // 14 products and a rest stay below 2^64
+        acc %= (uint64_t)MODULO; // 16 products and a rest stay below 2^64
     }
     __syncthreads();
     return lane < 55 ? (int32_t)acc : 0;
@@ -231,6 +231,13 @@ __device__ __forceinline__ int32_t ranf_advance(int32_t x, const uint32_t *__res
     return x;
 }
 
+// faster-threading's seeds pass the modulus (seed + 123456 b >= 1e9), which
+// leaves values outside [0, 1e9) in the first rounds of one batch in five.
+// Rounds and jumps don't commute there, so such a batch takes a jump at one
+// place only, round RANF_LATE (ranf_seed_kernel's `later`), and rounds from it
+// or from the origin to every other place, however the batch is split.
+__device__ __forceinline__ bool ranf_odd(int32_t x) { return __any((uint32_t)x >= (uint32_t)MODULO); }
+
 // What bounds a round: a chain of one LDS permute and nine dependent integer
 // instructions, about 180 cycles, which three wavefronts per SIMD hide behind
 // the events (14 rounds of about 48 issue cycles for 64 events of 2500).
@@ -243,6 +250,7 @@ struct RanfPart {
     uint32_t o = 0;       // the place of the next unread value in it: X[55 - o], o up to 55
     uint64_t round = 0;   // the number of the last round the part reads
     bool have = false;
+    uint32_t late = 0;    // rounds to RANF_LATE in an odd batch, otherwise more than the part's
     RanfLanes l = ranf_lanes();
 
     // To the first draw of n > 0 events from event `first` of batch b on.  win:
@@ -260,6 +268,17 @@ struct RanfPart {
             const uint32_t lane = threadIdx.x & 63u;
             x = lane < 55 ? (own ? R.origin[56 * b + lane + 1] : R.round[lane + 1]) : 0;
         }
+        late = 0x7fffffffu;
+        if (own && ranf_odd(x)) {
+            if (skip >= RANF_LATE) {
+                x = later(R, b);
+                skip -= RANF_LATE;
+            } else {
+                late = RANF_LATE - (uint32_t)skip;
+            }
+            for (; skip; --skip)
+                x = ranf_next_round(x, l);
+        }
         if (skip < 4) // (a round costs a twentieth of a jump)
             for (; skip; --skip)
                 x = ranf_next_round(x, l);
@@ -268,14 +287,31 @@ struct RanfPart {
         round = (q + 12ull * n - 1) / 55;
         have = true;
     }
-    // The next `need` (12 .. 768) values into lds[base ..] in stream order.
-    // Lanes with nothing to write do so to lds[dump].
-    __device__ __forceinline__ void fill(uint32_t need, int32_t *lds, uint32_t base, uint32_t dump)
+    __device__ __forceinline__ int32_t later(const RanfSource &R, uint64_t b) const
+    {
+        const uint32_t lane = threadIdx.x & 63u;
+        return lane < 55 ? R.later[56 * b + lane + 1] : 0;
+    }
+    // The next `need` (12 .. 768) values of batch b into lds[base ..] in stream
+    // order.  Lanes with nothing to write do so to lds[dump].
+    __device__ __forceinline__ void fill(const RanfSource &R, uint64_t b, uint32_t need, int32_t *lds, uint32_t base,
+                                         uint32_t dump)
     {
         const int lane = (int)(threadIdx.x & 63u), at = 54 - lane - (int)o;
         lds[lane < 55 && at >= 0 ? base + (uint32_t)at : dump] = x;
         uint32_t p = lane < 55 ? base + (uint32_t)(at + 55) : dump;
         const uint32_t step = lane < 55 ? 55u : 0u, rounds = (o + need + 54) / 55 - 1;
+        if (late <= rounds) { // an odd batch's round RANF_LATE is among them
+            for (uint32_t r = 1; r <= rounds; ++r) {
+                x = r == late ? later(R, b) : ranf_next_round(x, l);
+                lds[p < base + need ? p : dump] = x;
+                p += step;
+            }
+            late = 0x7fffffffu;
+            o = o + need - 55 * rounds;
+            return;
+        }
+        late -= rounds;
         for (uint32_t r = 1; r < rounds; ++r) {
             x = ranf_next_round(x, l);
             lds[p] = x;
@@ -393,7 +429,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                 qnext = a.evq[wbase + (size_t)((k + 1) * 64 + lane)];
             int4 rd[3]; // RANF: the lane's 12 draws
             if (SOURCE == 1) {
-                ranf.fill(12 * min(64u, n - 64 * k), qints, RING, RING_DUMP);
+                ranf.fill(a.ranf, b, 12 * min(64u, n - 64 * k), qints, RING, RING_DUMP);
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < 3; ++j)
@@ -882,12 +918,21 @@ template <int BITS> __global__ __launch_bounds__(64) void ranf_expand_kernel(Ran
     if (r_begin * 55 >= q_end)
         return; // whole workgroup
     int32_t x = lane < 55 ? a.origin[56 * piece + lane + 1] : 0;
-    x = ranf_advance(x, a.r16, seg * (uint64_t)a.R, win);
+    const RanfLanes l = ranf_lanes();
+    uint64_t skip = r_begin;
+    if (a.later && ranf_odd(x)) { // (R divides RANF_LATE)
+        if (skip >= RANF_LATE) {
+            x = lane < 55 ? a.later[56 * piece + lane + 1] : 0;
+            skip -= RANF_LATE;
+        }
+        for (; skip; --skip)
+            x = ranf_next_round(x, l);
+    }
+    x = ranf_advance(x, a.r16, skip, win);
     // (the empty asm makes the wait for a load of x come here: in the rounds'
     // loop, where the compiler would place it, it waits for each round's store)
     asm volatile("" : "+v"(x));
     int32_t *out = a.out + piece * a.piece_stride;
-    const RanfLanes l = ranf_lanes();
     __shared__ uint64_t bm[2][BITS ? 32 : 1];
     using BT = typename std::conditional<BITS == 2, float, double>::type;
     RanfBits<BT> bits;
@@ -1805,12 +1850,13 @@ void launch_xo_expand(const XoPieceArgs &a, hipStream_t st)
 }
 
 
-// seeded_new (ranf.rs:36-66) for jump mode, one thread per batch.
-__global__ void ranf_seed_kernel(int32_t seed0, uint64_t b_first, uint64_t nb, int32_t *origin, int32_t *p0)
+// seeded_new (ranf.rs:36-66) for jump mode, one thread per batch; then the
+// wavefront makes the round RANF_LATE of its odd batches (ranf_odd).
+__global__ __launch_bounds__(64) void ranf_seed_kernel(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16,
+                                                       int32_t *origin, int32_t *p0, int32_t *later)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nb)
-        return;
+    __shared__ int32_t win[112];
+    const uint64_t i0 = (uint64_t)blockIdx.x * 64, i = i0 + threadIdx.x;
     const uint64_t b = b_first + i;
     int32_t x[56];
     const int32_t seed = (int32_t)((uint32_t)seed0 + (uint32_t)(123456ull * b));
@@ -1841,15 +1887,30 @@ __global__ void ranf_seed_kernel(int32_t seed0, uint64_t b_first, uint64_t nb, i
                 x[t] += MODULO;
         }
     }
-    for (int k = 0; k < 56; ++k)
-        origin[56 * i + k] = x[k];
-    p0[i] = 0;
+    bool odd = false;
+    if (i < nb) {
+        for (int k = 0; k < 56; ++k) {
+            origin[56 * i + k] = x[k];
+            odd |= (uint32_t)x[k] >= (uint32_t)MODULO;
+        }
+        p0[i] = 0;
+    }
+    uint64_t odds = __ballot(odd);
+    __syncthreads(); // the lanes' origins, read by the others below
+    const uint32_t lane = threadIdx.x, ck = ranf_jump_lane(r16 + 55 * RANF_LATE_R16);
+    for (; odds; odds &= odds - 1) {
+        const uint64_t at = 56 * (i0 + (uint64_t)__builtin_ctzll(odds)) + lane + 1;
+        const int32_t y = ranf_jump(lane < 55 ? origin[at] : 0, ck, win);
+        if (lane < 55)
+            later[at] = y;
+    }
 }
 
-void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, int32_t *origin, int32_t *p0, hipStream_t st)
+void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16, int32_t *origin, int32_t *p0,
+                      int32_t *later, hipStream_t st)
 {
     const unsigned blocks = (unsigned)((nb + 63) / 64);
-    hipLaunchKernelGGL(ranf_seed_kernel, dim3(blocks), dim3(64), 0, st, seed0, b_first, nb, origin, p0);
+    hipLaunchKernelGGL(ranf_seed_kernel, dim3(blocks), dim3(64), 0, st, seed0, b_first, nb, r16, origin, p0, later);
 }
 
 // ---- in-order merge --------------------------------------------------------
@@ -2106,7 +2167,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
             int4 rd[3]; // RANF: the lane's 12 draws, through the half that is free
             if (SOURCE == 1) {
                 const uint32_t ring = head ? 0 : HALF;
-                ranf.fill(12 * min(64u, n - 64 * i), qints, ring, DUMP);
+                ranf.fill(a.ranf, b, 12 * min(64u, n - 64 * i), qints, ring, DUMP);
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < 3; ++j)
