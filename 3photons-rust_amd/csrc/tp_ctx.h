@@ -188,15 +188,16 @@ struct PartCost {
 };
 // Measured at 100 to 10 000 batches with every run length.  A wavefront with a
 // SIMD to itself takes 1.45 of an iteration's issue time (RANF, 1000 batches:
-// 481 us in one part each, 405 in two, 381 in three, 368 in four, 378 in eight),
-// a part some 3.5 iterations beside its events (10 000 batches: 2.53 ms whole,
-// 2.72 in two parts); event loops that read their draws from HBM wait 2.6
-// iterations a round (faster-evgen, 1000 batches: 780 us whole, 540 in two
-// parts, 414 in three, which fill the chip once, 478 in four); the weighted
-// loop's rows of uniforms come in best in long runs (2000 batches: 4.12 ms whole
-// with the flow, 4.21 in two parts; 1000: 2.20 and 2.11); the all-f32 loop waits
-// 0.8, its separate sums take 42 us per 1536 batches (1000 batches: 560 us in
-// two parts, 494 in four, 475 in eight; 10 000: 3.13 ms whole, 3.72 in three).
+// 444 us in one part each, 344 in two, 317 in three, 307 in four, 308 in eight,
+// 336 in sixteen), a part some 3.5 iterations beside its events (10 000 batches:
+// 2.76 ms whole, 2.98 in two parts); event loops that read their draws from HBM
+// wait 2.6 iterations a round (faster-evgen, 1000 batches with the walk: 1234 us
+// whole, 1009 in two parts, 879 in three, which fill the chip once, 951 in
+// four); the weighted loop's rows of uniforms come in best in long runs (with
+// the flow, 2000 batches take 2 % longer in two parts, 1000 batches 4 % less);
+// the all-f32 loop waits 0.8, its separate sums take 42 us per 1536 batches
+// (1000 batches: 819 us whole, 492 in two parts, 418 in four, 395 in eight;
+// 10 000: 2.99 ms whole, 3.63 in three).
 inline PartCost event_part_cost(int source)
 {
     return source < 2 ? PartCost{3.5, 0.45, false} : source == 2 ? PartCost{3.5, 0.45, false, 0.85} : PartCost{1.5, 2.6, true};

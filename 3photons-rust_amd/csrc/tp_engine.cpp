@@ -231,7 +231,7 @@ int check_common(Ctx *c, const tp_params *params, int rng_kind, const void *stat
 // RANF with `faster-evgen`: the event starts of the reference's
 // simulate_event_batch walk, then each chunk of batches is simulated from
 // them with its stream expanded into HBM.  Runs of FE_DEVICE_WALK_MIN events
-// or more walk the stream on the device (fe_walk_kernel: segment walkers
+// (xoshiro streams: FE_XO_DEVICE_WALK_MIN) or more walk the stream on the device (fe_walk_kernel: segment walkers
 // joined where they meet); shorter runs, and any chunk whose device walkers
 // do not all join, take the host walk, 20 to 90 ns an event.  The device's takes
 // its launches and a segment's length at least.  Closures of 2000, 8000, 32 000

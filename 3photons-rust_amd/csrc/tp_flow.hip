@@ -624,8 +624,8 @@ __global__ __launch_bounds__(64 * BWD_WAVES) __attribute__((amdgpu_waves_per_eu(
 // block per (layer, sample range): chunks of 64 samples of all 304 saved rows
 // are staged through LDS (the next chunk is loaded into registers while the
 // current one is multiplied), so every saved value is read from HBM once, and
-// that read is what bounds the kernel (48 us for 65 536 samples, 4.9 TB/s).  A row block of 16 samples lies there
-// sample by sample; the transposing LDS read gives lane 16 g + r row r's
+// that read is what bounds the kernel (48 us for 65 536 samples, 5.0 TB/s).  A
+// row block of 16 samples lies there sample by sample; the transposing LDS read gives lane 16 g + r row r's
 // samples 4g .. 4g + 3, the operand layout of the products.
 // The layer's 38 output tiles -- 28 weight tiles and 10 bias tiles, whose
 // B operand is a column of ones -- are spread over the four wavefronts by the

@@ -1,14 +1,18 @@
 // tp_kernels.hip -- gfx950 kernels of the 3photons event loop.
 //
 //  fused_kernel      one wavefront per 10 000-event batch or part of one,
-//                    grid-strided over parts; uniforms from xoshiro256+ in registers or from
-//                    the expanded RANF stream, RAMBO -> cuts in registers,
+//                    grid-strided over parts; uniforms from xoshiro256+ or RANF made in the
+//                    loop, or read from HBM (faster-evgen, flow); RAMBO -> cuts in registers,
 //                    passing events compacted through an LDS queue, spinors
 //                    -> amplitudes -> weight on full wavefronts, 12 running
 //                    sums per lane, butterfly reduction to one accumulator
 //                    per part (batch_sums_kernel adds a batch's parts).
-//  ranf_expand       RANF stream into HBM, one wavefront per segment of R
-//                    rounds, 55 lanes = the 55 values of a round.
+//  ranf_expand       RANF stream and accept bits into HBM for faster-evgen, one
+//                    wavefront per segment of R rounds, 55 lanes = the 55
+//                    values of a round; xo_expand, xo128_expand the same for
+//                    pieces of the xoshiro streams; fe_* walk them.
+//  f32_events        the all-f32 event loop, f32_accumulate its in-order sums.
+//  adjoint_*         values and derivatives at given or drawn points.
 //  ranf_seed         jump-mode origins, seeded_new(seed + 123456 b) per batch.
 //  merge_kernel      in-order left fold of the batch accumulators.
 //
@@ -349,11 +353,11 @@ struct RanfPart {
 // wavefront per batch left a run of 1e7 events with one wavefront per SIMD of
 // the three that fit and a closure call with one on the whole chip, most of
 // whose time was the lanes' own skips of the stream (a call of 4321 events
-// 381 -> 42 us, 1.23e6 events with jump seeding 677 -> 93 us, 1e9 events
-// 26.8 -> 25.8 ms with parts and shared skips).
+// 381 -> 25 us, 1.23e6 events with jump seeding 677 -> 78 us, 1e9 events
+// 26.8 -> 25.4 ms with parts and shared skips).
 constexpr int QCAP = 128;
 
-// Three wavefronts per SIMD (163 VGPRs at f64, no scratch): the LDS queue
+// Three wavefronts per SIMD (167 VGPRs at f64, no scratch): the LDS queue
 // (12.4 KB per workgroup) caps a CU at 12 resident workgroups anyway, and the
 // third wave hides the transcendental-table, LDS and f64 latencies better than
 // two (measured 3 % faster at f64).

@@ -124,8 +124,8 @@ typedef struct {
     uint64_t events;
     uint64_t batches;
     uint64_t host_walk_chunks; /* faster-evgen with skip-ahead seeding: chunks of batches whose event
-                                  starts came from the host walk (runs below 2^20 events, the
-                                  closure, or device walkers that did not all meet) */
+                                  starts came from the host walk (runs and calls below 8192 events,
+                                  16384 on xoshiro streams, or device walkers that did not all meet) */
     uint64_t chunks;           /* faster-evgen: chunks of batches the run was split into (each one's
                                   stream expanded, walked and simulated in turn); 0 otherwise */
 } tp_stats;
@@ -182,7 +182,7 @@ int tp_run_device(void *ctx, const tp_params *params, int rng_kind, int seeding,
  * runs the xoshiro256+ stream only (rng_kind TP_RNG_XOSHIRO, precision
  * TP_PREC_F64 or TP_PREC_MIXED, both seedings, no faster-evgen; anything else
  * returns TP_ERR_UNSUPPORTED) and at most 2^32 - 1 batches (TP_ERR_ARG
- * beyond).  Its skip-ahead tables sit in a static device array of 24 MiB
+ * beyond).  Its skip-ahead tables sit in a static device array of 33 MiB
  * per GPU, filled once by tp_create and only read afterwards, so calls that
  * overlap on one GPU share it without racing; the sums of batches split over
  * several wavefronts go through 6.5 MiB of the context's own, also allocated
