@@ -124,6 +124,13 @@ RanfPoly ranf_poly_xpow(uint64_t n)
     return result;
 }
 
+// Values outside [0, 1e9), which seeds past the modulus leave in the first
+// rounds: sums of unreduced products and several jumps for one would give others.
+static bool past_modulus(const int32_t *x)
+{
+    return std::any_of(x + 1, x + 56, [](int32_t v) { return static_cast<uint32_t>(v) >= RANF_MODULO; });
+}
+
 void ranf_apply_round_jump(const uint32_t *c, const int32_t *x_in, int32_t *x_out)
 {
     // Window Y[0..109] = X_r[1..55], X_{r+1}[1..55]; X_{r+m}[i] = sum_k c_k Y[i-1+k].
@@ -136,9 +143,10 @@ void ranf_apply_round_jump(const uint32_t *c, const int32_t *x_in, int32_t *x_ou
         y[55 + i] = static_cast<uint64_t>(next[i + 1]);
     }
     uint64_t acc[55] = {0};
+    const bool past = past_modulus(x_in);
     for (int k = 0; k < 55; ++k) {
         for (int i = 0; i < 55; ++i)
-            acc[i] += c[k] * y[i + k];
+            acc[i] += past ? c[k] * y[i + k] % RANF_MODULO : c[k] * y[i + k];
         if (k % 8 == 7 || k == 54)
             for (uint64_t &v : acc)
                 v %= RANF_MODULO;
@@ -158,6 +166,12 @@ void ranf_advance(RanfState &g, uint64_t n)
     uint64_t rounds = (rest + 54) / 55;
     const uint32_t *tab = ranf_round_digits().data(); // of the hexadecimal digits of `rounds`
     int32_t out[56];
+    if (past_modulus(g.numbers)) { // one jump
+        ranf_apply_round_jump(ranf_poly_rounds(rounds).data(), g.numbers, out);
+        std::memcpy(g.numbers, out, sizeof out);
+        g.index = static_cast<uint32_t>(55 * rounds - rest);
+        return;
+    }
     for (uint64_t e = rounds; e; e >>= 4, tab += 15 * 55)
         if (e & 15u) {
             ranf_apply_round_jump(tab + ((e & 15u) - 1) * 55, g.numbers, out);
