@@ -211,6 +211,13 @@ int ensure_r16(Ctx *c)
     return TP_OK;
 }
 
+// A state whose round holds values outside [0, 1e9): seeded past the modulus
+// (tpk::RanfSource::later).
+bool ranf_past_modulus(const tp_ranf_state *rs)
+{
+    return std::any_of(rs->numbers + 1, rs->numbers + 56, [](int32_t x) { return (uint32_t)x >= 1000000000u; });
+}
+
 int check_common(Ctx *c, const tp_params *params, int rng_kind, const void *state)
 {
     if (!params || !state)
@@ -581,6 +588,10 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
 int enqueue_ranf_faster_evgen(Ctx *c, tpk::FusedArgs &a, tpk::F32Args *fa, const tp_ranf_state *rs,
                               uint64_t num_events, uint32_t batch_size, void *per_batch_dev)
 {
+    // The host walk's rounds and the kernels' differ there: an event replayed
+    // from the other's start re-rolls on past its stored values.
+    if (ranf_past_modulus(rs))
+        return fail(c, TP_ERR_UNSUPPORTED, "faster-evgen needs a RANF state of values in [0, 1e9) (a seed below 1e9)");
     HIPCHK(c, hipStreamSynchronize(c->stream)); // the staging vectors below are reused
     tp::RanfState g0;
     std::memcpy(g0.numbers, rs->numbers, sizeof g0.numbers);
@@ -760,7 +771,13 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
             HIPCHK(c, hipMemcpyAsync(c->origin.p, c->origin0, sizeof c->origin0, hipMemcpyHostToDevice, c->stream));
             HIPCHK(c, hipMemcpyAsync(c->p0.p, &c->p00, sizeof c->p00, hipMemcpyHostToDevice, c->stream));
             const uint64_t p00 = (uint64_t)c->p00;
-            rc = expand(0, 1, 0ull - p00, PS - p00, false);
+            const bool past = ranf_past_modulus(rs);
+            if (past) {
+                tpk::launch_ranf_late(rs->numbers, static_cast<const uint32_t *>(c->r16.p),
+                                      static_cast<int32_t *>(c->origin.p), later, c->stream);
+                HIPCHK(c, hipGetLastError());
+            }
+            rc = expand(0, 1, 0ull - p00, PS - p00, past);
             if (!rc && cnb > 1)
                 rc = expand(1, cnb - 1, 0, PS, true);
         } else {
@@ -1101,6 +1118,15 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         HIPCHK(c, hipGetLastError());
         R.origin = origin;
         R.later = origin + 56 * nb;
+    }
+    if (ranf_past_modulus(rs) && (R.later || (nb == 1 && R.p0 + 12ull * num_events <= 2 * 55ull * tpk::RANF_LATE))) {
+        if (!R.later && (rc = ensure(c, c->origin, 2 * 56 * sizeof(int32_t))))
+            return rc;
+        int32_t *const origin = static_cast<int32_t *>(c->origin.p);
+        if (!R.later)
+            R.later = origin + 56;
+        tpk::launch_ranf_late(rs->numbers, R.r16, origin, const_cast<int32_t *>(R.later), c->stream);
+        HIPCHK(c, hipGetLastError());
     }
     if (const int e = mark(c, 1))
         return e;

@@ -138,6 +138,7 @@ void launch_ranf_expand(const RanfArgs &a, uint64_t npieces, hipStream_t st);
 // Per-batch RANF origins of jump mode: seeded_new(seed0 + 123456*b).
 void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16, int32_t *origin, int32_t *p0,
                       int32_t *later, hipStream_t st);
+void launch_ranf_late(const int32_t round[56], const uint32_t *r16, int32_t *origin, int32_t *later, hipStream_t st);
 // In-order left fold of nb accumulators (resacc.rs:133-139) into *merged.
 // In-order fold of nb accumulators; f32 = 1 adds in float (all-f32 mode).
 void launch_merge(const void *per_batch, uint64_t nb, void *merged, hipStream_t st, int f32 = 0);

@@ -273,7 +273,7 @@ struct RanfPart {
             x = lane < 55 ? (own ? R.origin[56 * b + lane + 1] : R.round[lane + 1]) : 0;
         }
         late = 0x7fffffffu;
-        if (own && ranf_odd(x)) {
+        if (R.later && ranf_odd(x)) {
             if (skip >= RANF_LATE) {
                 x = later(R, b);
                 skip -= RANF_LATE;
@@ -1908,6 +1908,29 @@ __global__ __launch_bounds__(64) void ranf_seed_kernel(int32_t seed0, uint64_t b
         if (lane < 55)
             later[at] = y;
     }
+}
+
+// The same for a caller's state: its round to `origin`, round RANF_LATE to `later`.
+struct RanfRound {
+    int32_t x[56];
+};
+__global__ __launch_bounds__(64) void ranf_late_kernel(RanfRound r, const uint32_t *r16, int32_t *origin, int32_t *later)
+{
+    __shared__ int32_t win[112];
+    const uint32_t lane = threadIdx.x;
+    const int32_t x = lane < 55 ? r.x[lane + 1] : 0;
+    const int32_t y = ranf_jump(x, ranf_jump_lane(r16 + 55 * RANF_LATE_R16), win);
+    if (lane < 55) {
+        origin[lane + 1] = x;
+        later[lane + 1] = y;
+    }
+}
+void launch_ranf_late(const int32_t round[56], const uint32_t *r16, int32_t *origin, int32_t *later, hipStream_t st)
+{
+    RanfRound r;
+    for (int i = 0; i < 56; ++i)
+        r.x[i] = round[i];
+    hipLaunchKernelGGL(ranf_late_kernel, dim3(1), dim3(64), 0, st, r, r16, origin, later);
 }
 
 void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16, int32_t *origin, int32_t *p0,
