@@ -707,7 +707,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
     if (!rc)
         rc = ensure(c, c->draws, chunk * PS * sizeof(int32_t));
     if (!rc)
-        rc = ensure(c, c->origin, 2 * chunk * 56 * sizeof(int32_t)); // origins, then their rounds RANF_LATE
+        rc = ensure(c, c->origin, chunk * 56 * sizeof(int32_t));
     if (!rc)
         rc = ensure(c, c->p0, chunk * sizeof(int32_t));
     if (!rc)
@@ -731,12 +731,10 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
     c->p00 = static_cast<int32_t>(55u - rs->index);
     c->fe_flag_host = 0;
     HIPCHK(c, hipMemcpyAsync(c->fe_flag.p, &c->fe_flag_host, sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
-    int32_t *const later = static_cast<int32_t *>(c->origin.p) + 56 * chunk;
-    auto expand = [&](uint64_t first_piece, uint64_t npieces, uint64_t d_begin, uint64_t d_end, bool own) -> int {
+    auto expand = [&](uint64_t first_piece, uint64_t npieces, uint64_t d_begin, uint64_t d_end) -> int {
         tpk::RanfArgs r;
         std::memset(&r, 0, sizeof r);
         r.origin = static_cast<const int32_t *>(c->origin.p) + 56 * first_piece;
-        r.later = own && batch_size <= TP_BATCH_SIZE ? later + 56 * first_piece : nullptr;
         r.p0 = static_cast<const int32_t *>(c->p0.p) + first_piece;
         r.r16 = static_cast<const uint32_t *>(c->r16.p);
         r.R = (int32_t)R;
@@ -762,7 +760,7 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
             if (const int e = mark(c, 0))
                 return e;
         tpk::launch_ranf_seed(rs->seed, b0, cnb, static_cast<const uint32_t *>(c->r16.p),
-                              static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p), later, c->stream);
+                              static_cast<int32_t *>(c->origin.p), static_cast<int32_t *>(c->p0.p), nullptr, c->stream);
         HIPCHK(c, hipGetLastError());
         if (b0 == 0) {
             // batch 0 runs on the caller's state, which may be inside its
@@ -771,17 +769,11 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
             HIPCHK(c, hipMemcpyAsync(c->origin.p, c->origin0, sizeof c->origin0, hipMemcpyHostToDevice, c->stream));
             HIPCHK(c, hipMemcpyAsync(c->p0.p, &c->p00, sizeof c->p00, hipMemcpyHostToDevice, c->stream));
             const uint64_t p00 = (uint64_t)c->p00;
-            const bool past = ranf_past_modulus(rs);
-            if (past) {
-                tpk::launch_ranf_late(rs->numbers, static_cast<const uint32_t *>(c->r16.p),
-                                      static_cast<int32_t *>(c->origin.p), later, c->stream);
-                HIPCHK(c, hipGetLastError());
-            }
-            rc = expand(0, 1, 0ull - p00, PS - p00, past);
+            rc = expand(0, 1, 0ull - p00, PS - p00);
             if (!rc && cnb > 1)
-                rc = expand(1, cnb - 1, 0, PS, true);
+                rc = expand(1, cnb - 1, 0, PS);
         } else {
-            rc = expand(0, cnb, 0, PS, true);
+            rc = expand(0, cnb, 0, PS);
         }
         if (rc)
             return rc;

@@ -83,7 +83,6 @@ struct FusedArgs {
 // skip-ahead mode, or one reseeded batch stream in jump mode.
 struct RanfArgs {
     const int32_t *origin; // [npieces][56] round X[1..55] at [1..55]
-    const int32_t *later;  // the same for round RANF_LATE of reseeded streams, as RanfSource; may be null
     const int32_t *p0;     // [npieces] values of the origin round already consumed
     uint64_t d_begin, d_end; // window of draws (piece-relative) to write
     uint64_t seg_first;    // first segment index of the window

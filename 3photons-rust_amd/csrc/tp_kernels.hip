@@ -235,12 +235,24 @@ __device__ __forceinline__ int32_t ranf_advance(int32_t x, const uint32_t *__res
     return x;
 }
 
-// faster-threading's seeds pass the modulus (seed + 123456 b >= 1e9), which
-// leaves values outside [0, 1e9) in the first rounds of one batch in five.
-// Rounds and jumps don't commute there, so such a batch takes a jump at one
-// place only, round RANF_LATE (ranf_seed_kernel's `later`), and rounds from it
-// or from the origin to every other place, however the batch is split.
+// A stream seeded past the modulus (faster-threading's seed + 123456 b does in
+// long runs) holds values outside [0, 1e9) in its first rounds, an odd stream.
+// Rounds and jumps don't commute there, so jumps are taken to whole segments of
+// RANF_LATE rounds only, each straight from round 0, and rounds to every other
+// place: the values don't depend on how the stream is split.
 __device__ __forceinline__ bool ranf_odd(int32_t x) { return __any((uint32_t)x >= (uint32_t)MODULO); }
+// Round RANF_LATE seg of an odd stream from its round 0: first the jump by the
+// lowest binary digit of seg (the rounds it leads to are in range, and further
+// jumps may be taken in any steps).  win: 110 ints of LDS, free before and after.
+__device__ __forceinline__ int32_t ranf_odd_segment(int32_t x, const uint32_t *__restrict__ r16, uint64_t seg, int32_t *win)
+{
+    static_assert(RANF_LATE == 1u << 11, "seg's binary digit k is digit 11 + k of the rounds");
+    if (!seg)
+        return x;
+    const uint32_t bit = 11u + (uint32_t)__builtin_ctzll(seg);
+    x = ranf_jump(x, ranf_jump_lane(r16 + 55 * (15 * (bit / 4) + (1u << bit % 4) - 1)), win);
+    return ranf_advance(x, r16, RANF_LATE * (seg & (seg - 1)), win);
+}
 
 // What bounds a round: a chain of one LDS permute and nine dependent integer
 // instructions, about 180 cycles, which three wavefronts per SIMD hide behind
@@ -924,12 +936,11 @@ template <int BITS> __global__ __launch_bounds__(64) void ranf_expand_kernel(Ran
     int32_t x = lane < 55 ? a.origin[56 * piece + lane + 1] : 0;
     const RanfLanes l = ranf_lanes();
     uint64_t skip = r_begin;
-    if (a.later && ranf_odd(x)) { // (R divides RANF_LATE)
-        if (skip >= RANF_LATE) {
-            x = lane < 55 ? a.later[56 * piece + lane + 1] : 0;
-            skip -= RANF_LATE;
-        }
-        for (; skip; --skip)
+    if (ranf_odd(x)) { // (R divides RANF_LATE)
+        const uint64_t odd_seg = skip / RANF_LATE;
+        x = ranf_odd_segment(x, a.r16, odd_seg, win);
+        skip %= RANF_LATE;
+        for (; skip && !odd_seg; --skip)
             x = ranf_next_round(x, l);
     }
     x = ranf_advance(x, a.r16, skip, win);
@@ -1855,7 +1866,7 @@ void launch_xo_expand(const XoPieceArgs &a, hipStream_t st)
 
 
 // seeded_new (ranf.rs:36-66) for jump mode, one thread per batch; then the
-// wavefront makes the round RANF_LATE of its odd batches (ranf_odd).
+// wavefront makes the round RANF_LATE of its odd batches (ranf_odd), if asked to.
 __global__ __launch_bounds__(64) void ranf_seed_kernel(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16,
                                                        int32_t *origin, int32_t *p0, int32_t *later)
 {
@@ -1902,7 +1913,7 @@ __global__ __launch_bounds__(64) void ranf_seed_kernel(int32_t seed0, uint64_t b
     uint64_t odds = __ballot(odd);
     __syncthreads(); // the lanes' origins, read by the others below
     const uint32_t lane = threadIdx.x, ck = ranf_jump_lane(r16 + 55 * RANF_LATE_R16);
-    for (; odds; odds &= odds - 1) {
+    for (odds = later ? odds : 0; odds; odds &= odds - 1) {
         const uint64_t at = 56 * (i0 + (uint64_t)__builtin_ctzll(odds)) + lane + 1;
         const int32_t y = ranf_jump(lane < 55 ? origin[at] : 0, ck, win);
         if (lane < 55)
