@@ -253,7 +253,7 @@ inline Split split_for_f32(const Ctx *c, int source, uint64_t nb, uint32_t n)
 inline void set_ranf_jump(tpk::RanfSource &R, const Split &s, uint64_t nb, uint32_t batch_size, uint32_t n)
 {
     R.jump_rounds = 0;
-    if (R.origin || nb * s.parts <= (uint64_t)s.grid)
+    if (R.origin || R.later || nb * s.parts <= (uint64_t)s.grid)
         return;
     // the least number of rounds from the last one of a part to the first of
     // the wavefront's next (a part of whole runs: that or one more)

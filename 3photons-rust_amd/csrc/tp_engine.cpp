@@ -1111,13 +1111,16 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
         R.origin = origin;
         R.later = origin + 56 * nb;
     }
-    if (ranf_past_modulus(rs) && (R.later || (nb == 1 && R.p0 + 12ull * num_events <= 2 * 55ull * tpk::RANF_LATE))) {
-        if (!R.later && (rc = ensure(c, c->origin, 2 * 56 * sizeof(int32_t))))
-            return rc;
-        int32_t *const origin = static_cast<int32_t *>(c->origin.p);
-        if (!R.later)
-            R.later = origin + 56;
-        tpk::launch_ranf_late(rs->numbers, R.r16, origin, const_cast<int32_t *>(R.later), c->stream);
+    if (ranf_past_modulus(rs)) {
+        uint64_t segs = 1; // of RANF_LATE rounds: the first one's end of batch 0, or all of the one stream
+        if (!R.origin) {
+            segs = (R.p0 + 12 * num_events - 1) / 55 / tpk::RANF_LATE + 1;
+            rc = ensure(c, c->origin, segs * 56 * sizeof(int32_t));
+            if (rc)
+                return rc;
+            R.later = static_cast<const int32_t *>(c->origin.p);
+        }
+        tpk::launch_ranf_late(rs->numbers, R.r16, R.origin ? 1 : 0, segs, const_cast<int32_t *>(R.later), c->stream);
         HIPCHK(c, hipGetLastError());
     }
     if (const int e = mark(c, 1))

@@ -14,13 +14,16 @@ namespace tpk {
 // The RANF stream of a run.  Batch b's events draw from position p0 + 12
 // batch_size b on of the stream whose round 0 is `round` (X[1..55]); with jump
 // seeding (origin non-null) batch b > 0 has a stream of its own, round 0 at
-// origin[56 b] and positions from 0.  A batch whose origin holds values outside
-// [0, 1e9) goes on from later[56 b] at round RANF_LATE.
+// origin[56 b] and positions from 0.  A stream whose round 0 holds values outside
+// [0, 1e9) goes on at each multiple s of RANF_LATE rounds from `later`: at
+// later[56 b] (s = 1, no batch gets further) with jump seeding, else at
+// later[56 (s - late_first)].
 constexpr uint32_t RANF_LATE = 2048, RANF_LATE_R16 = 2 * 15 + 7; // 8 * 16^2: its place in r16
 struct RanfSource {
     int32_t round[56];
     uint32_t p0;
     const int32_t *origin, *later;
+    uint64_t late_first;
     const uint32_t *r16;  // x^(55 v 16^j) mod the recurrence's polynomial, 55 coefficients each, v = 1..15,
                           // for the digits of a number of rounds
     uint32_t jump[55];    // x^(55 jump_rounds): from the end of a wavefront's part to near its next one
@@ -137,7 +140,8 @@ void launch_ranf_expand(const RanfArgs &a, uint64_t npieces, hipStream_t st);
 // Per-batch RANF origins of jump mode: seeded_new(seed0 + 123456*b).
 void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16, int32_t *origin, int32_t *p0,
                       int32_t *later, hipStream_t st);
-void launch_ranf_late(const int32_t round[56], const uint32_t *r16, int32_t *origin, int32_t *later, hipStream_t st);
+// The rounds RANF_LATE s, s = first .. first + n - 1, of a caller's such stream.
+void launch_ranf_late(const int32_t round[56], const uint32_t *r16, uint64_t first, uint64_t n, int32_t *later, hipStream_t st);
 // In-order left fold of nb accumulators (resacc.rs:133-139) into *merged.
 // In-order fold of nb accumulators; f32 = 1 adds in float (all-f32 mode).
 void launch_merge(const void *per_batch, uint64_t nb, void *merged, hipStream_t st, int f32 = 0);

@@ -266,7 +266,8 @@ struct RanfPart {
     uint32_t o = 0;       // the place of the next unread value in it: X[55 - o], o up to 55
     uint64_t round = 0;   // the number of the last round the part reads
     bool have = false;
-    uint32_t late = 0;    // rounds to RANF_LATE in an odd batch, otherwise more than the part's
+    uint32_t late = 0;    // rounds to the next segment of RANF_LATE in an odd stream, otherwise more than the part's
+    uint64_t seg = 0;     // odd stream: the current segment
     RanfLanes l = ranf_lanes();
 
     // To the first draw of n > 0 events from event `first` of batch b on.  win:
@@ -286,14 +287,14 @@ struct RanfPart {
         }
         late = 0x7fffffffu;
         if (R.later && ranf_odd(x)) {
-            if (skip >= RANF_LATE) {
+            seg = skip / RANF_LATE;
+            skip %= RANF_LATE;
+            late = RANF_LATE - (uint32_t)skip;
+            if (seg)
                 x = later(R, b);
-                skip -= RANF_LATE;
-            } else {
-                late = RANF_LATE - (uint32_t)skip;
-            }
-            for (; skip; --skip)
-                x = ranf_next_round(x, l);
+            else
+                for (; skip; --skip)
+                    x = ranf_next_round(x, l);
         }
         if (skip < 4) // (a round costs a twentieth of a jump)
             for (; skip; --skip)
@@ -306,7 +307,7 @@ struct RanfPart {
     __device__ __forceinline__ int32_t later(const RanfSource &R, uint64_t b) const
     {
         const uint32_t lane = threadIdx.x & 63u;
-        return lane < 55 ? R.later[56 * b + lane + 1] : 0;
+        return lane < 55 ? R.later[56 * (R.origin ? b : seg - R.late_first) + lane + 1] : 0;
     }
     // The next `need` (12 .. 768) values of batch b into lds[base ..] in stream
     // order.  Lanes with nothing to write do so to lds[dump].
@@ -317,13 +318,18 @@ struct RanfPart {
         lds[lane < 55 && at >= 0 ? base + (uint32_t)at : dump] = x;
         uint32_t p = lane < 55 ? base + (uint32_t)(at + 55) : dump;
         const uint32_t step = lane < 55 ? 55u : 0u, rounds = (o + need + 54) / 55 - 1;
-        if (late <= rounds) { // an odd batch's round RANF_LATE is among them
+        if (late <= rounds) { // an odd stream's next segment starts among them
             for (uint32_t r = 1; r <= rounds; ++r) {
-                x = r == late ? later(R, b) : ranf_next_round(x, l);
+                if (--late == 0) {
+                    ++seg;
+                    late = RANF_LATE;
+                    x = later(R, b);
+                } else {
+                    x = ranf_next_round(x, l);
+                }
                 lds[p < base + need ? p : dump] = x;
                 p += step;
             }
-            late = 0x7fffffffu;
             o = o + need - 55 * rounds;
             return;
         }
@@ -1921,27 +1927,24 @@ __global__ __launch_bounds__(64) void ranf_seed_kernel(int32_t seed0, uint64_t b
     }
 }
 
-// The same for a caller's state: its round to `origin`, round RANF_LATE to `later`.
+// The segment starts of a caller's odd stream, a wavefront each.
 struct RanfRound {
     int32_t x[56];
 };
-__global__ __launch_bounds__(64) void ranf_late_kernel(RanfRound r, const uint32_t *r16, int32_t *origin, int32_t *later)
+__global__ __launch_bounds__(64) void ranf_late_kernel(RanfRound r, const uint32_t *r16, uint64_t first, int32_t *later)
 {
     __shared__ int32_t win[112];
     const uint32_t lane = threadIdx.x;
-    const int32_t x = lane < 55 ? r.x[lane + 1] : 0;
-    const int32_t y = ranf_jump(x, ranf_jump_lane(r16 + 55 * RANF_LATE_R16), win);
-    if (lane < 55) {
-        origin[lane + 1] = x;
-        later[lane + 1] = y;
-    }
+    const int32_t y = ranf_odd_segment(lane < 55 ? r.x[lane + 1] : 0, r16, first + blockIdx.x, win);
+    if (lane < 55)
+        later[56 * (uint64_t)blockIdx.x + lane + 1] = y;
 }
-void launch_ranf_late(const int32_t round[56], const uint32_t *r16, int32_t *origin, int32_t *later, hipStream_t st)
+void launch_ranf_late(const int32_t round[56], const uint32_t *r16, uint64_t first, uint64_t n, int32_t *later, hipStream_t st)
 {
     RanfRound r;
     for (int i = 0; i < 56; ++i)
         r.x[i] = round[i];
-    hipLaunchKernelGGL(ranf_late_kernel, dim3(1), dim3(64), 0, st, r, r16, origin, later);
+    hipLaunchKernelGGL(ranf_late_kernel, dim3((unsigned)n), dim3(64), 0, st, r, r16, first, later);
 }
 
 void launch_ranf_seed(int32_t seed0, uint64_t b_first, uint64_t nb, const uint32_t *r16, int32_t *origin, int32_t *p0,
