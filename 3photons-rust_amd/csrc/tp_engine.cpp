@@ -246,6 +246,14 @@ int check_common(Ctx *c, const tp_params *params, int rng_kind, const void *stat
 // and 175, 175, 178, 221; xoshiro256+ 153, 363, 1149, 9880 us and about 800 (a
 // segment has 1024 events there).
 constexpr uint64_t FE_DEVICE_WALK_MIN = 8192, FE_XO_DEVICE_WALK_MIN = 16384;
+// From RANF states past the modulus only the device walk serves: it reads the
+// bits of the very values that its events replay, while the host walk's rounds
+// differ from the kernels' there, and an event replayed from the other's start
+// re-rolls on past its stored values.  Runs of FE_PAST_MIN events or more have
+// always been walked on the device; shorter ones and closures are refused.
+constexpr uint64_t FE_PAST_MIN = 1u << 20;
+constexpr const char *FE_PAST_TEXT = "faster-evgen of fewer than 2^20 events on one stream needs a RANF state of values in "
+                                     "[0, 1e9) (a seed below 1e9)";
 constexpr uint64_t FE_WALK_BATCHES = 12288; // batches per chunk: four strides of the event-loop grid
 constexpr double FE_POSITIONS_PER_EVENT = 18.5; // stream positions allowed for per event (mean 17.9)
 constexpr uint64_t FE_MAX_WALKERS = 1u << 18;
@@ -528,6 +536,8 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
             q_next = c->fe_qnext;
         }
         if (!ok) { // host walk of this chunk from q_start
+            if (!host_walk)
+                return fail(c, TP_ERR_UNSUPPORTED, FE_PAST_TEXT);
             ++c->fe_host_chunks;
             c->fe_starts.resize(n);
             host_walk(q_start, n, c->fe_starts.data(), &q_next);
@@ -588,10 +598,9 @@ int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, t
 int enqueue_ranf_faster_evgen(Ctx *c, tpk::FusedArgs &a, tpk::F32Args *fa, const tp_ranf_state *rs,
                               uint64_t num_events, uint32_t batch_size, void *per_batch_dev)
 {
-    // The host walk's rounds and the kernels' differ there: an event replayed
-    // from the other's start re-rolls on past its stored values.
-    if (ranf_past_modulus(rs))
-        return fail(c, TP_ERR_UNSUPPORTED, "faster-evgen needs a RANF state of values in [0, 1e9) (a seed below 1e9)");
+    const bool past = ranf_past_modulus(rs);
+    if (past && num_events < FE_PAST_MIN)
+        return fail(c, TP_ERR_UNSUPPORTED, FE_PAST_TEXT);
     HIPCHK(c, hipStreamSynchronize(c->stream)); // the staging vectors below are reused
     tp::RanfState g0;
     std::memcpy(g0.numbers, rs->numbers, sizeof g0.numbers);
@@ -612,9 +621,11 @@ int enqueue_ranf_faster_evgen(Ctx *c, tpk::FusedArgs &a, tpk::F32Args *fa, const
     HIPCHK(c, hipMemcpyAsync(c->origin.p, c->origin0, sizeof c->origin0, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->p0.p, &c->p00, sizeof c->p00, hipMemcpyHostToDevice, c->stream));
     const bool f32 = fa != nullptr;
-    const FeHostWalk walk = [&](uint64_t q, uint64_t n, uint64_t *starts, uint64_t *q_next) {
-        tp::ranf_walk_faster_evgen_from(g0, q, n, starts, q_next, 16, f32);
-    };
+    FeHostWalk walk; // none past the modulus
+    if (!past)
+        walk = [&](uint64_t q, uint64_t n, uint64_t *starts, uint64_t *q_next) {
+            tp::ranf_walk_faster_evgen_from(g0, q, n, starts, q_next, 16, f32);
+        };
     uint64_t q_end = 0;
     rc = enqueue_fe_chunks(c, fs, walk, a, fa, fs.p0_master, num_events, batch_size, per_batch_dev, &q_end);
     if (rc)

@@ -84,7 +84,10 @@ typedef struct {
     int32_t faster_evgen;                 /* 1 = `faster-evgen` generation (evgen.rs:143-173, 221-249),
                                              0 = default.  Available for every stream (RANF,
                                              xoshiro256+, xoshiro128+ in f32) in f64 and f32, with
-                                             either seeding; not in mixed precision */
+                                             either seeding; not in mixed precision, and from a RANF
+                                             state with values outside [0, 1e9) (a seed past 1e9)
+                                             not in calls of fewer than 2^20 events on its stream
+                                             (every closure; TP_ERR_UNSUPPORTED) */
     int32_t reserved;                     /* 0 */
 } tp_params;
 
