@@ -130,6 +130,9 @@ using namespace tpe;
 // Batches per launch of the xoshiro128+ events in registers:
 // 24576 * 10000 events * 24 B = 5.9 GB of per-event values.
 constexpr uint64_t F32_CHUNK_BATCHES = 24576;
+// Batches per launch of a RANF run whose streams' rounds lie in memory: 448
+// bytes each with jump seeding, 239 from a state past the modulus: 470 MB.
+constexpr uint64_t RANF_CHUNK_BATCHES = 1u << 20;
 
 int xo_tables(Ctx *c)
 {
@@ -1110,46 +1113,60 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     std::memcpy(R.round, rs->numbers, sizeof R.round);
     R.p0 = 55u - rs->index;
     R.r16 = static_cast<const uint32_t *>(c->r16.p);
-    if (seeding == TP_SEED_JUMP) {
-        rc = ensure(c, c->origin, 2 * nb * 56 * sizeof(int32_t)); // origins, then their rounds RANF_LATE
-        if (!rc)
-            rc = ensure(c, c->p0, nb * sizeof(int32_t));
-        if (rc)
-            return rc;
-        int32_t *const origin = static_cast<int32_t *>(c->origin.p);
-        tpk::launch_ranf_seed(rs->seed, 0, nb, R.r16, origin, static_cast<int32_t *>(c->p0.p), origin + 56 * nb, c->stream);
-        HIPCHK(c, hipGetLastError());
-        R.origin = origin;
-        R.later = origin + 56 * nb;
-    }
-    if (ranf_past_modulus(rs)) {
-        uint64_t segs = 1; // of RANF_LATE rounds: the first one's end of batch 0, or all of the one stream
-        if (!R.origin) {
-            segs = (R.p0 + 12 * num_events - 1) / 55 / tpk::RANF_LATE + 1;
+    // Rounds held in memory, a few hundred bytes a batch, limit a launch to
+    // RANF_CHUNK_BATCHES: the batches' own ones, or an odd stream's segments.
+    const bool jump = seeding == TP_SEED_JUMP, past = ranf_past_modulus(rs);
+    const uint64_t chunk = jump || past ? std::min(nb, RANF_CHUNK_BATCHES) : nb;
+    const uint32_t n = (uint32_t)std::min<uint64_t>(num_events, batch_size);
+    for (uint64_t b0 = 0; b0 < nb; b0 += chunk) {
+        const uint64_t cnb = std::min(nb - b0, chunk);
+        if (jump) {
+            rc = ensure(c, c->origin, 2 * chunk * 56 * sizeof(int32_t)); // origins, then their rounds RANF_LATE
+            if (!rc)
+                rc = ensure(c, c->p0, chunk * sizeof(int32_t));
+            if (rc)
+                return rc;
+            int32_t *const origin = static_cast<int32_t *>(c->origin.p);
+            R.origin = origin;
+            R.later = origin + 56 * chunk;
+            R.first = b0;
+            tpk::launch_ranf_seed(rs->seed, b0, cnb, R.r16, origin, static_cast<int32_t *>(c->p0.p), origin + 56 * chunk,
+                                  c->stream);
+            HIPCHK(c, hipGetLastError());
+            if (past && b0 == 0) { // the caller's stream, whose batch 0 may reach round RANF_LATE
+                tpk::launch_ranf_late(rs->numbers, R.r16, 1, 1, origin + 56 * chunk, c->stream);
+                HIPCHK(c, hipGetLastError());
+            }
+        } else if (past) {
+            const uint64_t end = std::min<uint64_t>(num_events, (b0 + cnb) * batch_size);
+            R.first = (R.p0 + 12ull * batch_size * b0) / 55 / tpk::RANF_LATE;
+            const uint64_t segs = (R.p0 + 12 * end - 1) / 55 / tpk::RANF_LATE + 1 - R.first;
             rc = ensure(c, c->origin, segs * 56 * sizeof(int32_t));
             if (rc)
                 return rc;
             R.later = static_cast<const int32_t *>(c->origin.p);
+            tpk::launch_ranf_late(rs->numbers, R.r16, R.first, segs, static_cast<int32_t *>(c->origin.p), c->stream);
+            HIPCHK(c, hipGetLastError());
         }
-        tpk::launch_ranf_late(rs->numbers, R.r16, R.origin ? 1 : 0, segs, const_cast<int32_t *>(R.later), c->stream);
-        HIPCHK(c, hipGetLastError());
-    }
-    if (const int e = mark(c, 1))
-        return e;
-    const uint32_t n = (uint32_t)std::min<uint64_t>(num_events, batch_size);
-    if (f32) {
-        // (a run whose batches are split has at most MAX_PARTS of them: its
-        // per-event values stay below 13.2 GB)
-        fa.nb = nb;
-        fa.out = per_batch_dev;
-        rc = launch_f32_batches(c, fa, n);
-        if (rc)
-            return rc;
-    } else {
-        a.nb = nb;
-        a.out = per_batch_dev;
-        if (const int e = launch_event_loop(c, a, 1, n))
-            return e;
+        if (b0 == 0)
+            if (const int e = mark(c, 1))
+                return e;
+        if (f32) {
+            // (a launch whose batches are split has at most MAX_PARTS of them:
+            // its per-event values stay below 13.2 GB)
+            fa.nb = cnb;
+            fa.b_first = b0;
+            fa.out = static_cast<tp_acc *>(per_batch_dev) + b0;
+            rc = launch_f32_batches(c, fa, n);
+            if (rc)
+                return rc;
+        } else {
+            a.nb = cnb;
+            a.b_first = b0;
+            a.out = static_cast<tp_acc *>(per_batch_dev) + b0;
+            if (const int e = launch_event_loop(c, a, 1, n))
+                return e;
+        }
     }
     if (const int e = mark(c, 2))
         return e;

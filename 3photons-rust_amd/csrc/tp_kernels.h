@@ -14,16 +14,16 @@ namespace tpk {
 // The RANF stream of a run.  Batch b's events draw from position p0 + 12
 // batch_size b on of the stream whose round 0 is `round` (X[1..55]); with jump
 // seeding (origin non-null) batch b > 0 has a stream of its own, round 0 at
-// origin[56 b] and positions from 0.  A stream whose round 0 holds values outside
-// [0, 1e9) goes on at each multiple s of RANF_LATE rounds from `later`: at
-// later[56 b] (s = 1, no batch gets further) with jump seeding, else at
-// later[56 (s - late_first)].
+// origin[56 (b - first)] and positions from 0.  A stream whose round 0 holds
+// values outside [0, 1e9) goes on at each multiple s of RANF_LATE rounds from
+// `later`: at later[56 (b - first)] (s = 1, no batch gets further) with jump
+// seeding, else at later[56 (s - first)].
 constexpr uint32_t RANF_LATE = 2048, RANF_LATE_R16 = 2 * 15 + 7; // 8 * 16^2: its place in r16
 struct RanfSource {
     int32_t round[56];
     uint32_t p0;
     const int32_t *origin, *later;
-    uint64_t late_first;
+    uint64_t first;       // the first batch that origin and later hold, or the first s that later does
     const uint32_t *r16;  // x^(55 v 16^j) mod the recurrence's polynomial, 55 coefficients each, v = 1..15,
                           // for the digits of a number of rounds
     uint32_t jump[55];    // x^(55 jump_rounds): from the end of a wavefront's part to near its next one

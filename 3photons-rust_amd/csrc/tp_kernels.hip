@@ -283,7 +283,7 @@ struct RanfPart {
             skip -= round + R.jump_rounds;
         } else {
             const uint32_t lane = threadIdx.x & 63u;
-            x = lane < 55 ? (own ? R.origin[56 * b + lane + 1] : R.round[lane + 1]) : 0;
+            x = lane < 55 ? (own ? R.origin[56 * (b - R.first) + lane + 1] : R.round[lane + 1]) : 0;
         }
         late = 0x7fffffffu;
         if (R.later && ranf_odd(x)) {
@@ -307,7 +307,7 @@ struct RanfPart {
     __device__ __forceinline__ int32_t later(const RanfSource &R, uint64_t b) const
     {
         const uint32_t lane = threadIdx.x & 63u;
-        return lane < 55 ? R.later[56 * (R.origin ? b : seg - R.late_first) + lane + 1] : 0;
+        return lane < 55 ? R.later[56 * ((R.origin ? b : seg) - R.first) + lane + 1] : 0;
     }
     // The next `need` (12 .. 768) values of batch b into lds[base ..] in stream
     // order.  Lanes with nothing to write do so to lds[dump].
