@@ -1116,25 +1116,27 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     // Rounds held in memory, a few hundred bytes a batch, limit a launch to
     // RANF_CHUNK_BATCHES: the batches' own ones, or an odd stream's segments.
     const bool jump = seeding == TP_SEED_JUMP, past = ranf_past_modulus(rs);
+    // Batches' seeds in [0, 1e9) give values in [0, 1e9): at most 8101 batches,
+    // 6200 from the default seed.
+    const bool odd = past || (jump && (rs->seed < 0 || nb > 8101 || rs->seed + 123456ll * (int64_t)(nb - 1) > 999999999));
     const uint64_t chunk = jump || past ? std::min(nb, RANF_CHUNK_BATCHES) : nb;
     const uint32_t n = (uint32_t)std::min<uint64_t>(num_events, batch_size);
     for (uint64_t b0 = 0; b0 < nb; b0 += chunk) {
         const uint64_t cnb = std::min(nb - b0, chunk);
         if (jump) {
-            rc = ensure(c, c->origin, 2 * chunk * 56 * sizeof(int32_t)); // origins, then their rounds RANF_LATE
+            rc = ensure(c, c->origin, (odd ? 2 : 1) * chunk * 56 * sizeof(int32_t)); // origins, then their rounds RANF_LATE
             if (!rc)
                 rc = ensure(c, c->p0, chunk * sizeof(int32_t));
             if (rc)
                 return rc;
-            int32_t *const origin = static_cast<int32_t *>(c->origin.p);
+            int32_t *const origin = static_cast<int32_t *>(c->origin.p), *const later = odd ? origin + 56 * chunk : nullptr;
             R.origin = origin;
-            R.later = origin + 56 * chunk;
+            R.later = later;
             R.first = b0;
-            tpk::launch_ranf_seed(rs->seed, b0, cnb, R.r16, origin, static_cast<int32_t *>(c->p0.p), origin + 56 * chunk,
-                                  c->stream);
+            tpk::launch_ranf_seed(rs->seed, b0, cnb, R.r16, origin, static_cast<int32_t *>(c->p0.p), later, c->stream);
             HIPCHK(c, hipGetLastError());
             if (past && b0 == 0) { // the caller's stream, whose batch 0 may reach round RANF_LATE
-                tpk::launch_ranf_late(rs->numbers, R.r16, 1, 1, origin + 56 * chunk, c->stream);
+                tpk::launch_ranf_late(rs->numbers, R.r16, 1, 1, later, c->stream);
                 HIPCHK(c, hipGetLastError());
             }
         } else if (past) {

@@ -17,7 +17,8 @@ namespace tpk {
 // origin[56 (b - first)] and positions from 0.  A stream whose round 0 holds
 // values outside [0, 1e9) goes on at each multiple s of RANF_LATE rounds from
 // `later`: at later[56 (b - first)] (s = 1, no batch gets further) with jump
-// seeding, else at later[56 (s - first)].
+// seeding, else at later[56 (s - first)].  Without such a stream later is null
+// (the event loops then run kernels that leave the rule out).
 constexpr uint32_t RANF_LATE = 2048, RANF_LATE_R16 = 2 * 15 + 7; // 8 * 16^2: its place in r16
 struct RanfSource {
     int32_t round[56];

@@ -261,13 +261,17 @@ __device__ __forceinline__ int32_t ranf_odd_segment(int32_t x, const uint32_t *_
 // again: 1e9 events 43.4 -> 28.3 ms with the event loop's own gains, the
 // expansion having been 10.4 ms of them; 1e7 events 586 -> 414 us.
 //
-struct RanfPart {
+// ODD: the run has streams with values outside [0, 1e9) (RanfSource::later),
+// in kernels of their own: the places where such a stream's jumps may go cost
+// every other run 2 % in the all-f32 loop, whose registers are full (1e7 events
+// 395 us without them, 410 with).
+template <bool ODD> struct RanfPart {
     int32_t x = 0;        // lane l: X[l + 1] of the current round
     uint32_t o = 0;       // the place of the next unread value in it: X[55 - o], o up to 55
     uint64_t round = 0;   // the number of the last round the part reads
     bool have = false;
-    uint32_t late = 0;    // rounds to the next segment of RANF_LATE in an odd stream, otherwise more than the part's
-    uint64_t seg = 0;     // odd stream: the current segment
+    uint32_t late = 0;    // ODD: rounds to the next segment of RANF_LATE in an odd stream, otherwise more than the part's
+    uint32_t next = 0;    // ODD: the row of RanfSource::later where it starts
     RanfLanes l = ranf_lanes();
 
     // To the first draw of n > 0 events from event `first` of batch b on.  win:
@@ -278,7 +282,7 @@ struct RanfPart {
         const bool own = R.origin && b > 0;
         const uint64_t q = (own ? 0 : R.p0) + 12ull * (first + (R.origin ? 0 : b * batch_size));
         uint64_t skip = q / 55;
-        if (have && R.jump_rounds && round + R.jump_rounds <= skip) { // on from the previous part
+        if (!ODD && have && R.jump_rounds && round + R.jump_rounds <= skip) { // on from the previous part
             x = ranf_jump(x, ranf_jump_lane(R.jump), win);
             skip -= round + R.jump_rounds;
         } else {
@@ -286,15 +290,17 @@ struct RanfPart {
             x = lane < 55 ? (own ? R.origin[56 * (b - R.first) + lane + 1] : R.round[lane + 1]) : 0;
         }
         late = 0x7fffffffu;
-        if (R.later && ranf_odd(x)) {
-            seg = skip / RANF_LATE;
+        if (ODD && ranf_odd(x)) {
+            const uint64_t seg = skip / RANF_LATE;
             skip %= RANF_LATE;
             late = RANF_LATE - (uint32_t)skip;
+            next = (uint32_t)((R.origin ? b : seg) - R.first); // (with jump seeding one row serves the batch)
             if (seg)
-                x = later(R, b);
+                x = later(R);
             else
                 for (; skip; --skip)
                     x = ranf_next_round(x, l);
+            next += R.origin ? 0 : 1;
         }
         if (skip < 4) // (a round costs a twentieth of a jump)
             for (; skip; --skip)
@@ -304,36 +310,33 @@ struct RanfPart {
         round = (q + 12ull * n - 1) / 55;
         have = true;
     }
-    __device__ __forceinline__ int32_t later(const RanfSource &R, uint64_t b) const
+    __device__ __forceinline__ int32_t later(const RanfSource &R) const
     {
-        const uint32_t lane = threadIdx.x & 63u;
-        return lane < 55 ? R.later[56 * ((R.origin ? b : seg) - R.first) + lane + 1] : 0;
+        uint32_t lane = threadIdx.x & 63u;
+        asm volatile("" : "+v"(lane)); // (its address is formed here, not kept in registers over the events)
+        return lane < 55 ? R.later[56 * (uint64_t)next + lane + 1] : 0;
     }
-    // The next `need` (12 .. 768) values of batch b into lds[base ..] in stream
+    // The next `need` (12 .. 768) values into lds[base ..] in stream
     // order.  Lanes with nothing to write do so to lds[dump].
-    __device__ __forceinline__ void fill(const RanfSource &R, uint64_t b, uint32_t need, int32_t *lds, uint32_t base,
-                                         uint32_t dump)
+    __device__ __forceinline__ void fill(const RanfSource &R, uint32_t need, int32_t *lds, uint32_t base, uint32_t dump)
     {
         const int lane = (int)(threadIdx.x & 63u), at = 54 - lane - (int)o;
         lds[lane < 55 && at >= 0 ? base + (uint32_t)at : dump] = x;
         uint32_t p = lane < 55 ? base + (uint32_t)(at + 55) : dump;
         const uint32_t step = lane < 55 ? 55u : 0u, rounds = (o + need + 54) / 55 - 1;
-        if (late <= rounds) { // an odd stream's next segment starts among them
+        if (ODD && __builtin_expect(late <= rounds, 0)) { // the next segment starts among them (no two do)
             for (uint32_t r = 1; r <= rounds; ++r) {
-                if (--late == 0) {
-                    ++seg;
-                    late = RANF_LATE;
-                    x = later(R, b);
-                } else {
-                    x = ranf_next_round(x, l);
-                }
+                x = r == late ? later(R) : ranf_next_round(x, l);
                 lds[p < base + need ? p : dump] = x;
                 p += step;
             }
+            late += RANF_LATE - rounds;
+            next += R.origin ? 0 : 1;
             o = o + need - 55 * rounds;
             return;
         }
-        late -= rounds;
+        if (ODD)
+            late -= rounds;
         for (uint32_t r = 1; r < rounds; ++r) {
             x = ranf_next_round(x, l);
             lds[p] = x;
@@ -393,7 +396,7 @@ __device__ __forceinline__ const Params &fresh_params()
     return *(const Params *)k;
 }
 
-template <int SOURCE, int PREC>
+template <int SOURCE, int PREC, bool ODD = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void fused_kernel(FusedArgs a)
 {
     // momenta, structure of arrays, slots 0..63 and 64..127; between
@@ -408,7 +411,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
     const uint32_t lane = threadIdx.x;
     const uint64_t lanemask_lt = (1ull << lane) - 1ull;
     uint64_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}; // xoshiro state at the part's first draw (uniform)
-    RanfPart ranf;
+    RanfPart<ODD> ranf;
     bool have = false;
     for (uint64_t t = blockIdx.x; t < a.nb * a.parts; t += gridDim.x) {
         const uint64_t lb = a.parts == 1 ? t : t / a.parts;
@@ -451,7 +454,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
                 qnext = a.evq[wbase + (size_t)((k + 1) * 64 + lane)];
             int4 rd[3]; // RANF: the lane's 12 draws
             if (SOURCE == 1) {
-                ranf.fill(a.ranf, b, 12 * min(64u, n - 64 * k), qints, RING, RING_DUMP);
+                ranf.fill(a.ranf, 12 * min(64u, n - 64 * k), qints, RING, RING_DUMP);
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < 3; ++j)
@@ -729,7 +732,11 @@ void launch_fused(const FusedArgs &a, int source, int grid, hipStream_t st)
         else
             hipLaunchKernelGGL((fused_kernel<0, 1>), g, b, 0, st, a);
     } else if (source == 1) {
-        if (a.precision == 0)
+        if (a.ranf.later && a.precision == 0)
+            hipLaunchKernelGGL((fused_kernel<1, 0, true>), g, b, 0, st, a);
+        else if (a.ranf.later)
+            hipLaunchKernelGGL((fused_kernel<1, 1, true>), g, b, 0, st, a);
+        else if (a.precision == 0)
             hipLaunchKernelGGL((fused_kernel<1, 0>), g, b, 0, st, a);
         else
             hipLaunchKernelGGL((fused_kernel<1, 1>), g, b, 0, st, a);
@@ -2096,7 +2103,7 @@ __device__ __forceinline__ const FParams &fresh_fparams() // as fresh_params
     return *(const FParams *)k;
 }
 
-template <int SOURCE, bool SUMS>
+template <int SOURCE, bool SUMS, bool ODD = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void f32_events_kernel(F32Args a)
 {
     constexpr uint32_t HALF = 12 * 64, DUMP = 2 * HALF;
@@ -2106,7 +2113,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
     const uint32_t lane = threadIdx.x;
     const uint64_t lanemask_lt = (1ull << lane) - 1ull;
     uint32_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}; // xoshiro128+ state at the part's first draw (uniform)
-    RanfPart ranf;
+    RanfPart<ODD> ranf;
     bool have = false;
     for (uint64_t t = blockIdx.x; t < a.nb * a.parts; t += gridDim.x) {
         const uint64_t lb = a.parts == 1 ? t : t / a.parts;
@@ -2208,7 +2215,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
             int4 rd[3]; // RANF: the lane's 12 draws, through the half that is free
             if (SOURCE == 1) {
                 const uint32_t ring = head ? 0 : HALF;
-                ranf.fill(a.ranf, b, 12 * min(64u, n - 64 * i), qints, ring, DUMP);
+                ranf.fill(a.ranf, 12 * min(64u, n - 64 * i), qints, ring, DUMP);
                 __syncthreads();
 #pragma unroll
                 for (int j = 0; j < 3; ++j)
@@ -2440,18 +2447,20 @@ int f32_blocks_per_cu(int source)
     return source == 0 ? f32_blocks<0>() : source == 1 ? f32_blocks<1>() : source == 2 ? f32_blocks<2>() : f32_blocks<3>();
 }
 
-template <int SOURCE> static void launch_f32_source(const F32Args &a, int grid, hipStream_t st)
+template <int SOURCE, bool ODD = false> static void launch_f32_source(const F32Args &a, int grid, hipStream_t st)
 {
     if (f32_sums_in_kernel(a))
-        hipLaunchKernelGGL((f32_events_kernel<SOURCE, true>), dim3(grid), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((f32_events_kernel<SOURCE, true, ODD>), dim3(grid), dim3(64), 0, st, a);
     else
-        hipLaunchKernelGGL((f32_events_kernel<SOURCE, false>), dim3(grid), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((f32_events_kernel<SOURCE, false, ODD>), dim3(grid), dim3(64), 0, st, a);
 }
 
 void launch_f32_events(const F32Args &a, int grid, hipStream_t st)
 {
     if (a.source == 0)
         hipLaunchKernelGGL((f32_events_kernel<0, false>), dim3(grid), dim3(64), 0, st, a);
+    else if (a.source == 1 && a.ranf.later)
+        launch_f32_source<1, true>(a, grid, st);
     else if (a.source == 1)
         launch_f32_source<1>(a, grid, st);
     else if (a.source == 2)

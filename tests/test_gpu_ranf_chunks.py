@@ -109,3 +109,21 @@ def test_one_odd_stream(engine, valeurs):
         scale = np.abs(ref)
         scale[1:6], scale[11] = np.sqrt(count * ref[6:11]), np.sqrt(count * ref[12])
         assert a[0] == ref[0] and np.all(np.abs(a - ref) <= 1e-9 * scale), (b, a, ref)
+
+
+# the last batch's seed is the last in [0, 1e9), the first past it, or one past 2^31; and the most batches that all lie inside
+@pytest.mark.parametrize("prec", [tp.PREC_F64, tp.PREC_MIXED, tp.PREC_F32])
+@pytest.mark.parametrize("first, batches", [(999_999_999 - 5 * 123456, 6), (10**9 - 5 * 123456, 6), (999_999_999 - 5 * 123456, 7),
+                                            (2**31 - 3 * 123456, 6), (63_999, 8101), (64_000, 8101), (0, 8102)])
+def test_seeds_at_the_modulus(engine, valeurs, first, batches, prec):
+    """Batches' seeds first + 123456 b: each batch is the closure on its state."""
+    params = tp.params_from_config(tp.Configuration.load(valeurs), precision=prec)
+    print(f"jump-seeded run precision {prec} seed {first} batches {batches}", flush=True)
+    per, _, _ = engine.run(params, tp.RNG_RANF, tp.SEED_JUMP, tp.rng_state(tp.RNG_RANF, first), 10_000 * batches)
+    for b in sorted({0, *range(batches - 6, batches)}):
+        acc = engine.simulate_batch(params, tp.RNG_RANF, tp.rng_state(tp.RNG_RANF, (first + 123456 * b) % 2**32), 10_000)
+        got = tp.TpAcc.from_buffer_copy(per[b])
+        if prec == tp.PREC_F32:
+            assert bytes(acc) == bytes(got), b
+        else:
+            close(acc.as_array(), got.as_array())
