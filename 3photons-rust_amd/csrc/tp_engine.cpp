@@ -1565,6 +1565,9 @@ extern "C" int tp_events(void *ctx, const tp_params *params, int rng_kind, const
     });
 }
 
+// Points of the stream that tp_adjoint expands at a time, 96 bytes each (1.6 GB).  2^22 took
+// about as long (2^24 points in f64 4.04 and 4.09 ms, in f32 4.40 and 4.35).
+constexpr uint64_t ADJ_STREAM_POINTS = 1u << 24;
 // Points per lane of the kernel that expands tp_adjoint's stream: the longest
 // run that still gives each SIMD a wavefront (whole calls at 2^20 points: 295 us
 // in runs of 10 or 20, 309 of 5, 349 of 1; at 1001: 30 us of 1, 35 of 10).
@@ -1602,17 +1605,17 @@ extern "C" int tp_adjoint(void *ctx, const tp_params *params, int rng_kind, cons
         a.P = make_params(params);
         a.hk = tpd::helicity_constants(params->e_total, params->g_a, params->g_beta_p, params->g_beta_m, 1.);
         a.w = params->ev_weight;
-        a.n = n;
+        const uint64_t step = u_in ? n : std::min(n, ADJ_STREAM_POINTS);
         if (!u_in) {
             std::memcpy(a.s0, static_cast<const tp_xoshiro_state *>(rng_state)->s, sizeof a.s0);
             rc = xo_tables(c);
             if (!rc)
-                rc = ensure(c, c->adj_u, 12 * n * sizeof(double)); // the stream's points, expanded first
+                rc = ensure(c, c->adj_u, 12 * step * sizeof(double)); // the stream's points, expanded first
             if (rc)
                 return rc;
             a.u_gen = static_cast<double *>(c->adj_u.p);
             a.m16 = c->xo->m16;
-            a.run = adjoint_run(c, n);
+            a.run = adjoint_run(c, step);
             a.lanes = reinterpret_cast<const uint64_t *>(
                 xo_lane_table(reinterpret_cast<const uint32_t *>(c->xo->lanes), 2 * tpk::XO_LANE_WORDS, a.run));
         }
@@ -1642,10 +1645,19 @@ extern "C" int tp_adjoint(void *ctx, const tp_params *params, int rng_kind, cons
         }
         if (rc == TP_OK) {
             HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-            tpk::launch_adjoint(a, precision, c->stream);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess)
-                rc = fail(c, TP_ERR_HIP, std::string("adjoint kernel: ") + hipGetErrorString(e));
+            auto past = [es](void *p, uint64_t values) { return p ? static_cast<char *>(p) + values * es : nullptr; };
+            for (uint64_t at = 0; at < n && rc == TP_OK; at += step) {
+                tpk::AdjArgs k = a;
+                k.first = at;
+                k.n = std::min(step, n - at);
+                k.F = past(a.F, 5 * at);
+                k.dF_du = past(a.dF_du, 60 * at);
+                k.dF_dp = past(a.dF_dp, 60 * at);
+                tpk::launch_adjoint(k, precision, c->stream);
+                hipError_t e = hipGetLastError();
+                if (e != hipSuccess)
+                    rc = fail(c, TP_ERR_HIP, std::string("adjoint kernel: ") + hipGetErrorString(e));
+            }
             HIPCHK(c, hipEventRecord(c->ev[2], c->stream));
         }
         if (rc == TP_OK && !on_device)

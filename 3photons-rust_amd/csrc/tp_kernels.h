@@ -326,6 +326,7 @@ struct AdjArgs {
     const double *u_in;
     double *u_gen;
     uint64_t s0[4];
+    uint64_t first;        // of the stream's points, 12 draws each
     const uint64_t *m16, *lanes; // as FusedArgs
     uint32_t run;          // one of XO_RUNS
     void *F, *dF_du, *dF_dp; // [n][5], [n][5][12], [n][5][12] of double or float

@@ -2632,7 +2632,7 @@ __global__ __launch_bounds__(64) void adjoint_points_kernel(AdjArgs a)
 {
     const uint64_t base = 64ull * a.run * blockIdx.x;
     uint64_t sw[4] = {a.s0[0], a.s0[1], a.s0[2], a.s0[3]}, s[4];
-    xo_advance_uniform(a.m16, 12 * base, sw);
+    xo_advance_uniform(a.m16, 12 * (a.first + base), sw);
     xo_lane_states(a.lanes, sw, s);
     const uint64_t first = base + (uint64_t)a.run * threadIdx.x, last = min(first + a.run, a.n);
     for (uint64_t k = first; k < last; ++k) {
