@@ -303,6 +303,7 @@ inline int launch_f32_batches(Ctx *c, tpk::F32Args &a, uint32_t n)
     const Split s = split_for_f32(c, a.source, a.nb, n);
     a.parts = s.parts;
     a.run = s.run;
+    a.wide = tpd::f32_wide_range(a.P.e_total, a.P.e_min, a.P.cut_beam);
     if (a.source == 0)
         a.lanes = xo_lane_table(c->xo->lanes128, tpk::XO128_LANE_WORDS, s.run);
     if (a.source == 0 && !a.lanes)

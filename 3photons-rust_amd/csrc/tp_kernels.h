@@ -160,6 +160,7 @@ struct F32Args {
     int32_t source;        // 0 xoshiro128+ in registers, 1 RANF, 2 faster-evgen on
                            // RANF draws, 3 faster-evgen on xoshiro128+ uniforms (x32draws)
     uint32_t parts, run;
+    bool wide;             // f32_wide_range of P
     uint32_t s0[4];        // xoshiro128+ state of the run, and its skip tables as in FusedArgs
     const uint32_t *m16, *b16;
     const uint32_t *lanes;

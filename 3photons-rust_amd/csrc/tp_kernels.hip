@@ -2103,7 +2103,7 @@ __device__ __forceinline__ const FParams &fresh_fparams() // as fresh_params
     return *(const FParams *)k;
 }
 
-template <int SOURCE, bool SUMS, bool ODD = false>
+template <int SOURCE, bool SUMS, bool ODD = false, bool WIDE = false>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void f32_events_kernel(F32Args a)
 {
     constexpr uint32_t HALF = 12 * 64, DUMP = 2 * HALF;
@@ -2153,7 +2153,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         pq[i][j] = half[64 * (4 * i + j) + lane];
-                matrix_elements_f32(fresh_fparams(), pq, m);
+                matrix_elements_f32<WIDE>(fresh_fparams(), pq, m);
             };
             if (SUMS) {
                 // summand j of event e at column (e + 4 j) % 64 of row j: the 12
@@ -2226,10 +2226,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
                 const RerollBits rb{a.acc1, a.bbase, a.bstride ? (lb + 1) * a.bstride : a.blimit};
                 if constexpr (SOURCE == 2) {
                     RanfWalkF32 w{a.draws, a.qbase, qk, rb};
-                    pass = generate_faster_f32(fresh_fparams(), w, p);
+                    pass = generate_faster_f32<WIDE>(fresh_fparams(), w, p);
                 } else {
                     Xo128WalkF32 w{a.x32draws, a.qbase, qk, rb};
-                    pass = generate_faster_f32(fresh_fparams(), w, p);
+                    pass = generate_faster_f32<WIDE>(fresh_fparams(), w, p);
                 }
             } else if (i < len) {
                 float u[12];
@@ -2246,7 +2246,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 8))) void
                         u[4 * j + 3] = (float)rd[j].w * 1e-9f;
                     }
                 }
-                pass = generate_f32(fresh_fparams(), u, p);
+                pass = generate_f32<WIDE>(fresh_fparams(), u, p);
             }
             if (SOURCE == 0 && i < len && !pass) {
                 float *o = a.ev + 6 * (size_t)(base + lane * a.run + i);
@@ -2447,24 +2447,32 @@ int f32_blocks_per_cu(int source)
     return source == 0 ? f32_blocks<0>() : source == 1 ? f32_blocks<1>() : source == 2 ? f32_blocks<2>() : f32_blocks<3>();
 }
 
-template <int SOURCE, bool ODD = false> static void launch_f32_source(const F32Args &a, int grid, hipStream_t st)
+template <int SOURCE, bool ODD = false, bool WIDE = false> static void launch_f32_source(const F32Args &a, int grid, hipStream_t st)
 {
     if (f32_sums_in_kernel(a))
-        hipLaunchKernelGGL((f32_events_kernel<SOURCE, true, ODD>), dim3(grid), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((f32_events_kernel<SOURCE, true, ODD, WIDE>), dim3(grid), dim3(64), 0, st, a);
     else
-        hipLaunchKernelGGL((f32_events_kernel<SOURCE, false, ODD>), dim3(grid), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((f32_events_kernel<SOURCE, false, ODD, WIDE>), dim3(grid), dim3(64), 0, st, a);
 }
 
 void launch_f32_events(const F32Args &a, int grid, hipStream_t st)
 {
-    if (a.source == 0)
+    if (a.source == 0 && a.wide)
+        hipLaunchKernelGGL((f32_events_kernel<0, false, false, true>), dim3(grid), dim3(64), 0, st, a);
+    else if (a.source == 0)
         hipLaunchKernelGGL((f32_events_kernel<0, false>), dim3(grid), dim3(64), 0, st, a);
+    else if (a.source == 1 && a.wide) // (ODD serves streams inside [0, 1e9) too)
+        launch_f32_source<1, true, true>(a, grid, st);
     else if (a.source == 1 && a.ranf.later)
         launch_f32_source<1, true>(a, grid, st);
     else if (a.source == 1)
         launch_f32_source<1>(a, grid, st);
+    else if (a.source == 2 && a.wide)
+        launch_f32_source<2, false, true>(a, grid, st);
     else if (a.source == 2)
         launch_f32_source<2>(a, grid, st);
+    else if (a.wide)
+        launch_f32_source<3, false, true>(a, grid, st);
     else
         launch_f32_source<3>(a, grid, st);
 }

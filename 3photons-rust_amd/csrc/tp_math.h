@@ -126,10 +126,10 @@ TPM_FN double sqrt_nonneg(double x)
 }
 // a / b and sqrt(x) in f32, the values of '/' and sqrtf(): their sequences
 // without the scaling that only acts where an exponent (of b, of a below -103, of
-// the quotient, of x below -96) comes near the ends of the range, which the
-// all-f32 event loop's values stay away from; zeros, infinities and NaN come out
-// as in those.  8 and 9 instructions instead of 11 and 16, and quotients by one
-// divisor share its reciprocal.
+// the quotient, of x below -96) comes near the ends of the range: the callers see
+// to it that theirs do not (tpd::f32_wide_range); zeros, infinities and NaN come
+// out as in those.  8 and 9 instructions instead of 11 and 16, and quotients by
+// one divisor share its reciprocal.
 TPM_FN float div_f(float a, float b)
 {
     float y = __builtin_amdgcn_rcpf(b);

@@ -63,28 +63,34 @@ template <class T> __device__ __forceinline__ C<T> cmul(C<T> a, C<T> b)
 }
 // IEEE division and square root: in f64 through tpm::div_n / tpm::sqrt_n
 // (the same correctly rounded results in the event loop's range, fewer
-// instructions), in f32 through tpm::div_f / tpm::sqrt_f.
-template <class T> __device__ __forceinline__ T dv(T a, T b)
+// instructions), in f32 through tpm::div_f / tpm::sqrt_f, or with WIDE the
+// plain operations: for runs whose values f32_wide_range cannot keep away from
+// the ends of f32's exponents.
+template <bool WIDE = false, class T> __device__ __forceinline__ T dv(T a, T b)
 {
     if constexpr (std::is_same<T, double>::value)
         return tpm::div_n(a, b);
+    else if constexpr (WIDE)
+        return a / b;
     else
         return tpm::div_f(a, b);
 }
-template <class T> __device__ __forceinline__ T sq(T x)
+template <bool WIDE = false, class T> __device__ __forceinline__ T sq(T x)
 {
     if constexpr (std::is_same<T, double>::value)
         return tpm::sqrt_n(x);
+    else if constexpr (WIDE)
+        return sqrtf(x);
     else
         return tpm::sqrt_f(x);
 }
 // num-complex naive division (spinor.rs divides with it).
-template <class T> __device__ __forceinline__ C<T> cdiv(C<T> a, C<T> b)
+template <bool WIDE = false, class T> __device__ __forceinline__ C<T> cdiv(C<T> a, C<T> b)
 {
     T n = b.re * b.re + b.im * b.im;
     T re = a.re * b.re + a.im * b.im;
     T im = a.im * b.re - a.re * b.im;
-    return C<T>{dv(re, n), dv(im, n)};
+    return C<T>{dv<WIDE>(re, n), dv<WIDE>(im, n)};
 }
 template <class T> __device__ __forceinline__ C<T> cadd(C<T> a, C<T> b) { return C<T>{a.re + b.re, a.im + b.im}; }
 template <class T> __device__ __forceinline__ C<T> csq(C<T> z) { return cmul(z, z); }
@@ -269,7 +275,7 @@ template <bool FAST, class T> __device__ __forceinline__ T mul_add(T a, T b, T c
 }
 
 // The all-f32 parity path's spinor products: the reference's plain operations.
-template <class T>
+template <class T, bool WIDE = false>
 __device__ __forceinline__ void spinor_products(T xx0, T f0re, T f0im, T xx1, T f1re, T f1im, const T p[3][4],
                                                 Spin<T> &S)
 {
@@ -277,13 +283,13 @@ __device__ __forceinline__ void spinor_products(T xx0, T f0re, T f0im, T xx1, T 
     C<T> fx[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        xx[k] = sq(p[k][3] + p[k][2]);
+        xx[k] = sq<WIDE>(p[k][3] + p[k][2]);
         // f32::MIN_POSITIVE / f64::MIN_POSITIVE
         const T minpos = sizeof(T) == 8 ? (T)2.2250738585072014e-308 : (T)1.17549435e-38f;
         if (xx[k] > minpos)
-            fx[k] = mk<T>(dv(p[k][0], xx[k]), dv(p[k][1], xx[k]));
+            fx[k] = mk<T>(dv<WIDE>(p[k][0], xx[k]), dv<WIDE>(p[k][1], xx[k]));
         else
-            fx[k] = mk<T>(sq((T)2. * p[k][3]), (T)0.);
+            fx[k] = mk<T>(sq<WIDE>((T)2. * p[k][3]), (T)0.);
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -334,12 +340,12 @@ template <bool FAST, class T> __device__ __forceinline__ C<T> xmul(C<T> a, C<T> 
     else
         return cmul(a, b);
 }
-template <bool FAST, class T> __device__ __forceinline__ C<T> xdiv(C<T> a, C<T> b)
+template <bool FAST, bool WIDE = false, class T> __device__ __forceinline__ C<T> xdiv(C<T> a, C<T> b)
 {
     if constexpr (FAST)
         return cdiv_fast(a, b);
     else
-        return cdiv(a, b);
+        return cdiv<WIDE>(a, b);
 }
 template <bool FAST, class T> __device__ __forceinline__ T xnorm(C<T> z) { return mul_add<FAST>(z.re, z.re, z.im, z.im); }
 template <bool FAST, class T> __device__ __forceinline__ C<T> xsq(C<T> z) { return xmul<FAST>(z, z); }
@@ -367,19 +373,19 @@ template <bool FAST, class T> __device__ __forceinline__ C<T> kmul(C<T> c, T k, 
         return cmul(c, z);
 }
 
-template <class T, bool FAST>
+template <class T, bool FAST, bool WIDE = false>
 __device__ __forceinline__ C<T> a_ppm(const Spin<T> &S, const AmpK<T> &K, int k1, int k2, int k3)
 {
     C<T> num = kmul<FAST>(K.ns01, K.ka_s, xsq<FAST>(S.s[0][k3]));
     C<T> den = xmul<FAST>(xmul<FAST>(xmul<FAST>(S.s[0][k1], S.s[0][k2]), S.s[1][k1]), S.s[1][k2]);
-    return xdiv<FAST>(num, den);
+    return xdiv<FAST, WIDE>(num, den);
 }
-template <class T, bool FAST>
+template <class T, bool FAST, bool WIDE = false>
 __device__ __forceinline__ C<T> a_pmm(const Spin<T> &S, const AmpK<T> &K, int k1, int k2, int k3)
 {
     C<T> num = kmul<FAST>(K.nt01, K.ka_t, xsq<FAST>(tof(S.s[1][k1])));
     C<T> den = xmul<FAST>(xmul<FAST>(xmul<FAST>(tof(S.s[1][k2]), tof(S.s[1][k3])), tof(S.s[0][k2])), tof(S.s[0][k3]));
-    return xdiv<FAST>(num, den);
+    return xdiv<FAST, WIDE>(num, den);
 }
 template <class T, bool FAST>
 __device__ __forceinline__ C<T> bp_ppm(const Spin<T> &S, const AmpK<T> &K, int k1, int k2, int k3)
@@ -438,7 +444,7 @@ template <class T> __device__ __forceinline__ C<T> a_pmm_d(const Spin<T> &S, con
 // interference terms are summed without their factor 2, which multiplies the
 // sums at the end: doubling is exact in binary, so every partial sum is the
 // reference's halved and the results are the same bits.
-template <class T, bool FAST>
+template <class T, bool FAST, bool WIDE = false>
 __device__ __forceinline__ void helicity_sums(const Spin<T> &S, const AmpK<T> &K, T m[5])
 {
     // (A, B+) for h = MMP, MPM, MPP, PMM, PMP, PPM, each folded into the sums
@@ -474,12 +480,12 @@ __device__ __forceinline__ void helicity_sums(const Spin<T> &S, const AmpK<T> &K
         fold(4, a_ppm_d(S, K, d24, 3), bp_ppm<T, FAST>(S, K, 2, 4, 3));
         fold(5, a_ppm_d(S, K, d23, 4), bp_ppm<T, FAST>(S, K, 2, 3, 4));
     } else {
-        fold(0, a_pmm<T, FAST>(S, K, 4, 2, 3), bp_pmm<T, FAST>(S, K, 4, 2, 3));
-        fold(1, a_pmm<T, FAST>(S, K, 3, 2, 4), bp_pmm<T, FAST>(S, K, 3, 2, 4));
-        fold(2, a_ppm<T, FAST>(S, K, 3, 4, 2), bp_ppm<T, FAST>(S, K, 3, 4, 2));
-        fold(3, a_pmm<T, FAST>(S, K, 2, 3, 4), bp_pmm<T, FAST>(S, K, 2, 3, 4));
-        fold(4, a_ppm<T, FAST>(S, K, 2, 4, 3), bp_ppm<T, FAST>(S, K, 2, 4, 3));
-        fold(5, a_ppm<T, FAST>(S, K, 2, 3, 4), bp_ppm<T, FAST>(S, K, 2, 3, 4));
+        fold(0, a_pmm<T, FAST, WIDE>(S, K, 4, 2, 3), bp_pmm<T, FAST>(S, K, 4, 2, 3));
+        fold(1, a_pmm<T, FAST, WIDE>(S, K, 3, 2, 4), bp_pmm<T, FAST>(S, K, 3, 2, 4));
+        fold(2, a_ppm<T, FAST, WIDE>(S, K, 3, 4, 2), bp_ppm<T, FAST>(S, K, 3, 4, 2));
+        fold(3, a_pmm<T, FAST, WIDE>(S, K, 2, 3, 4), bp_pmm<T, FAST>(S, K, 2, 3, 4));
+        fold(4, a_ppm<T, FAST, WIDE>(S, K, 2, 4, 3), bp_ppm<T, FAST>(S, K, 2, 4, 3));
+        fold(5, a_ppm<T, FAST, WIDE>(S, K, 2, 3, 4), bp_ppm<T, FAST>(S, K, 2, 3, 4));
     }
     C<T> Bm = bm_mmm<T, FAST>(S, K);
     C<T> Bp = bm_ppp<T, FAST>(S, K);
@@ -809,6 +815,23 @@ struct FParams {
     int sort;
 };
 
+// Whether tpm::div_f and tpm::sqrt_f may round otherwise than '/' and sqrtf()
+// in an all-f32 run, whose kernels then take those (WIDE).  The events' divisors
+// that come near the ends of f32's exponents first are |D|^2 of products D of
+// four spinor products with the beams; each one's square lies between
+// e_total e_min (1 - cut_beam) and 4 e_total^2 for a photon inside the cuts.
+// Where |D|^2 lies within 2^-76 .. 2^100, it and the quotients stay clear of the
+// exponents that the scaling acts on, and the momenta and their roots all the
+// more; the rest of an event does not depend on the energy.  With the shipped
+// cuts that is e_total from 0.02 to 2896 GeV (1e8 events on RANF 3.1 ms, 3.4 with
+// WIDE); f32 holds the sums from some 1e-4 to 1e5.  (The f32 adjoint divides by
+// single products' squares, and its reciprocals of |D|^2 are the hardware's.)
+__host__ __device__ inline bool f32_wide_range(double e_total, double e_min, double cut_beam)
+{
+    const double lo = e_total * e_min * (1. - cut_beam), hi = 4. * (e_total * e_total);
+    return !(e_min > 0. && cut_beam < 1. && (lo * lo) * (lo * lo) >= 0x1.0p-76 && (hi * hi) * (hi * hi) <= 0x1.0p100);
+}
+
 // sin, cos and ln of an f32 argument are evaluated in f64 and rounded once:
 // the correctly rounded f32 result in all but astronomically rare cases,
 // which is what the host libm's f32 functions return (within their < 1 ulp
@@ -830,6 +853,7 @@ __device__ __forceinline__ void raw_photon_f32(float uc, float uphi, float ue1, 
     q[3] = en;
 }
 
+template <bool WIDE>
 __device__ __forceinline__ void conformal_f32(const FParams &P, const float q[3][4], float p[3][4])
 {
     float r[4];
@@ -837,7 +861,7 @@ __device__ __forceinline__ void conformal_f32(const FParams &P, const float q[3]
     for (int k = 0; k < 4; ++k)
         r[k] = (q[0][k] + q[1][k]) + q[2][k];
     float rn2 = r[3] * r[3] - ((r[0] * r[0] + r[1] * r[1]) + r[2] * r[2]);
-    float alpha = tpm::div_f(P.e_total, rn2);
+    float alpha = dv<WIDE>(P.e_total, rn2);
     float rn = tpm::sqrt_f(rn2);
     float beta = tpm::div_f(1.f, rn + r[3]);
 #pragma unroll
@@ -891,25 +915,27 @@ __device__ __forceinline__ bool keep_f32(const FParams &P, const float p[3][4])
 
 // One f32 event from 12 uniforms: photon momenta (sorted when P.sort) and
 // the cut decision.
+template <bool WIDE = false>
 __device__ __forceinline__ bool generate_f32(const FParams &P, const float u[12], float p[3][4])
 {
     float q[3][4];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
         raw_photon_f32(u[4 * i], u[4 * i + 1], u[4 * i + 2], u[4 * i + 3], q[i]);
-    conformal_f32(P, q, p);
+    conformal_f32<WIDE>(P, q, p);
     if (P.sort)
         sort3(p);
     return keep_f32(P, p);
 }
 
 // Helicity sums m[5] of an f32 event that passed the cuts.
+template <bool WIDE = false>
 __device__ __forceinline__ void matrix_elements_f32(const FParams &P, const float p[3][4], float m[5])
 {
     Spin<float> S;
-    spinor_products<float>(P.xx0, P.f0re, P.f0im, P.xx1, P.f1re, P.f1im, p, S);
+    spinor_products<float, WIDE>(P.xx0, P.f0re, P.f0im, P.xx1, P.f1re, P.f1im, p, S);
     const AmpK<float> K{mk(P.ns01re, P.ns01im), mk(P.nt01re, P.nt01im), P.g_a, P.g_bp, P.g_bm, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    helicity_sums<float, false>(S, K, m);
+    helicity_sums<float, false, WIDE>(S, K, m);
 }
 
 // ---- faster-evgen in f32 (evgen.rs:143-173, 221-249 with Float = f32) -------
@@ -1029,11 +1055,11 @@ template <class Walk> __device__ __forceinline__ void raw_photons_faster_f32(Wal
     }
 }
 
-template <class Walk> __device__ __forceinline__ bool generate_faster_f32(const FParams &P, Walk &w, float p[3][4])
+template <bool WIDE, class Walk> __device__ __forceinline__ bool generate_faster_f32(const FParams &P, Walk &w, float p[3][4])
 {
     float q[3][4];
     raw_photons_faster_f32(w, q);
-    conformal_f32(P, q, p);
+    conformal_f32<WIDE>(P, q, p);
     if (P.sort)
         sort3(p);
     return keep_f32(P, p);
