@@ -138,7 +138,10 @@ TPM_FN void helicity_sums_closed(const HelicityK &K, const double p[3][4], doubl
 // m[5]: the sums; g[c][k] = d m_c / d (X, Y, ez) of photon k.  `along`: bit k is
 // set for a photon with the spinor (0, sqrt(2 E)), which depends on E alone; its
 // X and Y derivatives are 0 and g[c][k][2] is the one by E (a photon with E
-// below -Z counts as one too, and its sums and derivatives are NaN).
+// below -Z counts as one too, and its sums and derivatives are NaN).  A photon
+// without energy (RAMBO's from u1 u2 = 1, which given points may have and only
+// cuts that are off let pass) has the spinor (0, 0), a factor of every B and a
+// divisor of A: the sums of the B are 0 (bit 3), all else NaN.
 TPM_FN void helicity_gradients(const HelicityK &K, const double p[3][4], double m[5], double g[5][3][3], int &along)
 {
     using tpm::fma_;
@@ -151,10 +154,14 @@ TPM_FN void helicity_gradients(const HelicityK &K, const double p[3][4], double 
         py[k] = p[k][1];
     }
     if (!(ez[0] > 0. && ez[1] > 0. && ez[2] > 0.)) { // as in helicity_sums_closed
+        bool spinors = true;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             if (!(ez[k] > 0.))
                 along |= 1 << k;
+            if (ez[k] == 0. && p[k][3] == 0.)
+                along |= 8;
+            spinors = spinors && ez[k] >= 0.;
             if (ez[k] == 0.) {
                 ez[k] = p[k][3] * 0x1.0p-120;
                 px[k] = tpm::sqrt_n(2. * p[k][3] * ez[k]);
@@ -163,6 +170,7 @@ TPM_FN void helicity_gradients(const HelicityK &K, const double p[3][4], double 
             if (!(ez[k] > 0.))
                 ez[k] = __builtin_nan("");
         }
+        along = spinors ? along : along & 7;
     }
     double iz[3], zr[3], zi[3], u[3], v[3], rho[3], fr[3], fi[3], Gr[3], Gi[3], ur[3], ui[3], vr[3], vi[3];
 #pragma unroll
@@ -283,6 +291,8 @@ TPM_FN void helicity_gradients(const HelicityK &K, const double p[3][4], double 
             g[c][k][2] = fma_(-zr[k], wr[c][k], fma_(-zi[k], wi[c][k], we[c][k])) * iz[k];
         }
     if (along) {
+        if (along & 8)
+            m[1] = m[2] = 0.;
 #pragma unroll
         for (int k = 0; k < 3; ++k)
             if (along >> k & 1) // X = sqrt(ez) sqrt(2 E): d/dE = d/dX ez / X
