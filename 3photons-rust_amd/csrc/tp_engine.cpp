@@ -1199,7 +1199,7 @@ constexpr size_t NS_LANES = NS_B + 2 * 15 * tpk::XO_B_DIGITS * tpk::XO_MAT_WORDS
 constexpr size_t NS_128 = NS_LANES + tpk::XO_NTABLES * tpk::XO_LANE_WORDS;  // xoshiro128+ (u32 words), as above
 constexpr size_t NS128_B = 15 * tpk::XO_M_DIGITS * tpk::XO128_MAT_WORDS;
 constexpr size_t NS128_LANES = NS128_B + 2 * 15 * tpk::XO_B_DIGITS * tpk::XO128_MAT_WORDS;
-constexpr size_t NS_WORDS = NS_128 + (NS128_LANES + tpk::XO_NTABLES * tpk::XO128_LANE_WORDS) / 2; // 33 MiB
+constexpr size_t NS_WORDS = NS_128 + (NS128_LANES + tpk::XO_NTABLES * tpk::XO128_LANE_WORDS) / 2; // 31.7 MiB
 static_assert(sizeof(tp::Gf2Mat128) == tpk::XO128_MAT_WORDS * sizeof(uint32_t), "matrix layout");
 static_assert(sizeof(tp::Gf2Mat) == tpk::XO_MAT_WORDS * sizeof(uint64_t), "matrix layout");
 static __device__ __align__(256) uint64_t scratch[NS_WORDS];

@@ -121,7 +121,9 @@ constexpr int XO_NRUNS = sizeof XO_RUNS / sizeof XO_RUNS[0];
 // faster-evgen, 12 * XO_EXPAND_RUN draws each.
 constexpr uint32_t XO_EXPAND_RUN = 32;
 constexpr int XO_NTABLES = XO_NRUNS + 1;
-constexpr int XO_M_DIGITS = 12, XO_B_DIGITS = 8;         // exponents below 2^48 draws, 2^32 batches
+// Exponents below 2^52 draws and 2^32 batches: no run is longer, as the
+// accumulators of 2.8e9 batches fill 288 GB (faster-evgen: 4.7e14 draws).
+constexpr int XO_M_DIGITS = 13, XO_B_DIGITS = 8;
 constexpr size_t XO_MAT_WORDS = 1024;                    // 256 columns of 4 words
 constexpr size_t XO_LANE_WORDS = 64 * 16 * 64 * 4;       // per run length: 2 MiB
 // tab16[(15 j + v - 1) * 1024 ..] = B^(v 16^j) from pow2[k * 1024 ..] = B^(2^k), k < 4 digits.
