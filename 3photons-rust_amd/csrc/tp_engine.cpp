@@ -241,14 +241,18 @@ int check_common(Ctx *c, const tp_params *params, int rng_kind, const void *stat
 // RANF with `faster-evgen`: the event starts of the reference's
 // simulate_event_batch walk, then each chunk of batches is simulated from
 // them with its stream expanded into HBM.  Runs of FE_DEVICE_WALK_MIN events
-// (xoshiro streams: FE_XO_DEVICE_WALK_MIN) or more walk the stream on the device (fe_walk_kernel: segment walkers
-// joined where they meet); shorter runs, and any chunk whose device walkers
-// do not all join, take the host walk, 20 to 90 ns an event.  The device's takes
-// its launches and a segment's length at least.  Closures of 2000, 8000, 32 000
-// and 300 000 events on the host and on the device: RANF 120, 190, 706, 5900 us
-// and 175, 175, 178, 221; xoshiro256+ 153, 363, 1149, 9880 us and about 800 (a
-// segment has 1024 events there).
-constexpr uint64_t FE_DEVICE_WALK_MIN = 8192, FE_XO_DEVICE_WALK_MIN = 16384;
+// or more, by the kind of stream (FeStream), walk it on the device
+// (fe_walk_kernel: segment walkers joined where they meet); shorter runs, and
+// any chunk whose device walkers do not all join, take the host walk, 15 to 90
+// ns an event.  The device's takes its launches and a segment's length at least,
+// 1024 events on the xoshiro streams.  Closures on the host and on the device:
+// RANF of 2000, 8000, 32 000 and 300 000 events 120, 190, 706, 5900 us and 175,
+// 175, 178, 221; xoshiro256+ of 8000, 12 000 and 16 383 events 306, 420, 544 us,
+// of 16 384 and 32 000 608 and 630, which meet near 19 000 (host and device of
+// another machine near 21 000); xoshiro128+, whose values the host rounds one by
+// one, 753, 1105, 1488 us, and on the device 683 of 12 000 events and 881 of
+// 32 000, which meet below 8000.
+constexpr uint64_t FE_DEVICE_WALK_MIN[4] = {8192, 8192, 20000, 8192};
 // From RANF states past the modulus only the device walk serves: it reads the
 // bits of the very values that its events replay, while the host walk's rounds
 // differ from the kernels' there, and an event replayed from the other's start
@@ -516,7 +520,7 @@ using FeHostWalk = std::function<void(uint64_t q, uint64_t n, uint64_t *starts, 
 int enqueue_fe_chunks(Ctx *c, const FeStream &fs, const FeHostWalk &host_walk, tpk::FusedArgs &a, tpk::F32Args *fa,
                       uint64_t q_start, uint64_t num_events, uint32_t batch_size, void *per_batch_dev, uint64_t *q_end)
 {
-    const bool device_walk = num_events >= (fs.kind < 2 ? FE_DEVICE_WALK_MIN : FE_XO_DEVICE_WALK_MIN);
+    const bool device_walk = num_events >= FE_DEVICE_WALK_MIN[fs.kind];
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     c->fe_host_chunks = 0;

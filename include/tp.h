@@ -128,7 +128,7 @@ typedef struct {
     uint64_t batches;
     uint64_t host_walk_chunks; /* faster-evgen with skip-ahead seeding: chunks of batches whose event
                                   starts came from the host walk (runs and calls below 8192 events,
-                                  16384 on xoshiro streams, or device walkers that did not all meet) */
+                                  20000 on xoshiro256+ streams, or device walkers that did not all meet) */
     uint64_t chunks;           /* faster-evgen: chunks of batches the run was split into (each one's
                                   stream expanded, walked and simulated in turn); 0 otherwise */
 } tp_stats;
