@@ -715,11 +715,9 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
                                    uint64_t num_events, uint32_t batch_size, void *per_batch_dev)
 {
     const bool f32 = params->precision == TP_PREC_F32;
-    if (batch_size > 10u * TP_BATCH_SIZE)
-        return fail(c, TP_ERR_ARG, "faster-evgen with jump seeding runs batches of at most 100 000 events");
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
-    const uint64_t PS = FE_JUMP_PIECE * ((batch_size + TP_BATCH_SIZE - 1) / TP_BATCH_SIZE);
+    const uint64_t PS = FE_JUMP_PIECE;
     const uint64_t max_rounds = PS / 55 + 2, R = ranf_seg_rounds(c, chunk * max_rounds);
     int rc = ensure_r16(c);
     if (!rc)
@@ -866,8 +864,6 @@ int enqueue_ranf_faster_evgen_jump(Ctx *c, const tp_params *params, tpk::FusedAr
 int enqueue_xo_faster_evgen_jump(Ctx *c, tpk::FusedArgs &a, const tp_xoshiro_state *x, uint64_t num_events,
                                  uint32_t batch_size, void *per_batch_dev)
 {
-    if (batch_size > TP_BATCH_SIZE)
-        return fail(c, TP_ERR_ARG, "faster-evgen with jump seeding runs batches of at most 10 000 events");
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     int rc = ensure(c, c->xo_draws, chunk * FE_XO_PIECE * sizeof(double));
@@ -967,8 +963,6 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
         c->fe_xo_end = q_end;
         return TP_OK;
     }
-    if (batch_size > TP_BATCH_SIZE)
-        return fail(c, TP_ERR_ARG, "faster-evgen with jump seeding runs batches of at most 10 000 events");
     const uint64_t nb = (num_events + batch_size - 1) / batch_size;
     const uint64_t chunk = std::min<uint64_t>(nb, FE_WALK_BATCHES);
     int rc = ensure(c, c->evq, chunk * batch_size * sizeof(uint64_t));
@@ -1057,11 +1051,10 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     a.num_events = num_events;
     a.batch_size = batch_size;
     a.precision = params->precision;
-    int rc = ensure_mt(c);
-    if (rc)
-        return rc;
-    a.mt = static_cast<const uint64_t *>(c->mt.p);
-    a.km = c->km;
+    // (faster-evgen's pieces of a batch's stream hold whole batches; closures
+    // have one stream)
+    if (params->faster_evgen && seeding == TP_SEED_JUMP && batch_size != TP_BATCH_SIZE)
+        return fail(c, TP_ERR_INTERNAL, "faster-evgen with jump seeding runs batches of 10 000 events");
     if (rng_kind == TP_RNG_XOSHIRO128 && params->faster_evgen)
         return enqueue_xo128_faster_evgen(c, params, seeding, static_cast<const tp_xoshiro128_state *>(state0),
                                           num_events, batch_size, per_batch_dev);
@@ -1087,9 +1080,8 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
     if (rng_kind == TP_RNG_XOSHIRO) {
         const tp_xoshiro_state *x = static_cast<const tp_xoshiro_state *>(state0);
         std::memcpy(a.s0, x->s, sizeof a.s0);
-        rc = xo_event_args(c, a, seeding, nb);
-        if (rc)
-            return rc;
+        if (const int e = xo_event_args(c, a, seeding, nb))
+            return e;
         a.out = per_batch_dev;
         if (const int e = mark(c, 1))
             return e;
@@ -1109,7 +1101,7 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
             fa.source = 2;
         return enqueue_ranf_faster_evgen(c, a, f32 ? &fa : nullptr, rs, num_events, batch_size, per_batch_dev);
     }
-    rc = ensure_r16(c);
+    int rc = ensure_r16(c);
     if (rc)
         return rc;
     // the event loop makes its draws itself
