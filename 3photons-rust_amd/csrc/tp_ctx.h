@@ -39,10 +39,8 @@ template <int N> struct ScopedBufs {
 };
 
 // xoshiro skip tables of one device, filled once by the first tp_create on
-// it and only read afterwards (tp_kernels.h).
+// it (the next caller, if that fails) and only read afterwards (tp_kernels.h).
 struct XoTables {
-    int rc = TP_ERR_INTERNAL;
-    std::string err;
     const uint64_t *m16 = nullptr;     // M^(v 16^j), M one draw
     const uint64_t *b16[2] = {nullptr, nullptr}; // B^(v 16^j): M^(12 * 10 000), the 2^128 jump (by seeding)
     const uint64_t *lanes = nullptr;   // lane tables of every run length, then of the pieces of a stream
@@ -51,7 +49,7 @@ struct XoTables {
 
 struct Ctx {
     int device = 0;
-    const XoTables *xo = nullptr;
+    const XoTables *xo = nullptr;   // null where their set-up has failed so far
     int cus = 1;                    // compute units of the device
     int blocks_per_cu[5][2] = {{1, 1}, {1, 1}, {1, 1}, {1, 1}, {1, 1}}; // resident fused workgroups per CU [source][precision]
     int f32_blocks[4] = {1, 1, 1, 1}; // resident all-f32 wavefronts per CU [source]

@@ -19,6 +19,7 @@
 #include "tp_kernels.h"
 #include "tp_rng_host.h"
 #include "tp_ctx.h"
+#include "tp_once.h"
 
 namespace tpe {
 tpd::Params make_params(const tp_params *p)
@@ -134,13 +135,9 @@ constexpr uint64_t F32_CHUNK_BATCHES = 24576;
 // bytes each with jump seeding, 239 from a state past the modulus: 470 MB.
 constexpr uint64_t RANF_CHUNK_BATCHES = 1u << 20;
 
-int xo_tables(Ctx *c)
-{
-    if (!c->xo || c->xo->rc != TP_OK)
-        return fail(c, c->xo ? c->xo->rc : TP_ERR_UNSUPPORTED,
-                    "xoshiro table set-up failed: " + (c->xo ? c->xo->err : std::string("device ordinal above 63")));
-    return TP_OK;
-}
+// The context's xoshiro tables; with `make`, they are set up (again) where that
+// has not been done.
+int xo_tables(Ctx *c, bool make = true);
 
 // All-f32 run with the xoshiro128+ stream.
 int enqueue_xo128_f32(Ctx *c, const tp_params *params, int seeding, const tp_xoshiro128_state *x,
@@ -1028,9 +1025,9 @@ int enqueue_xo128_faster_evgen(Ctx *c, const tp_params *params, int seeding, con
 // The stream tables and batch range of a xoshiro256+ run of nb batches.  (The
 // powers of B are those of batches of 10 000 events; a closure call of another
 // size is one batch and uses none.)
-int xo_event_args(Ctx *c, tpk::FusedArgs &a, int seeding, uint64_t nb)
+int xo_event_args(Ctx *c, tpk::FusedArgs &a, int seeding, uint64_t nb, bool make = true)
 {
-    const int rc = xo_tables(c);
+    const int rc = xo_tables(c, make);
     if (rc)
         return rc;
     a.m16 = c->xo->m16;
@@ -1203,25 +1200,24 @@ static __device__ __align__(256) uint64_t scratch[NS_WORDS];
 namespace {
 constexpr int NS_MAX_DEVICES = 64;
 struct XoSetup {
-    std::once_flag once;
+    OnceDone once;
     XoTables t;
 };
 XoSetup g_xo[NS_MAX_DEVICES];
 
-// Once per device, with the device current: the array's address and its
-// tables, from the powers of two of the three matrices.
-void xo_setup(XoTables &T, hipStream_t st)
+// With the device current: the array's address and its tables, from the powers
+// of two of the three matrices.
+bool xo_setup(XoTables &T, hipStream_t st, std::string &err)
 {
     void *ptr = nullptr, *pow2 = nullptr;
+    err.clear();
     auto check = [&](hipError_t e, const char *what) {
-        if (e != hipSuccess && T.err.empty()) {
-            T.err = std::string(what) + ": " + hipGetErrorString(e);
-            T.rc = TP_ERR_HIP;
-        }
+        if (e != hipSuccess && err.empty())
+            err = std::string(what) + ": " + hipGetErrorString(e);
         return e == hipSuccess;
     };
     if (!check(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)"))
-        return;
+        return false;
     const std::vector<tp::Gf2Mat> &mt = tp::xoshiro_step_pow2();
     const int digits[3] = {tpk::XO_M_DIGITS, tpk::XO_B_DIGITS, tpk::XO_B_DIGITS};
     std::vector<tp::Gf2Mat> mats(mt.begin(), mt.begin() + 4 * digits[0]);
@@ -1274,7 +1270,7 @@ void xo_setup(XoTables &T, hipStream_t st)
     if (pow2)
         (void)hipFree(pow2);
     if (!ok)
-        return;
+        return false;
     T.m16 = t + NS_M;
     T.b16[TP_SEED_SKIPAHEAD] = t + NS_B;
     T.b16[TP_SEED_JUMP] = t + NS_B + 15 * tpk::XO_B_DIGITS * tpk::XO_MAT_WORDS;
@@ -1283,7 +1279,21 @@ void xo_setup(XoTables &T, hipStream_t st)
     T.b16_128[TP_SEED_SKIPAHEAD] = t128 + NS128_B;
     T.b16_128[TP_SEED_JUMP] = t128 + NS128_B + 15 * tpk::XO_B_DIGITS * tpk::XO128_MAT_WORDS;
     T.lanes128 = t128 + NS128_LANES;
-    T.rc = TP_OK;
+    return true;
+}
+
+int xo_tables(Ctx *c, bool make)
+{
+    if (c->xo)
+        return TP_OK;
+    if (c->device >= NS_MAX_DEVICES)
+        return fail(c, TP_ERR_UNSUPPORTED, "xoshiro table set-up failed: device ordinal above 63");
+    XoSetup &S = g_xo[c->device];
+    std::string err = "not made in this process";
+    if (!(make ? S.once.run([&] { return xo_setup(S.t, c->stream, err); }) : S.once.done()))
+        return fail(c, TP_ERR_HIP, "xoshiro table set-up failed: " + err);
+    c->xo = &S.t;
+    return TP_OK;
 }
 } // namespace
 
@@ -1319,10 +1329,7 @@ extern "C" int tp_create(int device, void **ctx_out)
                 c->blocks_per_cu[src][prec] = tpk::fused_blocks_per_cu(src, prec);
         for (int src = 0; src < 4; ++src)
             c->f32_blocks[src] = tpk::f32_blocks_per_cu(src);
-        if (device < NS_MAX_DEVICES) { // xoshiro tables (device current)
-            std::call_once(g_xo[device].once, [&] { xo_setup(g_xo[device].t, c->stream); });
-            c->xo = &g_xo[device].t;
-        }
+        (void)xo_tables(c); // (device current; a call that needs them reports what failed)
         int rc = ensure(c, c->parts, MAX_PARTS * sizeof(tp_acc));
         if (!rc && hipHostMalloc(reinterpret_cast<void **>(&c->host_acc), HOST_ACCS * sizeof(tp_acc), hipHostMallocMapped | hipHostMallocCoherent) !=
                        hipSuccess) {
@@ -1809,7 +1816,7 @@ extern "C" int tp_run_device_noalloc(void *ctx, const tp_params *params, int rng
         a.batch_size = TP_BATCH_SIZE;
         a.precision = params->precision;
         std::memcpy(a.s0, static_cast<const tp_xoshiro_state *>(rng_state0)->s, sizeof a.s0);
-        rc = xo_event_args(c, a, seeding, nb);
+        rc = xo_event_args(c, a, seeding, nb, false);
         if (rc)
             return rc;
         a.out = per_batch_dev;
