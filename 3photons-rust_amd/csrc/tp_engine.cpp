@@ -272,7 +272,7 @@ constexpr uint64_t FE_SEG = 24 * 55, FE_OVERLAP = 24 * 55;
 // simulated 1.5e9-draw stream, 12 of them past 512).  On one stream its
 // walkers, which have to meet the next one within its segment, therefore take
 // 1024 events each; a batch's own stream is walked by chains of walkers that
-// may leave some out, 256 events each, going up to 1024 events (17 500
+// may leave some out, 1024 events each too, going up to 1024 events (17 500
 // positions) past their segment; 16.64 positions per event on average, 17.0
 // allowed for.
 constexpr double FE_XO_POSITIONS_PER_EVENT = 17.0;
@@ -1148,7 +1148,7 @@ int enqueue_run(Ctx *c, const tp_params *params, int rng_kind, int seeding, cons
                 return e;
         if (f32) {
             // (a launch whose batches are split has at most MAX_PARTS of them:
-            // its per-event values stay below 13.2 GB)
+            // its per-event values stay below 6.6 GB)
             fa.nb = cnb;
             fa.b_first = b0;
             fa.out = static_cast<tp_acc *>(per_batch_dev) + b0;

@@ -268,10 +268,11 @@ __device__ __forceinline__ double sigmoid_u(float z)
 
 // ---- forward ----------------------------------------------------------------
 // The forward and inverse kernels load the forward weights of all L layers
-// into LDS once (97.5 KB, one block per CU) and then stride over the samples
+// into LDS once (99.75 KiB, one block per CU) and then stride over the samples
 // with no further barrier: a block takes waves x tiles x 16 samples per pass.
-// Bound by VALU issue (some 120 instructions per tile, layer and wavefront next
-// to 16 matrix instructions) where the wavefronts cover each other's latencies,
+// Bound by VALU issue (204 instructions per tile and layer, draws and densities
+// among them, next to 16 matrix instructions: 79 % of the issue slots at 4 cycles
+// each) where the wavefronts cover each other's latencies,
 // so three wavefronts per SIMD with two tiles each take the long runs and four
 // with one tile the batches that would leave CUs idle otherwise.  1.4e7 samples
 // drawn and 6e6 inverted, with the weighted event loop: 4.05 ms; 4.11 at two

@@ -16,9 +16,11 @@
 //  ranf_seed         jump-mode origins, seeded_new(seed + 123456 b) per batch.
 //  merge_kernel      in-order left fold of the batch accumulators.
 //
-// Compiled with -ffp-contract=off: the f64 path keeps the reference's
-// operation order (HadrienG2/3photons-rust src/evgen.rs, evcut.rs, spinor.rs,
-// matelems.rs, resacc.rs).
+// Compiled with -ffp-contract=off: nothing is fused but what the code writes as
+// fma.  The f64 path keeps the reference's operation order through RAMBO and the
+// sort (HadrienG2/3photons-rust src/evgen.rs); its cuts' products are fused, its
+// helicity sums closed forms (evcut.rs, spinor.rs, matelems.rs), its sums taken
+// per lane and part (resacc.rs).  The all-f32 path keeps the order throughout.
 #include "tp_kernels.h"
 #include "tp_xoshiro.h"
 

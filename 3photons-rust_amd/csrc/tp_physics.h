@@ -6,9 +6,10 @@
 // L1-resident log and sin/cos tables of tp_math.h, whose routines return the
 // correctly rounded value but within ~0.002 ulp of a rounding boundary (the
 // reference calls the host libm; the two agree on > 99.8 % of arguments).  The
-// f64 path keeps the reference's operation order through RAMBO, the sort and
-// the cuts (the translation unit is compiled with -ffp-contract=off) and takes
-// its helicity sums in closed form (tp_helicity.h); the all-f32 path keeps the
+// f64 path keeps the reference's operation order through RAMBO and the sort
+// (the translation unit is compiled with -ffp-contract=off), fuses the cuts'
+// products (keep_f64) and takes its helicity sums in closed form
+// (tp_helicity.h); the all-f32 path keeps the
 // reference's order throughout, apart from known zeros and exact negations:
 //   * s(j,i) is taken as -s(i,j) (exactly equal but for the sign of a zero);
 //   * the helicity sums skip the zero amplitudes (adding +-0 to a non-zero sum

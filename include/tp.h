@@ -59,7 +59,11 @@ typedef enum { TP_RNG_RANF = 0, TP_RNG_XOSHIRO = 1, TP_RNG_XOSHIRO128 = 2 } tp_r
 typedef enum { TP_SEED_SKIPAHEAD = 0, TP_SEED_JUMP = 1 } tp_seeding;
 
 /* Arithmetic of the per-event path.
- *   TP_PREC_F64   -- IEEE double, no contraction, reference operation order.
+ *   TP_PREC_F64   -- IEEE double: RAMBO and the sort in the reference's operation
+ *                    order, the cuts' products fused (a decision can differ from
+ *                    the reference's, and from tp_adjoint's unfused cuts, where
+ *                    the compared values lie within an ulp or so: about one event
+ *                    in 1e15), the helicity sums in closed form.
  *   TP_PREC_MIXED -- f64 RAMBO, cuts and weight; f32 spinor products and
  *                    helicity amplitudes; Kahan-compensated f64 batch sums.
  *   TP_PREC_F32   -- the reference's `f32` feature (numeric.rs:6-14):
@@ -147,7 +151,14 @@ int tp_rng_seed(int rng_kind, uint64_t seed, void *state);
 
 /* RandomGenerator::skip (ranf.rs:122-127, standard.rs:37-43): advance the
  * state as n calls of random() would, in O(log n) (polynomial / GF(2)
- * skip-ahead instead of stepping). */
+ * skip-ahead instead of stepping).  RANF states with values outside [0, 1e9),
+ * which seeds of 1e9 and more can leave (faster-threading reaches them at batch
+ * 6200 from the default seed), are an exception: the recurrence holds modulo 1e9,
+ * but the reference's rounds go on with the values as they are, so stepping and
+ * the polynomial part ways there.  A skip of such a state is one polynomial jump
+ * (not what stepping gives in most of them), and every run, closure and
+ * tp_events call draws from it by one rule of its own: rounds from the state up
+ * to round 2048, and each later stretch of 2048 rounds from a jump. */
 int tp_rng_skip(int rng_kind, void *state, uint64_t n);
 /* RandomGenerator::jump (ranf.rs:135-140 reseed with seed+123456,
  * standard.rs:51-55 the 2^128 jump). */
@@ -185,7 +196,7 @@ int tp_run_device(void *ctx, const tp_params *params, int rng_kind, int seeding,
  * runs the xoshiro256+ stream only (rng_kind TP_RNG_XOSHIRO, precision
  * TP_PREC_F64 or TP_PREC_MIXED, both seedings, no faster-evgen; anything else
  * returns TP_ERR_UNSUPPORTED) and at most 2^32 - 1 batches (TP_ERR_ARG
- * beyond).  Its skip-ahead tables sit in a static device array of 33 MiB
+ * beyond).  Its skip-ahead tables sit in a static device array of 31.7 MiB
  * per GPU, filled once by tp_create and only read afterwards, so calls that
  * overlap on one GPU share it without racing; the sums of batches split over
  * several wavefronts go through 6.5 MiB of the context's own, also allocated
